@@ -1,0 +1,114 @@
+"""The whole-sweep LSTM kernel that keeps its weights in registers (zr_lstm_resident.hip), against the oracle: hidden
+sizes around the edges of its row tiles, k-groups and register classes, batches around the edges of its column tiles,
+more layers than fit in one launch, initial states, padding, cell clipping, kept gates, and giving up a wait."""
+import numpy as np
+import pytest
+
+import oracle_lib as o
+from gpu_util import Layer, assert_close
+from zoph_rnn_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+def _case(H, mb, T, L, V=211, seed=41):
+    g = synth.rng(seed, H + 31 * mb + L)
+    ids = g.integers(0, V, size=(T, mb)).astype(np.int32)
+    if mb > 1:
+        ids[: T // 2, 1] = -1
+    ids[T - 1, mb - 1] = -1
+    return dict(H=H, mb=mb, T=T, L=L, V=V, ids=ids, embed=synth.uniform(g, (H, V), -0.5, 0.5),
+                layers=[synth.lstm_layer(g, H, forget_bias_one=True) for _ in range(L)],
+                h0=[np.tanh(synth.uniform(g, (H, mb), -1, 1)) for _ in range(L)],
+                c0=[synth.uniform(g, (H, mb), -0.5, 0.5) for _ in range(L)])
+
+
+def _run(ctx, c, clip=0.9, times=1):
+    """h, c and gates of every node, [L][T](, 4), H x mb."""
+    H, mb, T, L, V, ids = c["H"], c["mb"], c["T"], c["L"], c["V"], c["ids"]
+    layers = [Layer(ctx, ly) for ly in c["layers"]]
+    d_nn, d_m = ctx.empty(ids.size, np.int32), ctx.empty(ids.size, np.int32)
+    ctx.vocab_prep(ctx.array(ids.reshape(-1)), ids.size, V, d_nn, d_m)
+    d_embed = ctx.array(c["embed"])
+    d_h0, d_c0 = [ctx.array(a) for a in c["h0"]], [ctx.array(a) for a in c["c0"]]
+    n = H * mb
+    h, x = [ctx.empty((n * T,)) for _ in range(L)], [ctx.empty((n * T,)) for _ in range(L)]
+    g = [ctx.empty((4 * n * T,)) for _ in range(L)]
+    try:
+        for _ in range(times):
+            ctx.lstm_stack_forward_train([ly.w for ly in layers], d_embed, V, d_nn, d_m, T, mb, d_h0, d_c0, h, x, g, clip=clip)
+        path = ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH)
+        abandoned = ctx.query(capi.ZR_QUERY_LSTM_SWEEP_ABANDONED)
+    finally:
+        for ly in layers:
+            ly.close()
+    shape = lambda a, k: a.get().reshape(T, *k, mb, H).swapaxes(-1, -2)  # noqa: E731
+    return np.stack([shape(a, ()) for a in h]), np.stack([shape(a, ()) for a in x]), np.stack([shape(a, (4,)) for a in g]), path, abandoned
+
+
+def _want(c, clip=0.9):
+    nn, m = o.vocab_prep(c["ids"])
+    return o.lstm_stack_forward(c["embed"], c["layers"], nn, m, h0=c["h0"], c0=c["c0"], clip=clip)
+
+
+# H: one row tile, a row tail of every kind (H % 8 = 1, 4, 7), the last and first size of each register class;
+# mb: 1, the last and first of 16 and 32 columns, several column tiles; L: one, several, more than fit at once
+@pytest.mark.parametrize("H,mb,T,L", [(8, 1, 1, 1), (9, 16, 4, 2), (15, 17, 3, 3), (100, 8, 6, 1), (127, 33, 4, 2),
+                                      (129, 5, 3, 8), (255, 32, 3, 2), (257, 31, 3, 1), (300, 20, 5, 2), (500, 37, 4, 2),
+                                      (508, 64, 3, 4), (516, 16, 3, 1), (1000, 12, 3, 4), (1001, 1, 3, 2), (1024, 16, 3, 3)])
+def test_sweep_with_weights_in_registers(ctx, H, mb, T, L):
+    c = _case(H, mb, T, L)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    try:
+        h, x, g, path, abandoned = _run(ctx, c)
+        h2, x2, g2, _, _ = _run(ctx, c, times=3)  # flags of one launch must not reach the next
+    finally:
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
+    assert path == capi.ZR_LSTM_STACK_PATH_SWEEP and not abandoned
+    assert h.tobytes() == h2.tobytes() and x.tobytes() == x2.tobytes() and g.tobytes() == g2.tobytes()
+    want_h, want_c = _want(c)
+    assert_close(h, want_h, what="h")
+    assert_close(x, want_c, what="c")
+    # the kept gates reproduce the states: c = clip(f c_prev + i c~), h = o tanh(c), 0 where masked
+    m = (c["ids"] >= 0).astype(np.float32)[None, :, None, :]
+    c_prev = np.concatenate([np.stack(c["c0"])[:, None], want_c[:, :-1]], axis=1)
+    cell = np.clip(g[:, :, 1] * c_prev + g[:, :, 0] * g[:, :, 2], -0.9, 0.9)
+    assert_close(m * cell, want_c, what="c from the gates")
+    assert_close(m * g[:, :, 3] * np.tanh(cell), want_h, what="h from the gates")
+
+
+def test_library_picks_it_for_a_small_model(ctx):
+    c = _case(100, 8, 5, 2)
+    h, x, _, path, _ = _run(ctx, c)
+    assert path == capi.ZR_LSTM_STACK_PATH_SWEEP
+    want_h, want_c = _want(c)
+    assert_close(h, want_h, what="h")
+    assert_close(x, want_c, what="c")
+
+
+def test_abandoned_wait_is_reported_and_leaves_nan(ctx):
+    """H = 100 has no other single-launch schedule: with one poll per wait the upper layer gives up, every workgroup
+    leaves, the outputs are NaN, and the next sweep with the default limit is complete again."""
+    c = _case(100, 24, 6, 3)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 1)
+    try:
+        h, x, g, path, abandoned = _run(ctx, c)
+        assert path == capi.ZR_LSTM_STACK_PATH_SWEEP and abandoned == 1
+        assert np.all(np.isnan(h)) and np.all(np.isnan(x)) and np.all(np.isnan(g))
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)
+        h, x, g, path, abandoned = _run(ctx, c)
+        assert path == capi.ZR_LSTM_STACK_PATH_SWEEP and abandoned == 0
+    finally:
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)
+    want_h, want_c = _want(c)
+    assert_close(h, want_h, what="h")
+    assert_close(x, want_c, what="c")

@@ -8,6 +8,7 @@
 #include "../../include/zoph_rnn.h"
 
 #define ZR_MAX_COUNTERS 4096
+#define ZR_MAX_STEP_FLAGS 16384
 #define ZR_MAX_PACKED_D 8
 
 struct zr_ctx {
@@ -24,12 +25,14 @@ struct zr_ctx {
   int lstm_kernel;   // 0 auto, 1 register-streaming kernel, 2 LDS / split-K kernel
   int lstm_kparts;   // K parts per segment for the split-K kernel (0 auto)
   int* d_counters;   // ZR_MAX_COUNTERS arrival counters, zero between launches
+  int* d_step_flags; // ZR_MAX_STEP_FLAGS flags of lstm_resident_kernel (the first 32 hold its departure count), zero between launches
   int lstm_sweep;    // whole-sweep LSTM kernel: 0 auto, 1 never, 2 whenever the launch fits on the device
   int sweep_spin;    // polls before a waiting workgroup of that kernel gives up (0: default)
   int step_wait_extra;  // arrivals the decoder step's layer waits expect beyond the real ones (tests of giving up)
   int stack_helpers;    // 1 (default): the decoder step may run 32-column tiles with helper workgroups (zr_lstm.hip)
   int cu_count;      // compute units of the device (filled with sweep_capacity)
   int sweep_capacity[3];  // resident workgroups of lstm_sweep_kernel<TN> (0: not asked yet, -1: unknown)
+  int resident_capacity[4][3];  // the same for lstm_resident_kernel, by size class and column class
   int stack_step_capacity;  // the same for lstm_decoder_stack_kernel (the lesser of its two tile widths)
   int attn_step_capacity[3];  // the same for attn_step_kernel<8 / 16 / 32>
   int attn_single;      // ZR_OPT_ATTN_SINGLE_LAUNCH
@@ -206,6 +209,18 @@ int zr_lstm_decoder_step_packed(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
 int zr_softmax_forward_packed(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, int H, const float* d_h,
                               const float* d_h_packed, int mb, int mode, float* d_out, float* d_logits_scratch,
                               const unsigned short* d_h_hi = nullptr, const unsigned short* d_h_lo = nullptr);
+
+// The whole sweep with the weights held in registers (zr_lstm_resident.hip), as one launch or, when not all layers fit on
+// the device at once, a few.  The plan: which kernel, how many layers a launch; its value is the estimated time in us
+// (negative: the shape does not fit).  The caller poisons the outputs of an abandoned sweep (lstm_sweep_poison_kernel).
+struct ZrResidentPlan {
+  int size_class, col_class, n_tiles, at_once, flag_stride;
+};
+double zr_lstm_resident_plan(zr_ctx* ctx, int nl, int H, int mb, int T, ZrResidentPlan* plan);
+int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, const zr_lstm_weights* const layers[],
+                           const float* d_embed, int V, const int* d_ids_nonneg, const int* d_mask01, int T, int mb,
+                           const float* const d_h0[], const float* const d_c0[], float clip_threshold,
+                           float* const d_h_all[], float* const d_c_all[], float* const d_gates_all[]);
 
 // The attention step in one launch (zr_attn_step.hip).  a->d_hpack must hold h_t k-interleaved.  *took = 0: the
 // conditions do not hold and nothing was launched (the caller goes on with one launch per stage).

@@ -1352,21 +1352,28 @@ __global__ void __launch_bounds__(256) lstm_sweep_poison_kernel(SweepPoison P) {
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < P.count[a]; i += stride) P.out[a][i] = nan;
 }
 
+int poison_if_abandoned(zr_ctx* ctx, int nl, int T, int H, int mb, float* const d_h_all[], float* const d_c_all[],
+                        float* const d_gates_all[]) {
+  SweepPoison Q = {};
+  const long long per = (long long)T * H * mb;
+  for (int l = 0; l < nl; ++l) {
+    Q.out[Q.n_out] = d_h_all[l], Q.count[Q.n_out++] = per;
+    Q.out[Q.n_out] = d_c_all[l], Q.count[Q.n_out++] = per;
+    if (d_gates_all && d_gates_all[l]) Q.out[Q.n_out] = d_gates_all[l], Q.count[Q.n_out++] = 4 * per;
+  }
+  Q.status = ctx->d_flags + 2;
+  // (as many workgroups as a rarely needed fill of the outputs can use, and no more: all of them start every time)
+  const long long blocks = (per + 4095) / 4096;
+  lstm_sweep_poison_kernel<<<(unsigned)(blocks < 512 ? blocks : 512), 256, 0, ctx->stream>>>(Q);
+  ZR_LAUNCH_CHECK("lstm_sweep_poison_kernel");
+  return ZR_OK;
+}
+
 template <int TN>
 int launch_sweep_v(zr_ctx* ctx, LstmSweep& P, int grid) {
   lstm_sweep_kernel<TN><<<grid, 256, 0, ctx->stream>>>(P);
   ZR_LAUNCH_CHECK("lstm_sweep_kernel");
-  SweepPoison Q = {};
-  const long long per = (long long)P.T * P.H * P.mb;
-  for (int l = 0; l < P.nl; ++l) {
-    Q.out[Q.n_out] = P.h_all[l], Q.count[Q.n_out++] = per;
-    Q.out[Q.n_out] = P.c_all[l], Q.count[Q.n_out++] = per;
-    if (P.gates_all[l]) Q.out[Q.n_out] = P.gates_all[l], Q.count[Q.n_out++] = 4 * per;
-  }
-  Q.status = P.status;
-  lstm_sweep_poison_kernel<<<512, 256, 0, ctx->stream>>>(Q);
-  ZR_LAUNCH_CHECK("lstm_sweep_poison_kernel");
-  return ZR_OK;
+  return poison_if_abandoned(ctx, P.nl, P.T, P.H, P.mb, P.h_all, P.c_all, P.gates_all);
 }
 
 // Resident workgroups of lstm_decoder_stack_kernel (either tile width) the device can hold at once (0: unknown /
@@ -1812,68 +1819,97 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
     vec = vec && aligned16(d_h0[l]) && aligned16(d_h_all[l]);
   }
   const size_t n = (size_t)H * mb;
-  // One launch for the whole sweep when its workgroups -- one tile of one layer each, kept for all T steps -- fill
-  // most of the chip and fit on it together; otherwise one launch per diagonal.
-  if (vec && H % 8 == 0 && !layers[0]->bf16 && ctx->lstm_fused && ctx->lstm_sweep != 1 && nl <= kMaxUnits) {
-    const int j_tiles = (H + 31) / 32, n32 = (mb + 31) / 32;
-    const int groups = nl * j_tiles;
-    const int padded = (groups + 7) / 8 * 8;
-    int tn = 0;
+  // Left to itself the library takes a single-launch schedule only when this is the only context on the device: two such
+  // launches from two streams could each hold part of the CUs and wait for the rest (their bounded waits would end it,
+  // with an error).  Nor on a caller-provided stream: the caller's other streams may hold compute units for as long as
+  // they like.
+  const bool alone = zr_live_contexts(ctx->device) == 1 && ctx->stream == ctx->own_stream;
+  const bool single_ok = !layers[0]->bf16 && ctx->lstm_fused && (ctx->lstm_sweep == 2 || (ctx->lstm_sweep == 0 && alone));
+  // Whole-sweep kernel with streamed weights: when its workgroups -- one tile of one layer each, kept for all T steps --
+  // fill most of the chip and fit on it together.
+  const int j_tiles = (H + 31) / 32, n32 = (mb + 31) / 32;
+  const int groups = nl * j_tiles;
+  const int padded = (groups + 7) / 8 * 8;
+  int tn = 0;
+  if (single_ok && vec && H % 8 == 0 && nl <= kMaxUnits) {
     if ((long long)padded * n32 <= sweep_capacity<1>(ctx)) tn = 1;
     else if ((long long)padded * ((n32 + 1) / 2) <= sweep_capacity<2>(ctx)) tn = 2;
-    const int n_tiles = tn ? (n32 + tn - 1) / tn : 0;
-    const long long tiles = (long long)groups * n_tiles;
-    // Left to itself the library takes the single launch only when it fills most of the chip and this is the only
-    // context on the device: two such launches from two streams could each hold part of the CUs and wait for the
-    // rest (their bounded waits would end it, with an error).
-    // Nor on a caller-provided stream: the caller's other streams may hold compute units for as long as they like.
-    const bool fills = tn && tiles * 10 >= 6LL * ctx->cu_count && zr_live_contexts(ctx->device) == 1 &&
-                       ctx->stream == ctx->own_stream;
     // the kernel addresses its operands as descriptor base + 32-bit byte offsets
     const long long lim = 1LL << 32;
     const bool offsets_fit = (long long)V * H * 4 < lim && (long long)n * 4 < lim &&
                              8LL * layers[0]->kp * layers[0]->ldw * 4 < lim;
-    if (tn && offsets_fit && (fills || ctx->lstm_sweep == 2) && nl * n_tiles <= 512 &&
-        (long long)T * j_tiles < kSweepGaveUp) {
-      LstmSweep P = {};
-      const size_t ctr_bytes = sizeof(int) * 512 * kSweepCtrStride;
-      void* p = nullptr;
-      rc = zr_ctx_scratch(ctx, 1, ctr_bytes + sizeof(float) * (size_t)nl * T * n, &p);
-      if (rc) return rc;
-      P.counters = (int*)p;
-      P.hp = (float*)((char*)p + ctr_bytes);
-      rc = zr_memset_zero(ctx, P.counters, sizeof(int) * (size_t)nl * n_tiles * kSweepCtrStride);
-      if (rc) return rc;
-      for (int l = 0; l < nl; ++l) {
-        P.W[l] = (const float*)layers[l]->d_W;
-        P.bias[l] = layers[l]->d_bias;
-        P.h0[l] = d_h0[l];
-        P.c0[l] = d_c0[l];
-        P.h_all[l] = d_h_all[l];
-        P.c_all[l] = d_c_all[l];
-        P.gates_all[l] = d_gates_all ? d_gates_all[l] : nullptr;
-      }
-      P.embed = d_embed;
-      P.ids = d_ids_nonneg;
-      P.mask01 = d_mask01;
-      P.status = ctx->d_flags + 2;
-      P.nl = nl;
-      P.T = T;
-      P.V = V;
-      P.H = H;
-      P.mb = mb;
-      P.ldw = layers[0]->ldw;
-      P.kp = layers[0]->kp;
-      P.j_tiles = j_tiles;
-      P.n_tiles = n_tiles;
-      P.clip = clip_threshold;
-      P.spin_limit = ctx->sweep_spin > 0 ? ctx->sweep_spin : (1 << 20);
-      // Without the invalidation a consumer relies on never having cached a line before its producer wrote it: true
-      // when no 128-byte line of the k-interleaved copies is shared between two producers, i.e. mb % 8 == 0.
-      P.fence = (mb % 8 == 0) ? 0 : 1;
-      ctx->last_stack_path = ZR_LSTM_STACK_PATH_SWEEP;
-      return tn == 1 ? launch_sweep_v<1>(ctx, P, padded * n_tiles) : launch_sweep_v<2>(ctx, P, padded * n_tiles);
+    const long long tiles = tn ? (long long)groups * ((n32 + tn - 1) / tn) : 0;
+    const bool fills = tiles * 10 >= 6LL * ctx->cu_count;
+    if (!offsets_fit || !(fills || ctx->lstm_sweep == 2) || (tn && nl * ((n32 + tn - 1) / tn) > 512) ||
+        (long long)T * j_tiles >= kSweepGaveUp)
+      tn = 0;
+  }
+  // Resident-weight sweep: small models and narrow batches, where the sweep above (if it fits) runs on few workgroups with
+  // long K loops and a launch per diagonal costs more than its work.  Taken when its estimated time is the least.  The
+  // estimates of the other two, us a step, and what was measured (layers x H at columns):
+  //   streamed sweep: 5 + the K loop of a workgroup (H/8 groups of both segments over 4 waves, 16 TN instructions of 64
+  //     cycles each at 2.3 GHz), half a step more per layer to fill: 4 x 1000 at 128 61 / 61, 3 x 640 at 130 41 / 46;
+  //   a launch per diagonal: 8 + the longer of its weights at 5 TB/s and its products at 100 TFLOP/s: 4 x 1000 at 16
+  //     34 / 30, 1 x 1000 at 128 28 / 25, 2 x 1000 at 33 28 / 25.
+  if (single_ok && (ctx->lstm_sweep == 2 || (!ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts))) {
+    ZrResidentPlan plan;
+    const double resident_us = zr_lstm_resident_plan(ctx, nl, H, mb, T, &plan);
+    const double k_groups = 2.0 * ((H + 7) / 8);
+    double other_us = -1.0;
+    if (tn) other_us = (T + 0.5 * nl) * (5.0 + k_groups / 4 * 16 * tn * 64 / 2300.0);
+    if (!ctx->lstm_sweep) {
+      const double weights = 32.0 * H * H * nl, flops = 16.0 * H * H * (32.0 * n32) * nl;
+      const double diag_us = (T + nl - 1) * (8.0 + (weights / 5e6 > flops / 100e6 ? weights / 5e6 : flops / 100e6));
+      if (other_us < 0.0 || diag_us < other_us) other_us = diag_us;
     }
+    if (resident_us > 0.0 && (other_us < 0.0 || resident_us < other_us)) {
+      rc = zr_lstm_resident_sweep(ctx, plan, nl, layers, d_embed, V, d_ids_nonneg, d_mask01, T, mb, d_h0, d_c0,
+                                  clip_threshold, d_h_all, d_c_all, d_gates_all);
+      if (rc) return rc;
+      ctx->last_stack_path = ZR_LSTM_STACK_PATH_SWEEP;
+      return poison_if_abandoned(ctx, nl, T, H, mb, d_h_all, d_c_all, d_gates_all);
+    }
+  }
+  if (tn) {
+    const int n_tiles = (n32 + tn - 1) / tn;
+    LstmSweep P = {};
+    const size_t ctr_bytes = sizeof(int) * 512 * kSweepCtrStride;
+    void* p = nullptr;
+    rc = zr_ctx_scratch(ctx, 1, ctr_bytes + sizeof(float) * (size_t)nl * T * n, &p);
+    if (rc) return rc;
+    P.counters = (int*)p;
+    P.hp = (float*)((char*)p + ctr_bytes);
+    rc = zr_memset_zero(ctx, P.counters, sizeof(int) * (size_t)nl * n_tiles * kSweepCtrStride);
+    if (rc) return rc;
+    for (int l = 0; l < nl; ++l) {
+      P.W[l] = (const float*)layers[l]->d_W;
+      P.bias[l] = layers[l]->d_bias;
+      P.h0[l] = d_h0[l];
+      P.c0[l] = d_c0[l];
+      P.h_all[l] = d_h_all[l];
+      P.c_all[l] = d_c_all[l];
+      P.gates_all[l] = d_gates_all ? d_gates_all[l] : nullptr;
+    }
+    P.embed = d_embed;
+    P.ids = d_ids_nonneg;
+    P.mask01 = d_mask01;
+    P.status = ctx->d_flags + 2;
+    P.nl = nl;
+    P.T = T;
+    P.V = V;
+    P.H = H;
+    P.mb = mb;
+    P.ldw = layers[0]->ldw;
+    P.kp = layers[0]->kp;
+    P.j_tiles = j_tiles;
+    P.n_tiles = n_tiles;
+    P.clip = clip_threshold;
+    P.spin_limit = ctx->sweep_spin > 0 ? ctx->sweep_spin : (1 << 20);
+    // Without the invalidation a consumer relies on never having cached a line before its producer wrote it: true
+    // when no 128-byte line of the k-interleaved copies is shared between two producers, i.e. mb % 8 == 0.
+    P.fence = (mb % 8 == 0) ? 0 : 1;
+    ctx->last_stack_path = ZR_LSTM_STACK_PATH_SWEEP;
+    return tn == 1 ? launch_sweep_v<1>(ctx, P, padded * n_tiles) : launch_sweep_v<2>(ctx, P, padded * n_tiles);
   }
   // Every h is also written in a k-interleaved layout ([H/4][mb][4]) into a small ping-pong buffer per layer: its
   // two consumers on the next diagonal, (l+1, t) and (l, t+1), then fetch activations with contiguous 16-byte

@@ -1,0 +1,507 @@
+// Whole stacked-LSTM sweep with the weights held in registers.
+//
+// lstm_sweep_kernel (zr_lstm.hip) streams every weight tile from the caches in every time step and gives a workgroup 32
+// hidden rows: right when the batch is wide enough for the matrix cores to be the bound, but a small model or a narrow
+// batch then runs on a handful of workgroups (H = 500, two layers: 32), each with a K loop far longer than the time
+// step's arithmetic needs.  Here a workgroup owns 8 hidden rows of one layer -- 32 weight rows, its 8 rows of the four
+// gates, the width of one matrix instruction -- for one column tile and all T steps, and its 8 waves keep their share of
+// those 32 x 2H weights in vector registers: 2H x 32 floats over 512 threads is H/8 registers a thread, 128 at H = 1024.
+// A time step then moves activations only.
+//
+// What bounds it: the chain of time steps -- h of (l, t-1) must be published by every row tile of the layer, seen by the
+// others and multiplied before (l, t) can publish -- so everything that is not on that chain is kept off it:
+//   * the product with the input from below (embedding columns, or h of (l-1, t), which is there a step early) runs
+//     first, in the shadow of the hand-over of h of (l, t-1);
+//   * a wave waits only for the producers of its own K slice: a row tile of 8 is one k-group, the flags of the 16
+//     producers (at most) of a wave's groups lie side by side and one load by one wave looks at all of them;
+//   * h travels in a k-interleaved copy [k/4][columns][4] whose pad rows are written as zeros (any H, no K tails) and
+//     whose columns are padded to four, so that every 128-byte line of it has one producer and is read only after that
+//     producer's flag: no cache invalidation inside the launch;
+//   * h, c and the kept gate values are stored after the publish.
+// Batches of up to 16 columns use the 16 x 16 x 4 instruction (NARROW), half the matrix time of a half-empty 32-column
+// tile.  Progress, bounded waits and the abandon protocol are those of lstm_sweep_kernel; a workgroup that gives up marks
+// its own flag, which makes everybody who depends on it give up in turn.  The last workgroup out clears the flags.
+//
+// Measured, whole sweep, against one launch per diagonal: 1 layer of H = 100, 8 columns, 20 steps 55 us (253); 2 of 500,
+// 20 columns, 35 steps 180 us (1130); 4 of 1000, 16 columns, 50 steps 700 us (1600), 1 column, 25 steps 370 us (800).
+// Tried: finishing waves that publish on their own while the others run ahead into the next step (300 against 180 us at
+// H = 500: the waves that are ahead poll, and their polls hold up the publishing stores); a first look at the flags of
+// the layer below a step early (no change).
+#include "zr_internal.h"
+#include "zr_math.h"
+#include "zr_mfma_core.h"
+
+namespace {
+
+constexpr int kMaxLayers = 8;
+constexpr int kWaves = 8;                 // waves per workgroup = K slices
+constexpr int kRows = 8;                  // hidden rows per workgroup
+constexpr int kRedLd = 36;                // LDS row of 32 partial sums, padded: conflict-free for the cell's reads
+constexpr int kResidentGaveUp = 1 << 28;  // flag value of a workgroup that stopped waiting
+
+struct LstmResident {
+  const float* W[kMaxLayers];     // per layer: [2][4] packed fp32 matrices
+  const float* bias[kMaxLayers];  // per layer: [4][H]
+  const float* h0[kMaxLayers];
+  const float* c0[kMaxLayers];
+  float* h_all[kMaxLayers];
+  float* c_all[kMaxLayers];
+  float* gates_all[kMaxLayers];   // null: gates not kept
+  const float* embed;
+  const int* ids;                 // [T][mb], already non-negative
+  const int* mask01;              // [T][mb]
+  float* hp;                      // [layers][T + 1] slots of k-interleaved h: slot 0 = initial state, slot t + 1 = h_t
+  long long slot;                 // floats per slot: ceil8(H) * mbp
+  int* flags;                     // [layers of this launch][n_tiles] at flag_stride, zero at launch: slots published
+  int flag_stride, n_flags;
+  int* departures;                // workgroups that have left the kernel (zero at launch)
+  int* status;                    // set to 1 when a wait was abandoned
+  int l_begin;                    // first layer of this launch (the layers below it are complete)
+  int T, V, H, mb, mbp, ldw, kp, j_tiles, n_tiles;
+  float clip;
+  int spin_limit;
+};
+
+typedef zr_f32x4 zr_f32x4_u __attribute__((aligned(4)));  // 16-byte load from a 4-byte aligned address
+
+// NG: k-groups per wave and segment (H <= 64 * NG, NARROW: 128 * NG).  TN: 32-column tiles per workgroup (NARROW: one
+// 16-column tile).
+template <int NG, int TN, bool NARROW>
+__global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_resident_kernel(LstmResident P) {
+  static_assert(!NARROW || TN == 1, "a narrow tile is one tile of 16 columns");
+  constexpr int KB = NARROW ? 4 : 2;             // k-blocks of 4 per k-group
+  constexpr int NB = NARROW ? 2 : 1;             // 16-row halves of the 32 weight rows
+  constexpr int COLS = NARROW ? 16 : 32 * TN;    // columns of the workgroup's tile
+  constexpr int NPROD = NARROW ? 2 * NG : NG;    // producers of a wave's K slice
+  constexpr int NOUT = (kRows * COLS + 511) / 512;  // (row, column) pairs a thread finishes
+  __shared__ float red[kWaves * COLS * kRedLd];
+  __shared__ int s_abort, s_last;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int kslice = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int H = P.H, mb = P.mb;
+  const int nt = (int)blockIdx.x % P.n_tiles;
+  const int jt = ((int)blockIdx.x / P.n_tiles) % P.j_tiles;
+  const int l = P.l_begin + (int)blockIdx.x / (P.n_tiles * P.j_tiles);
+  const int j0 = jt * kRows;
+  const int n0 = nt * COLS;
+  const int cl = NARROW ? (lane & 15) : (lane & 31);  // this lane's column of the activations, row of the weights
+  const int kq = NARROW ? (lane >> 4) : (lane >> 5);  // its k-block inside a group
+  const bool from_embed = l == 0;
+  if (tid == 0) s_abort = 0;
+
+  auto work = [&]() {
+    // ---- weights into registers: w[segment][group][half][k]
+    float w[2][NG][NB][4];
+    const long long HH = (long long)P.kp * P.ldw;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < NG; ++i)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const int c = cl + 16 * b;
+          const float* m = P.W[l] + (s * 4 + (c >> 3)) * HH + 4 * (j0 + (c & 7));
+          const int k0 = 4 * (KB * (kslice + kWaves * i) + kq);
+          if (s == 0 && from_embed) {
+            // embedding columns are read as they lie, so a lane's four k must stay inside the column: the last
+            // k-block of a column is moved down to end at H - 1, and what it covers twice counts once
+            const int ks = k0 < H - 4 ? k0 : H - 4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int k = ks + e;
+              w[s][i][b][e] = k >= k0 ? m[(long long)(k >> 2) * (4 * P.ldw) + (k & 3)] : 0.0f;
+            }
+          } else {
+            zr_f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (k0 < P.kp) v = *(const zr_f32x4*)(m + (long long)(k0 >> 2) * (4 * P.ldw));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[s][i][b][e] = v[e];
+          }
+        }
+
+    // ---- the outputs this thread finishes: (row, column) pairs, rows of four fastest (the order h travels in)
+    int oj[NOUT], on[NOUT];
+    bool ok[NOUT], tile_ok[NOUT];
+    float bi[NOUT], bf[NOUT], bc[NOUT], bo[NOUT], c_state[NOUT];
+    unsigned hp_off[NOUT];  // element inside a slot
+#pragma unroll
+    for (int u = 0; u < NOUT; ++u) {
+      const int o = tid + 512 * u;
+      oj[u] = ((o >> 2) / COLS) * 4 + (o & 3);
+      on[u] = (o >> 2) % COLS;
+      const int j = j0 + oj[u], n = n0 + on[u];
+      tile_ok[u] = o < kRows * COLS && n < mb;
+      ok[u] = tile_ok[u] && j < H;
+      const int jc = j < H ? j : H - 1, nc = n < mb ? n : mb - 1;
+      bi[u] = P.bias[l][jc], bf[u] = P.bias[l][H + jc], bc[u] = P.bias[l][2 * H + jc], bo[u] = P.bias[l][3 * H + jc];
+      c_state[u] = P.c0[l][(long long)nc * H + jc];
+      hp_off[u] = (unsigned)(((j >> 2) * P.mbp + n) * 4 + (j & 3));
+    }
+    int* flags_here = P.flags + ((l - P.l_begin) * P.n_tiles + nt) * P.flag_stride;
+    const int* flags_below = flags_here - P.n_tiles * P.flag_stride;
+    // Flags of a (layer, column tile): [K slice][producer of the slice].
+    int pslice, pindex;  // where this workgroup stands as a producer
+    if constexpr (NARROW)
+      pslice = (jt >> 1) & 7, pindex = (jt >> 4) * 2 + (jt & 1);
+    else
+      pslice = jt & 7, pindex = jt >> 3;
+    int* my_flag = flags_here + pslice * NPROD + pindex;
+    // the producer this lane looks at, for the lanes below NPROD
+    const int pj = NARROW ? 2 * (kslice + kWaves * (lane >> 1)) + (lane & 1) : kslice + kWaves * lane;
+    const bool looks = lane < NPROD && pj < P.j_tiles;
+    const int look = kslice * NPROD + (lane < NPROD ? lane : 0);
+    bool dead = false;  // this wave has given up a wait: it goes on without waiting to the next barrier
+    auto wait_for = [&](const int* flags, int target) {
+      if (dead) return;
+      int spins = 0;
+      bool gave_up = false;
+      for (;;) {
+        const int v =
+            looks ? __hip_atomic_load(flags + look, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kResidentGaveUp - 1;
+        if (__all(v >= target)) {
+          gave_up = __any(v >= kResidentGaveUp);
+          break;
+        }
+        if (++spins > P.spin_limit) {
+          gave_up = true;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      if (gave_up) {
+        dead = true;
+        if (lane == 0) s_abort = 1;
+      }
+      asm volatile("" ::: "memory");  // nothing behind the wait is read before it
+    };
+
+    // ---- the initial state goes out as slot 0
+    float* hp_mine = P.hp + (long long)l * (P.T + 1) * P.slot;
+    const float* hp_below = hp_mine - (long long)(P.T + 1) * P.slot;
+#pragma unroll
+    for (int u = 0; u < NOUT; ++u)
+      if (tile_ok[u])
+        __hip_atomic_store(hp_mine + hp_off[u], ok[u] ? P.h0[l][(long long)(n0 + on[u]) * H + j0 + oj[u]] : 0.0f,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    zr_publish_barrier();
+    if (tid == 0) __hip_atomic_store(my_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+    // ---- this lane's activation columns
+    int cols[TN], idv[TN];
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) {
+      const int c = n0 + tn * 32 + cl;
+      cols[tn] = c < mb ? c : mb - 1;
+    }
+    auto clamp_id = [&](int v) { return v < 0 ? 0 : (v >= P.V ? P.V - 1 : v); };
+    // The embedding columns of a step's words, read as they lie.  AHEAD: a step ahead (H = 1000, 16 columns: 6.8 us a step
+    // against 7.5; no gain at smaller sizes, whose shorter segments leave nothing to hide the earlier loads behind).
+    constexpr bool AHEAD = NARROW && NG == 8;
+    zr_f32x4 x_ahead[AHEAD ? NG : 1][TN];
+    const float* col[TN];
+    auto next_words = [&](int t) {
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) {
+        col[tn] = P.embed + (long long)idv[tn] * H;
+        idv[tn] = clamp_id(P.ids[(long long)(t + 1 < P.T ? t + 1 : t) * mb + cols[tn]]);
+      }
+    };
+    auto load_embed = [&](zr_f32x4 (&x)[TN], int i) {
+      const int k0 = 4 * (KB * (kslice + kWaves * i) + kq);
+      const int ks = k0 < H - 4 ? k0 : H - 4;
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) x[tn] = *(const zr_f32x4_u*)(col[tn] + ks);
+    };
+    if (from_embed) {
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) idv[tn] = clamp_id(P.ids[cols[tn]]);
+      next_words(0);
+      if constexpr (AHEAD) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) load_embed(x_ahead[i], i);
+      }
+    }
+    const unsigned kb_step = (unsigned)(kWaves * KB * P.mbp * 4);  // elements from a wave's group to its next
+    const unsigned kb_first = (unsigned)((KB * kslice + kq) * P.mbp * 4);
+    // A narrow group is two row tiles; when only the first exists its last k-block stands in for the second's (it meets
+    // zero weights).  Groups past the end are not read at all: a line read before its producer's flag would go stale.
+    const unsigned kb_last = (unsigned)((2 * P.j_tiles - 1) * P.mbp * 4);
+    const int n_groups = (2 * P.j_tiles + KB - 1) / KB;
+
+    typedef float acc16 __attribute__((ext_vector_type(16)));
+    for (int t = 0; t < P.T; ++t) {
+      acc16 acc[TN];
+      zr_f32x4 acc4[NB];
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[tn][r] = 0.0f;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc4[b] = {0.0f, 0.0f, 0.0f, 0.0f};
+
+      auto mma = [&](const zr_f32x4 (&x)[TN], const float (&wg)[NB][4]) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (NARROW) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) acc4[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0][e], wg[b][e], acc4[b], 0, 0, 0);
+          } else {
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn)
+              acc[tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[tn][e], wg[0][e], acc[tn], 0, 0, 0);
+          }
+        }
+      };
+      // One segment.  All of a wave's activations are in flight at once where the registers allow it, else a few groups
+      // ahead of the ones being multiplied.
+      auto segment = [&](const float (&ws)[NG][NB][4], auto load) {
+        constexpr int CH = NG <= 8 ? NG : (TN == 1 ? 4 : 2);
+        constexpr int NC = NG / CH;
+        zr_f32x4 x[NC > 1 ? 2 : 1][CH][TN];
+#pragma unroll
+        for (int i = 0; i < CH; ++i) load(x[0][i], i);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          if (c + 1 < NC) {
+#pragma unroll
+            for (int i = 0; i < CH; ++i) load(x[(c + 1) & (NC > 1 ? 1 : 0)][i], (c + 1) * CH + i);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < CH; ++i) mma(x[c & (NC > 1 ? 1 : 0)][i], ws[c * CH + i]);
+        }
+      };
+      auto load_packed = [&](const float* base) {
+        return [=, &cols](zr_f32x4 (&x)[TN], int i) {
+          if (kslice + kWaves * i < n_groups) {
+            unsigned kb = kb_first + (unsigned)i * kb_step;
+            if constexpr (NARROW) kb = kb < kb_last ? kb : kb_last;
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn) x[tn] = *(const zr_f32x4*)(base + (kb + 4u * (unsigned)cols[tn]));
+          } else {
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn) x[tn] = zr_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+          }
+        };
+      };
+
+      // the input from below
+      if (from_embed) {
+        if constexpr (AHEAD) {
+#pragma unroll
+          for (int i = 0; i < NG; ++i) mma(x_ahead[i], w[0][i]);
+        } else {
+          segment(w[0], load_embed);
+        }
+      } else {
+        if (l > P.l_begin) wait_for(flags_below, t + 2);
+        segment(w[0], load_packed(hp_below + (long long)(t + 1) * P.slot));
+      }
+      float mask_v[NOUT];
+#pragma unroll
+      for (int u = 0; u < NOUT; ++u) mask_v[u] = tile_ok[u] ? (float)P.mask01[(long long)t * mb + n0 + on[u]] : 0.0f;
+      // the layer's own previous step
+      wait_for(flags_here, t + 1);
+      segment(w[1], load_packed(hp_mine + (long long)t * P.slot));
+
+      // what the next step reads from below: asked for now, in flight while this step is finished
+      if (t + 1 < P.T) {
+        if (from_embed) {
+          next_words(t + 1);
+          if constexpr (AHEAD) {
+#pragma unroll
+            for (int i = 0; i < NG; ++i) load_embed(x_ahead[i], i);
+          }
+        }
+      }
+
+      // partial sums of the 8 K slices through LDS, then the cell
+      float* mine = red + kslice * (COLS * kRedLd);
+      if constexpr (NARROW) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) mine[(4 * kq + r) * kRedLd + cl + 16 * b] = acc4[b][r];
+      } else {
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) mine[(tn * 32 + 8 * (r >> 2) + 4 * kq + (r & 3)) * kRedLd + cl] = acc[tn][r];
+      }
+      __syncthreads();
+      if (s_abort) {  // every wave of the workgroup sees the same value: waits come before this barrier
+        if (tid == 0) __hip_atomic_store(my_flag, kResidentGaveUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) __hip_atomic_store(P.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return;
+      }
+      float h_v[NOUT], g_v[NOUT][4];
+      float* hp_out = hp_mine + (long long)(t + 1) * P.slot;
+#pragma unroll
+      for (int u = 0; u < NOUT; ++u) {
+        if (!tile_ok[u]) continue;
+        float z[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float* p = red + on[u] * kRedLd + g * 8 + oj[u];
+          float sum = 0.0f;
+#pragma unroll
+          for (int q = 0; q < kWaves; ++q) sum += p[q * (COLS * kRedLd)];
+          z[g] = sum;
+        }
+        float c;
+        zr_lstm_cell(z[0] + bi[u], z[1] + bf[u], z[2] + bc[u], z[3] + bo[u], c_state[u], mask_v[u], P.clip, g_v[u][0],
+                     g_v[u][1], g_v[u][2], g_v[u][3], c, h_v[u]);
+        c_state[u] = c;
+        __hip_atomic_store(hp_out + hp_off[u], ok[u] ? h_v[u] : 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      zr_publish_barrier();
+      if (tid == 0) __hip_atomic_store(my_flag, t + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int u = 0; u < NOUT; ++u) {
+        if (!ok[u]) continue;
+        const long long n_el = (long long)H * mb;
+        const long long ix = (long long)(n0 + on[u]) * H + j0 + oj[u];
+        P.h_all[l][(long long)t * n_el + ix] = h_v[u];
+        P.c_all[l][(long long)t * n_el + ix] = c_state[u];
+        if (P.gates_all[l]) {
+          float* gt = P.gates_all[l] + (long long)t * 4 * n_el + ix;
+#pragma unroll
+          for (int g = 0; g < 4; ++g) gt[g * n_el] = g_v[u][g];
+        }
+      }
+    }
+  };
+  __syncthreads();  // s_abort
+  work();
+
+  // Departure: the last workgroup out returns the flags to zero for the next launch (this one's own last flag has
+  // landed by then).
+  zr_publish_barrier();
+  if (tid == 0) {
+    const int before = __hip_atomic_fetch_add(P.departures, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = before == (int)gridDim.x - 1 ? 1 : 0;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  for (int i = tid; i < P.n_flags; i += 512) __hip_atomic_store(P.flags + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) __hip_atomic_store(P.departures, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+typedef void (*ResidentKernel)(LstmResident);
+// [size class][column class]: H <= 128, 256, 512, 1024; 16, 32, 64 columns a workgroup (64 columns of H > 512: the
+// registers hold 128 weights a thread and not the 32 accumulators on top)
+const ResidentKernel kKernels[4][3] = {
+    {lstm_resident_kernel<1, 1, true>, lstm_resident_kernel<2, 1, false>, lstm_resident_kernel<2, 2, false>},
+    {lstm_resident_kernel<2, 1, true>, lstm_resident_kernel<4, 1, false>, lstm_resident_kernel<4, 2, false>},
+    {lstm_resident_kernel<4, 1, true>, lstm_resident_kernel<8, 1, false>, lstm_resident_kernel<8, 2, false>},
+    {lstm_resident_kernel<8, 1, true>, lstm_resident_kernel<16, 1, false>, nullptr}};
+constexpr int kColumns[3] = {16, 32, 64};
+
+int resident_capacity(zr_ctx* ctx, int size_class, int col_class) {
+  int& cached = ctx->resident_capacity[size_class][col_class];
+  if (!kKernels[size_class][col_class]) return 0;
+  if (cached == 0) {
+    int cus = 0, per_cu = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kKernels[size_class][col_class], 64 * kWaves, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      cached = -1;
+    } else {
+      ctx->cu_count = cus;
+      cached = cus * per_cu > 0 ? cus * per_cu : -1;
+    }
+  }
+  return cached > 0 ? cached : 0;
+}
+
+}  // namespace
+
+double zr_lstm_resident_plan(zr_ctx* ctx, int nl, int H, int mb, int T, ZrResidentPlan* plan) {
+  plan->at_once = 0;
+  if (H < 8 || H > 1024 || nl > kMaxLayers || T >= kResidentGaveUp / 2) return -1.0;
+  const int size_class = H <= 128 ? 0 : (H <= 256 ? 1 : (H <= 512 ? 2 : 3));
+  const int j_tiles = (H + kRows - 1) / kRows;
+  const int nprod = 2 << size_class;  // NPROD of the kernel, in every column class
+  const int flag_stride = (kWaves * nprod + 31) / 32 * 32;
+  const long long slot = (long long)j_tiles * kRows * ((mb + 3) & ~3);
+  if (slot * 4 >= (1LL << 32)) return -1.0;
+  // Column class and layers per launch: the cheapest by the time a step takes -- a hand-over of 3.2 us and the matrix
+  // instructions of both segments at 2.3 GHz, two waves to a SIMD and as many workgroups to a compute unit as the launch
+  // needs, times what the shorter prefetch of the wider tiles costs.  Measured against the estimate, us a step: H = 500,
+  // 16 columns 4.9 / 5.0, 32 columns 8.2 / 8.5; H = 1000, 16 columns 6.8 / 6.8, 32 columns 15.8 / 15.6.
+  double best = -1.0;
+  for (int c = 0; c < 3; ++c) {
+    const int n_tiles = (mb + kColumns[c] - 1) / kColumns[c];
+    int at_once = resident_capacity(ctx, size_class, c) / (j_tiles * n_tiles);
+    if (at_once > nl) at_once = nl;
+    while (at_once > 0 && at_once * n_tiles * flag_stride > ZR_MAX_STEP_FLAGS - 32) --at_once;
+    if (at_once < 1) continue;
+    const int per_cu = (at_once * j_tiles * n_tiles + ctx->cu_count - 1) / ctx->cu_count;
+    const int groups = c == 0 ? (H + 127) / 128 : (H + 63) / 64;  // of a wave and segment
+    const double stretch = c == 0 ? 1.0 : (c == 2 ? 1.6 : (size_class == 3 ? 1.75 : 1.5));
+    const double step = 3.2 + stretch * per_cu * 2.0 * groups * 4 * (c == 2 ? 128 : 64) * 2 / 2300.0;
+    const double us = (double)((nl + at_once - 1) / at_once) * (T + at_once - 1) * step;
+    if (best < 0.0 || us < best) {
+      best = us;
+      plan->size_class = size_class;
+      plan->col_class = c;
+      plan->n_tiles = n_tiles;
+      plan->at_once = at_once;
+      plan->flag_stride = flag_stride;
+    }
+  }
+  return best;
+}
+
+int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, const zr_lstm_weights* const layers[],
+                           const float* d_embed, int V, const int* d_ids_nonneg, const int* d_mask01, int T, int mb,
+                           const float* const d_h0[], const float* const d_c0[], float clip_threshold,
+                           float* const d_h_all[], float* const d_c_all[], float* const d_gates_all[]) {
+  const int H = layers[0]->H;
+  const int j_tiles = (H + kRows - 1) / kRows;
+  const int per_layer = j_tiles * plan.n_tiles;
+  const int mbp = (mb + 3) & ~3;
+  const long long slot = (long long)j_tiles * kRows * mbp;
+  void* p = nullptr;
+  int rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (size_t)(nl * (long long)(T + 1) * slot), &p);
+  if (rc) return rc;
+  LstmResident P = {};
+  for (int l = 0; l < nl; ++l) {
+    P.W[l] = (const float*)layers[l]->d_W;
+    P.bias[l] = layers[l]->d_bias;
+    P.h0[l] = d_h0[l];
+    P.c0[l] = d_c0[l];
+    P.h_all[l] = d_h_all[l];
+    P.c_all[l] = d_c_all[l];
+    P.gates_all[l] = d_gates_all ? d_gates_all[l] : nullptr;
+  }
+  P.embed = d_embed;
+  P.ids = d_ids_nonneg;
+  P.mask01 = d_mask01;
+  P.hp = (float*)p;
+  P.slot = slot;
+  P.flags = ctx->d_step_flags + 32;
+  P.flag_stride = plan.flag_stride;
+  P.departures = ctx->d_step_flags;
+  P.status = ctx->d_flags + 2;
+  P.T = T;
+  P.V = V;
+  P.H = H;
+  P.mb = mb;
+  P.mbp = mbp;
+  P.ldw = layers[0]->ldw;
+  P.kp = layers[0]->kp;
+  P.j_tiles = j_tiles;
+  P.n_tiles = plan.n_tiles;
+  P.clip = clip_threshold;
+  P.spin_limit = ctx->sweep_spin > 0 ? ctx->sweep_spin : (1 << 20);
+  for (int l = 0; l < nl; l += plan.at_once) {
+    const int now = nl - l < plan.at_once ? nl - l : plan.at_once;
+    P.l_begin = l;
+    P.n_flags = now * plan.n_tiles * plan.flag_stride;
+    kKernels[plan.size_class][plan.col_class]<<<now * per_layer, 64 * kWaves, 0, ctx->stream>>>(P);
+    ZR_LAUNCH_CHECK("lstm_resident_kernel");
+  }
+  return ZR_OK;
+}

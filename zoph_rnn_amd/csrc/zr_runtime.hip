@@ -102,14 +102,15 @@ int zr_ctx_create(int device, zr_ctx** out) {
     return zr_set_error(ZR_EHIP, "hipStreamCreate failed: %s", hipGetErrorString(e));
   }
   c->stream = c->own_stream;
-  e = hipMalloc((void**)&c->d_flags, (4 + ZR_MAX_COUNTERS) * sizeof(int));
+  e = hipMalloc((void**)&c->d_flags, (32 + ZR_MAX_COUNTERS + ZR_MAX_STEP_FLAGS) * sizeof(int));
   if (e != hipSuccess) {
     (void)hipStreamDestroy(c->own_stream);
     delete c;
     return zr_set_error(ZR_ENOMEM, "flag allocation failed: %s", hipGetErrorString(e));
   }
-  (void)hipMemset(c->d_flags, 0, (4 + ZR_MAX_COUNTERS) * sizeof(int));
-  c->d_counters = c->d_flags + 4;
+  (void)hipMemset(c->d_flags, 0, (32 + ZR_MAX_COUNTERS + ZR_MAX_STEP_FLAGS) * sizeof(int));
+  c->d_counters = c->d_flags + 32;  // (a line apart from the flags)
+  c->d_step_flags = c->d_counters + ZR_MAX_COUNTERS;
   {
     const int rc = static_scratch_address(device, &c->d_static_scratch);
     if (rc) {
