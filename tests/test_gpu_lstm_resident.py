@@ -1,4 +1,5 @@
-"""The whole-sweep LSTM kernel that keeps its weights in registers (zr_lstm_resident.hip), against the oracle: hidden
+"""The LSTM kernels on narrow row tiles: the whole sweep with weights in registers (zr_lstm_resident.hip) and one node
+(zr_lstm_rows.hip), against the oracle: hidden
 sizes around the edges of its row tiles, k-groups and register classes, batches around the edges of its column tiles,
 more layers than fit in one launch, initial states, padding, cell clipping, kept gates, and giving up a wait."""
 import numpy as np
@@ -112,3 +113,40 @@ def test_abandoned_wait_is_reported_and_leaves_nan(ctx):
     want_h, want_c = _want(c)
     assert_close(h, want_h, what="h")
     assert_close(x, want_c, what="c")
+
+
+# One node on tiles of 4 or 8 hidden rows (zr_lstm_rows.hip): row tails of every kind, columns around the edges of 16-, 32-
+# and 64-column tiles, K tails of the last load (H % 4 and H % 8), with the embedding gather and with feed-input
+@pytest.mark.parametrize("H,mb", [(8, 1), (9, 17), (11, 16), (100, 8), (127, 33), (130, 129), (257, 64), (500, 37), (510, 70),
+                                  (513, 16), (1000, 12), (1000, 33), (1001, 130), (2000, 5)])
+def test_node_on_narrow_row_tiles(ctx, H, mb):
+    g = synth.rng(43, H + mb)
+    V = 97
+    ly = synth.lstm_layer(g, H, feed_input=True, forget_bias_one=True)
+    embed = synth.uniform(g, (H, V), -0.5, 0.5)
+    ids = g.integers(0, V, size=mb).astype(np.int32)
+    hp, ht = np.tanh(synth.uniform(g, (H, mb), -1, 1)), np.tanh(synth.uniform(g, (H, mb), -1, 1))
+    cp = synth.uniform(g, (H, mb), -0.5, 0.5)
+    mask = (g.random(mb) < 0.8).astype(np.int32)
+    layer = Layer(ctx, ly)
+    d_h, d_c = ctx.empty((H, mb)), ctx.empty((H, mb))
+    d_g = [ctx.empty((H, mb)) for _ in range(4)]
+    x = np.asfortranarray(embed[:, ids])
+    try:
+        for feed in (False, True):
+            want = o.lstm_step(ly["M"], ly["Wh"], ly["b"], x, hp, cp, mask, clip=0.9, **(dict(Q=ly["Q"], htild=ht) if feed else {}))
+            for gather in (False, True):
+                args = dict(clip=0.9, gates=d_g, d_htild=ctx.array(ht) if feed else None)
+                if gather:
+                    ctx.lstm_step_embed(layer.w, ctx.array(embed), V, ctx.array(ids), ctx.array(hp), ctx.array(cp),
+                                        ctx.array(mask), mb, d_h, d_c, **args)
+                else:
+                    ctx.lstm_step(layer.w, ctx.array(x), ctx.array(hp), ctx.array(cp), ctx.array(mask), mb, d_h, d_c, **args)
+                ctx.sync()
+                what = "feed %d gather %d" % (feed, gather)
+                assert_close(d_h.get(), want["h"], what="h " + what)
+                assert_close(d_c.get(), want["c"], what="c " + what)
+                for a, k in zip(d_g, ("i", "f", "c_tilde", "o")):
+                    assert_close(a.get(), want[k], what=k + " " + what)
+    finally:
+        layer.close()

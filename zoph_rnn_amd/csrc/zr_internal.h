@@ -30,7 +30,7 @@ struct zr_ctx {
   int sweep_spin;    // polls before a waiting workgroup of that kernel gives up (0: default)
   int step_wait_extra;  // arrivals the decoder step's layer waits expect beyond the real ones (tests of giving up)
   int stack_helpers;    // 1 (default): the decoder step may run 32-column tiles with helper workgroups (zr_lstm.hip)
-  int cu_count;      // compute units of the device (filled with sweep_capacity)
+  int cu_count;      // compute units of the device
   int sweep_capacity[3];  // resident workgroups of lstm_sweep_kernel<TN> (0: not asked yet, -1: unknown)
   int resident_capacity[4][3];  // the same for lstm_resident_kernel, by size class and column class
   int stack_step_capacity;  // the same for lstm_decoder_stack_kernel (the lesser of its two tile widths)
@@ -221,6 +221,14 @@ int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, cons
                            const float* d_embed, int V, const int* d_ids_nonneg, const int* d_mask01, int T, int mb,
                            const float* const d_h0[], const float* const d_c0[], float clip_threshold,
                            float* const d_h_all[], float* const d_c_all[], float* const d_gates_all[]);
+
+// One node on tiles of 4 or 8 hidden rows (zr_lstm_rows.hip).  shape: 0 = 4 rows x 16 columns, 1 = 8 x 16, 2 = 8 x 32,
+// 3 = 8 x 64.  H >= 8; d_hp: h also k-interleaved [H/4][mb][4] (null: not wanted).
+int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const float* const in[3], const int* d_gather_ids,
+                      int V, const float* d_cprev, const int* d_mask01, float clip, int mb, float* d_h, float* d_c,
+                      float* const d_gates[4], float* d_hp, int shape);
+// The shape for a node of this size (-1: leave it to lstm_fused_kernel).
+int zr_lstm_rows_shape(int H, int mb, int cu_count);
 
 // The attention step in one launch (zr_attn_step.hip).  a->d_hpack must hold h_t k-interleaved.  *took = 0: the
 // conditions do not hold and nothing was launched (the caller goes on with one launch per stage).

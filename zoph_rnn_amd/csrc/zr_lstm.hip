@@ -1600,6 +1600,12 @@ static int lstm_step_impl(zr_ctx* ctx, const zr_lstm_weights* w, const float* d_
     const float* b[4] = {w->d_bias, w->d_bias + H, w->d_bias + 2 * (size_t)H, w->d_bias + 3 * (size_t)H};
     return zr_lstm_gates(ctx, (const float*)pre, b, d_cprev, d_mask01, clip_threshold, H, mb, d_h, d_c, d_gates);
   }
+  if (!w->bf16 && !ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts) {
+    const int shape = zr_lstm_rows_shape(H, mb, ctx->cu_count);
+    if (shape >= 0)
+      return zr_lstm_rows_step(ctx, w, nseg, U.in, d_gather_ids, V, d_cprev, d_mask01, clip_threshold, mb, d_h, d_c,
+                               d_gates, U.hp, shape);
+  }
   return launch_fused(ctx, L, vec);
 }
 
@@ -1826,7 +1832,7 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
   const bool alone = zr_live_contexts(ctx->device) == 1 && ctx->stream == ctx->own_stream;
   const bool single_ok = !layers[0]->bf16 && ctx->lstm_fused && (ctx->lstm_sweep == 2 || (ctx->lstm_sweep == 0 && alone));
   // Whole-sweep kernel with streamed weights: when its workgroups -- one tile of one layer each, kept for all T steps --
-  // fill most of the chip and fit on it together.
+  // fit on the chip together.
   const int j_tiles = (H + 31) / 32, n32 = (mb + 31) / 32;
   const int groups = nl * j_tiles;
   const int padded = (groups + 7) / 8 * 8;
@@ -1838,31 +1844,36 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
     const long long lim = 1LL << 32;
     const bool offsets_fit = (long long)V * H * 4 < lim && (long long)n * 4 < lim &&
                              8LL * layers[0]->kp * layers[0]->ldw * 4 < lim;
-    const long long tiles = tn ? (long long)groups * ((n32 + tn - 1) / tn) : 0;
-    const bool fills = tiles * 10 >= 6LL * ctx->cu_count;
-    if (!offsets_fit || !(fills || ctx->lstm_sweep == 2) || (tn && nl * ((n32 + tn - 1) / tn) > 512) ||
-        (long long)T * j_tiles >= kSweepGaveUp)
-      tn = 0;
+    if (!offsets_fit || (tn && nl * ((n32 + tn - 1) / tn) > 512) || (long long)T * j_tiles >= kSweepGaveUp) tn = 0;
   }
-  // Resident-weight sweep: small models and narrow batches, where the sweep above (if it fits) runs on few workgroups with
-  // long K loops and a launch per diagonal costs more than its work.  Taken when its estimated time is the least.  The
-  // estimates of the other two, us a step, and what was measured (layers x H at columns):
-  //   streamed sweep: 5 + the K loop of a workgroup (H/8 groups of both segments over 4 waves, 16 TN instructions of 64
-  //     cycles each at 2.3 GHz), half a step more per layer to fill: 4 x 1000 at 128 61 / 61, 3 x 640 at 130 41 / 46;
-  //   a launch per diagonal: 8 + the longer of its weights at 5 TB/s and its products at 100 TFLOP/s: 4 x 1000 at 16
-  //     34 / 30, 1 x 1000 at 128 28 / 25, 2 x 1000 at 33 28 / 25.
-  if (single_ok && (ctx->lstm_sweep == 2 || (!ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts))) {
-    ZrResidentPlan plan;
-    const double resident_us = zr_lstm_resident_plan(ctx, nl, H, mb, T, &plan);
-    const double k_groups = 2.0 * ((H + 7) / 8);
-    double other_us = -1.0;
-    if (tn) other_us = (T + 0.5 * nl) * (5.0 + k_groups / 4 * 16 * tn * 64 / 2300.0);
+  // Which schedule: the least estimated time, us a step (for the sweep with resident weights see zr_lstm_resident_plan).
+  // Against what was measured (layers x H at columns):
+  //   streamed sweep: 5 + the K loop of a workgroup (the groups of 8 k of both segments over 4 waves, 16 TN instructions
+  //     of 64 cycles each at 2.3 GHz), half a step more per layer to fill: 4 x 1000 at 128 61 / 61, 2 x 600 at 100 22 / 25;
+  //   a launch per diagonal: 10 + the longer of the weights at 5 TB/s and the K loop of a 32-column tile, divided over as
+  //     many workgroups as bring the launch nearest to one per compute unit, times the rounds those then need: 4 x 1000 at
+  //     16 36 / 30, 1 x 1000 at 128 24 / 25, 2 x 1000 at 33 24 / 25, 2 x 600 at 100 27 / 32; H % 8 != 0 has no K split
+  //     and slower loads: 4 x 300 at 200 38 / 38.
+  if (single_ok) {
+    const double k_loop = 2.0 * ((H + 7) / 8) / 4 * 16 * 64 / 2300.0;
+    double diag_us = -1.0;
     if (!ctx->lstm_sweep) {
-      const double weights = 32.0 * H * H * nl, flops = 16.0 * H * H * (32.0 * n32) * nl;
-      const double diag_us = (T + nl - 1) * (8.0 + (weights / 5e6 > flops / 100e6 ? weights / 5e6 : flops / 100e6));
-      if (other_us < 0.0 || diag_us < other_us) other_us = diag_us;
+      const double weights_us = 32.0 * H * H * nl / 5e6;
+      const long long tiles = (long long)groups * n32;
+      const long long parts = tiles >= ctx->cu_count ? 1 : (ctx->cu_count + tiles / 2) / tiles;
+      const double loop_us = (double)((tiles * parts + ctx->cu_count - 1) / ctx->cu_count) * k_loop / parts;
+      diag_us = (T + nl - 1) * (10.0 + (weights_us > loop_us ? weights_us : loop_us)) * (H % 8 ? 1.4 : 1.0);
     }
-    if (resident_us > 0.0 && (other_us < 0.0 || resident_us < other_us)) {
+    const double sweep_us = tn ? (T + 0.5 * nl) * (5.0 + k_loop * tn) : -1.0;
+    if (tn && diag_us > 0.0 && diag_us < sweep_us) tn = 0;
+    const double other_us = tn ? sweep_us : diag_us;
+    ZrResidentPlan plan;
+    plan.at_once = 0;
+    if (ctx->lstm_sweep == 2 || (!ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts)) {
+      const double resident_us = zr_lstm_resident_plan(ctx, nl, H, mb, T, &plan);
+      if (resident_us < 0.0 || (other_us > 0.0 && other_us <= resident_us)) plan.at_once = 0;
+    }
+    if (plan.at_once) {
       rc = zr_lstm_resident_sweep(ctx, plan, nl, layers, d_embed, V, d_ids_nonneg, d_mask01, T, mb, d_h0, d_c0,
                                   clip_threshold, d_h_all, d_c_all, d_gates_all);
       if (rc) return rc;

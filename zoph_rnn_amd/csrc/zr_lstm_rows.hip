@@ -1,0 +1,275 @@
+// One LSTM node (one layer, one time step) on narrow tiles: a workgroup owns ROWS hidden rows -- 4 * ROWS weight rows, all
+// four gates -- for one column tile, and its 8 waves split the K range of all segments together.
+//
+// lstm_fused_kernel (zr_lstm.hip) gives a workgroup 32 rows x 4 gates: a single node of a small model is then a dozen or two
+// workgroups whose K loops are many times longer than the weights' way from memory, and dividing K across workgroups as
+// well costs a round of partial tiles through memory.  Tiles of 4 or 8 rows put a node on 8 (4) times as many workgroups
+// with no exchange between them: one LDS sum of the 8 waves and the cell.
+// What bounds it: the weights' way from the memory-side cache at narrow batches, the matrix pipe at wide ones.
+//
+// Inputs are read as they lie (columns of H floats, gathered from the embedding for a bottom layer), four consecutive k a
+// lane with one 16-byte load that only needs 4-byte alignment, so any H >= 8 runs here: the last load of a column is moved
+// down to end inside it and its values are shifted back before they are used.
+#include "zr_internal.h"
+#include "zr_math.h"
+#include "zr_mfma_core.h"
+
+namespace {
+
+constexpr int kWaves = 8;
+constexpr int kRedLd = 36;  // LDS row of 32 partial sums, padded
+
+struct LstmRows {
+  const float* W;      // [nseg][4] packed fp32 matrices
+  const float* bias;   // [4][H]
+  const float* in[3];  // segment inputs, columns of H floats
+  const int* ids;      // non-null: column n of segment 0 is in[0] + clamp(ids[n]) * H
+  const float* cprev;
+  const int* mask01;
+  float *h, *c;
+  float* gates[4];     // all null or all non-null
+  float* hp;           // optional: h also k-interleaved, [H/4][mb][4]
+  int nseg, V, H, mb, ldw, kp, j_tiles, n_tiles;
+  float clip;
+};
+
+typedef zr_f32x4 zr_f32x4_u __attribute__((aligned(4)));
+
+// NARROW: 16 columns on the 16 x 16 x 4 instruction; else TN tiles of 32 columns on the 32 x 32 x 2 one (ROWS = 8).
+template <int ROWS, int TN, bool NARROW>
+__global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
+  static_assert(NARROW ? TN == 1 : ROWS == 8, "tile shape");
+  constexpr int KB = NARROW ? 4 : 2;            // k-blocks of 4 per k-group
+  constexpr int NB = NARROW ? ROWS / 4 : 1;     // weight sub-tiles
+  constexpr int COLS = NARROW ? 16 : 32 * TN;
+  constexpr int NOUT = (ROWS * COLS + 511) / 512;
+  constexpr int PF = NARROW || TN == 2 ? 8 : 10;  // k-groups in flight
+  constexpr int NS = PF + 1;
+  __shared__ float red[kWaves * COLS * kRedLd];
+  // Workgroup ids congruent mod 8 share a die: the column tiles of a row tile, which read the same weights, go together.
+  const int id = blockIdx.x;
+  const int jt = (id / (8 * P.n_tiles)) * 8 + (id & 7);
+  const int nt = (id >> 3) % P.n_tiles;
+  if (jt >= P.j_tiles) return;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int kslice = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int H = P.H, mb = P.mb;
+  const int j0 = jt * ROWS;
+  const int n0 = nt * COLS;
+  const int cl = NARROW ? (lane & 15) : (lane & 31);
+  const int kq = NARROW ? (lane >> 4) : (lane >> 5);
+
+  // the outputs this thread finishes; their operands are fetched ahead of the K loop
+  int oj[NOUT], on[NOUT];
+  bool ok[NOUT];
+  float bi[NOUT], bf[NOUT], bc[NOUT], bo[NOUT], cprev_v[NOUT], mask_v[NOUT];
+#pragma unroll
+  for (int u = 0; u < NOUT; ++u) {
+    const int o = tid + 512 * u;
+    oj[u] = o % ROWS;
+    on[u] = o / ROWS;
+    const int j = j0 + oj[u], n = n0 + on[u];
+    ok[u] = o < ROWS * COLS && n < mb && j < H;
+    const int jc = j < H ? j : H - 1, nc = n < mb ? n : mb - 1;
+    bi[u] = P.bias[jc], bf[u] = P.bias[H + jc], bc[u] = P.bias[2 * H + jc], bo[u] = P.bias[3 * H + jc];
+    cprev_v[u] = P.cprev[(long long)nc * H + jc];
+    mask_v[u] = (float)P.mask01[nc];
+  }
+
+  // this lane's columns and weight rows
+  long long col_off[TN], col_off0[TN];
+#pragma unroll
+  for (int tn = 0; tn < TN; ++tn) {
+    int c = n0 + tn * 32 + cl;
+    c = c < mb ? c : mb - 1;
+    col_off[tn] = (long long)c * H;
+    col_off0[tn] = col_off[tn];
+    if (P.ids) {
+      const int v = P.ids[c];
+      col_off0[tn] = (long long)(v < 0 ? 0 : (v >= P.V ? P.V - 1 : v)) * H;
+    }
+  }
+  const long long HH = (long long)P.kp * P.ldw;
+  unsigned woff[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int c = cl + 16 * b;
+    woff[b] = (unsigned)((c / ROWS) * HH + 4 * (j0 + c % ROWS));
+  }
+  const int G = (P.kp + 4 * KB - 1) / (4 * KB);  // k-groups per segment
+  const int total = P.nseg * G;
+  const int kb_max = (P.kp >> 2) - 1;
+
+  struct Frag {
+    zr_f32x4 w[NB], x[TN];
+  };
+  Frag f[NS];
+  // The k-groups of all segments in one row, dealt to the waves in turn: group r is (segment r / G, group r % G).
+  int ls = kslice / G, lg = kslice - ls * G, lr = kslice;  // the next group to load
+  auto load = [&](Frag& q) {
+    const float* Ws = P.W + 4 * HH * ls;
+    const int kb = KB * lg + kq;
+    const int kbc = NARROW && kb > kb_max ? kb_max : kb;  // (a narrow group may be half: its x is zero there)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) q.w[b] = *(const zr_f32x4*)(Ws + (woff[b] + (unsigned)(kbc * 4 * P.ldw)));
+    const int k0 = 4 * kb;
+    const int ks = k0 < H - 4 ? k0 : H - 4;
+    const float* xs = P.in[ls];
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) q.x[tn] = *(const zr_f32x4_u*)(xs + ((ls == 0 ? col_off0[tn] : col_off[tn]) + ks));
+    // past the end: the last group again (not multiplied)
+    if (lr + kWaves < total) {
+      lr += kWaves;
+      lg += kWaves;
+      while (lg >= G) lg -= G, ++ls;
+    }
+  };
+  typedef float acc16 __attribute__((ext_vector_type(16)));
+  acc16 acc[TN];
+  zr_f32x4 acc4[NB];
+#pragma unroll
+  for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[tn][r] = 0.0f;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) acc4[b] = {0.0f, 0.0f, 0.0f, 0.0f};
+  int mg = kslice % G;  // the group (inside its segment) multiplied next
+  auto mma = [&](Frag& q) {
+    if (4 * KB * (mg + 1) > H) {  // the column ends inside this group: shift the moved loads back, zero what lies behind
+      const int k0 = 4 * (KB * mg + kq);
+      const int d = k0 < H - 4 ? 0 : k0 - (H - 4);
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) {
+        const zr_f32x4 v = q.x[tn];
+        q.x[tn][0] = d == 0 ? v[0] : (d == 1 ? v[1] : (d == 2 ? v[2] : (d == 3 ? v[3] : 0.0f)));
+        q.x[tn][1] = d == 0 ? v[1] : (d == 1 ? v[2] : (d == 2 ? v[3] : 0.0f));
+        q.x[tn][2] = d == 0 ? v[2] : (d == 1 ? v[3] : 0.0f);
+        q.x[tn][3] = d == 0 ? v[3] : 0.0f;
+      }
+    }
+    mg += kWaves;
+    while (mg >= G) mg -= G;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (NARROW) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc4[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x[0][e], q.w[b][e], acc4[b], 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+          acc[tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(q.x[tn][e], q.w[0][e], acc[tn], 0, 0, 0);
+      }
+    }
+  };
+  if (kslice < total) {
+    const int n_mine = (total - kslice + kWaves - 1) / kWaves;
+#pragma unroll
+    for (int s = 0; s < PF; ++s) load(f[s]);
+    int it = 0;
+    for (; it + NS <= n_mine; it += NS) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        load(f[(s + PF) % NS]);
+        mma(f[s]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < PF; ++s)
+      if (it + s < n_mine) mma(f[s]);
+  }
+
+  // partial sums of the K slices through LDS, then the cell
+  float* mine = red + kslice * (COLS * kRedLd);
+  if constexpr (NARROW) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mine[(4 * kq + r) * kRedLd + cl + 16 * b] = acc4[b][r];
+  } else {
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mine[(tn * 32 + 8 * (r >> 2) + 4 * kq + (r & 3)) * kRedLd + cl] = acc[tn][r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NOUT; ++u) {
+    if (!ok[u]) continue;
+    float z[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float* p = red + on[u] * kRedLd + g * ROWS + oj[u];
+      float sum = 0.0f;
+#pragma unroll
+      for (int q = 0; q < kWaves; ++q) sum += p[q * (COLS * kRedLd)];
+      z[g] = sum;
+    }
+    float gi, gf, gc, go, c, h;
+    zr_lstm_cell(z[0] + bi[u], z[1] + bf[u], z[2] + bc[u], z[3] + bo[u], cprev_v[u], mask_v[u], P.clip, gi, gf, gc, go, c, h);
+    const int j = j0 + oj[u], n = n0 + on[u];
+    const long long ix = (long long)n * H + j;
+    P.c[ix] = c;
+    P.h[ix] = h;
+    if (P.hp) P.hp[((long long)(j >> 2) * mb + n) * 4 + (j & 3)] = h;
+    if (P.gates[0]) P.gates[0][ix] = gi, P.gates[1][ix] = gf, P.gates[2][ix] = gc, P.gates[3][ix] = go;
+  }
+}
+
+}  // namespace
+
+// Tile by size, one node of H = 1000 / 500 / 300 at up to 128 columns, us (the register-streaming kernel of zr_lstm.hip
+// with K split across workgroups: 16-27 / 30-33 / 23-30):
+//   4 x 16:  13.0 at 12 columns /  6.4 at 12, 8.6 at 37 /  5.5 at 20      8 x 16:  11.5 at 12, 12.0 at 32 / 7.4 at 37 / 6.1
+//   8 x 32:  17.0 at 64 / 11.7 at 128 / 7.7 at 100                        8 x 64:  26.5 at 128 (26.7) / 16.8 at 128
+// The smallest tile that keeps the workgroups within one per compute unit wins, except that 4 x 16 tiles of H > 512 read the
+// activations once too often (13.0 against 11.5).  Wide tiles of a long K range lose to the streaming kernel (H = 2000, 64
+// columns: 71 against 48), and so does any that needs a second round of workgroups (H = 1000, 192 columns: 42-65 against
+// 37) -- where that kernel has its whole-group form, H % 8 == 0.
+int zr_lstm_rows_shape(int H, int mb, int cu_count) {
+  if (H < 8) return -1;
+  for (int shape = H > 512 ? 1 : 0; shape < 4; ++shape) {
+    const int rows = shape == 0 ? 4 : 8, cols = shape <= 1 ? 16 : (shape == 2 ? 32 : 64);
+    const long long wgs = (long long)((H + rows - 1) / rows) * ((mb + cols - 1) / cols);
+    if (wgs <= cu_count) return (shape >= 2 && H > 1024 && H % 8 == 0) ? -1 : shape;
+  }
+  return H % 8 == 0 ? -1 : 3;
+}
+
+int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const float* const in[3], const int* d_gather_ids,
+                      int V, const float* d_cprev, const int* d_mask01, float clip, int mb, float* d_h, float* d_c,
+                      float* const d_gates[4], float* d_hp, int shape) {
+  LstmRows P = {};
+  P.W = (const float*)w->d_W;
+  P.bias = w->d_bias;
+  for (int s = 0; s < nseg; ++s) P.in[s] = in[s];
+  P.ids = d_gather_ids;
+  P.cprev = d_cprev;
+  P.mask01 = d_mask01;
+  P.h = d_h;
+  P.c = d_c;
+  for (int g = 0; g < 4; ++g) P.gates[g] = d_gates ? d_gates[g] : nullptr;
+  P.hp = d_hp;
+  P.nseg = nseg;
+  P.V = V;
+  P.H = w->H;
+  P.mb = mb;
+  P.ldw = w->ldw;
+  P.kp = w->kp;
+  P.clip = clip;
+  const int rows = shape == 0 ? 4 : 8, cols = shape <= 1 ? 16 : (shape == 2 ? 32 : 64);
+  P.j_tiles = (P.H + rows - 1) / rows;
+  P.n_tiles = (mb + cols - 1) / cols;
+  const unsigned grid = (unsigned)((P.j_tiles + 7) / 8 * 8 * P.n_tiles);
+  if (shape == 0)
+    lstm_rows_kernel<4, 1, true><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+  else if (shape == 1)
+    lstm_rows_kernel<8, 1, true><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+  else if (shape == 2)
+    lstm_rows_kernel<8, 1, false><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+  else
+    lstm_rows_kernel<8, 2, false><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+  ZR_LAUNCH_CHECK("lstm_rows_kernel");
+  return ZR_OK;
+}

@@ -120,6 +120,11 @@ int zr_ctx_create(int device, zr_ctx** out) {
       return rc;
     }
   }
+  e = hipDeviceGetAttribute(&c->cu_count, hipDeviceAttributeMultiprocessorCount, device);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    c->cu_count = 256;
+  }
   c->lstm_fused = 1;
   // ZR_LSTM_SWEEP in the environment presets ZR_OPT_LSTM_SWEEP for every context of the process (0, 1 or 2): lets a
   // whole program, e.g. a test run, be put on one path or the other without touching its code
