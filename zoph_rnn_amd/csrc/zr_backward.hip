@@ -336,35 +336,50 @@ __global__ void sumsq_accumulate_kernel(const double* __restrict__ partial, int 
 // W += lr * clip(scale * g).  mode ZR_CLIP_MATRIX_NORM: the gradient is shrunk by threshold / ||scale * g|| when that norm
 // (from `partial`) exceeds threshold; ZR_CLIP_WHOLE_NORM: the same with the norm sqrt(*sumsq) the caller accumulated
 // over every gradient of the model; ZR_CLIP_ELEMENT: every element of scale * g is clamped to +-threshold.
+// vec: W and g 16-byte aligned.
 __global__ void __launch_bounds__(256) sgd_apply_kernel(float* __restrict__ W, const float* __restrict__ g, long long n,
-                                                        float scale, int mode, float threshold, float lr,
+                                                        int vec, float scale, int mode, float threshold, float lr,
                                                         const double* __restrict__ partial, int n_partial,
                                                         const double* __restrict__ sumsq) {
+  // Every workgroup adds the partial sums itself, its first wave four a lane and then across the lanes (a single thread
+  // running through all 256 took 15 us, three times the update of a 1000 x 1000 matrix).
   __shared__ float coef_s;
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {
     float coef = 1.0f;
     if (mode == ZR_CLIP_MATRIX_NORM) {
       double ss = 0.0;
-      for (int i = 0; i < n_partial; ++i) ss += partial[i];
+      for (int i = threadIdx.x; i < n_partial; i += 64) ss += partial[i];
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
       const float norm = (float)sqrt(ss) * fabsf(scale);
       if (norm > threshold) coef = threshold / norm;
     } else if (mode == ZR_CLIP_WHOLE_NORM) {
       const float norm = (float)sqrt(*sumsq);
       if (norm > threshold) coef = threshold / norm;
     }
-    coef_s = coef;
+    if (threadIdx.x == 0) coef_s = coef;
   }
   __syncthreads();
   const long long first = (long long)blockIdx.x * 256 + threadIdx.x, stride = (long long)gridDim.x * 256;
-  if (mode == ZR_CLIP_ELEMENT) {
-    for (long long i = first; i < n; i += stride) {
-      const float x = scale * g[i];
-      W[i] += lr * (x > threshold ? threshold : (x < -threshold ? -threshold : x));  // a NaN stays a NaN (clip_mat_kernel)
-    }
-    return;
-  }
   const float f = lr * coef_s * scale;
-  for (long long i = first; i < n; i += stride) W[i] += f * g[i];
+  auto updated = [&](float w, float x) {
+    if (mode != ZR_CLIP_ELEMENT) return w + f * x;
+    x *= scale;
+    return w + lr * (x > threshold ? threshold : (x < -threshold ? -threshold : x));  // a NaN stays a NaN (clip_mat_kernel)
+  };
+  long long done = 0;
+  if (vec) {
+    const long long n4 = n >> 2;
+    for (long long i = first; i < n4; i += stride) {
+      const zr_f32x4 x = ((const zr_f32x4*)g)[i];
+      zr_f32x4 w = ((zr_f32x4*)W)[i];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) w[c] = updated(w[c], x[c]);
+      ((zr_f32x4*)W)[i] = w;
+    }
+    done = n4 << 2;
+  }
+  for (long long i = done + first; i < n; i += stride) W[i] = updated(W[i], g[i]);
 }
 
 
@@ -1241,9 +1256,10 @@ int zr_sgd_update_clipped(zr_ctx* ctx, float* d_W, const float* d_grad, long lon
     sumsq_partial_kernel<<<n_partial, 1024, 0, ctx->stream>>>(d_grad, n, aligned16(d_grad) ? 1 : 0, (double*)scratch);
     ZR_LAUNCH_CHECK("sumsq_partial_kernel");
   }
-  const long long blocks = (n + 255) / 256;
+  const int vec = aligned16(d_W) && aligned16(d_grad) ? 1 : 0;
+  const long long blocks = ((vec ? (n + 3) / 4 : n) + 255) / 256;
   sgd_apply_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, ctx->stream>>>(
-      d_W, d_grad, n, scale, clip_mode, threshold, learning_rate, (const double*)scratch, n_partial, d_sumsq);
+      d_W, d_grad, n, vec, scale, clip_mode, threshold, learning_rate, (const double*)scratch, n_partial, d_sumsq);
   ZR_LAUNCH_CHECK("sgd_apply_kernel");
   return ZR_OK;
 }
