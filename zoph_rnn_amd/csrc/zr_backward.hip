@@ -155,13 +155,12 @@ __global__ void __launch_bounds__(256) lstm_node_backward_group_kernel(NodeBackw
 
 // Sum over the unmasked columns of log((double) p[target, column]): train_perplexity_kernel
 // (src/custom_kernels.h:478-488), one workgroup, fixed summation order.
-__global__ void __launch_bounds__(256) train_logprob_kernel(const float* __restrict__ prob, int V, int n,
-                                                            const int* __restrict__ target,
+__global__ void __launch_bounds__(256) train_logprob_kernel(const float* __restrict__ p_target, int n,
                                                             const int* __restrict__ mask01, double* __restrict__ out) {
   __shared__ double part[256];
   double s = 0.0;
   for (int i = threadIdx.x; i < n; i += 256)
-    if (mask01[i] == 1) s += log((double)prob[(size_t)i * V + target[i]]);
+    if (mask01[i] == 1) s += log((double)p_target[i]);
   part[threadIdx.x] = s;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
@@ -260,31 +259,6 @@ __global__ void __launch_bounds__(256) embed_grad_kernel(const float* __restrict
   int id = ids[k];
   id = id < 0 ? 0 : (id >= V ? V - 1 : id);
   atomicAdd(&dW[(size_t)id * H + j], err[(size_t)k * H + j]);
-}
-
-// p (V x n probabilities) -> e = onehot(target) - p on unmasked columns, 0 on masked ones, in place.
-// VEC: four consecutive rows per thread with 16-byte accesses (V % 4 == 0, p 16-byte aligned).
-template <bool VEC>
-__global__ void __launch_bounds__(256) softmax_error_kernel(float* __restrict__ p, int V, const int* __restrict__ target,
-                                                            const int* __restrict__ mask01) {
-  const int col = blockIdx.y;
-  const bool on = mask01[col] == 1;
-  const int tg = target[col];
-  if (VEC) {
-    const int v = (blockIdx.x * 256 + threadIdx.x) * 4;
-    if (v >= V) return;
-    zr_f32x4* q = (zr_f32x4*)(p + (size_t)col * V + v);
-    const zr_f32x4 x = *q;
-    zr_f32x4 e;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) e[c] = on ? (v + c == tg ? 1.0f : 0.0f) - x[c] : 0.0f;
-    *q = e;
-  } else {
-    const int v = blockIdx.x * 256 + threadIdx.x;
-    if (v >= V) return;
-    const size_t ix = (size_t)col * V + v;
-    p[ix] = on ? (v == tg ? 1.0f : 0.0f) - p[ix] : 0.0f;
-  }
 }
 
 // sum of squares, two deterministic stages.  1024 threads per block and 16-byte loads (when g is 16-byte aligned)
@@ -801,6 +775,25 @@ static int weight_gradients(zr_ctx* ctx, int H, int T, int mb, const float* d_dg
   const long long K = (long long)T * mb;
   ZR_CHECK_ARG(K < (1LL << 31) / 4, "zr_lstm_weight_gradients: T * mb = %lld too large", K);
   void* scratch = nullptr;
+  if (zr_split_gemm_takes(4 * H, H, (int)K)) {
+    // the split product reads both operands as they lie; the previous states [h0, h_1 .. h_{T-1}] side by side
+    const size_t first = sizeof(float) * (size_t)H * mb;
+    const float* h_prev = d_h0;
+    if (T > 1) {
+      rc = zr_ctx_scratch(ctx, 1, first * T, &scratch);
+      if (rc) return rc;
+      ZR_HIP(hipMemcpyAsync(scratch, d_h0, first, hipMemcpyDeviceToDevice, ctx->stream));
+      ZR_HIP(hipMemcpyAsync((char*)scratch + first, d_h_all, first * (T - 1), hipMemcpyDeviceToDevice, ctx->stream));
+      h_prev = (const float*)scratch;
+    }
+    rc = zr_split_gemm(ctx, 4 * H, H, (int)K, d_dgates, 4 * H, ZR_SPLIT_ROW_FAST, d_in_all, H, ZR_SPLIT_ROW_FAST, d_dM_stack,
+                       4 * H, nullptr, nullptr, accumulate);
+    if (rc) return rc;
+    rc = zr_split_gemm(ctx, 4 * H, H, (int)K, d_dgates, 4 * H, ZR_SPLIT_ROW_FAST, h_prev, H, ZR_SPLIT_ROW_FAST, d_dWh_stack,
+                       4 * H, nullptr, nullptr, accumulate);
+    if (rc) return rc;
+    return row_sum_launch(ctx, d_dgates, 4 * H, K, d_db, accumulate);
+  }
   rc = zr_ctx_scratch(ctx, 0, sizeof(float) * (size_t)K * H, &scratch);  // the transposed right-hand side, K x H
   if (rc) return rc;
   float* xt = (float*)scratch;
@@ -1118,38 +1111,48 @@ static int softmax_backward(zr_ctx* ctx, const float* d_D, const float* d_b_d, i
   ZR_CHECK_ARG(V > 0 && H > 0 && n > 0 && n <= 65535, "zr_softmax_backward: V = %d, H = %d, n = %d", V, H, n);
   ZR_CHECK_ARG(d_D && d_b_d && d_h && d_target && d_mask01 && d_prob_scratch && d_err_h && d_dD && d_db,
                "zr_softmax_backward: null pointer");
-  rc = zr_softmax_forward(ctx, d_D, d_b_d, V, H, d_h, n, ZR_SOFTMAX_PROB, d_prob_scratch, nullptr);
-  if (rc) return rc;
-  // err_h = D^T e, computed as (e^T D)^T: with e^T as the left operand the product is tall (n rows) with contiguous
-  // rows, the shape the large-matrix kernels are built for; the two transposes move 2 x V*n + 2 x n*H floats.
+  // logits, then in one pass over them the errors e = onehot - p (0 on masked columns), the sums of e over each chunk of
+  // columns and the targets' probabilities
+  const int chunks = zr_softmax_error_chunks(n);
   void *s0 = nullptr, *s1 = nullptr;
-  rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (size_t)V * n, &s1);
-  if (rc) return rc;
-  rc = zr_ctx_scratch(ctx, 0, sizeof(float) * (size_t)n * H + sizeof(double), &s0);
+  const size_t sums = ((size_t)V * chunks + 3) & ~(size_t)3;
+  const float* e = d_prob_scratch;
+  rc = zr_softmax_error(ctx, d_D, d_b_d, V, H, d_h, n, d_target, d_mask01, d_prob_scratch, sizeof(float) * (sums + n) + 16, &s0);
   if (rc) return rc;
   if (h_loss) {
-    // before the probabilities are turned into errors.  The cell is the head of scratch 0; the copy out is queued
-    // ahead of the kernels that reuse that buffer, and waited for at the end of this call.
-    train_logprob_kernel<<<1, 256, 0, ctx->stream>>>(d_prob_scratch, V, n, d_target, d_mask01, (double*)s0);
+    double* cell = (double*)((char*)s0 + ((sizeof(float) * (sums + n) + 7) & ~(size_t)7));
+    train_logprob_kernel<<<1, 256, 0, ctx->stream>>>((const float*)s0 + sums, n, d_mask01, cell);
     ZR_LAUNCH_CHECK("train_logprob_kernel");
-    ZR_HIP(hipMemcpyAsync(h_loss, s0, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    // queued ahead of the kernels that reuse that buffer, and waited for at the end of this call
+    ZR_HIP(hipMemcpyAsync(h_loss, cell, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   }
-  if (V % 4 == 0 && aligned16(d_prob_scratch)) {
-    dim3 egrid((V / 4 + 255) / 256, n);
-    softmax_error_kernel<true><<<egrid, 256, 0, ctx->stream>>>(d_prob_scratch, V, d_target, d_mask01);
-  } else {
-    dim3 egrid((V + 255) / 256, n);
-    softmax_error_kernel<false><<<egrid, 256, 0, ctx->stream>>>(d_prob_scratch, V, d_target, d_mask01);
+  row_sum_pass(ctx, (const float*)s0, V, chunks, chunks, d_db, accumulate);
+  ZR_LAUNCH_CHECK("row_sum_kernel");
+  const bool split_err = zr_split_gemm_takes(H, n, V), split_dD = zr_split_gemm_takes(V, H, n);
+  if (split_err) {
+    rc = zr_split_gemm(ctx, H, n, V, d_D, V, ZR_SPLIT_K_FAST, e, V, ZR_SPLIT_K_FAST, d_err_h, H, nullptr, nullptr, 0);
+    if (rc) return rc;
   }
-  ZR_LAUNCH_CHECK("softmax_error_kernel");
-  float* et = (float*)s1;   // n x V
-  float* ct = (float*)s0;   // n x H
+  if (split_dD) {
+    rc = zr_split_gemm(ctx, V, H, n, e, V, ZR_SPLIT_ROW_FAST, d_h, H, ZR_SPLIT_ROW_FAST, d_dD, V, nullptr, nullptr, accumulate);
+    if (rc) return rc;
+  }
   ZrGemmDesc g = {};
   g.nseg = 1;
   g.K[0] = V;
   g.batch = 1;
   g.epilogue = ZR_EPI_STORE;
-  if (n >= 1024) {
+  if (split_err) {
+    // done
+  } else if (n >= 1024) {
+    // D^T e, computed as (e^T D)^T: with e^T as the left operand the product is tall (n rows) with contiguous rows; the
+    // two transposes move 2 x V*n + 2 x n*H floats.
+    rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (size_t)V * n, &s1);
+    if (rc) return rc;
+    rc = zr_ctx_scratch(ctx, 0, sizeof(float) * (size_t)n * H, &s0);
+    if (rc) return rc;
+    float* et = (float*)s1;  // n x V
+    float* ct = (float*)s0;  // n x H
     rc = transpose_launch(ctx, d_prob_scratch, V, n, et, n, 0);
     if (rc) return rc;
     g.M = n;
@@ -1177,7 +1180,13 @@ static int softmax_backward(zr_ctx* ctx, const float* d_D, const float* d_b_d, i
     rc = zr_gemm_launch(ctx, g);
     if (rc) return rc;
   }
+  if (split_dD) {
+    if (h_loss) ZR_HIP(hipStreamSynchronize(ctx->stream));
+    return ZR_OK;
+  }
   // dD = e h^T : right-hand side h^T as an n x H column-major matrix
+  rc = zr_ctx_scratch(ctx, 0, sizeof(float) * (size_t)n * H, &s0);
+  if (rc) return rc;
   float* ht = (float*)s0;  // the product above has been queued: the buffer is free again in stream order
   rc = transpose_launch(ctx, d_h, H, n, ht, n, 0);
   if (rc) return rc;
@@ -1196,8 +1205,6 @@ static int softmax_backward(zr_ctx* ctx, const float* d_D, const float* d_b_d, i
   w.epilogue = ZR_EPI_STORE;
   w.accumulate = accumulate;
   rc = zr_gemm_launch(ctx, w);
-  if (rc) return rc;
-  rc = row_sum_launch(ctx, d_prob_scratch, V, n, d_db, accumulate);
   if (rc) return rc;
   if (h_loss) ZR_HIP(hipStreamSynchronize(ctx->stream));
   return ZR_OK;

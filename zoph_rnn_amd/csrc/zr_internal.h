@@ -183,6 +183,18 @@ static inline size_t zr_softmax_blocks_offset_floats(int V, int cols) { return (
 // softmax_colstats_kernel on [cols][nblocks][2] pairs -> colstats[cols][2] (zr_softmax.hip)
 int zr_softmax_colstats_launch(zr_ctx* ctx, const float* d_partials, int nblocks, int cols, float* d_colstats);
 
+// Large fp32 products on the bf16 matrix cores, every operand as three bf16 terms (zr_split_gemm.hip):
+// C = A B (+ bias[m]) (+ C when accumulate); partials non-null: the soft-max-partial epilogue of ZrGemmDesc instead.
+// `a` and `b` say where an operand's element (row, k) lies (a row of B is a column of C).  May use scratch slot 0.
+enum ZrSplitLayout {
+  ZR_SPLIT_K_FAST = 0,    // [row*ld + k]
+  ZR_SPLIT_ROW_FAST = 1,  // [row + k*ld]
+  ZR_SPLIT_PACK4 = 2      // the k-interleaved fp32 copy (ZrGemmDesc::a_pack = 1); A only, with B ZR_SPLIT_K_FAST
+};
+bool zr_split_gemm_takes(int M, int N, int K);  // whether a product of this size is faster that way
+int zr_split_gemm(zr_ctx* ctx, int M, int N, int K, const float* A, long long lda, int a_layout, const float* B,
+                  long long ldb, int b_layout, float* C, long long ldc, const float* bias, float* partials, int accumulate);
+
 struct zr_lstm_weights {
   int H;
   int nseg;        // 2 (M, Wh) or 3 (+Q)
@@ -209,6 +221,13 @@ int zr_lstm_decoder_step_packed(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
 int zr_softmax_forward_packed(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, int H, const float* d_h,
                               const float* d_h_packed, int mb, int mode, float* d_out, float* d_logits_scratch,
                               const unsigned short* d_h_hi = nullptr, const unsigned short* d_h_lo = nullptr);
+
+// The output layer's errors: logits into d_out, then in place e = onehot(target) - p, 0 on masked columns.  Scratch slot 0,
+// of at least `bytes` (handed back in *out), starts with the sums of e over chunks of columns, [zr_softmax_error_chunks(n)]
+// [V], and, V * chunks rounded up to 4 floats on, the probability of every column's target.
+int zr_softmax_error_chunks(int n);
+int zr_softmax_error(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, int H, const float* d_h, int n,
+                     const int* d_target, const int* d_mask01, float* d_out, size_t bytes, void** out);
 
 // The whole sweep with the weights held in registers (zr_lstm_resident.hip), as one launch or, when not all layers fit on
 // the device at once, a few.  The plan: which kernel, how many layers a launch; its value is the estimated time in us

@@ -57,6 +57,42 @@ softmax_normalize_kernel(const float* in, float* out, int V, const float* __rest
   }
 }
 
+// x (V x n logits) -> e = onehot(target) - p in place, p = exp(x - max) / sum as softmax_normalize_kernel has it, 0 on masked
+// columns; the sums of e over the workgroup's ERROR_COLS columns to sums[blockIdx.y][V], and every column's target
+// probability.  The three readers of the probabilities (errors, gradient of the bias, loss) were passes of their own over
+// the matrix: at 50000 x 6400 normalise 483, error 499, bias sums 250 us, bound by memory; this pass reads and writes once.
+// VEC: four consecutive rows per thread with 16-byte accesses (V % 4 == 0, x and sums 16-byte aligned).
+constexpr int ERROR_COLS = 32;
+template <bool VEC>
+__global__ void __launch_bounds__(256)
+softmax_error_kernel(float* __restrict__ x, int V, int n, const float* __restrict__ colstats, const int* __restrict__ target,
+                     const int* __restrict__ mask01, float* __restrict__ sums, float* __restrict__ p_target) {
+  constexpr int W = VEC ? 4 : 1;
+  typedef float vec __attribute__((ext_vector_type(W)));
+  const int v = (blockIdx.x * 256 + threadIdx.x) * W;
+  if (v >= V) return;
+  const int n0 = blockIdx.y * ERROR_COLS, n1 = min(n, n0 + ERROR_COLS);
+  vec s = {};
+#pragma unroll 4
+  for (int c = n0; c < n1; ++c) {
+    vec* q = (vec*)(x + (size_t)c * V + v);
+    const vec in = *q;
+    const float mx = colstats[2 * c], sum = colstats[2 * c + 1];
+    const bool on = mask01[c] == 1;
+    const int tg = min(max(target[c], 0), V - 1);
+    vec e;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const float p = expf(in[i] - mx) / sum;
+      if (v + i == tg) p_target[c] = p;
+      e[i] = on ? (v + i == target[c] ? 1.0f : 0.0f) - p : 0.0f;
+    }
+    *q = e;
+    s += e;
+  }
+  *(vec*)(sums + (size_t)blockIdx.y * V + v) = s;
+}
+
 // Double-precision column statistics straight from the logits (outputdist_perplexity_kernel accumulates in
 // double, reference: src/custom_kernels.h:583-660).  One workgroup per column, two passes over the column.
 __global__ void __launch_bounds__(256)
@@ -329,6 +365,32 @@ int zr_softmax_forward_packed(zr_ctx* ctx, const float* d_D, const float* d_b_d,
       softmax_normalize_kernel<1, false><<<grid, 256, 0, ctx->stream>>>(logits, d_out, V, colstats);
   }
   ZR_LAUNCH_CHECK("softmax_normalize_kernel");
+  return ZR_OK;
+}
+
+int zr_softmax_error_chunks(int n) { return (n + ERROR_COLS - 1) / ERROR_COLS; }
+
+int zr_softmax_error(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, int H, const float* d_h, int n,
+                     const int* d_target, const int* d_mask01, float* d_out, size_t bytes, void** out) {
+  float* partials = nullptr;
+  int nblocks = 0;
+  int rc = logits_with_partials(ctx, d_D, d_b_d, V, H, d_h, n, d_out, &partials, &nblocks);
+  if (rc) return rc;
+  float* colstats = (float*)stats_ptr(partials, nblocks, n);
+  softmax_colstats_kernel<<<n, 256, 0, ctx->stream>>>(partials, nblocks, colstats);
+  ZR_LAUNCH_CHECK("softmax_colstats_kernel");
+  rc = zr_ctx_scratch(ctx, 0, bytes, out);
+  if (rc) return rc;
+  float* sums = (float*)*out;
+  float* p_target = sums + (((size_t)V * zr_softmax_error_chunks(n) + 3) & ~(size_t)3);
+  if (V % 4 == 0 && (((uintptr_t)d_out & 15u) == 0)) {
+    const dim3 grid((V / 4 + 255) / 256, zr_softmax_error_chunks(n));
+    softmax_error_kernel<true><<<grid, 256, 0, ctx->stream>>>(d_out, V, n, colstats, d_target, d_mask01, sums, p_target);
+  } else {
+    const dim3 grid((V + 255) / 256, zr_softmax_error_chunks(n));
+    softmax_error_kernel<false><<<grid, 256, 0, ctx->stream>>>(d_out, V, n, colstats, d_target, d_mask01, sums, p_target);
+  }
+  ZR_LAUNCH_CHECK("softmax_error_kernel");
   return ZR_OK;
 }
 
