@@ -121,6 +121,24 @@ class DeviceArray:
             _chk(load().zr_memset_zero(ctx.h, C.c_void_p(self.ptr), C.c_size_t((self.nbytes + 3) // 4 * 4)))
 
     @classmethod
+    def block(cls, ctx, specs):
+        """Arrays of the given (shape, dtype), side by side in one allocation, each 256-byte aligned; the allocation lives
+        as long as any of them."""
+        arrays, offset = [], 0
+        for shape, dtype in specs:
+            d = cls.__new__(cls)
+            d.ctx, d.shape, d.dtype = ctx, tuple(int(s) for s in shape), np.dtype(dtype)
+            d.nbytes = int(np.prod(d.shape, dtype=np.int64)) * d.dtype.itemsize
+            d.ptr, d._owned = offset, False
+            offset += (max(d.nbytes, 4) + 255) // 256 * 256
+            arrays.append(d)
+        whole = cls(ctx, (offset,), np.uint8)
+        for d in arrays:
+            d.ptr += whole.ptr
+            d._block = whole
+        return arrays
+
+    @classmethod
     def from_numpy(cls, ctx, a, dtype=None):
         a = np.asarray(a, dtype=dtype if dtype is not None else a.dtype)
         d = cls(ctx, a.shape, a.dtype)
@@ -196,6 +214,9 @@ class Context:
 
     def empty(self, shape, dtype=np.float32):
         return DeviceArray(self, shape, dtype)
+
+    def block(self, specs):
+        return DeviceArray.block(self, specs)
 
     def zeros(self, shape, dtype=np.float32):
         return DeviceArray(self, shape, dtype, zero=True)

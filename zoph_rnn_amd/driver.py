@@ -51,27 +51,39 @@ class BeamDecode:
         self.D = attention_D
         self.max_len = max_steps + 3
         H, cols, L = w.H, self.cols, w.L
-        self.tables = [ctx.empty((H, cols)) for _ in range(src_len)]
+        off = capi.softmax_blocks_offset(w.Vt, cols)
+        # Everything in one allocation: as arrays of their own (88 for 16 sentences of 50 words) giving them back took 8 ms
+        # of the 37 ms of a translation.
+        n_src = n_sent * src_len
+        state, i32 = ((H, cols), np.float32), np.int32
+        arrays = iter(ctx.block([state] * (src_len + 4 * L + 2) + [((H * n_src,), np.float32)] * (2 * L) +
+                                [((H, n_sent), np.float32), ((off + 2 * capi.softmax_block_count(w.Vt) * cols,), np.float32)] +
+                                [((cols,), i32)] * 5 + [((2 * cols,), i32)] + [((n_src,), i32)] * 3))
+
+        def take(n):
+            return [next(arrays) for _ in range(n)]
+
+        self.tables = take(src_len)
         self.attn = ctx.attn_create(H, cols, attention_D, w.attn["W_a"], w.attn["W_p"], w.attn["v_p"],
                                     w.attn["out_bias"], w.attn["W_c1"], w.attn["W_c2"], self.tables)
         ctx.attn_prepare(self.attn)
         self.bm = ctx.beam_create(beam, w.Vt, n_sent, self.max_len, penalty)
-        self.h = [[ctx.empty((H, cols)) for _ in range(L)] for _ in range(2)]  # ping-pong: previous / new state
-        self.c = [[ctx.empty((H, cols)) for _ in range(L)] for _ in range(2)]
-        self.h_tild = [ctx.empty((H, cols)) for _ in range(2)]
-        self.x = ctx.empty((H, cols))
+        self.h, self.c = [take(L) for _ in range(2)], [take(L) for _ in range(2)]  # ping-pong: previous / new state
+        self.h_tild = take(2)
+        self._h_all, self._c_all = take(L), take(L)
+        self._zero, self.logits = take(2)
+        self.d_words, self.d_words_nn, self.d_back, self.d_ones, self._rep = take(5)
+        self.d_batch_info, self._ids, self._nn, self._mask = take(4)
+        ctx.memset_zero(self._zero)
         # the logits and, behind them, the output product's (max, sum exp) pair per 32-row block and column
         # (ZR_SOFTMAX_LOGITS_BLOCKS): the beam folds the pairs itself, reads only the blocks that can hold one of a
         # column's beam + 1 largest entries and normalises only what it selects -- no probability matrix is written,
         # and the logits are not read again as a whole
-        off = capi.softmax_blocks_offset(w.Vt, cols)
-        self.logits = ctx.empty((off + 2 * capi.softmax_block_count(w.Vt) * cols,))
         self.blocks = self.logits.at(off)
-        self.d_words = ctx.array(np.zeros(cols, np.int32))  # <START> = 0
-        self.d_words_nn = ctx.array(np.zeros(cols, np.int32))
+        self.d_words.set(np.zeros(cols, np.int32))  # <START> = 0
+        self.d_words_nn.set(np.zeros(cols, np.int32))
         ctx.beam_set_input_ids(self.bm, self.d_words_nn)
-        self.d_back = ctx.empty(cols, np.int32)
-        self.d_ones = ctx.array(np.ones(cols, np.int32))
+        self.d_ones.set(np.ones(cols, np.int32))
         self.cur = 0
         self.step_index = 0
         self.history = []
@@ -80,16 +92,14 @@ class BeamDecode:
         """src_ids: (S, n_sent) time-major, reversed and left padded with -1 as the reference lays sources out."""
         ctx, w, S, n_sent, beam = self.ctx, self.w, self.S, self.n_sent, self.beam
         H, L = w.H, w.L
-        ids = np.ascontiguousarray(src_ids, np.int32)
-        d_nn, d_m = ctx.empty(ids.size, np.int32), ctx.empty(ids.size, np.int32)
-        ctx.vocab_prep(ctx.array(ids.reshape(-1)), ids.size, w.Vs, d_nn, d_m)
-        z = ctx.zeros((H, n_sent))
-        h_all = [ctx.empty((H * n_sent * S,)) for _ in range(L)]
-        c_all = [ctx.empty((H * n_sent * S,)) for _ in range(L)]
+        d_nn, d_m, z, h_all, c_all = self._nn, self._mask, self._zero, self._h_all, self._c_all
+        self._ids.set(np.ascontiguousarray(src_ids, np.int32).reshape(-1))
+        ctx.vocab_prep(self._ids, S * n_sent, w.Vs, d_nn, d_m)
         ctx.lstm_stack_forward(w.src, w.src_embed, w.Vs, d_nn, d_m, S, n_sent, [z] * L, [z] * L, h_all, c_all)
         # every sentence's states replicated over its beam columns (forward_prop_source, src/model.hpp:2394-2445,
         # and transfer_decoding_states_GPU for the final state of each layer)
-        rep = ctx.array(np.repeat(np.arange(n_sent, dtype=np.int32), beam))
+        rep = self._rep
+        rep.set(np.repeat(np.arange(n_sent, dtype=np.int32), beam))
         n = H * n_sent
         for t in range(S):
             ctx.gather_columns(h_all[L - 1].at(t * n), H, rep, self.cols, self.tables[t])
@@ -97,9 +107,8 @@ class BeamDecode:
             ctx.gather_columns(h_all[l].at((S - 1) * n), H, rep, self.cols, self.h[0][l])
             ctx.gather_columns(c_all[l].at((S - 1) * n), H, rep, self.cols, self.c[0][l])
         lens = np.repeat(np.asarray(src_lens, np.int32), beam)
-        self.d_batch_info = ctx.array(np.concatenate([lens, S - lens]).astype(np.int32))
+        self.d_batch_info.set(np.concatenate([lens, S - lens]).astype(np.int32))
         ctx.sync()
-        self._enc_keep = (h_all, c_all, d_nn, d_m, z, rep)
 
     def _forward(self):
         """forward_prop_target (src/model.hpp:2573-2688): new state into the other ping-pong half, logits and their per-block pairs."""
