@@ -41,15 +41,19 @@ struct SplitArgs {
 constexpr int KC = 32;  // k values per step
 constexpr int TM = 128; // rows of a workgroup's tile
 
-// One operand in LDS: [term][k-group of 8][row], 16 bytes an item; four spare items keep the k-groups on different banks.
+// One operand in LDS: [term][k-group of 8][row], 16 bytes an item.
 template <int ROWS>
 struct Oper {
-  static constexpr int KG = ROWS + 4, TERM = 4 * KG, SIZE = 3 * TERM;
+  static constexpr int KG = ROWS, TERM = 4 * KG, SIZE = 3 * TERM;
 };
 
-// Where row r of an operand's tile lies inside a k-group: the low two bits are turned by (r / 16) % 4, so that threads
-// that each store one row of four (rows 4q + j, one j at a time) hit different banks; 16 neighbouring rows still do.
-__device__ __forceinline__ int lds_row(int r) { return (r & ~3) | ((r + (r >> 4)) & 3); }
+// Where row r of an operand's tile lies inside a k-group.  The low two bits are turned by (r / 16) % 4, so that threads
+// that each store one row of four (rows 4q + j, one j at a time) hit different banks.  The k-groups are turned against each
+// other by 8 and 4 items: a read of a fragment serves rows of two neighbouring k-groups at a time (one per half of the
+// wave; with the groups 4 items apart half of every read met a conflict), a store threads of all four.
+__device__ __forceinline__ int lds_row(int r, int kg) {
+  return ((r & ~3) | ((r + (r >> 4)) & 3)) ^ (8 * (kg & 1) + 4 * (kg >> 1));
+}
 
 // One operand's share of a step, ROWS rows x 32 k, by 256 threads.
 // ZR_SPLIT_K_FAST:   element (row, k) at p[row*ld + k]; a thread holds k-group t%4 of rows t/4 + 64*i, v[2*i + k%8/4][k%4].
@@ -121,7 +125,8 @@ __device__ __forceinline__ void load_operand(f32x4u (&v)[ROWS / 32], const float
 // Two values' leading bf16 terms (rounded to nearest) in one register; the values become what is left of them.
 __device__ __forceinline__ unsigned next_terms(float& a, float& b) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  const unsigned t = __builtin_bit_cast(unsigned, bf16x2{(__bf16)a, (__bf16)b});
+  unsigned t = __builtin_bit_cast(unsigned, bf16x2{(__bf16)a, (__bf16)b});
+  asm("" : "+v"(t));  // one conversion for both values: without this the compiler converts one of them a second time
   a -= __uint_as_float(t << 16);
   b -= __uint_as_float(t & 0xffff0000u);
   return t;
@@ -133,8 +138,8 @@ __device__ __forceinline__ void store_operand(u32x4* s, const f32x4u (&v)[ROWS /
   if (LAYOUT != ZR_SPLIT_ROW_FAST) {
 #pragma unroll
     for (int i = 0; i < ROWS / 64; ++i) {
-      u32x4* d = LAYOUT == ZR_SPLIT_PACK4 ? s + (t >> 6) * O::KG + lds_row((t & 63) + 64 * i)
-                                          : s + (t & 3) * O::KG + lds_row((t >> 2) + 64 * i);
+      u32x4* d = LAYOUT == ZR_SPLIT_PACK4 ? s + (t >> 6) * O::KG + lds_row((t & 63) + 64 * i, t >> 6)
+                                          : s + (t & 3) * O::KG + lds_row((t >> 2) + 64 * i, t & 3);
       u32x4 term[3];
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
@@ -150,7 +155,7 @@ __device__ __forceinline__ void store_operand(u32x4* s, const f32x4u (&v)[ROWS /
     for (int i = 0; i < ROWS / 128; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        u32x2* d = (u32x2*)(s + (t >> 6) * O::KG + lds_row(4 * ((t >> 1) & 31) + 128 * i + e)) + (t & 1);
+        u32x2* d = (u32x2*)(s + (t >> 6) * O::KG + lds_row(4 * ((t >> 1) & 31) + 128 * i + e, t >> 6)) + (t & 1);
         u32x2 term[3];
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
@@ -236,11 +241,11 @@ __global__ void __launch_bounds__(256, TNW == 2 ? 3 : 2) split_gemm_kernel(Split
 
   f32x4u va[TM / 32], vb[TN / 32];
   const int wm = 64 * (wave & 1), wn = 32 * TNW * (wave >> 1);
-  int ra[2], rb[TNW];
+  int ra[2], rb[TNW];  // of k-groups 0 and 1; those of 2 and 3 are turned by another 4 items
 #pragma unroll
-  for (int i = 0; i < 2; ++i) ra[i] = half * OA::KG + lds_row(wm + 32 * i + jl);
+  for (int i = 0; i < 2; ++i) ra[i] = half * OA::KG + lds_row(wm + 32 * i + jl, half);
 #pragma unroll
-  for (int j = 0; j < TNW; ++j) rb[j] = OA::SIZE + half * OB::KG + lds_row(wn + 32 * j + jl);
+  for (int j = 0; j < TNW; ++j) rb[j] = OA::SIZE + half * OB::KG + lds_row(wn + 32 * j + jl, half);
   load_operand<TM, AL>(va, a.A, a.lda, m0, a.M, k_begin, k_end, tid);
   load_operand<TN, BL>(vb, a.B, a.ldb, n0, a.N, k_begin, k_end, tid);
   for (int k0 = k_begin; k0 < k_end; k0 += KC) {
@@ -258,12 +263,12 @@ __global__ void __launch_bounds__(256, TNW == 2 ? 3 : 2) split_gemm_kernel(Split
 #pragma unroll
       for (int q = 2; q >= 0; --q)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) x[i][q] = __builtin_bit_cast(bf16x8, s[ra[i] + q * OA::TERM + 2 * st * OA::KG]);
+        for (int i = 0; i < 2; ++i) x[i][q] = __builtin_bit_cast(bf16x8, s[(ra[i] ^ (4 * st)) + q * OA::TERM + 2 * st * OA::KG]);
 #pragma unroll
       for (int j = 0; j < TNW; ++j) {
         bf16x8 y[3];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) y[q] = __builtin_bit_cast(bf16x8, s[rb[j] + q * OB::TERM + 2 * st * OB::KG]);
+        for (int q = 0; q < 3; ++q) y[q] = __builtin_bit_cast(bf16x8, s[(rb[j] ^ (4 * st)) + q * OB::TERM + 2 * st * OB::KG]);
         constexpr int P[6] = {2, 0, 1, 1, 0, 0}, Q[6] = {0, 2, 1, 0, 1, 0};  // the smallest products first
 #pragma unroll
         for (int p = 0; p < 6; ++p)
