@@ -247,6 +247,62 @@ __global__ void __launch_bounds__(256) row_sum_kernel(const float* __restrict__ 
   }
 }
 
+// C_g (M x N) += A_g (M x K) B_g^T for up to two independent problems (blockIdx.z), all column-major without padding: the
+// weight gradients of a single attention or feed-input node, K = the minibatch.  Both operands have their rows contiguous
+// for every k, which is how the matrix instruction wants them: a half-wave reads 32 rows of one column, no transpose and no
+// LDS.  A wave has a 32 x 32 tile, A's rows on the lanes so that C is read and written 32 consecutive floats at a time.
+// Bound by the trip to memory for the operands and C, and by the launch.
+// Two of 500 x 500 at 64 columns 7.1 us, the launch included; the 20 target nodes of an encoder-decoder training step (2 x 500,
+// 64 columns) took 9.15 ms with a transpose and a tiled product each, 8.35 with this (W_c1^T e and W_c2^T e joined as well).
+struct OuterProducts {
+  const float* A[2];
+  const float* B[2];
+  float* C[2];
+};
+__global__ void __launch_bounds__(256) outer_accumulate_kernel(OuterProducts P, int M, int N, int K) {
+  constexpr int U = 16;  // instructions (of two k) a round; the next round's operands are in flight meanwhile
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, half = lane >> 5;
+  const int m0 = blockIdx.x * 64 + 32 * (wave & 1), n0 = blockIdx.y * 64 + 32 * (wave >> 1);
+  if (m0 >= M || n0 >= N) return;
+  const int m = m0 + r;
+  const float* a = P.A[blockIdx.z] + (m < M ? m : M - 1);
+  const float* b = P.B[blockIdx.z] + (n0 + r < N ? n0 + r : N - 1);
+  float* c = P.C[blockIdx.z] + m;
+  float av[U], bv[U];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + 2 * u + half;
+      const bool in = k < K;
+      const size_t at = (size_t)(in ? k : K - 1);
+      const float x = a[at * M], y = b[at * N];
+      av[u] = in ? x : 0.0f;
+      bv[u] = in ? y : 0.0f;
+    }
+  };
+  fetch(0);
+  float old[16];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int n = n0 + 8 * (q >> 2) + 4 * half + (q & 3);
+    old[q] = m < M && n < N ? c[(size_t)n * M] : 0.0f;
+  }
+  zr_f32x16 acc = {};
+  for (int k0 = 0; k0 < K; k0 += 2 * U) {
+    float ac[U], bc[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) ac[u] = av[u], bc[u] = bv[u];
+    if (k0 + 2 * U < K) fetch(k0 + 2 * U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(bc[u], ac[u], acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int n = n0 + 8 * (q >> 2) + 4 * half + (q & 3);
+    if (m < M && n < N) c[(size_t)n * M] = old[q] + acc[q];
+  }
+}
+
 // Embedding gradient: column id[k] of dW += err column k for every unmasked position.  Float atomics: the order of
 // the additions into one column is not fixed (the reference's sparse W gradient kernels use atomicAdd as well).
 __global__ void __launch_bounds__(256) embed_grad_kernel(const float* __restrict__ err, const int* __restrict__ ids,
@@ -551,6 +607,16 @@ int row_sum_launch(zr_ctx* ctx, const float* a, int rows, long long n, float* ou
     row_sum_pass(ctx, (const float*)scratch, rows, chunks, chunks, out, accumulate);
   }
   ZR_LAUNCH_CHECK("row_sum_kernel");
+  return ZR_OK;
+}
+
+// outer_accumulate_kernel's range: at 256 columns its lead over a transpose and the LDS-tiled product is nearly gone for the
+// stacked (4H x H) gradient (H = 1000, zr_lstm_feed_backward, us: 128 columns 61 / 79, 256 86 / 88).
+bool outer_takes(int M, int N, int K) { return K <= 256 && !zr_split_gemm_takes(M, N, K); }
+
+int outer_launch(zr_ctx* ctx, const OuterProducts& P, int count, int M, int N, int K) {
+  outer_accumulate_kernel<<<dim3((M + 63) / 64, (N + 63) / 64, count), 256, 0, ctx->stream>>>(P, M, N, K);
+  ZR_LAUNCH_CHECK("outer_accumulate_kernel");
   return ZR_OK;
 }
 
@@ -983,11 +1049,34 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
 
   attn_bwd_e_kernel<<<eg, 256, 0, ctx->stream>>>(d_err_htild, d_h_tild, d_mask01, H, (long long)n, e);
   ZR_LAUNCH_CHECK("attn_bwd_e_kernel");
-  if ((rc = outer_acc(e, d_c_t, grads->d_W_c1))) return rc;                     // :437
-  if ((rc = outer_acc(e, d_h_t, grads->d_W_c2))) return rc;                     // :443
+  const bool outer = outer_takes(H, H, mb);
+  if (outer) {
+    rc = outer_launch(ctx, OuterProducts{{e, e}, {d_c_t, d_h_t}, {grads->d_W_c1, grads->d_W_c2}}, 2, H, H, mb);
+    if (rc) return rc;
+  } else {
+    if ((rc = outer_acc(e, d_c_t, grads->d_W_c1))) return rc;                   // :437
+    if ((rc = outer_acc(e, d_h_t, grads->d_W_c2))) return rc;                   // :443
+  }
   if ((rc = row_sum_launch(ctx, e, H, mb, grads->d_out_bias, 1))) return rc;    // :456
-  if ((rc = product(a->W_c1, 1, e, err_ct, 0, ZR_EPI_STORE))) return rc;        // :464
-  if ((rc = product(a->W_c2, 1, e, d_err_h_t, 0, ZR_EPI_STORE))) return rc;     // :476
+  {
+    // W_c1^T e and W_c2^T e (:464, :476), one launch
+    ZrGemmDesc g = {};
+    g.M = H;
+    g.N = mb;
+    g.nseg = 1;
+    g.K[0] = H;
+    g.lda[0] = H;
+    g.trans_a = 1;
+    g.ldb[0] = H;
+    g.ldc = H;
+    g.batch = 1;
+    g.epilogue = ZR_EPI_STORE;
+    g.groups = 2;
+    g.gA[0] = a->W_c1, g.gA[1] = a->W_c2;
+    g.gB[0] = g.gB[1] = e;
+    g.gC[0] = err_ct, g.gC[1] = d_err_h_t;
+    if ((rc = zr_gemm_launch(ctx, g))) return rc;
+  }
   attn_bwd_align_kernel<<<dim3(W, mb), 256, 0, ctx->stream>>>(err_ct, a->d_table, a->d_err_table, d_batch_info, d_indices,
                                                               d_alignments, H, mb, W, a->longest_sent, err_as);
   ZR_LAUNCH_CHECK("attn_bwd_align_kernel");
@@ -998,13 +1087,17 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   attn_bwd_vp_wp_kernel<<<eg, 256, 0, ctx->stream>>>(a->d_tanh1, a->v_p, col, H, mb, (long long)n, tv, tw);
   ZR_LAUNCH_CHECK("attn_bwd_vp_wp_kernel");
   if ((rc = row_sum_launch(ctx, tv, H, mb, grads->d_v_p, 1))) return rc;        // :536
-  if ((rc = outer_acc(tw, d_h_t, grads->d_W_p))) return rc;                     // :545
+  if (!outer && (rc = outer_acc(tw, d_h_t, grads->d_W_p))) return rc;           // :545
   if ((rc = product(a->W_p, 1, tw, d_err_h_t, 1, ZR_EPI_STORE))) return rc;     // :551
   if ((rc = product(a->W_a, 1, d_h_t, a->d_q, 0, ZR_EPI_STORE))) return rc;     // W_a^T h of the forward pass again
   attn_bwd_hs_kernel<<<mb, 256, 0, ctx->stream>>>(a->d_q, a->d_table, a->d_err_table, d_batch_info, d_indices, scal, H, mb,
                                                   W, a->longest_sent, hs_sum);
   ZR_LAUNCH_CHECK("attn_bwd_hs_kernel");
-  if ((rc = outer_acc(d_h_t, hs_sum, grads->d_W_a))) return rc;                 // :632
+  if (outer)
+    rc = outer_launch(ctx, OuterProducts{{tw, d_h_t}, {d_h_t, hs_sum}, {grads->d_W_p, grads->d_W_a}}, 2, H, H, mb);
+  else
+    rc = outer_acc(d_h_t, hs_sum, grads->d_W_a);                                // :632
+  if (rc) return rc;
   return product(a->W_a, 0, hs_sum, d_err_h_t, 1, ZR_EPI_STORE);                // :636
 }
 
@@ -1063,6 +1156,7 @@ int zr_lstm_feed_backward(zr_ctx* ctx, const float* const d_Q[4], int H, int mb,
   }
   // Q gradients, stacked over the gates like the M and W_h gradients: dQ (4H x H) += dgates (4H x mb) * h~^T
   // (src/LSTM.hpp:1014-1050)
+  if (outer_takes(4 * H, H, mb)) return outer_launch(ctx, OuterProducts{{d_dgates}, {d_htild}, {d_dQ_stack}}, 1, 4 * H, H, mb);
   void* scratch = nullptr;
   rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (size_t)H * mb, &scratch);
   if (rc) return rc;
