@@ -938,14 +938,21 @@ int zr_lstm_node_backward(zr_ctx* ctx, const zr_lstm_train* layer, int mb, const
   g.N = mb;
   g.nseg = 1;
   g.K[0] = 4 * H;
-  g.A[0] = layer->d_stack;
-  g.lda[0] = H;
+  if (H % 4 == 0) {  // the k-interleaved copy, as in the sweep over the whole grid: one 16-byte load per four k
+    g.a_pack = 1;
+    g.A[0] = layer->d_stack_pack;
+    g.lda[0] = layer->ldp;
+    g.strideA = (long long)layer->kp * layer->ldp;
+  } else {
+    g.A[0] = layer->d_stack;
+    g.lda[0] = H;
+    g.strideA = 4LL * H * H;
+  }
   g.B[0] = d_dgates;
   g.ldb[0] = 4 * H;
   g.C = out;
   g.ldc = H;
   g.batch = d_err_below ? 2 : 1;
-  g.strideA = 4LL * H * H;
   g.strideC = (long long)n;
   g.epilogue = ZR_EPI_STORE;
   rc = zr_gemm_launch(ctx, g);
