@@ -98,10 +98,11 @@ const char* zr_version(void);
                                         3: weights streamed to registers, K split inside and across workgroups */
 #define ZR_OPT_LSTM_KPARTS 6         /* kernels 2 and 3: K parts per weight segment (0 = auto) */
 #define ZR_OPT_LSTM_SWEEP 7          /* zr_lstm_stack_forward as ONE launch whose workgroups hand h to each other
-                                        through device memory: 0 auto (when they fill most of the device, are all
-                                        resident at once, the context is the process's only one on its device and
-                                        runs on its own stream),
-                                        1 never (one launch per diagonal), 2 whenever they fit.  The environment
+                                        through device memory: 0 auto (the least estimated time of: the sweep with
+                                        streamed weights, the sweep with its weights in registers, one launch per
+                                        diagonal; a sweep only when its workgroups are all resident at once, the
+                                        context is the process's only one on its device and runs on its own stream),
+                                        1 never (one launch per diagonal), 2 a sweep whenever one fits.  The environment
                                         variable ZR_LSTM_SWEEP presets this option for every context created */
 #define ZR_OPT_LSTM_SWEEP_SPIN 8     /* polls a workgroup of that launch spends on one wait before it gives up
                                         (0 = default, about a second); giving up is reported by zr_ctx_sync */
@@ -224,7 +225,7 @@ int zr_lstm_gates(zr_ctx* ctx, const float* d_preact, const float* const d_b[4],
  * forward_prop_source, :2367-2452): layer 0 gathers its input from d_embed by token id, layer l>0 reads layer
  * l-1's h_t.  Nodes that do not depend on each other run side by side: either the whole sweep is ONE launch whose
  * workgroups keep their tile of one layer for all T steps and hand h_t to each other through device memory (taken
- * when they fill most of the GPU and are all resident at once; see ZR_OPT_LSTM_SWEEP), or one launch per diagonal
+ * when they are all resident at once and that is estimated to be faster; see ZR_OPT_LSTM_SWEEP), or one launch per diagonal
  * l + t = d.  The single launch keeps its hand-over buffer and arrival counters in the context's scratch memory.
  *   d_ids_nonneg, d_mask01: time-major [b + t*mb] (src/fileHelper.h:488), outputs of zr_vocab_prep
  *   d_h0/d_c0: arrays of L device pointers (initial state per layer, H x mb) -- zeros for encoder / LM
