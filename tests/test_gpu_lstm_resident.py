@@ -85,6 +85,37 @@ def test_sweep_with_weights_in_registers(ctx, H, mb, T, L):
     assert_close(m * g[:, :, 3] * np.tanh(cell), want_h, what="h from the gates")
 
 
+@pytest.mark.parametrize("H,mb,T,L", [(100, 35, 6, 2), (100, 68, 5, 1), (300, 36, 6, 2), (500, 34, 5, 2), (500, 41, 5, 1),
+                                      (500, 76, 4, 1)])
+def test_back_to_back_with_different_inputs(ctx, H, mb, T, L):
+    """Three and five column tiles of batches that are 1 to 4 columns beyond a multiple of eight, whose k-blocks in the
+    hand-over copy would share cache lines were they padded to four columns: sweeps over different words and initial states
+    queued one after another into the same scratch slots, so that a state left there by an earlier sweep is a wrong one."""
+    cases = [_case(H, mb, T, L, seed=50 + i) for i in range(3)]
+    for c in cases[1:]:
+        c["layers"], c["embed"] = cases[0]["layers"], cases[0]["embed"]
+    V, n = cases[0]["V"], H * mb
+    layers, d_embed, runs = [Layer(ctx, ly) for ly in cases[0]["layers"]], ctx.array(cases[0]["embed"]), []
+    for c in cases:
+        d_nn, d_m = ctx.empty(c["ids"].size, np.int32), ctx.empty(c["ids"].size, np.int32)
+        ctx.vocab_prep(ctx.array(c["ids"].reshape(-1)), c["ids"].size, V, d_nn, d_m)
+        runs.append(dict(nn=d_nn, m=d_m, h0=[ctx.array(a) for a in c["h0"]], c0=[ctx.array(a) for a in c["c0"]],
+                         h=[ctx.empty((n * T,)) for _ in range(L)], c=[ctx.empty((n * T,)) for _ in range(L)]))
+    ctx.sync()
+    try:
+        for r in runs + runs[:2]:
+            ctx.lstm_stack_forward([ly.w for ly in layers], d_embed, V, r["nn"], r["m"], T, mb, r["h0"], r["c0"], r["h"], r["c"])
+            assert ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH) == capi.ZR_LSTM_STACK_PATH_SWEEP
+        ctx.sync()
+    finally:
+        for ly in layers:
+            ly.close()
+    for i, (c, r) in enumerate(zip(cases, runs)):
+        want_h, want_c = _want(c, clip=None)
+        for got, want, what in ((r["h"], want_h, "h"), (r["c"], want_c, "c")):
+            assert_close(np.stack([a.get().reshape(T, mb, H).swapaxes(1, 2) for a in got]), want, what="%s of sweep %d" % (what, i))
+
+
 def test_library_picks_it_for_a_small_model(ctx):
     c = _case(100, 8, 5, 2)
     h, x, _, path, _ = _run(ctx, c)

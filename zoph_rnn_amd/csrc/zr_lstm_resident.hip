@@ -15,8 +15,8 @@
 //   * a wave waits only for the producers of its own K slice: a row tile of 8 is one k-group, the flags of the 16
 //     producers (at most) of a wave's groups lie side by side and one load by one wave looks at all of them;
 //   * h travels in a k-interleaved copy [k/4][columns][4] whose pad rows are written as zeros (any H, no K tails) and
-//     whose columns are padded to four, so that every 128-byte line of it has one producer and is read only after that
-//     producer's flag: no cache invalidation inside the launch;
+//     whose columns are padded to eight, so that every 128-byte line of it has one producer, with any number of column
+//     tiles, and is read only after that producer's flag: no cache invalidation inside the launch (zr_resident_layout.h);
 //   * h, c and the kept gate values are stored after the publish.
 // Batches of up to 16 columns use the 16 x 16 x 4 instruction (NARROW), half the matrix time of a half-empty 32-column
 // tile.  Progress, bounded waits and the abandon protocol are those of lstm_sweep_kernel; a workgroup that gives up marks
@@ -30,12 +30,13 @@
 #include "zr_internal.h"
 #include "zr_math.h"
 #include "zr_mfma_core.h"
+#include "zr_resident_layout.h"
 
 namespace {
 
 constexpr int kMaxLayers = 8;
 constexpr int kWaves = 8;                 // waves per workgroup = K slices
-constexpr int kRows = 8;                  // hidden rows per workgroup
+constexpr int kRows = kResidentRows;
 constexpr int kRedLd = 36;                // LDS row of 32 partial sums, padded: conflict-free for the cell's reads
 constexpr int kResidentGaveUp = 1 << 28;  // flag value of a workgroup that stopped waiting
 
@@ -51,7 +52,7 @@ struct LstmResident {
   const int* ids;                 // [T][mb], already non-negative
   const int* mask01;              // [T][mb]
   float* hp;                      // [layers][T + 1] slots of k-interleaved h: slot 0 = initial state, slot t + 1 = h_t
-  long long slot;                 // floats per slot: ceil8(H) * mbp
+  long long slot;                 // floats per slot (zr_resident_slot)
   int* flags;                     // [layers of this launch][n_tiles] at flag_stride, zero at launch: slots published
   int flag_stride, n_flags;
   int* departures;                // workgroups that have left the kernel (zero at launch)
@@ -136,7 +137,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
       const int jc = j < H ? j : H - 1, nc = n < mb ? n : mb - 1;
       bi[u] = P.bias[l][jc], bf[u] = P.bias[l][H + jc], bc[u] = P.bias[l][2 * H + jc], bo[u] = P.bias[l][3 * H + jc];
       c_state[u] = P.c0[l][(long long)nc * H + jc];
-      hp_off[u] = (unsigned)(((j >> 2) * P.mbp + n) * 4 + (j & 3));
+      hp_off[u] = zr_resident_at(j, n, P.mbp);
     }
     int* flags_here = P.flags + ((l - P.l_begin) * P.n_tiles + nt) * P.flag_stride;
     const int* flags_below = flags_here - P.n_tiles * P.flag_stride;
@@ -424,7 +425,7 @@ double zr_lstm_resident_plan(zr_ctx* ctx, int nl, int H, int mb, int T, ZrReside
   const int j_tiles = (H + kRows - 1) / kRows;
   const int nprod = 2 << size_class;  // NPROD of the kernel, in every column class
   const int flag_stride = (kWaves * nprod + 31) / 32 * 32;
-  const long long slot = (long long)j_tiles * kRows * ((mb + 3) & ~3);
+  const long long slot = zr_resident_slot(H, mb);
   if (slot * 4 >= (1LL << 32)) return -1.0;
   // Column class and layers per launch: the cheapest by the time a step takes -- a hand-over of 3.2 us and the matrix
   // instructions of both segments at 2.3 GHz, two waves to a SIMD and as many workgroups to a compute unit as the launch
@@ -461,8 +462,7 @@ int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, cons
   const int H = layers[0]->H;
   const int j_tiles = (H + kRows - 1) / kRows;
   const int per_layer = j_tiles * plan.n_tiles;
-  const int mbp = (mb + 3) & ~3;
-  const long long slot = (long long)j_tiles * kRows * mbp;
+  const long long slot = zr_resident_slot(H, mb);
   void* p = nullptr;
   int rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (size_t)(nl * (long long)(T + 1) * slot), &p);
   if (rc) return rc;
@@ -489,7 +489,7 @@ int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, cons
   P.V = V;
   P.H = H;
   P.mb = mb;
-  P.mbp = mbp;
+  P.mbp = zr_resident_columns(mb);
   P.ldw = layers[0]->ldw;
   P.kp = layers[0]->kp;
   P.j_tiles = j_tiles;
