@@ -64,6 +64,8 @@ int zr_ctx_set_option(zr_ctx* ctx, int option, int value);
  *     the flag -- and with it the data flags that launches queued behind the abandoned one raised on its NaN outputs --
  *     so a following zr_ctx_sync no longer reports it.  A decoder step called with d_c[l] == d_cprev[l] (cell state
  *     updated in place) has overwritten its own input by then: running it again needs the caller's copy of c_{t-1}.
+ *   ZR_QUERY_LSTM_SWEEP_KERNEL: which single-launch sweep the last zr_lstm_stack_forward(_train) call on this context ran
+ *     -- ZR_LSTM_SWEEP_STREAMED or ZR_LSTM_SWEEP_RESIDENT; 0 if none has, or it took one launch per diagonal.  Does not wait.
  *   ZR_QUERY_SCRATCH_KIB: device memory the context has allocated for scratch buffers so far, in KiB (0 for a context
  *     that has only served calls that allocate nothing).  Does not wait.
  *   ZR_QUERY_ATTN_PATH: which schedule the last zr_attn_step (or the attention part of zr_decoder_step) on this
@@ -74,6 +76,9 @@ int zr_ctx_query(zr_ctx* ctx, int what, int* h_value);
 #define ZR_QUERY_LSTM_SWEEP_ABANDONED 2
 #define ZR_QUERY_ATTN_PATH 3
 #define ZR_QUERY_SCRATCH_KIB 4
+#define ZR_QUERY_LSTM_SWEEP_KERNEL 5
+#define ZR_LSTM_SWEEP_STREAMED 1 /* weights streamed from the caches in every time step */
+#define ZR_LSTM_SWEEP_RESIDENT 2 /* weights held in registers */
 #define ZR_ATTN_PATH_SINGLE_LAUNCH 1  /* projections, window / scores / context and output product in one launch */
 #define ZR_ATTN_PATH_THREE_LAUNCHES 2 /* the same three stages as one launch each */
 #define ZR_ATTN_PATH_SEPARATE 3       /* unprepared or bf16 matrices: products and the middle as separate launches */
@@ -102,8 +107,10 @@ const char* zr_version(void);
                                         streamed weights, the sweep with its weights in registers, one launch per
                                         diagonal; a sweep only when its workgroups are all resident at once, the
                                         context is the process's only one on its device and runs on its own stream),
-                                        1 never (one launch per diagonal), 2 a sweep whenever one fits.  The environment
-                                        variable ZR_LSTM_SWEEP presets this option for every context created */
+                                        1 never (one launch per diagonal), 2 a sweep whenever one fits, with streamed
+                                        weights if that one does, 3 the same with its weights in registers if that
+                                        one does.  The environment variable ZR_LSTM_SWEEP presets this option for every
+                                        context created */
 #define ZR_OPT_LSTM_SWEEP_SPIN 8     /* polls a workgroup of that launch spends on one wait before it gives up
                                         (0 = default, about a second); giving up is reported by zr_ctx_sync */
 

@@ -11,6 +11,8 @@ from zoph_rnn_amd import capi, synth
 
 pytestmark = pytest.mark.gpu
 
+RESIDENT = (capi.ZR_LSTM_STACK_PATH_SWEEP, capi.ZR_LSTM_SWEEP_RESIDENT)
+
 
 @pytest.fixture(scope="module")
 def ctx():
@@ -45,7 +47,7 @@ def _run(ctx, c, clip=0.9, times=1):
     try:
         for _ in range(times):
             ctx.lstm_stack_forward_train([ly.w for ly in layers], d_embed, V, d_nn, d_m, T, mb, d_h0, d_c0, h, x, g, clip=clip)
-        path = ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH)
+        path = (ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH), ctx.query(capi.ZR_QUERY_LSTM_SWEEP_KERNEL))
         abandoned = ctx.query(capi.ZR_QUERY_LSTM_SWEEP_ABANDONED)
     finally:
         for ly in layers:
@@ -66,13 +68,13 @@ def _want(c, clip=0.9):
                                       (508, 64, 3, 4), (516, 16, 3, 1), (1000, 12, 3, 4), (1001, 1, 3, 2), (1024, 16, 3, 3)])
 def test_sweep_with_weights_in_registers(ctx, H, mb, T, L):
     c = _case(H, mb, T, L)
-    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 3)
     try:
         h, x, g, path, abandoned = _run(ctx, c)
         h2, x2, g2, _, _ = _run(ctx, c, times=3)  # flags of one launch must not reach the next
     finally:
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
-    assert path == capi.ZR_LSTM_STACK_PATH_SWEEP and not abandoned
+    assert path == RESIDENT and not abandoned
     assert h.tobytes() == h2.tobytes() and x.tobytes() == x2.tobytes() and g.tobytes() == g2.tobytes()
     want_h, want_c = _want(c)
     assert_close(h, want_h, what="h")
@@ -105,7 +107,7 @@ def test_back_to_back_with_different_inputs(ctx, H, mb, T, L):
     try:
         for r in runs + runs[:2]:
             ctx.lstm_stack_forward([ly.w for ly in layers], d_embed, V, r["nn"], r["m"], T, mb, r["h0"], r["c0"], r["h"], r["c"])
-            assert ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH) == capi.ZR_LSTM_STACK_PATH_SWEEP
+            assert ctx.query(capi.ZR_QUERY_LSTM_SWEEP_KERNEL) == capi.ZR_LSTM_SWEEP_RESIDENT
         ctx.sync()
     finally:
         for ly in layers:
@@ -119,25 +121,25 @@ def test_back_to_back_with_different_inputs(ctx, H, mb, T, L):
 def test_library_picks_it_for_a_small_model(ctx):
     c = _case(100, 8, 5, 2)
     h, x, _, path, _ = _run(ctx, c)
-    assert path == capi.ZR_LSTM_STACK_PATH_SWEEP
+    assert path == RESIDENT
     want_h, want_c = _want(c)
     assert_close(h, want_h, what="h")
     assert_close(x, want_c, what="c")
 
 
 def test_abandoned_wait_is_reported_and_leaves_nan(ctx):
-    """H = 100 has no other single-launch schedule: with one poll per wait the upper layer gives up, every workgroup
-    leaves, the outputs are NaN, and the next sweep with the default limit is complete again."""
+    """With one poll per wait the upper layer gives up, every workgroup leaves, the outputs are NaN, and the next sweep
+    with the default limit is complete again."""
     c = _case(100, 24, 6, 3)
-    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 3)
     ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 1)
     try:
         h, x, g, path, abandoned = _run(ctx, c)
-        assert path == capi.ZR_LSTM_STACK_PATH_SWEEP and abandoned == 1
+        assert path == RESIDENT and abandoned == 1
         assert np.all(np.isnan(h)) and np.all(np.isnan(x)) and np.all(np.isnan(g))
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)
         h, x, g, path, abandoned = _run(ctx, c)
-        assert path == capi.ZR_LSTM_STACK_PATH_SWEEP and abandoned == 0
+        assert path == RESIDENT and abandoned == 0
     finally:
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)

@@ -246,6 +246,15 @@ def test_lstm_step_full_size_layer(ctx):
 
 
 # ------------------------------------------------------------------------------------------------ A6/A7/A11 stack
+# ZR_OPT_LSTM_SWEEP -> the kernel it asks for
+SWEEPS = {2: capi.ZR_LSTM_SWEEP_STREAMED, 3: capi.ZR_LSTM_SWEEP_RESIDENT}
+
+
+def _assert_sweep(ctx, sweep):
+    assert ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH) == capi.ZR_LSTM_STACK_PATH_SWEEP
+    assert ctx.query(capi.ZR_QUERY_LSTM_SWEEP_KERNEL) == SWEEPS[sweep]
+
+
 def _run_stack(ctx, cfg_layers, embed, ids, h0=None, c0=None, clip=0.0, expect_path=None):
     """expect_path: the schedule zr_lstm_stack_forward must have taken (capi.ZR_LSTM_STACK_PATH_*), asserted."""
     H, V = embed.shape
@@ -1029,9 +1038,11 @@ def test_stack_forward_with_split_kernel_forced(ctx):
 
 @pytest.mark.parametrize("H,mb,T,L", [(64, 5, 7, 3), (104, 40, 9, 4), (256, 70, 6, 2), (1000, 128, 5, 4),
                                       (72, 33, 12, 1), (512, 128, 4, 8), (8, 1, 3, 2), (32, 2, 1, 1), (40, 9, 1, 5)])
-def test_stack_forward_whole_sweep_launch(ctx, H, mb, T, L):
-    """The single-launch sweep (workgroups hand h to each other through device memory) against the oracle and against
-    one launch per diagonal: column and row tails, one to eight layers, initial states, padding, cell clipping."""
+@pytest.mark.parametrize("sweep", [2, 3])
+def test_stack_forward_whole_sweep_launch(ctx, H, mb, T, L, sweep):
+    """The single-launch sweeps (workgroups hand h to each other through device memory; weights streamed or in registers)
+    against the oracle and against one launch per diagonal: column and row tails, one to eight layers, initial states,
+    padding, cell clipping."""
     g = synth.rng(19, H + mb)
     V = 311
     embed = U(g, (H, V))
@@ -1042,28 +1053,32 @@ def test_stack_forward_whole_sweep_launch(ctx, H, mb, T, L):
     ids[: T - 1, mb - 1] = -1
     h0 = [np.tanh(U(g, (H, mb), -1, 1)) for _ in range(L)]
     c0 = [U(g, (H, mb), -0.5, 0.5) for _ in range(L)]
+    # 1000 x 128 is more than registers hold: option 3 then takes the sweep that fits
+    kernel = capi.ZR_LSTM_SWEEP_STREAMED if (H, mb) == (1000, 128) else SWEEPS[sweep]
     out = {}
-    for mode in (2, 1):
+    for mode in (sweep, 1):
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, mode)
         try:
-            path = capi.ZR_LSTM_STACK_PATH_SWEEP if mode == 2 else capi.ZR_LSTM_STACK_PATH_DIAGONALS
+            path = capi.ZR_LSTM_STACK_PATH_SWEEP if mode != 1 else capi.ZR_LSTM_STACK_PATH_DIAGONALS
             out[mode] = _run_stack(ctx, layers, embed, ids, h0=h0, c0=c0, clip=0.9, expect_path=path)
-            again = _run_stack(ctx, layers, embed, ids, h0=h0, c0=c0, clip=0.9, expect_path=path) if mode == 2 else None
+            assert ctx.query(capi.ZR_QUERY_LSTM_SWEEP_KERNEL) == (kernel if mode != 1 else 0)
+            again = _run_stack(ctx, layers, embed, ids, h0=h0, c0=c0, clip=0.9, expect_path=path) if mode != 1 else None
         finally:
             ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
         if again is not None:  # fixed summation order: the same bits on every run
-            assert again[0].tobytes() == out[2][0].tobytes() and again[1].tobytes() == out[2][1].tobytes()
+            assert again[0].tobytes() == out[sweep][0].tobytes() and again[1].tobytes() == out[sweep][1].tobytes()
     nn, m = o.vocab_prep(ids)
     want_h, want_c = o.lstm_stack_forward(embed, layers, nn, m, h0=h0, c0=c0, clip=0.9)
-    for mode in (2, 1):
+    for mode in (sweep, 1):
         assert_close(out[mode][0], want_h, what="stack h (sweep option %d)" % mode)
         assert_close(out[mode][1], want_c, what="stack c (sweep option %d)" % mode)
-    assert mb == 1 or np.all(out[2][0][:, : min(2, T), :, 1] == 0)
-    assert np.all(out[2][1][:, : T - 1, :, mb - 1] == 0)
+    assert mb == 1 or np.all(out[sweep][0][:, : min(2, T), :, 1] == 0)
+    assert np.all(out[sweep][1][:, : T - 1, :, mb - 1] == 0)
 
 
-def test_whole_sweep_launch_keeps_gates_for_training(ctx):
-    """zr_lstm_stack_forward_train through the single-launch sweep: every node's four gate activations, h and c against
+@pytest.mark.parametrize("sweep", [2, 3])
+def test_whole_sweep_launch_keeps_gates_for_training(ctx, sweep):
+    """zr_lstm_stack_forward_train through either single-launch sweep: every node's four gate activations, h and c against
     the oracle's node-by-node forward pass."""
     g = synth.rng(22, 1)
     H, mb, T, V, L = 96, 24, 5, 131, 2
@@ -1079,11 +1094,11 @@ def test_whole_sweep_launch_keeps_gates_for_training(ctx):
     h_all = [ctx.empty((n * T,)) for _ in range(L)]
     c_all = [ctx.empty((n * T,)) for _ in range(L)]
     g_all = [ctx.empty((4 * n * T,)) for _ in range(L)]
-    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, sweep)
     try:
         ctx.lstm_stack_forward_train([ly.w for ly in layers], ctx.array(embed), V, d_nn, d_m, T, mb, [z] * L, [z] * L,
                                      h_all, c_all, g_all)
-        assert ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH) == capi.ZR_LSTM_STACK_PATH_SWEEP
+        _assert_sweep(ctx, sweep)
         ctx.sync()
     finally:
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
@@ -1110,11 +1125,12 @@ def test_whole_sweep_launch_keeps_gates_for_training(ctx):
         ly.close()
 
 
-def test_whole_sweep_launch_back_to_back_with_different_inputs(ctx):
+@pytest.mark.parametrize("sweep", [2, 3])
+def test_whole_sweep_launch_back_to_back_with_different_inputs(ctx, sweep):
     """Sweeps of the same shape with different token ids and initial states, queued back to back through the same
     hand-over buffers with nothing but the counter-clearing fill between them (the whole hand-over buffer, 1.5 MB, stays
-    cache resident): a later sweep must not see anything of an earlier one (mb % 8 == 0: the consumers do not
-    invalidate their caches inside the launch)."""
+    cache resident): a later sweep must not see anything of an earlier one (neither kernel's consumers invalidate their
+    caches inside the launch here: with streamed weights because mb % 8 == 0, with resident ones always)."""
     H, mb, T, V, L = 256, 64, 6, 211, 4
     g = synth.rng(21, 1)
     embed = U(g, (H, V))
@@ -1133,12 +1149,12 @@ def test_whole_sweep_launch_back_to_back_with_different_inputs(ctx):
                          d_c0=[ctx.array(a) for a in c0], h_all=[ctx.empty((n * T,)) for _ in range(L)],
                          c_all=[ctx.empty((n * T,)) for _ in range(L)]))
     ctx.sync()
-    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, sweep)
     try:
         for r in runs:  # queued without a synchronisation or any other work in between
             ctx.lstm_stack_forward([ly.w for ly in layers], d_embed, V, r["d_nn"], r["d_m"], T, mb, r["d_h0"], r["d_c0"],
                                    r["h_all"], r["c_all"])
-            assert ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH) == capi.ZR_LSTM_STACK_PATH_SWEEP
+            _assert_sweep(ctx, sweep)
         ctx.sync()
     finally:
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
@@ -1154,11 +1170,12 @@ def test_whole_sweep_launch_back_to_back_with_different_inputs(ctx):
 
 
 @pytest.mark.parametrize("H,mb,T,L", [(200, 70, 20, 3), (256, 64, 12, 4)])
-def test_whole_sweep_launch_many_repetitions_identical(ctx, H, mb, T, L):
+@pytest.mark.parametrize("sweep", [2, 3])
+def test_whole_sweep_launch_many_repetitions_identical(ctx, H, mb, T, L, sweep):
     """The same sweep 400 times in a row: the order of the sums is fixed, so whatever the timing of the hand-overs
     between workgroups, every repetition gives the first one's bits (checked every 50 launches), the first one agrees
-    with the oracle, and no wait is ever abandoned (zr_ctx_sync would report it).  mb = 70 takes the waits that
-    invalidate the caches, mb = 64 the ones that do not."""
+    with the oracle, and no wait is ever abandoned (zr_ctx_sync would report it).  With streamed weights mb = 70
+    takes the waits that invalidate the caches, mb = 64 the ones that do not."""
     g = synth.rng(23, H + mb)
     V = 257
     embed = U(g, (H, V))
@@ -1173,11 +1190,11 @@ def test_whole_sweep_launch_many_repetitions_identical(ctx, H, mb, T, L):
     h_all = [ctx.empty((H * mb * T,)) for _ in range(L)]
     c_all = [ctx.empty((H * mb * T,)) for _ in range(L)]
     first = None
-    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, sweep)
     try:
         for i in range(400):
             ctx.lstm_stack_forward([ly.w for ly in layers], d_embed, V, d_nn, d_m, T, mb, [z] * L, [z] * L, h_all, c_all)
-            assert ctx.query(capi.ZR_QUERY_LSTM_STACK_PATH) == capi.ZR_LSTM_STACK_PATH_SWEEP
+            _assert_sweep(ctx, sweep)
             if i % 50 == 0 or i == 399:
                 ctx.sync()
                 got = [a.get().tobytes() for a in h_all + c_all]
@@ -1196,7 +1213,8 @@ def test_whole_sweep_launch_many_repetitions_identical(ctx, H, mb, T, L):
         ly.close()
 
 
-def test_whole_sweep_launch_abandoned_wait_is_reported(ctx):
+@pytest.mark.parametrize("sweep", [2, 3])
+def test_whole_sweep_launch_abandoned_wait_is_reported(ctx, sweep):
     """With a single poll per wait the upper layers give up at once: every workgroup still leaves the kernel, and
     zr_ctx_sync reports the incomplete sweep; the next sweep with the default limit is complete again."""
     g = synth.rng(20, 1)
@@ -1204,7 +1222,7 @@ def test_whole_sweep_launch_abandoned_wait_is_reported(ctx):
     embed = U(g, (H, V))
     layers = [synth.lstm_layer(g, H) for _ in range(L)]
     ids = g.integers(0, V, size=(T, mb)).astype(np.int32)
-    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, sweep)
     ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 1)
     try:
         with pytest.raises(capi.ZrError, match="gave up waiting"):
@@ -1219,6 +1237,7 @@ def test_whole_sweep_launch_abandoned_wait_is_reported(ctx):
         h_all = [ctx.zeros((H_ * mb_ * T,)) for _ in range(L)]
         c_all = [ctx.zeros((H_ * mb_ * T,)) for _ in range(L)]
         ctx.lstm_stack_forward([ly.w for ly in lys], ctx.array(embed), V, d_nn, d_m, T, mb_, [z] * L, [z] * L, h_all, c_all)
+        _assert_sweep(ctx, sweep)
         assert ctx.query(capi.ZR_QUERY_LSTM_SWEEP_ABANDONED) == 1
         assert ctx.query(capi.ZR_QUERY_LSTM_SWEEP_ABANDONED) == 0  # the look clears the flag
         ctx.sync()  # ... so the synchronisation has nothing left to report
@@ -1227,6 +1246,7 @@ def test_whole_sweep_launch_abandoned_wait_is_reported(ctx):
             ly.close()
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)
         hs, cs = _run_stack(ctx, layers, embed, ids, expect_path=capi.ZR_LSTM_STACK_PATH_SWEEP)
+        _assert_sweep(ctx, sweep)
         assert ctx.query(capi.ZR_QUERY_LSTM_SWEEP_ABANDONED) == 0
     finally:
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)

@@ -26,7 +26,7 @@ struct zr_ctx {
   int lstm_kparts;   // K parts per segment for the split-K kernel (0 auto)
   int* d_counters;   // ZR_MAX_COUNTERS arrival counters, zero between launches
   int* d_step_flags; // ZR_MAX_STEP_FLAGS flags of lstm_resident_kernel (the first 32 hold its departure count), zero between launches
-  int lstm_sweep;    // whole-sweep LSTM kernel: 0 auto, 1 never, 2 whenever the launch fits on the device
+  int lstm_sweep;    // whole-sweep LSTM kernels: 0 auto, 1 never, 2 / 3 streamed / resident weights whenever the launch fits
   int sweep_spin;    // polls before a waiting workgroup of that kernel gives up (0: default)
   int step_wait_extra;  // arrivals the decoder step's layer waits expect beyond the real ones (tests of giving up)
   int stack_helpers;    // 1 (default): the decoder step may run 32-column tiles with helper workgroups (zr_lstm.hip)
@@ -39,6 +39,7 @@ struct zr_ctx {
   int last_attn_path;   // ZR_ATTN_PATH_* of the last attention step (0: none yet)
   int gemm_cfg;
   int bf16_terms;       // bf16-weight products: 2 (default, 0 = 2) = activations as two bf16 terms, 1 = rounded to bf16 once
+  int last_sweep_kernel;  // ZR_LSTM_SWEEP_STREAMED / _RESIDENT: the last zr_lstm_stack_forward(_train) call (0: neither)
   int last_stack_path;  // ZR_LSTM_STACK_PATH_* of the last zr_lstm_stack_forward(_train) call (0: none yet)
   // scratch owned by the context (grown on demand, never shrunk)
   void* d_scratch;

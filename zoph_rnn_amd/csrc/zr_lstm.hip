@@ -1685,7 +1685,7 @@ int zr_lstm_decoder_step_packed(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
     const bool offsets_fit = (long long)V * H * 4 < lim && (long long)n * 4 < lim &&
                              12LL * layers[0]->kp * layers[0]->ldw * 4 < lim;
     const long long n_counters = nl * tiles + (long long)nl * n_tiles * kSweepCtrStride;
-    if (cap > 0 && wgs <= cap && offsets_fit && n_counters < ZR_MAX_COUNTERS && (fills || ctx->lstm_sweep == 2)) {
+    if (cap > 0 && wgs <= cap && offsets_fit && n_counters < ZR_MAX_COUNTERS && (fills || ctx->lstm_sweep >= 2)) {
       const int NV = tn == 1 ? zr_visit_count<1, 4>() : zr_visit_count<2, 4>();
       LstmDecStack P = {};
       void* p = nullptr;
@@ -1830,7 +1830,7 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
   // with an error).  Nor on a caller-provided stream: the caller's other streams may hold compute units for as long as
   // they like.
   const bool alone = zr_live_contexts(ctx->device) == 1 && ctx->stream == ctx->own_stream;
-  const bool single_ok = !layers[0]->bf16 && ctx->lstm_fused && (ctx->lstm_sweep == 2 || (ctx->lstm_sweep == 0 && alone));
+  const bool single_ok = !layers[0]->bf16 && ctx->lstm_fused && (ctx->lstm_sweep >= 2 || (ctx->lstm_sweep == 0 && alone));
   // Whole-sweep kernel with streamed weights: when its workgroups -- one tile of one layer each, kept for all T steps --
   // fit on the chip together.
   const int j_tiles = (H + 31) / 32, n32 = (mb + 31) / 32;
@@ -1869,15 +1869,17 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
     const double other_us = tn ? sweep_us : diag_us;
     ZrResidentPlan plan;
     plan.at_once = 0;
-    if (ctx->lstm_sweep == 2 || (!ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts)) {
+    // option 2: the streamed sweep where it fits, 3: the one with resident weights where that fits
+    if (ctx->lstm_sweep == 2 ? !tn : ctx->lstm_sweep == 3 || (!ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts)) {
       const double resident_us = zr_lstm_resident_plan(ctx, nl, H, mb, T, &plan);
-      if (resident_us < 0.0 || (other_us > 0.0 && other_us <= resident_us)) plan.at_once = 0;
+      if (resident_us < 0.0 || (!ctx->lstm_sweep && other_us > 0.0 && other_us <= resident_us)) plan.at_once = 0;
     }
     if (plan.at_once) {
       rc = zr_lstm_resident_sweep(ctx, plan, nl, layers, d_embed, V, d_ids_nonneg, d_mask01, T, mb, d_h0, d_c0,
                                   clip_threshold, d_h_all, d_c_all, d_gates_all);
       if (rc) return rc;
       ctx->last_stack_path = ZR_LSTM_STACK_PATH_SWEEP;
+      ctx->last_sweep_kernel = ZR_LSTM_SWEEP_RESIDENT;
       return poison_if_abandoned(ctx, nl, T, H, mb, d_h_all, d_c_all, d_gates_all);
     }
   }
@@ -1920,12 +1922,14 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
     // when no 128-byte line of the k-interleaved copies is shared between two producers, i.e. mb % 8 == 0.
     P.fence = (mb % 8 == 0) ? 0 : 1;
     ctx->last_stack_path = ZR_LSTM_STACK_PATH_SWEEP;
+    ctx->last_sweep_kernel = ZR_LSTM_SWEEP_STREAMED;
     return tn == 1 ? launch_sweep_v<1>(ctx, P, padded * n_tiles) : launch_sweep_v<2>(ctx, P, padded * n_tiles);
   }
   // Every h is also written in a k-interleaved layout ([H/4][mb][4]) into a small ping-pong buffer per layer: its
   // two consumers on the next diagonal, (l+1, t) and (l, t+1), then fetch activations with contiguous 16-byte
   // loads.  The buffer written on diagonal d is read on d+1 only and overwritten on d+2.
   ctx->last_stack_path = ZR_LSTM_STACK_PATH_DIAGONALS;
+  ctx->last_sweep_kernel = 0;
   float* hp_buf = nullptr;
   if (vec && H % 8 == 0 && !layers[0]->bf16) {
     void* p = nullptr;

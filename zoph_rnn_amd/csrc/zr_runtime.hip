@@ -126,11 +126,11 @@ int zr_ctx_create(int device, zr_ctx** out) {
     c->cu_count = 256;
   }
   c->lstm_fused = 1;
-  // ZR_LSTM_SWEEP in the environment presets ZR_OPT_LSTM_SWEEP for every context of the process (0, 1 or 2): lets a
+  // ZR_LSTM_SWEEP in the environment presets ZR_OPT_LSTM_SWEEP for every context of the process (0 to 3): lets a
   // whole program, e.g. a test run, be put on one path or the other without touching its code
   if (const char* e = getenv("ZR_LSTM_SWEEP")) {
     const int v = atoi(e);
-    if (v >= 0 && v <= 2) c->lstm_sweep = v;
+    if (v >= 0 && v <= 3) c->lstm_sweep = v;
   }
   // the same for ZR_OPT_LSTM_SWEEP_SPIN and ZR_OPT_LSTM_STEP_WAIT_EXTRA (tests of a whole program's give-up handling)
   if (const char* e = getenv("ZR_LSTM_SWEEP_SPIN")) {
@@ -194,6 +194,9 @@ int zr_ctx_query(zr_ctx* ctx, int what, int* h_value) {
     case ZR_QUERY_LSTM_STACK_PATH:
       *h_value = ctx->last_stack_path;
       return ZR_OK;
+    case ZR_QUERY_LSTM_SWEEP_KERNEL:
+      *h_value = ctx->last_sweep_kernel;
+      return ZR_OK;
     case ZR_QUERY_SCRATCH_KIB:
       *h_value = (int)((ctx->scratch_bytes + ctx->scratch2_bytes + 1023) / 1024);
       return ZR_OK;
@@ -247,7 +250,7 @@ int zr_ctx_set_option(zr_ctx* ctx, int option, int value) {
       ctx->lstm_kparts = value;
       return ZR_OK;
     case ZR_OPT_LSTM_SWEEP:
-      ZR_CHECK_ARG(value >= 0 && value <= 2, "ZR_OPT_LSTM_SWEEP must be 0, 1 or 2");
+      ZR_CHECK_ARG(value >= 0 && value <= 3, "ZR_OPT_LSTM_SWEEP must be 0, 1, 2 or 3");
       ctx->lstm_sweep = value;
       return ZR_OK;
     case ZR_OPT_LSTM_SWEEP_SPIN:
