@@ -183,3 +183,53 @@ def test_node_on_narrow_row_tiles(ctx, H, mb):
                     assert_close(a.get(), want[k], what=k + " " + what)
     finally:
         layer.close()
+
+
+# Infinite values where a k-group is only partly filled: beside an infinity nothing may be multiplied by a zero that stands
+# for "not there".  H = 9, 100 and 101: the moved load of an embedding column's tail; 104: thirteen row tiles, whose last
+# 16-column k-group is half empty; 300 at 40 columns: 32-column tiles.
+@pytest.mark.parametrize("H,mb,L", [(9, 3, 1), (100, 8, 2), (101, 16, 1), (104, 8, 2), (300, 100, 1), (500, 12, 1), (1000, 12, 1)])
+def test_sweep_with_infinite_inputs_saturates(ctx, H, mb, L):
+    c = _case(H, mb, 4, L)
+    words = np.unique(c["ids"][c["ids"] >= 0])
+    for i, v in enumerate(words):  # at most one infinity a column: each gate's sum is then infinite and saturates
+        if i % 3:
+            c["embed"][H - 1 - (i % min(H, 6)), v] = np.inf if i % 2 else -np.inf
+    c["h0"][0][H - 1, 0] = np.inf
+    c["ids"][0, 0] = words[0]
+    want_h, want_c = _want(c)
+    assert np.isfinite(want_h).all() and np.isfinite(want_c).all()
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 3)
+    try:
+        h, x, _, path, _ = _run(ctx, c)
+    finally:
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
+    assert path == RESIDENT
+    assert_close(h, want_h, what="h")
+    assert_close(x, want_c, what="c")
+
+
+@pytest.mark.parametrize("H,mb", [(9, 3), (100, 8), (300, 20), (500, 12), (501, 37), (1000, 12), (1001, 70)])
+def test_node_with_infinite_inputs_saturates(ctx, H, mb):
+    g = synth.rng(47, H + mb)
+    ly = synth.lstm_layer(g, H, forget_bias_one=True)
+    x, hp = synth.uniform(g, (H, mb), -0.5, 0.5), np.tanh(synth.uniform(g, (H, mb), -1, 1))
+    cp, mask = synth.uniform(g, (H, mb), -0.5, 0.5), np.ones(mb, np.int32)
+    x[H - 1, 0], hp[H - 2, 1] = np.inf, -np.inf
+    for gate in range(4):
+        ly["M"][gate][H // 2, H - 1] = np.inf   # infinite weights meet column 0's infinity with one sign only
+        ly["Wh"][gate][H // 2 - 1, H - 3] = -np.inf
+    x[H - 1, 2:] = 0.25
+    want = o.lstm_step(ly["M"], ly["Wh"], ly["b"], x, hp, cp, mask)
+    fine = np.isfinite(want["h"])
+    assert fine.mean() > 0.85
+    layer = Layer(ctx, ly)
+    d_h, d_c = ctx.empty((H, mb)), ctx.empty((H, mb))
+    try:
+        ctx.lstm_step(layer.w, ctx.array(x), ctx.array(hp), ctx.array(cp), ctx.array(mask), mb, d_h, d_c)
+        ctx.sync()
+    finally:
+        layer.close()
+    assert np.array_equal(np.isfinite(d_h.get()), fine)
+    assert_close(np.where(fine, d_h.get(), 0), np.where(fine, want["h"], 0), what="h")
+    assert_close(np.where(fine, d_c.get(), 0), np.where(fine, want["c"], 0), what="c")

@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
   constexpr int COLS = NARROW ? 16 : 32 * TN;    // columns of the workgroup's tile
   constexpr int NPROD = NARROW ? 2 * NG : NG;    // producers of a wave's K slice
   constexpr int NOUT = (kRows * COLS + 511) / 512;  // (row, column) pairs a thread finishes
-  __shared__ float red[kWaves * COLS * kRedLd];
+  __shared__ float red[kWaves * COLS * kRedLd + kRows];  // (the last rows: read, not used, by threads that publish zeros)
   __shared__ int s_abort, s_last;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -104,14 +104,16 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
           const int c = cl + 16 * b;
           const float* m = P.W[l] + (s * 4 + (c >> 3)) * HH + 4 * (j0 + (c & 7));
           const int k0 = 4 * (KB * (kslice + kWaves * i) + kq);
-          if (s == 0 && from_embed) {
-            // embedding columns are read as they lie, so a lane's four k must stay inside the column: the last
-            // k-block of a column is moved down to end at H - 1, and what it covers twice counts once
+          if (s == 0 && from_embed && 4 * KB * (kslice + kWaves * i + 1) > H - 4) {  // uniform
+            // Embedding columns are read as they lie, so a lane's four k must stay inside the column: k-blocks that reach
+            // past its end, or lie behind it, are moved down to end at H - 1.  Every place that reads the same k keeps a part
+            // of its weight: not zero in all but one, for zero times an infinite activation is not zero.
             const int ks = k0 < H - 4 ? k0 : H - 4;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const int k = ks + e;
-              w[s][i][b][e] = k >= k0 ? m[(long long)(k >> 2) * (4 * P.ldw) + (k & 3)] : 0.0f;
+              w[s][i][b][e] = ldexpf(m[(long long)(k >> 2) * (4 * P.ldw) + (k & 3)],
+                                     -zr_resident_embed_halvings(H, NG * kWaves * KB, k0 >> 2, k));
             }
           } else {
             zr_f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -121,7 +123,9 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
           }
         }
 
-    // ---- the outputs this thread finishes: (row, column) pairs, rows of four fastest (the order h travels in)
+    // ---- the outputs this thread finishes: (row, column) pairs, rows of four fastest (the order h travels in).  A narrow
+    // k-group is two row tiles: behind an odd number of them the last one's workgroup also publishes a tile of zeros.
+    const int publishes = (NARROW && (P.j_tiles & 1) && jt == P.j_tiles - 1 ? 2 : 1) * kRows * COLS;
     int oj[NOUT], on[NOUT];
     bool ok[NOUT], tile_ok[NOUT];
     float bi[NOUT], bf[NOUT], bc[NOUT], bo[NOUT], c_state[NOUT];
@@ -132,7 +136,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
       oj[u] = ((o >> 2) / COLS) * 4 + (o & 3);
       on[u] = (o >> 2) % COLS;
       const int j = j0 + oj[u], n = n0 + on[u];
-      tile_ok[u] = o < kRows * COLS && n < mb;
+      tile_ok[u] = o < publishes && n < mb;
       ok[u] = tile_ok[u] && j < H;
       const int jc = j < H ? j : H - 1, nc = n < mb ? n : mb - 1;
       bi[u] = P.bias[l][jc], bf[u] = P.bias[l][H + jc], bc[u] = P.bias[l][2 * H + jc], bo[u] = P.bias[l][3 * H + jc];
@@ -225,9 +229,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
     }
     const unsigned kb_step = (unsigned)(kWaves * KB * P.mbp * 4);  // elements from a wave's group to its next
     const unsigned kb_first = (unsigned)((KB * kslice + kq) * P.mbp * 4);
-    // A narrow group is two row tiles; when only the first exists its last k-block stands in for the second's (it meets
-    // zero weights).  Groups past the end are not read at all: a line read before its producer's flag would go stale.
-    const unsigned kb_last = (unsigned)((2 * P.j_tiles - 1) * P.mbp * 4);
+    // Groups past the end are not read at all: a line read before its producer's flag would go stale.
     const int n_groups = (2 * P.j_tiles + KB - 1) / KB;
 
     typedef float acc16 __attribute__((ext_vector_type(16)));
@@ -276,8 +278,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
       auto load_packed = [&](const float* base) {
         return [=, &cols](zr_f32x4 (&x)[TN], int i) {
           if (kslice + kWaves * i < n_groups) {
-            unsigned kb = kb_first + (unsigned)i * kb_step;
-            if constexpr (NARROW) kb = kb < kb_last ? kb : kb_last;
+            const unsigned kb = kb_first + (unsigned)i * kb_step;
 #pragma unroll
             for (int tn = 0; tn < TN; ++tn) x[tn] = *(const zr_f32x4*)(base + (kb + 4u * (unsigned)cols[tn]));
           } else {

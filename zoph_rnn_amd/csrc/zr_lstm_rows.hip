@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
   auto load = [&](Frag& q) {
     const float* Ws = P.W + 4 * HH * ls;
     const int kb = KB * lg + kq;
-    const int kbc = NARROW && kb > kb_max ? kb_max : kb;  // (a narrow group may be half: its x is zero there)
+    const int kbc = NARROW && kb > kb_max ? kb_max : kb;  // (a narrow group may be half: made zero before it is multiplied)
 #pragma unroll
     for (int b = 0; b < NB; ++b) q.w[b] = *(const zr_f32x4*)(Ws + (woff[b] + (unsigned)(kbc * 4 * P.ldw)));
     const int k0 = 4 * kb;
@@ -138,6 +138,10 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
   auto mma = [&](Frag& q) {
     if (4 * KB * (mg + 1) > H) {  // the column ends inside this group: shift the moved loads back, zero what lies behind
       const int k0 = 4 * (KB * mg + kq);
+      if (NARROW && KB * mg + kq > kb_max) {  // (both operands: zero times an infinite weight is not zero)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) q.w[b] = zr_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
       const int d = k0 < H - 4 ? 0 : k0 - (H - 4);
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) {

@@ -12,9 +12,23 @@
 constexpr int kResidentRows = 8;  // hidden rows per workgroup
 
 constexpr int zr_resident_columns(int mb) { return (mb + 7) & ~7; }
-// floats of one hidden state (one layer, one time step)
+// floats of one hidden state (one layer, one time step): an even number of row tiles, two of which are a k-group of the
+// kernel's 16-column form
 constexpr long long zr_resident_slot(int H, int mb) {
-  return (long long)((H + kResidentRows - 1) / kResidentRows) * kResidentRows * zr_resident_columns(mb);
+  return (long long)((H + 2 * kResidentRows - 1) / (2 * kResidentRows)) * (2 * kResidentRows) * zr_resident_columns(mb);
 }
 // element (row k, column n) of a state; `columns` as above
 constexpr unsigned zr_resident_at(int k, int n, int columns) { return (unsigned)(((k >> 2) * columns + n) * 4 + (k & 3)); }
+
+// An embedding column of H values is read in `blocks` k-blocks of four; those that reach past its end or lie behind it are
+// moved down to end at H - 1 and read again what another block has read.  The part of weight k in block `block`, as the
+// number of times it is halved: the readers of one k, the block it lies in first and then the moved ones, have 1/2, 1/4, ...
+// of it and the last of them what is left.  The parts are powers of two and add up to one (to 2^-53, beyond 60 halvings).
+constexpr int zr_resident_embed_halvings(int H, int blocks, int block, int k) {
+  const int whole = H / 4;                 // blocks that lie inside the column as a whole
+  const int here = k < 4 * whole ? 1 : 0;  // k is also read where it lies
+  const int readers = k < H - 4 ? 1 : here + blocks - whole;
+  const int mine = block < whole ? 0 : here + block - whole;
+  const int halvings = mine < readers - 1 ? mine + 1 : readers - 1;
+  return halvings < 60 ? halvings : 60;
+}
