@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/zoph_rnn.h"
+#include "zr_rules.h"
 
 #define ZR_MAX_COUNTERS 4096
 #define ZR_MAX_STEP_FLAGS 16384
@@ -242,13 +243,10 @@ int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, cons
                            const float* const d_h0[], const float* const d_c0[], float clip_threshold,
                            float* const d_h_all[], float* const d_c_all[], float* const d_gates_all[]);
 
-// One node on tiles of 4 or 8 hidden rows (zr_lstm_rows.hip).  shape: 0 = 4 rows x 16 columns, 1 = 8 x 16, 2 = 8 x 32,
-// 3 = 8 x 64.  H >= 8; d_hp: h also k-interleaved [H/4][mb][4] (null: not wanted).
+// One node on tiles of 4 or 8 hidden rows (zr_lstm_rows.hip).  shape: as zr_lstm_rows_shape has it (zr_rules.h); d_hp: h also k-interleaved [H/4][mb][4] (null: not wanted).
 int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const float* const in[3], const int* d_gather_ids,
                       int V, const float* d_cprev, const int* d_mask01, float clip, int mb, float* d_h, float* d_c,
                       float* const d_gates[4], float* d_hp, int shape);
-// The shape for a node of this size (-1: leave it to lstm_fused_kernel).
-int zr_lstm_rows_shape(int H, int mb, int cu_count);
 
 // The attention step in one launch (zr_attn_step.hip).  a->d_hpack must hold h_t k-interleaved.  *took = 0: the
 // conditions do not hold and nothing was launched (the caller goes on with one launch per stage).

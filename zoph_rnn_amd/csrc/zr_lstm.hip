@@ -1601,7 +1601,7 @@ static int lstm_step_impl(zr_ctx* ctx, const zr_lstm_weights* w, const float* d_
     return zr_lstm_gates(ctx, (const float*)pre, b, d_cprev, d_mask01, clip_threshold, H, mb, d_h, d_c, d_gates);
   }
   if (!w->bf16 && !ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts) {
-    const int shape = zr_lstm_rows_shape(H, mb, ctx->cu_count);
+    const int shape = zr_lstm_rows_shape(H, mb, nseg, vec, ctx->cu_count);
     if (shape >= 0)
       return zr_lstm_rows_step(ctx, w, nseg, U.in, d_gather_ids, V, d_cprev, d_mask01, clip_threshold, mb, d_h, d_c,
                                d_gates, U.hp, shape);

@@ -223,24 +223,6 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
 
 }  // namespace
 
-// Tile by size, one node of H = 1000 / 500 / 300 at up to 128 columns, us (the register-streaming kernel of zr_lstm.hip
-// with K split across workgroups: 16-27 / 30-33 / 23-30):
-//   4 x 16:  13.0 at 12 columns /  6.4 at 12, 8.6 at 37 /  5.5 at 20      8 x 16:  11.5 at 12, 12.0 at 32 / 7.4 at 37 / 6.1
-//   8 x 32:  17.0 at 64 / 11.7 at 128 / 7.7 at 100                        8 x 64:  26.5 at 128 (26.7) / 16.8 at 128
-// The smallest tile that keeps the workgroups within one per compute unit wins, except that 4 x 16 tiles of H > 512 read the
-// activations once too often (13.0 against 11.5).  Wide tiles of a long K range lose to the streaming kernel (H = 2000, 64
-// columns: 71 against 48), and so does any that needs a second round of workgroups (H = 1000, 192 columns: 42-65 against
-// 37) -- where that kernel has its whole-group form, H % 8 == 0.
-int zr_lstm_rows_shape(int H, int mb, int cu_count) {
-  if (H < 8) return -1;
-  for (int shape = H > 512 ? 1 : 0; shape < 4; ++shape) {
-    const int rows = shape == 0 ? 4 : 8, cols = shape <= 1 ? 16 : (shape == 2 ? 32 : 64);
-    const long long wgs = (long long)((H + rows - 1) / rows) * ((mb + cols - 1) / cols);
-    if (wgs <= cu_count) return (shape >= 2 && H > 1024 && H % 8 == 0) ? -1 : shape;
-  }
-  return H % 8 == 0 ? -1 : 3;
-}
-
 int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const float* const in[3], const int* d_gather_ids,
                       int V, const float* d_cprev, const int* d_mask01, float clip, int mb, float* d_h, float* d_c,
                       float* const d_gates[4], float* d_hp, int shape) {
