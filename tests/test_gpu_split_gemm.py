@@ -86,7 +86,10 @@ def test_gemm_infinities_and_nan(ctx):
 
 
 @pytest.mark.parametrize("V,H,n,prepared", [(9001, 260, 520, True), (9001, 260, 520, False), (4133, 500, 1100, True),
-                                            (12000, 333, 257, True)])
+                                            (12000, 333, 257, True),
+                                            # the error pass with 2 columns a workgroup (a last chunk of one) and with 16
+                                            (1000, 64, 33, False), (1003, 30, 2, False), (1000, 100, 1000, True),
+                                            (4097, 52, 1001, False)])
 def test_output_layer(ctx, V, H, n, prepared):
     g = synth.rng(44, V + n)
     D = synth.uniform(g, (V, H), -0.2, 0.2)

@@ -1209,7 +1209,7 @@ static int softmax_backward(zr_ctx* ctx, const float* d_D, const float* d_b_d, i
                "zr_softmax_backward: null pointer");
   // logits, then in one pass over them the errors e = onehot - p (0 on masked columns), the sums of e over each chunk of
   // columns and the targets' probabilities
-  const int chunks = zr_softmax_error_chunks(n);
+  const int chunks = zr_softmax_error_chunks(V, n);
   void *s0 = nullptr, *s1 = nullptr;
   const size_t sums = ((size_t)V * chunks + 3) & ~(size_t)3;
   const float* e = d_prob_scratch;

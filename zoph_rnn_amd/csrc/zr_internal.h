@@ -225,9 +225,9 @@ int zr_softmax_forward_packed(zr_ctx* ctx, const float* d_D, const float* d_b_d,
                               const unsigned short* d_h_hi = nullptr, const unsigned short* d_h_lo = nullptr);
 
 // The output layer's errors: logits into d_out, then in place e = onehot(target) - p, 0 on masked columns.  Scratch slot 0,
-// of at least `bytes` (handed back in *out), starts with the sums of e over chunks of columns, [zr_softmax_error_chunks(n)]
-// [V], and, V * chunks rounded up to 4 floats on, the probability of every column's target.
-int zr_softmax_error_chunks(int n);
+// of at least `bytes` (handed back in *out), starts with the sums of e over chunks of columns, [zr_softmax_error_chunks
+// (V, n)][V], and, V * chunks rounded up to 4 floats on, the probability of every column's target.
+int zr_softmax_error_chunks(int V, int n);
 int zr_softmax_error(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, int H, const float* d_h, int n,
                      const int* d_target, const int* d_mask01, float* d_out, size_t bytes, void** out);
 

@@ -56,3 +56,15 @@ inline int zr_lstm_rows_shape(int H, int mb, int nseg, bool vec, int cus) {
   if (H % 8 == 0 && (rounds > 1 || H > 1024)) return -1;
   return rounds * (4.0 + 0.0115 * H * nseg) < zr_fused_node_us(H, mb, nseg, vec, cus) ? 3 : -1;
 }
+
+// ---- the output layer's error pass (softmax_error_kernel): columns a workgroup adds up, one after another
+
+// 32 keep the partial sums of the bias gradient small against the matrix.  Fewer where 1024-row blocks of 32 columns would
+// leave compute units without a workgroup: V = 1000, 33 columns are two workgroups, whose threads wait for 32 columns in turn
+// (the whole backward call 51 us against 41 with one column a workgroup and separate bias sums).
+inline int zr_softmax_error_cols(int V, int n) {
+  const long long row_blocks = (V + 1023) / 1024;
+  int cols = 32;
+  while (cols > 2 && row_blocks * ((n + cols - 1) / cols) < 256) cols /= 2;
+  return cols;
+}

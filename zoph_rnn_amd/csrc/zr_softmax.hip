@@ -58,20 +58,18 @@ softmax_normalize_kernel(const float* in, float* out, int V, const float* __rest
 }
 
 // x (V x n logits) -> e = onehot(target) - p in place, p = exp(x - max) / sum as softmax_normalize_kernel has it, 0 on masked
-// columns; the sums of e over the workgroup's ERROR_COLS columns to sums[blockIdx.y][V], and every column's target
-// probability.  The three readers of the probabilities (errors, gradient of the bias, loss) were passes of their own over
+// columns; the sums of e over the workgroup's `cols` columns to sums[blockIdx.y][V], and every column's target probability.  The three readers of the probabilities (errors, gradient of the bias, loss) were passes of their own over
 // the matrix: at 50000 x 6400 normalise 483, error 499, bias sums 250 us, bound by memory; this pass reads and writes once.
 // VEC: four consecutive rows per thread with 16-byte accesses (V % 4 == 0, x and sums 16-byte aligned).
-constexpr int ERROR_COLS = 32;
 template <bool VEC>
 __global__ void __launch_bounds__(256)
-softmax_error_kernel(float* __restrict__ x, int V, int n, const float* __restrict__ colstats, const int* __restrict__ target,
+softmax_error_kernel(float* __restrict__ x, int V, int n, int cols, const float* __restrict__ colstats, const int* __restrict__ target,
                      const int* __restrict__ mask01, float* __restrict__ sums, float* __restrict__ p_target) {
   constexpr int W = VEC ? 4 : 1;
   typedef float vec __attribute__((ext_vector_type(W)));
   const int v = (blockIdx.x * 256 + threadIdx.x) * W;
   if (v >= V) return;
-  const int n0 = blockIdx.y * ERROR_COLS, n1 = min(n, n0 + ERROR_COLS);
+  const int n0 = blockIdx.y * cols, n1 = min(n, n0 + cols);
   vec s = {};
 #pragma unroll 4
   for (int c = n0; c < n1; ++c) {
@@ -368,7 +366,7 @@ int zr_softmax_forward_packed(zr_ctx* ctx, const float* d_D, const float* d_b_d,
   return ZR_OK;
 }
 
-int zr_softmax_error_chunks(int n) { return (n + ERROR_COLS - 1) / ERROR_COLS; }
+int zr_softmax_error_chunks(int V, int n) { return (n + zr_softmax_error_cols(V, n) - 1) / zr_softmax_error_cols(V, n); }
 
 int zr_softmax_error(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, int H, const float* d_h, int n,
                      const int* d_target, const int* d_mask01, float* d_out, size_t bytes, void** out) {
@@ -382,13 +380,14 @@ int zr_softmax_error(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, i
   rc = zr_ctx_scratch(ctx, 0, bytes, out);
   if (rc) return rc;
   float* sums = (float*)*out;
-  float* p_target = sums + (((size_t)V * zr_softmax_error_chunks(n) + 3) & ~(size_t)3);
+  const int chunks = zr_softmax_error_chunks(V, n), cols = zr_softmax_error_cols(V, n);
+  float* p_target = sums + (((size_t)V * chunks + 3) & ~(size_t)3);
   if (V % 4 == 0 && (((uintptr_t)d_out & 15u) == 0)) {
-    const dim3 grid((V / 4 + 255) / 256, zr_softmax_error_chunks(n));
-    softmax_error_kernel<true><<<grid, 256, 0, ctx->stream>>>(d_out, V, n, colstats, d_target, d_mask01, sums, p_target);
+    const dim3 grid((V / 4 + 255) / 256, chunks);
+    softmax_error_kernel<true><<<grid, 256, 0, ctx->stream>>>(d_out, V, n, cols, colstats, d_target, d_mask01, sums, p_target);
   } else {
-    const dim3 grid((V + 255) / 256, zr_softmax_error_chunks(n));
-    softmax_error_kernel<false><<<grid, 256, 0, ctx->stream>>>(d_out, V, n, colstats, d_target, d_mask01, sums, p_target);
+    const dim3 grid((V + 255) / 256, chunks);
+    softmax_error_kernel<false><<<grid, 256, 0, ctx->stream>>>(d_out, V, n, cols, colstats, d_target, d_mask01, sums, p_target);
   }
   ZR_LAUNCH_CHECK("softmax_error_kernel");
   return ZR_OK;
