@@ -1344,7 +1344,8 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
     // Wide batches: the tall and row-range kernels serve up to 256 columns as well or better (50000 x 192 x 1000: 167
     // against 175 us), beyond that the split product does (33333 x 700 x 500: 174 against 602 us).
     if (d.nseg == 1 && zcount == 1 && !d.b_packed && d.groups == 0 && ctx->gemm_cfg == 0 && !ctx->fixed_scratch && d.N > 256 &&
-        (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) && zr_split_gemm_takes(d.M, d.N, d.K[0]))
+        (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) &&
+        zr_split_gemm_takes_product(d.M, d.N, d.K[0], false, d.epilogue == ZR_EPI_SOFTMAX_PARTIAL, ctx->cu_count))
       return zr_split_gemm(ctx, d.M, d.N, d.K[0], d.A[0], d.lda[0], ZR_SPLIT_PACK4, d.B[0], d.ldb[0], ZR_SPLIT_K_FAST, d.C,
                            d.ldc, d.bias, d.epilogue == ZR_EPI_SOFTMAX_PARTIAL ? d.partials : nullptr, d.accumulate);
     bool xpack = vec && d.M >= 2048 && d.groups == 0 && !d.b_packed;
@@ -1426,7 +1427,8 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
     return launch_pack4<2, 2, 2>(ctx, ga, d.epilogue, vec, zcount);
   }
   if (d.nseg == 1 && zcount == 1 && d.groups == 0 && ctx->gemm_cfg == 0 && !ctx->fixed_scratch &&
-      (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) && zr_split_gemm_takes(d.M, d.N, d.K[0]))
+      (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) &&
+      zr_split_gemm_takes_product(d.M, d.N, d.K[0], d.trans_a != 0, d.epilogue == ZR_EPI_SOFTMAX_PARTIAL, ctx->cu_count))
     return zr_split_gemm(ctx, d.M, d.N, d.K[0], d.A[0], d.lda[0], d.trans_a ? ZR_SPLIT_K_FAST : ZR_SPLIT_ROW_FAST, d.B[0],
                          d.ldb[0], ZR_SPLIT_K_FAST, d.C, d.ldc, d.bias,
                          d.epilogue == ZR_EPI_SOFTMAX_PARTIAL ? d.partials : nullptr, d.accumulate);

@@ -193,7 +193,6 @@ enum ZrSplitLayout {
   ZR_SPLIT_ROW_FAST = 1,  // [row + k*ld]
   ZR_SPLIT_PACK4 = 2      // the k-interleaved fp32 copy (ZrGemmDesc::a_pack = 1); A only, with B ZR_SPLIT_K_FAST
 };
-bool zr_split_gemm_takes(int M, int N, int K);  // whether a product of this size is faster that way
 int zr_split_gemm(zr_ctx* ctx, int M, int N, int K, const float* A, long long lda, int a_layout, const float* B,
                   long long ldb, int b_layout, float* C, long long ldc, const float* bias, float* partials, int accumulate);
 

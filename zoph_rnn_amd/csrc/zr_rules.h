@@ -68,3 +68,44 @@ inline int zr_softmax_error_cols(int V, int n) {
   while (cols > 2 && row_blocks * ((n + cols - 1) / cols) < 256) cols /= 2;
   return cols;
 }
+
+// ---- large fp32 products: the split product (zr_split_gemm.hip) or the fp32 kernels
+
+// Estimated microseconds of a split product's launch of `wgs` workgroups of `steps` steps of 32 k each, on tiles of 128 rows x
+// 64 * tnw columns.  A step of one workgroup alone on its compute unit, of two, of three sharing it (measured; 128-column
+// tiles hold three, 256-column tiles two).
+inline double zr_split_launch_us(int tnw, long long wgs, int steps, int cus) {
+  const double us128[4] = {0.0, 2.8, 3.7, 5.0}, us256[3] = {0.0, 3.7, 5.8};
+  const int cap = tnw == 4 ? 2 : 3;
+  const double* us = tnw == 4 ? us256 : us128;
+  const long long per_cu = (wgs + cus - 1) / cus;
+  return ((double)(per_cu / cap) * us[cap] + us[per_cu % cap]) * (steps + 1.5);
+}
+
+// Against the fp32 kernels (both with their launches' own preparation, us): 10001 x 300 x 700 63 / 97, 300 x 700 x 10001
+// 62 / 101, 4000 x 1000 x 6400 312 / 472, 33333 x 700 x 500 174 / 327; but 1000 x 128 x 4000 40 / 40 and 1200 x 300 x
+// 700 30 / 20: up to 10^9 multiply-adds, or with an output that fills few tiles, there is too little to win.
+inline bool zr_split_gemm_takes(int M, int N, int K) {
+  return M >= 256 && N >= 256 && K >= 256 && (double)M * N * K > 1.0e9;
+}
+
+// The same for a product as zr_gemm_launch has it, whose other choice is one launch without transposes.  Two places where
+// the line above lies too low:
+//   * Outputs of one to four 32 x 32 blocks a compute unit, row-major operands (M < 2048: beyond that the fp32 choice is
+//     another kernel): one wave per block leaves little idle there.  512 x 512 x 4096 37 / 31, 1000 x 1000 x 1000 41 / 34,
+//     1001 x 1001 x 1003 42 / 36, 1000 x 1000 x 1100 38 / 38; against it 1500 x 1500 x 500 40 / 64, 300 x 300 x 12000 51 / 89.
+//   * The logits with their block statistics, which cannot divide K: a few tiles then walk all of it.  The fp32 kernels
+//     reach half of 95 TFLOP/s or more.  2000 x 512 x 1000 (64 tiles) 82-92 / 38-42, 2000 x 1024 x 1000 (128) 96 / 64, 5000 x
+//     400 x 500 (160) 56 / 42; 5000 x 512 x 500 (160) 57 / 79, 2000 x 1100 x 1000 (144) 98 / 131.
+inline bool zr_split_gemm_takes_product(int M, int N, int K, bool k_fast_a, bool statistics, int cus) {
+  if (!zr_split_gemm_takes(M, N, K)) return false;
+  const double macs = (double)M * N * K;
+  if (statistics) {
+    const long long m_tiles = (M + 127) / 128;
+    const double narrow = zr_split_launch_us(2, m_tiles * ((N + 127) / 128), (K + 31) / 32, cus);
+    const double wide = zr_split_launch_us(4, m_tiles * ((N + 255) / 256), (K + 31) / 32, cus);
+    return (narrow < wide ? narrow : wide) <= 2.1 * macs * 2.0 / 95.0e6;
+  }
+  const long long blocks = (long long)((M + 31) / 32) * ((N + 31) / 32);
+  return k_fast_a || M >= 2048 || blocks < cus || blocks > 4 * cus || macs >= 1.1e9;
+}

@@ -394,24 +394,7 @@ void launch_layouts(const SplitArgs& a, int al, int bl, unsigned grid, hipStream
     launch<TNW, ZR_SPLIT_ROW_FAST, ZR_SPLIT_ROW_FAST>(a, grid, stream);
 }
 
-// Estimated microseconds of a launch of `wgs` workgroups of `steps` steps each.  A step of one workgroup alone on its
-// compute unit, of two, of three sharing it (measured; 128-column tiles hold three, 256-column tiles two).
-double launch_us(int tnw, long long wgs, int steps, int cus) {
-  static const double us128[4] = {0.0, 2.8, 3.7, 5.0}, us256[3] = {0.0, 3.7, 5.8};
-  const int cap = tnw == 4 ? 2 : 3;
-  const double* us = tnw == 4 ? us256 : us128;
-  const long long per_cu = (wgs + cus - 1) / cus;
-  return ((double)(per_cu / cap) * us[cap] + us[per_cu % cap]) * (steps + 1.5);
-}
-
 }  // namespace
-
-// Against the fp32 kernels (both with their launches' own preparation, us): 10001 x 300 x 700 63 / 97, 300 x 700 x 10001
-// 62 / 101, 4000 x 1000 x 6400 312 / 472, 33333 x 700 x 500 174 / 327; but 1000 x 128 x 4000 40 / 40 and 1200 x 300 x
-// 700 30 / 20: below 10^9 multiply-adds, or with an output that fills few tiles, there is too little to win.
-bool zr_split_gemm_takes(int M, int N, int K) {
-  return M >= 256 && N >= 256 && K >= 256 && (double)M * N * K >= 1.0e9;
-}
 
 int zr_split_gemm(zr_ctx* ctx, int M, int N, int K, const float* A, long long lda, int a_layout, const float* B,
                   long long ldb, int b_layout, float* C, long long ldc, const float* bias, float* partials, int accumulate) {
@@ -440,7 +423,7 @@ int zr_split_gemm(zr_ctx* ctx, int M, int N, int K, const float* A, long long ld
     for (int p = 1; p <= 64; ++p) {
       const size_t bytes = sizeof(float) * (size_t)M * N * p;
       if (p > 1 && (K < p * 4 * KC || bytes > most)) break;
-      const double us = launch_us(w, tiles * p, (K + p * KC - 1) / (p * KC), cus) + (p > 1 ? 6.0 + (double)bytes / 4.0e6 : 0.0);
+      const double us = zr_split_launch_us(w, tiles * p, (K + p * KC - 1) / (p * KC), cus) + (p > 1 ? 6.0 + (double)bytes / 4.0e6 : 0.0);
       if (best == 0.0 || us < best) best = us, tnw = w, a.parts = p;
     }
   }
