@@ -1,7 +1,7 @@
 """The weight gradients of a single node, C += A B^T over the minibatch, on the kernel that reads both operands as they lie:
 zr_lstm_feed_backward's (4H x H) and, two at a time, zr_attn_backward's (H x H, tests/test_gpu_backward.py holds their
-values).  Sizes at the edges of its 32 x 32 tiles and of its rounds of 32 columns, and one beyond its range (257 columns),
-which the transposing products serve.
+values).  Sizes at the edges of its 32 x 32 tiles, of its rounds of 32 columns and of its range (96 columns for the smaller H,
+256 from H = 274 on), beyond which the transposing products serve.
 Tolerance: K products summed one after another in fp32 and added to C are off by at most (K + 2) 2^-24 times the sum of the
 terms' magnitudes; the product instruction may add its two k at a time, which is not more."""
 import numpy as np
@@ -20,7 +20,7 @@ def ctx():
 
 
 @pytest.mark.parametrize("H,mb", [(8, 1), (9, 2), (8, 31), (31, 32), (33, 33), (63, 64), (65, 65), (100, 8), (129, 255), (300, 20),
-                                  (64, 256), (64, 257), (500, 64), (1000, 128)])
+                                  (64, 256), (64, 257), (500, 64), (1000, 128), (64, 96), (64, 97), (274, 255), (275, 256), (300, 257)])
 def test_feed_gradient_against_64_bits(ctx, H, mb):
     r = np.random.default_rng(1000 * H + mb)
     Q = [np.asfortranarray(r.uniform(-0.08, 0.08, (H, H)).astype(np.float32)) for _ in range(4)]

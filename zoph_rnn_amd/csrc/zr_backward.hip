@@ -610,10 +610,6 @@ int row_sum_launch(zr_ctx* ctx, const float* a, int rows, long long n, float* ou
   return ZR_OK;
 }
 
-// outer_accumulate_kernel's range: at 256 columns its lead over a transpose and the LDS-tiled product is nearly gone for the
-// stacked (4H x H) gradient (H = 1000, zr_lstm_feed_backward, us: 128 columns 61 / 79, 256 86 / 88).
-bool outer_takes(int M, int N, int K) { return K <= 256 && !zr_split_gemm_takes(M, N, K); }
-
 int outer_launch(zr_ctx* ctx, const OuterProducts& P, int count, int M, int N, int K) {
   outer_accumulate_kernel<<<dim3((M + 63) / 64, (N + 63) / 64, count), 256, 0, ctx->stream>>>(P, M, N, K);
   ZR_LAUNCH_CHECK("outer_accumulate_kernel");
@@ -1051,7 +1047,7 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
 
   attn_bwd_e_kernel<<<eg, 256, 0, ctx->stream>>>(d_err_htild, d_h_tild, d_mask01, H, (long long)n, e);
   ZR_LAUNCH_CHECK("attn_bwd_e_kernel");
-  const bool outer = outer_takes(H, H, mb);
+  const bool outer = zr_outer_takes(2, H, H, mb);
   if (outer) {
     rc = outer_launch(ctx, OuterProducts{{e, e}, {d_c_t, d_h_t}, {grads->d_W_c1, grads->d_W_c2}}, 2, H, H, mb);
     if (rc) return rc;
@@ -1158,7 +1154,7 @@ int zr_lstm_feed_backward(zr_ctx* ctx, const float* const d_Q[4], int H, int mb,
   }
   // Q gradients, stacked over the gates like the M and W_h gradients: dQ (4H x H) += dgates (4H x mb) * h~^T
   // (src/LSTM.hpp:1014-1050)
-  if (outer_takes(4 * H, H, mb)) return outer_launch(ctx, OuterProducts{{d_dgates}, {d_htild}, {d_dQ_stack}}, 1, 4 * H, H, mb);
+  if (zr_outer_takes(1, 4 * H, H, mb)) return outer_launch(ctx, OuterProducts{{d_dgates}, {d_htild}, {d_dQ_stack}}, 1, 4 * H, H, mb);
   void* scratch = nullptr;
   rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (size_t)H * mb, &scratch);
   if (rc) return rc;

@@ -109,3 +109,13 @@ inline bool zr_split_gemm_takes_product(int M, int N, int K, bool k_fast_a, bool
   const long long blocks = (long long)((M + 31) / 32) * ((N + 31) / 32);
   return k_fast_a || M >= 2048 || blocks < cus || blocks > 4 * cus || macs >= 1.1e9;
 }
+
+// ---- weight gradients of a single node (outer_accumulate_kernel), `count` products a launch, K = the minibatch
+
+// Against a transpose and the LDS-tiled product each, us of the whole call.  Two H x H at a time (zr_attn_backward): faster at
+// every size up to 256 columns, a third over all.  One 4H x H (zr_lstm_feed_backward): H = 1000, 128 columns 63 / 82, 200
+// 75 / 89; but small ones do not fill the chip with waves that each walk all columns: H = 64, 192 columns 20.8 / 19.1, 256
+// 23.2 / 19.5, H = 256, 192 columns 27.3 / 25.2, where 64 columns are 16.1 / 17.0 and 22.9 / 23.9.
+inline bool zr_outer_takes(int count, int M, int N, int K) {
+  return K <= (count > 1 || (long long)M * N >= 300000 ? 256 : 96) && !zr_split_gemm_takes(M, N, K);
+}
