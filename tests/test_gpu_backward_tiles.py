@@ -1,6 +1,7 @@
 """The error products of the backward pass, W_h^T dg and M^T dg, over the tiles they can run on: 32 x 32 with K split over
-eight waves, up to 256 of them a grouped launch (two nodes of H = 1000 at 64 columns are the last shape), 64 x 64 beyond, and
-hidden sizes that are no multiple of four.  Each is compared with the product in 64 bits of the gate errors the library itself left.
+eight waves, up to 256 of them a grouped launch (two nodes of H = 1000 at 64 columns) or, beyond 32 columns, 384 (the same at
+65 columns), 64 x 64 beyond, and hidden sizes that are no multiple of four.  Each is compared with the product in 64 bits of the
+gate errors the library itself left.
 Tolerance: K = 4H products and their sums, each rounded to fp32 at most once a term: (4H + 2) 2^-24 of the sum of the terms'
 magnitudes."""
 import numpy as np

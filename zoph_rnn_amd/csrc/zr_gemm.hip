@@ -1409,11 +1409,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
       const long long t32 = (long long)((d.M + 31) / 32) * ((d.N + 31) / 32) * zcount;
       long long ktot = 0;
       for (int s = 0; s < d.nseg; ++s) ktot += d.K[s];
-      // Grouped (the error products of a diagonal of the backward sweep, K = 4H): up to one such workgroup a compute unit;
-      // well above that 64 x 64 tiles read each operand half as often.  Sweep over 20-24 steps, us, 64 x 64 / 32 x 32 tiles
-      // by the 32 x 32 tiles of a full diagonal: 80 (2 x 300, 64 columns) 682 / 351, 128 (2 x 500, 64) 1156 / 540, 256 (2 x
-      // 1000, 64) 1662 / 721, 512 (2 x 1000, 128) 1718 / 1482, 768 (3 x 1000, 128) 1766 / 2151.
-      if (ctx->gemm_cfg == 0 && t32 <= (d.groups > 0 ? 256 : 768) && ktot >= 512) {
+      if (ctx->gemm_cfg == 0 && (d.groups > 0 ? zr_grouped_small_tiles(t32, d.N, ctx->cu_count) : t32 <= 768) && ktot >= 512) {
         ga.m_tiles = (ga.M + 31) / 32;
         ga.n_tiles = (ga.N + 31) / 32;
         if (vec) return launch_epi<1, 1, 8, 1, ZR_A_PACK4, true, 1>(ctx, ga, zcount, d.epilogue);

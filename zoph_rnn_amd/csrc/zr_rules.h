@@ -119,3 +119,17 @@ inline bool zr_split_gemm_takes_product(int M, int N, int K, bool k_fast_a, bool
 inline bool zr_outer_takes(int count, int M, int N, int K) {
   return K <= (count > 1 || (long long)M * N >= 300000 ? 256 : 96) && !zr_split_gemm_takes(M, N, K);
 }
+
+// ---- grouped products (the error products of a diagonal of the backward sweep, K = 4H): `tiles` of 32 x 32 with K over eight
+// waves, or 64 x 64 tiles (64 x 32 up to 32 columns)
+
+// Up to one such workgroup a compute unit the small tiles take half the time or less: whole sweeps of 20-24 steps, 80 tiles a
+// full diagonal (2 x 300, 64 columns) 682 -> 351 us, 128 (2 x 500, 64) 1156 -> 540, 256 (2 x 1000, 64) 1662 -> 721.  With up to
+// one and a half, in two rounds, a sweep is 9 to 13 % faster than on 64 x 64 tiles (2 x 768, 128 columns, 12 steps 789 -> 701;
+// 3 x 300, 192 columns 474 -> 482 the one exception of 37) -- but not up to 32 columns, where the larger tiles leave no more
+// idle (4 x 1200, 32 columns 746 -> 989).  Up to two workgroups a compute unit it goes either way: 2 x 1000, 128 columns
+// 970 -> 884, 4 x 500, 128 columns 665 -> 588, but 2 x 600, 192 columns 719 -> 804 and 4 x 300, 192 columns 531 -> 571, without
+// a size that tells them apart; beyond that it loses (3 x 1000, 128 columns 1098 -> 1317).
+inline bool zr_grouped_small_tiles(long long tiles, int columns, int cus) {
+  return tiles <= cus || (columns > 32 && 2 * tiles <= 3LL * cus);
+}
