@@ -231,12 +231,9 @@ int zr_softmax_error(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, i
                      const int* d_target, const int* d_mask01, float* d_out, size_t bytes, void** out);
 
 // The whole sweep with the weights held in registers (zr_lstm_resident.hip), as one launch or, when not all layers fit on
-// the device at once, a few.  The plan: which kernel, how many layers a launch; its value is the estimated time in us
-// (negative: the shape does not fit).  The caller poisons the outputs of an abandoned sweep (lstm_sweep_poison_kernel).
-struct ZrResidentPlan {
-  int size_class, col_class, n_tiles, at_once, flag_stride;
-};
-double zr_lstm_resident_plan(zr_ctx* ctx, int nl, int H, int mb, int T, ZrResidentPlan* plan);
+// the device at once, a few.  The plan (zr_rules.h): which kernel, how many layers a launch; us < 0: the shape does not fit.
+// The caller poisons the outputs of an abandoned sweep (lstm_sweep_poison_kernel).
+ZrResidentPlan zr_lstm_resident_plan(zr_ctx* ctx, int nl, int H, int mb, int T);
 int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, const zr_lstm_weights* const layers[],
                            const float* d_embed, int V, const int* d_ids_nonneg, const int* d_mask01, int T, int mb,
                            const float* const d_h0[], const float* const d_c0[], float clip_threshold,

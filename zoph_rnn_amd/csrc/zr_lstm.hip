@@ -1846,33 +1846,17 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
                              8LL * layers[0]->kp * layers[0]->ldw * 4 < lim;
     if (!offsets_fit || (tn && nl * ((n32 + tn - 1) / tn) > 512) || (long long)T * j_tiles >= kSweepGaveUp) tn = 0;
   }
-  // Which schedule: the least estimated time, us a step (for the sweep with resident weights see zr_lstm_resident_plan).
-  // Against what was measured (layers x H at columns):
-  //   streamed sweep: 5 + the K loop of a workgroup (the groups of 8 k of both segments over 4 waves, 16 TN instructions
-  //     of 64 cycles each at 2.3 GHz), half a step more per layer to fill: 4 x 1000 at 128 61 / 61, 2 x 600 at 100 22 / 25;
-  //   a launch per diagonal: 10 + the longer of the weights at 5 TB/s and the K loop of a 32-column tile, divided over as
-  //     many workgroups as bring the launch nearest to one per compute unit, times the rounds those then need: 4 x 1000 at
-  //     16 36 / 30, 1 x 1000 at 128 24 / 25, 2 x 1000 at 33 24 / 25, 2 x 600 at 100 27 / 32; H % 8 != 0 has no K split
-  //     and slower loads: 4 x 300 at 200 38 / 38.
+  // Which schedule: the least estimated time (zr_rules.h).
   if (single_ok) {
-    const double k_loop = 2.0 * ((H + 7) / 8) / 4 * 16 * 64 / 2300.0;
-    double diag_us = -1.0;
-    if (!ctx->lstm_sweep) {
-      const double weights_us = 32.0 * H * H * nl / 5e6;
-      const long long tiles = (long long)groups * n32;
-      const long long parts = tiles >= ctx->cu_count ? 1 : (ctx->cu_count + tiles / 2) / tiles;
-      const double loop_us = (double)((tiles * parts + ctx->cu_count - 1) / ctx->cu_count) * k_loop / parts;
-      diag_us = (T + nl - 1) * (10.0 + (weights_us > loop_us ? weights_us : loop_us)) * (H % 8 ? 1.4 : 1.0);
-    }
-    const double sweep_us = tn ? (T + 0.5 * nl) * (5.0 + k_loop * tn) : -1.0;
-    if (tn && diag_us > 0.0 && diag_us < sweep_us) tn = 0;
+    const double diag_us = zr_sweep_diagonals_us(nl, H, mb, T, vec, ctx->cu_count);
+    const double sweep_us = tn ? zr_sweep_streamed_us(nl, H, T, tn) : -1.0;
+    if (tn && !ctx->lstm_sweep && diag_us < sweep_us) tn = 0;
     const double other_us = tn ? sweep_us : diag_us;
-    ZrResidentPlan plan;
-    plan.at_once = 0;
+    ZrResidentPlan plan = {};
     // option 2: the streamed sweep where it fits, 3: the one with resident weights where that fits
     if (ctx->lstm_sweep == 2 ? !tn : ctx->lstm_sweep == 3 || (!ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts)) {
-      const double resident_us = zr_lstm_resident_plan(ctx, nl, H, mb, T, &plan);
-      if (resident_us < 0.0 || (!ctx->lstm_sweep && other_us > 0.0 && other_us <= resident_us)) plan.at_once = 0;
+      plan = zr_lstm_resident_plan(ctx, nl, H, mb, T);
+      if (plan.us < 0.0 || (!ctx->lstm_sweep && other_us <= plan.us)) plan.at_once = 0;
     }
     if (plan.at_once) {
       rc = zr_lstm_resident_sweep(ctx, plan, nl, layers, d_embed, V, d_ids_nonneg, d_mask01, T, mb, d_h0, d_c0,

@@ -398,7 +398,6 @@ const ResidentKernel kKernels[4][3] = {
     {lstm_resident_kernel<2, 1, true>, lstm_resident_kernel<4, 1, false>, lstm_resident_kernel<4, 2, false>},
     {lstm_resident_kernel<4, 1, true>, lstm_resident_kernel<8, 1, false>, lstm_resident_kernel<8, 2, false>},
     {lstm_resident_kernel<8, 1, true>, lstm_resident_kernel<16, 1, false>, nullptr}};
-constexpr int kColumns[3] = {16, 32, 64};
 
 int resident_capacity(zr_ctx* ctx, int size_class, int col_class) {
   int& cached = ctx->resident_capacity[size_class][col_class];
@@ -419,41 +418,15 @@ int resident_capacity(zr_ctx* ctx, int size_class, int col_class) {
 
 }  // namespace
 
-double zr_lstm_resident_plan(zr_ctx* ctx, int nl, int H, int mb, int T, ZrResidentPlan* plan) {
-  plan->at_once = 0;
-  if (H < 8 || H > 1024 || nl > kMaxLayers || T >= kResidentGaveUp / 2) return -1.0;
+ZrResidentPlan zr_lstm_resident_plan(zr_ctx* ctx, int nl, int H, int mb, int T) {
+  ZrResidentPlan plan = {};
+  plan.us = -1.0;
+  if (H < 8 || H > 1024 || nl > kMaxLayers || T >= kResidentGaveUp / 2) return plan;
+  if (zr_resident_slot(H, mb) * 4 >= (1LL << 32)) return plan;
   const int size_class = H <= 128 ? 0 : (H <= 256 ? 1 : (H <= 512 ? 2 : 3));
-  const int j_tiles = (H + kRows - 1) / kRows;
-  const int nprod = 2 << size_class;  // NPROD of the kernel, in every column class
-  const int flag_stride = (kWaves * nprod + 31) / 32 * 32;
-  const long long slot = zr_resident_slot(H, mb);
-  if (slot * 4 >= (1LL << 32)) return -1.0;
-  // Column class and layers per launch: the cheapest by the time a step takes -- a hand-over of 3.2 us and the matrix
-  // instructions of both segments at 2.3 GHz, two waves to a SIMD and as many workgroups to a compute unit as the launch
-  // needs, times what the shorter prefetch of the wider tiles costs.  Measured against the estimate, us a step: H = 500,
-  // 16 columns 4.9 / 5.0, 32 columns 8.2 / 8.5; H = 1000, 16 columns 6.8 / 6.8, 32 columns 15.8 / 15.6.
-  double best = -1.0;
-  for (int c = 0; c < 3; ++c) {
-    const int n_tiles = (mb + kColumns[c] - 1) / kColumns[c];
-    int at_once = resident_capacity(ctx, size_class, c) / (j_tiles * n_tiles);
-    if (at_once > nl) at_once = nl;
-    while (at_once > 0 && at_once * n_tiles * flag_stride > ZR_MAX_STEP_FLAGS - 32) --at_once;
-    if (at_once < 1) continue;
-    const int per_cu = (at_once * j_tiles * n_tiles + ctx->cu_count - 1) / ctx->cu_count;
-    const int groups = c == 0 ? (H + 127) / 128 : (H + 63) / 64;  // of a wave and segment
-    const double stretch = c == 0 ? 1.0 : (c == 2 ? 1.6 : (size_class == 3 ? 1.75 : 1.5));
-    const double step = 3.2 + stretch * per_cu * 2.0 * groups * 4 * (c == 2 ? 128 : 64) * 2 / 2300.0;
-    const double us = (double)((nl + at_once - 1) / at_once) * (T + at_once - 1) * step;
-    if (best < 0.0 || us < best) {
-      best = us;
-      plan->size_class = size_class;
-      plan->col_class = c;
-      plan->n_tiles = n_tiles;
-      plan->at_once = at_once;
-      plan->flag_stride = flag_stride;
-    }
-  }
-  return best;
+  int capacity[3];
+  for (int c = 0; c < 3; ++c) capacity[c] = resident_capacity(ctx, size_class, c);
+  return zr_sweep_resident_plan(nl, H, mb, T, capacity, ZR_MAX_STEP_FLAGS - 32, ctx->cu_count);
 }
 
 int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, const zr_lstm_weights* const layers[],

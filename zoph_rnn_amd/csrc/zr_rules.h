@@ -4,11 +4,14 @@
 
 // ---- one LSTM node: tiles of 4 or 8 hidden rows (zr_lstm_rows.hip) or launch_fused (zr_lstm.hip)
 
-// launch_fused's time for a single fp32 node, us.  vec: H % 4 == 0 and 16-byte aligned inputs.  Follows its own choice of
-// kernel; the constants are fitted to H = 300 .. 1500 at 64 .. 512 columns, two and three segments, and hold to about 10 %.
-inline double zr_fused_node_us(int H, int mb, int nseg, bool vec, int cus) {
-  const int j = (H + 31) / 32, n32 = (mb + 31) / 32;
+// launch_fused's time for `units` independent fp32 nodes in one launch, us.  vec: H % 4 == 0 and 16-byte aligned inputs.  Follows
+// its own choice of kernel; the constants are fitted to H = 64 .. 2000 at 1 .. 512 columns, one node with two and three segments
+// and up to four nodes with two, and hold to about 10 % (H below 200: 20 %).  No launch beats its weights at 7 TB/s.
+inline double zr_fused_us(int units, int H, int mb, int nseg, bool vec, int cus) {
+  const int j = units * ((H + 31) / 32), n32 = (mb + 31) / 32;
   const int whole = j * ((n32 + 1) / 2);
+  const double weights = 6.0 + 16.0 * units * nseg * H * H / 7.0e6;
+  double us;
   if (H % 8 == 0 && vec && whole < 200) {
     const int tiles = j * n32;
     int parts = (cus + tiles / 2) / tiles;
@@ -16,20 +19,27 @@ inline double zr_fused_node_us(int H, int mb, int nseg, bool vec, int cus) {
     if (parts > 8) parts = 8;
     if (parts >= 2) {  // K split across workgroups; the row tiles are dealt to the eight dies
       const int rounds = ((j + 7) / 8 * n32 * parts + cus / 8 - 1) / (cus / 8);
-      return rounds * (6.5 + 0.8 * parts + 0.018 * H / parts * nseg);
+      us = rounds * (6.5 + 0.8 * parts + 0.018 * H / parts * nseg);
+      return us > weights ? us : weights;
     }
   } else if (vec && n32 >= 3 && whole < 200) {  // weights through LDS
     const int tiles = j * ((n32 + 3) / 4);
     int parts = cus / (tiles * nseg);
     if (parts > 8) parts = 8;
+    if (parts > (H + 31) / 32) parts = (H + 31) / 32;
     if (parts < 1) parts = 1;
     const int rounds = (tiles * nseg * parts + cus - 1) / cus;
-    return rounds * (12.5 + 0.075 * H / parts + 3.0 * parts);
+    us = rounds * (12.5 + 0.075 * H / parts + 3.0 * parts);
+    return us > weights ? us : weights;
   }
+  const bool fast = H % 8 == 0 && vec;  // whole k-groups, wide loads
   const int tn = n32 >= 2 && whole > 128 ? 2 : 1;
   const int wgs = j * ((n32 + tn - 1) / tn);
-  if (wgs < 192) return 0.033 * H * nseg * tn;
-  return (wgs + cus - 1) / cus * (5.0 + (tn == 2 ? 0.036 : 0.0205) * H * nseg);
+  if (wgs < 192)
+    us = 6.0 + (fast ? (tn == 2 ? 0.014 : 0.0165) : (vec ? 0.026 : 0.030)) * H * nseg * tn;
+  else
+    us = (wgs + cus - 1) / cus * (6.5 + (tn == 2 ? (fast ? 0.0295 : 0.036) : (fast ? 0.0165 : 0.0205)) * H * nseg);
+  return us > weights ? us : weights;
 }
 
 // Tile by size, one node of H = 1000 / 500 / 300 at up to 128 columns, us (the register-streaming kernel of zr_lstm.hip
@@ -54,7 +64,75 @@ inline int zr_lstm_rows_shape(int H, int mb, int nseg, bool vec, int cus) {
     rounds = (int)((wgs + cus - 1) / cus);
   }
   if (H % 8 == 0 && (rounds > 1 || H > 1024)) return -1;
-  return rounds * (4.0 + 0.0115 * H * nseg) < zr_fused_node_us(H, mb, nseg, vec, cus) ? 3 : -1;
+  return rounds * (4.0 + 0.0115 * H * nseg) < zr_fused_us(1, H, mb, nseg, vec, cus) ? 3 : -1;
+}
+
+// ---- the sweep of a stack (zr_lstm_stack_forward): one launch per diagonal, one launch with streamed weights
+// (lstm_sweep_kernel), or with its weights in registers (lstm_resident_kernel).  Estimates in us; the least one is taken.
+// Against 1812 sizes (H = 64 .. 2000, 1 to 4 layers, 1 to 256 columns, 12 and 50 steps; all that fit measured for each) the
+// choice is 0.2 % from the best schedule on average, more than 10 % for about one size in a hundred.
+
+// One launch per diagonal: the first and last few have fewer layers than the others.
+inline double zr_sweep_diagonals_us(int nl, int H, int mb, int T, bool vec, int cus) {
+  const int full = nl < T ? nl : T;
+  double us = (T + nl - 1 - 2 * (full - 1)) * zr_fused_us(full, H, mb, 2, vec, cus);
+  for (int units = 1; units < full; ++units) us += 2.0 * zr_fused_us(units, H, mb, 2, vec, cus);
+  return us;
+}
+
+// Streamed weights on tiles of 32 * tn columns: a hand-over of 5 us, a little more with every layer, and the K loop of a workgroup (the groups of 8 k of both
+// segments over 4 waves, 16 tn instructions of 64 cycles each at 2.3 GHz), or the weights at 6 TB/s where they outgrow the
+// caches (4 layers of H = 2000 87 us a step, 61 by the K loop); half a step more per layer to fill.
+inline double zr_sweep_streamed_us(int nl, int H, int T, int tn) {
+  const double k_loop = 2.0 * ((H + 7) / 8) / 4 * 16 * 64 / 2300.0 * tn, weights = 32.0 * nl * H * H / 6.0e6;
+  return (T + 0.5 * nl) * (4.9 + 0.25 * nl + (k_loop > weights ? k_loop : weights));
+}
+
+// Resident weights, one launch of `layers` layers (the sweep's first or a later one): classes by H up to 128, 256, 512, 1024 and
+// by 16, 32, 64 columns a workgroup.  A time step takes what its class takes -- every workgroup has the registers, and walks
+// the k-groups, of the largest H of the class -- as long as each compute unit has one workgroup (H = 500: 4.1 us at 16 to 64
+// columns on 16-column tiles, 7.2-7.5 at 16 to 128 columns on 32-column tiles).  Later launches read h and no embedding.  With
+// two workgroups on some compute units a step takes about that much longer and the two get in each other's way (H = 500, 504
+// workgroups: 11.1), less so when they belong to different layers.  Filling the registers costs a few us a layer.
+inline double zr_sweep_resident_us(int size_class, int col_class, bool first, int layers, long long wgs, int T, int cus) {
+  const double step_first[4][3] = {{2.45, 3.1, 4.6}, {3.05, 4.15, 8.6}, {4.15, 6.9, 15.0}, {6.3, 11.5, 0.0}};
+  const double step_later[4][3] = {{2.4, 3.0, 4.6}, {3.0, 4.1, 6.7}, {4.1, 6.0, 11.0}, {6.0, 10.4, 0.0}};
+  const double two[3][2] = {{1.0, 1.0}, {1.4, 0.6}, {1.8, 0.5}}, two_wide[3][2] = {{1.3, 0.6}, {1.7, 0.3}, {1.7, 0.3}};
+  const double fill[4] = {1.0, 2.5, 4.5, 9.0};
+  double step = (first ? step_first : step_later)[size_class][col_class];
+  if (wgs > cus && size_class < 3) {
+    const double* f = (col_class ? two_wide : two)[size_class];
+    step *= f[0] + f[1] * ((double)wgs / cus - 1.0) - (col_class == 0 && size_class == 2 && layers > 1 ? 0.35 : 0.0);
+  }
+  return (T + layers - 1) * step + 6.0 + fill[size_class] * layers;
+}
+
+// Column class and layers a launch: the cheapest of those that fit.  capacity: workgroups of each column class the device holds
+// at once (0: no such kernel); flags: hand-over flags there are.  us < 0: none fits.
+constexpr int kResidentColumns[3] = {16, 32, 64};
+struct ZrResidentPlan {
+  int size_class, col_class, n_tiles, at_once, flag_stride;
+  double us;
+};
+inline ZrResidentPlan zr_sweep_resident_plan(int nl, int H, int mb, int T, const int capacity[3], int flags, int cus) {
+  ZrResidentPlan plan = {H <= 128 ? 0 : (H <= 256 ? 1 : (H <= 512 ? 2 : 3)), 0, 0, 0, 0, -1.0};
+  const int row_tiles = (H + 7) / 8;
+  const int producers = 2 << plan.size_class;  // of a wave's K slice, in every column class
+  plan.flag_stride = (8 * producers + 31) / 32 * 32;
+  for (int c = 0; c < 3; ++c) {
+    const int n_tiles = (mb + kResidentColumns[c] - 1) / kResidentColumns[c];
+    int at_once = capacity[c] / (row_tiles * n_tiles);
+    if (at_once > nl) at_once = nl;
+    while (at_once > 0 && (long long)at_once * n_tiles * plan.flag_stride > flags) --at_once;
+    if (at_once < 1) continue;
+    double us = 0.0;
+    for (int l = 0; l < nl; l += at_once) {
+      const int now = nl - l < at_once ? nl - l : at_once;
+      us += zr_sweep_resident_us(plan.size_class, c, l == 0, now, (long long)now * row_tiles * n_tiles, T, cus);
+    }
+    if (plan.us < 0.0 || us < plan.us) plan.us = us, plan.col_class = c, plan.n_tiles = n_tiles, plan.at_once = at_once;
+  }
+  return plan;
 }
 
 // ---- the output layer's error pass (softmax_error_kernel): columns a workgroup adds up, one after another
