@@ -53,6 +53,20 @@ def test_static_scratch_entry_point_matches_allocating_one_twice_in_a_row(prepar
         ctx.close()
 
 
+@pytest.mark.parametrize("prepared", [True, False])
+@pytest.mark.parametrize("V,H,mb", [(10001, 300, 400), (4133, 500, 1100), (33333, 260, 300)])
+def test_static_scratch_entry_point_takes_the_same_product_for_wide_batches(V, H, mb, prepared):
+    """Sizes at which the allocating entry point multiplies on the bf16 matrix cores (three exact terms an operand)."""
+    ctx = capi.Context(0)
+    try:
+        got, _ = _run(ctx, V, H, mb, capi.ZR_SOFTMAX_LOGPROB, prepared, 5, static=True)
+        assert ctx.query(capi.ZR_QUERY_SCRATCH_KIB) == 0
+        want, _ = _run(ctx, V, H, mb, capi.ZR_SOFTMAX_LOGPROB, prepared, 5, static=False)
+        assert np.array_equal(got, want), "static-scratch result differs from the allocating entry point"
+    finally:
+        ctx.close()
+
+
 def test_static_scratch_entry_point_rejects_what_does_not_fit():
     ctx = capi.Context(0)
     try:

@@ -1342,12 +1342,20 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
       ga.b_pack4 = 1;
     }
     // Wide batches: the tall and row-range kernels serve up to 256 columns as well or better (50000 x 192 x 1000: 167
-    // against 175 us), beyond that the split product does (33333 x 700 x 500: 174 against 602 us).
-    if (d.nseg == 1 && zcount == 1 && !d.b_packed && d.groups == 0 && ctx->gemm_cfg == 0 && !ctx->fixed_scratch && d.N > 256 &&
-        (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) &&
-        zr_split_gemm_takes_product(d.M, d.N, d.K[0], false, d.epilogue == ZR_EPI_SOFTMAX_PARTIAL, ctx->cu_count))
+    // against 175 us), beyond that the split product does (33333 x 700 x 500: 174 against 602 us).  With fixed scratch
+    // buffers only the statistics form, which needs none of them, and only where the fp32 kernels' copy of B would fit: the
+    // limit of the entry point does not follow the kernel.
+    if (d.nseg == 1 && zcount == 1 && !d.b_packed && d.groups == 0 && ctx->gemm_cfg == 0 && d.N > 256 &&
+        ((d.epilogue == ZR_EPI_STORE && !ctx->fixed_scratch) || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) &&
+        zr_split_gemm_takes_product(d.M, d.N, d.K[0], false, d.epilogue == ZR_EPI_SOFTMAX_PARTIAL, ctx->cu_count)) {
+      if (ctx->fixed_scratch && vec && d.M >= 2048 && d.K[0] % 8 == 0) {
+        void* p = nullptr;
+        const int rc = zr_ctx_scratch(ctx, 0, sizeof(float) * (size_t)d.K[0] * d.N, &p);
+        if (rc) return rc;
+      }
       return zr_split_gemm(ctx, d.M, d.N, d.K[0], d.A[0], d.lda[0], ZR_SPLIT_PACK4, d.B[0], d.ldb[0], ZR_SPLIT_K_FAST, d.C,
                            d.ldc, d.bias, d.epilogue == ZR_EPI_SOFTMAX_PARTIAL ? d.partials : nullptr, d.accumulate);
+    }
     bool xpack = vec && d.M >= 2048 && d.groups == 0 && !d.b_packed;
     size_t xfloats = 0;
     for (int s = 0; s < d.nseg; ++s) {
@@ -1422,8 +1430,8 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
     if (d.N <= 32) return launch_pack4<2, 1, 2>(ctx, ga, d.epilogue, vec, zcount);
     return launch_pack4<2, 2, 2>(ctx, ga, d.epilogue, vec, zcount);
   }
-  if (d.nseg == 1 && zcount == 1 && d.groups == 0 && ctx->gemm_cfg == 0 && !ctx->fixed_scratch &&
-      (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) &&
+  if (d.nseg == 1 && zcount == 1 && d.groups == 0 && ctx->gemm_cfg == 0 &&
+      ((d.epilogue == ZR_EPI_STORE && !ctx->fixed_scratch) || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) &&
       zr_split_gemm_takes_product(d.M, d.N, d.K[0], d.trans_a != 0, d.epilogue == ZR_EPI_SOFTMAX_PARTIAL, ctx->cu_count))
     return zr_split_gemm(ctx, d.M, d.N, d.K[0], d.A[0], d.lda[0], d.trans_a ? ZR_SPLIT_K_FAST : ZR_SPLIT_ROW_FAST, d.B[0],
                          d.ldb[0], ZR_SPLIT_K_FAST, d.C, d.ldc, d.bias,
