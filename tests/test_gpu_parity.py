@@ -919,7 +919,9 @@ def test_decoder_step_single_launch_abandoned_wait_is_reported(ctx, H, mb, L):
                                                    (256, 64, 3, 30, 50, 40000, True),
                                                    # v_p at a 4-byte offset (see below)
                                                    (1000, 128, 4, 20, 10, 5000, "v_p off by 4 bytes"),
-                                                   (64, 5, 2, 9, 3, 301, "v_p off by 4 bytes")])
+                                                   (64, 5, 2, 9, 3, 301, "v_p off by 4 bytes"),
+                                                   # an output layer for the split product, and one too small for it
+                                                   (512, 288, 2, 12, 5, 12000, True), (512, 288, 1, 7, 3, 4000, True)])
 def test_decoder_step_as_one_call_matches_the_three_calls(ctx, H, mb, L, S, D, V, prepared):
     """zr_decoder_step (forward_prop_target as one call, hand-overs kept in the matrix cores' layout) against
     zr_lstm_decoder_step + zr_attn_step + zr_softmax_forward on the same inputs: the same kernels read the same numbers,

@@ -159,7 +159,8 @@ softmax_loss_kernel(const float* __restrict__ logits, int V, int mb, const doubl
 }
 
 // d_h_packed: optional k-interleaved copy of d_h ([H/4][mb][4]); used when the product runs on the registered fp32 copy
-// of D and H % 8 == 0 (the product then skips its own re-layout of d_h).
+// of D and H % 8 == 0 (the product then skips its own re-layout of d_h), but not where the split product takes the call,
+// which reads d_h as it lies: with and without the copy the same kernel runs.
 // d_partials_ext: where the [mb][nblocks][2] pairs go instead of context scratch (ZR_SOFTMAX_LOGITS_BLOCKS: the caller's
 // buffer; no column statistics follow them there).
 int logits_with_partials(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, int H, const float* d_h, int mb,
@@ -185,8 +186,9 @@ int logits_with_partials(zr_ctx* ctx, const float* d_D, const float* d_b_d, int 
   for (int i = 0; i < ZR_MAX_PACKED_D; ++i) {
     const zr_ctx::PackedD& e = ctx->packed_d[i];
     if (e.key == d_D && e.V == V && e.H == H) {  // registered with zr_softmax_prepare: use the MFMA-layout copy
-      // ... unless the batch is thousands of columns wide (all time steps of a training minibatch at once): there
-      // the LDS-staged kernel on the plain matrix is faster than the register-streaming one on the fp32 copy
+      // ... unless the batch is thousands of columns wide (all time steps of a training minibatch at once) and too small a
+      // product for the split terms, which read either form: there the LDS-staged kernel on the plain matrix is faster than
+      // the register-streaming one on the fp32 copy
       if (!e.bf16 && mb > 1024) break;
       d.A[0] = (const float*)e.d_pack;
       d.lda[0] = e.ldp;
@@ -196,7 +198,8 @@ int logits_with_partials(zr_ctx* ctx, const float* d_D, const float* d_b_d, int 
   }
   d.B[0] = d_h;
   d.ldb[0] = H;
-  if (d_h_packed && d.a_pack == 1 && H % 8 == 0 && (((uintptr_t)d_h_packed & 15u) == 0)) {
+  const bool split = mb > 256 && zr_split_gemm_takes_product(V, mb, H, false, true, ctx->cu_count);
+  if (d_h_packed && d.a_pack == 1 && H % 8 == 0 && (((uintptr_t)d_h_packed & 15u) == 0) && !split) {
     d.B[0] = d_h_packed;
     d.b_packed = 1;
   }
