@@ -219,9 +219,11 @@ __global__ void __launch_bounds__(256) transpose_wide_kernel(const float* __rest
 
 // Row sums of a (rows x n, column-major): a workgroup adds 64 columns (chunk blockIdx.y) of 64 rows, its threads W rows
 // wide and 256 * W / 64 columns deep, and adds the threads' sums through LDS in a fixed order.  Several chunks leave
-// partial sums [chunk][rows], which the same kernel adds up.  Every thread has at most a few loads, all in flight at once:
-// 2000 x 64 (a training step's node) 17.8 us with one thread running down the columns, 4000 x 6400 64.4 + 27.2 us.
-// W = 4 needs rows % 4 == 0 and 16-byte alignment.
+// partial sums [chunk][rows], which a second pass of the same kernel adds up, all chunks in one workgroup's columns.  With W
+// = 4 a thread of the first pass has four loads, all in flight at once (W = 1: sixteen, four at a time); in the second it
+// has one for every sixteen chunks: 100 chunks of 4000 x 6400 seven, 65535 chunks, the most there can be, 4096.  2000 x 64 (a
+// training step's node) took 17.8 us with one thread running down the columns and takes 4.6, 4000 x 6400 64.4 + 27.2 and
+// 17.1 + 5.  W = 4 needs rows % 4 == 0 and 16-byte alignment.
 template <int W>
 __global__ void __launch_bounds__(256) row_sum_kernel(const float* __restrict__ a, int rows, long long n, long long chunk,
                                                       float* __restrict__ out, int accumulate) {

@@ -22,8 +22,8 @@
 // tile.  Progress, bounded waits and the abandon protocol are those of lstm_sweep_kernel; a workgroup that gives up marks
 // its own flag, which makes everybody who depends on it give up in turn.  The last workgroup out clears the flags.
 //
-// Measured, whole sweep, against one launch per diagonal: 1 layer of H = 100, 8 columns, 20 steps 55 us (253); 2 of 500,
-// 20 columns, 35 steps 180 us (1130); 4 of 1000, 16 columns, 50 steps 700 us (1600), 1 column, 25 steps 370 us (800).
+// Measured, whole sweep, against one launch per diagonal: 1 layer of H = 100, 8 columns, 20 steps 52 us (253); 2 of 500,
+// 20 columns, 35 steps 169 us (1130); 4 of 1000, 50 steps, 16 columns 706 us (1575), 1 column 670 us (1520).
 // Tried: finishing waves that publish on their own while the others run ahead into the next step (300 against 180 us at
 // H = 500: the waves that are ahead poll, and their polls hold up the publishing stores); a first look at the flags of
 // the layer below a step early (no change).

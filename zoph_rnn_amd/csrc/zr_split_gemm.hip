@@ -1,19 +1,22 @@
 // Large fp32 products on the bf16 matrix cores, without giving up any of the operands' 24 bits.
 //
 // x = x1 + x2 + x3 with x1 = x rounded to bf16, x2 = x - x1 rounded to bf16 and x3 the rest, which has at most 8 bits:
-// every subtraction is exact and nothing of x is lost.  x*y is taken as the six products x1y1, x1y2, x2y1, x2y2, x1y3 and
-// x3y1 (the three left out are below 2^-24 of x*y and of either sign), each exact, summed in the fp32 accumulator.  (A
-// product below about 2^-100 has its smaller terms among the subnormal numbers: its absolute error is of that size.)
+// every subtraction is exact and nothing of x is lost while the third term is a normal number, |x| above about 2^-110.
+// x*y is taken as the six products x1y1, x1y2, x2y1, x2y2, x1y3 and x3y1 (the three left out are below 2^-24 of x*y and of
+// either sign), each exact, summed in the fp32 accumulator.  (A product below about 2^-100 has its smaller terms among the
+// subnormal numbers: its absolute error is of that size.)  A sum of many terms carries no more error than with the fp32
+// instructions; a sum that is one large term may carry three roundings of it instead of one.
 // Six 32x32x16 bf16 instructions take 192 cycles of a matrix core for the work of eight 32x32x2 fp32 ones at 64 cycles
 // each.  Against 64 bits, normal operands, relative 2-norm, beside the fp32 instructions': K = 500 3.3e-7 / 3.8e-7, 1000
 // 4.7e-7 / 5.5e-7, 6400 1.3e-6 / 1.4e-6, 50000 1.9e-6 / 4.0e-6.
 //
 // What bounds it: the conversion (11 vector instructions for two values' three terms) and the LDS traffic beside the
-// matrix cores, which are busy about 45 % of the time.  The operands are read as fp32, as they lie, and split on their way
-// into LDS, 32 k at a time; every fragment read from LDS then feeds several of the six products.  A workgroup of four waves
-// has a tile of 128 x 128 (64 x 64 a wave, three workgroups a compute unit) or 128 x 256 (64 x 128 a wave, two), one LDS
-// buffer, and the next step's values in registers while it multiplies: the workgroups of a compute unit cover each other's
-// conversions and barriers.  50000 x 6400 x 1000: 128 x 128 tiles 3.94 ms, 128 x 256 3.49 (184 TFLOP/s of fp32 work;
+// matrix cores, which are busy 51 to 66 % of the time in the products of a large training step and 26 to 54 % in smaller
+// launches (a third of the cycles LDS is busy are bank conflicts).  The operands are read as fp32, as they lie, and split
+// on their way into LDS, 32 k at a time; every fragment read from LDS then feeds several of the six products.  A workgroup
+// of four waves has a tile of 128 x 128 (64 x 64 a wave, three workgroups a compute unit) or 128 x 256 (64 x 128 a wave,
+// two), one LDS buffer, and the next step's values in registers while it multiplies: the workgroups of a compute unit cover
+// each other's conversions and barriers.  50000 x 6400 x 1000: 128 x 128 tiles 3.94 ms, 128 x 256 3.49 (184 TFLOP/s of fp32 work;
 // the fp32 instructions' kernel 5.70); 4000 x 1000 x 6400 0.47 -> 0.31; 33333 x 700 x 500 0.60 -> 0.16.
 #include "zr_internal.h"
 
@@ -176,6 +179,8 @@ __device__ __forceinline__ long long element(long long row, long long k, long lo
 
 // The same sums with fp32 instructions straight from memory: for a wave whose accumulators came out infinite or NaN.
 // The terms of an infinite operand are infinity and NaN, so only this says what the sum of the operands' products is.
+// It is the slow way, for the waves concerned only: 4000 x 1000 x 6400 takes 319 us, 748 with one NaN in A, 945 with one
+// in B, 1049 with nothing finite in B (the fp32 kernels 500 in every case); 20000 x 6400 x 1000 1507, 1871, 1720, 4991 (2130).
 template <int TNW, int AL, int BL, bool ROWS_FIRST>
 __device__ __forceinline__ void plain_tile(const SplitArgs& a, zr_f32x16 (&acc)[2][TNW], int m0, int n0, int k_begin,
                                            int k_end, int lane) {
