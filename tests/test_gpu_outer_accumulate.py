@@ -42,3 +42,22 @@ def test_feed_gradient_against_64_bits(ctx, H, mb):
     ctx.sync()
     got = d_dQ.get()
     assert not np.isfinite(got[0]).any() and np.all(np.abs(got[1:] - want[1:]) <= bound[1:])
+
+
+@pytest.mark.parametrize("H,mb", [(64, 96), (300, 128), (500, 256), (1000, 200)])
+def test_feed_gradient_is_rounded_in_short_chains(ctx, H, mb):
+    """Four sums of a quarter of the products each, not one of all.  An addition rounds its result by a relative 2^-23 / sqrt(12)
+    * 0.73 = 2.5e-8 in the 2-norm (mantissas spread evenly in their logarithm); the n partial sums of a chain have
+    half the final square on average, and independent roundings add in squares: sqrt(n / 2) of them, n = mb / 4, and three for
+    the chains' sum.  A quarter above that passes (measured 5 % above); one chain would be twice it."""
+    r = np.random.default_rng(2000 * H + mb)
+    Q = [np.zeros((H, H), np.float32, order="F") for _ in range(4)]
+    dg = np.asfortranarray(r.uniform(-1, 1, (4 * H, mb)).astype(np.float32))
+    ht = np.asfortranarray(r.uniform(-1, 1, (H, mb)).astype(np.float32))
+    d_dQ = ctx.zeros((4 * H, H))
+    d_Q, d_dg, d_ht, d_err = [ctx.array(q) for q in Q], ctx.array(dg), ctx.array(ht), ctx.empty((H, mb))
+    ctx.lstm_feed_backward(d_Q, H, mb, d_dg, d_ht, d_err, d_dQ)
+    ctx.sync()
+    want = dg.astype(np.float64) @ ht.astype(np.float64).T
+    error = np.linalg.norm(d_dQ.get() - want) / np.linalg.norm(want)
+    assert error < 1.25 * 2.5e-8 * np.sqrt(mb / 8 + 3)

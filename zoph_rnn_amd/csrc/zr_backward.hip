@@ -253,6 +253,9 @@ __global__ void __launch_bounds__(256) row_sum_kernel(const float* __restrict__ 
 // weight gradients of a single attention or feed-input node, K = the minibatch.  Both operands have their rows contiguous
 // for every k, which is how the matrix instruction wants them: a half-wave reads 32 rows of one column, no transpose and no
 // LDS.  A wave has a 32 x 32 tile, A's rows on the lanes so that C is read and written 32 consecutive floats at a time.
+// Four accumulators, for every fourth instruction: a sum is rounded in chains of K / 4 products (error against 64 bits, 4000 x
+// 1000, 128 columns 1.1e-7, 256 1.5e-7; with one chain 2.0e-7 and 2.9e-7), and an instruction need not wait for the one before (8
+// columns of a 64 x 256 problem 15.4 -> 14.1 us, the attention node's whole backward pass 49.7 -> 45.8 at H = 100).
 // Bound by the trip to memory for the operands and C, and by the launch.
 // Two of 500 x 500 at 64 columns 7.1 us, the launch included; the 20 target nodes of an encoder-decoder training step (2 x 500,
 // 64 columns) took 9.15 ms with a transpose and a tiled product each, 8.35 with this (W_c1^T e and W_c2^T e joined as well).
@@ -289,19 +292,19 @@ __global__ void __launch_bounds__(256) outer_accumulate_kernel(OuterProducts P, 
     const int n = n0 + 8 * (q >> 2) + 4 * half + (q & 3);
     old[q] = m < M && n < N ? c[(size_t)n * M] : 0.0f;
   }
-  zr_f32x16 acc = {};
+  zr_f32x16 acc[4] = {};
   for (int k0 = 0; k0 < K; k0 += 2 * U) {
     float ac[U], bc[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) ac[u] = av[u], bc[u] = bv[u];
     if (k0 + 2 * U < K) fetch(k0 + 2 * U);
 #pragma unroll
-    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(bc[u], ac[u], acc, 0, 0, 0);
+    for (int u = 0; u < U; ++u) acc[u & 3] = __builtin_amdgcn_mfma_f32_32x32x2f32(bc[u], ac[u], acc[u & 3], 0, 0, 0);
   }
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     const int n = n0 + 8 * (q >> 2) + 4 * half + (q & 3);
-    if (m < M && n < N) c[(size_t)n * M] = old[q] + acc[q];
+    if (m < M && n < N) c[(size_t)n * M] = old[q] + ((acc[0][q] + acc[1][q]) + (acc[2][q] + acc[3][q]));
   }
 }
 
