@@ -233,3 +233,49 @@ def test_node_with_infinite_inputs_saturates(ctx, H, mb):
     assert np.array_equal(np.isfinite(d_h.get()), fine)
     assert_close(np.where(fine, d_h.get(), 0), np.where(fine, want["h"], 0), what="h")
     assert_close(np.where(fine, d_c.get(), 0), np.where(fine, want["c"], 0), what="c")
+
+
+def _sigmoid(v):
+    return 1.0 / (1.0 + np.exp(-v))
+
+
+def _cell_in_64_bits(z, c):
+    zi, zf, zc, zo = np.split(z, 4)
+    c = _sigmoid(zf) * c + _sigmoid(zi) * np.tanh(zc)
+    return _sigmoid(zo) * np.tanh(c), c
+
+
+def _wide(layer, key):
+    return np.concatenate([np.asarray(a, np.float64).reshape(layer["b"][0].size, -1) for a in layer[key]])
+
+
+def _rough_layer(g, H, **kw):
+    """Weights large enough that the products' rounding is most of the error of h."""
+    layer = synth.lstm_layer(g, H, **kw)
+    return {k: [synth.uniform(g, a.shape, -1.5 / H ** 0.5, 1.5 / H ** 0.5) for a in v] for k, v in layer.items()}
+
+
+# one size of every form whose sums go through LDS in pieces or have two accumulators, where the launches per diagonal divide K
+@pytest.mark.parametrize("H,mb", [(200, 16), (400, 8), (512, 16), (768, 1), (768, 40), (1000, 16), (1024, 8), (1024, 40)])
+def test_sweep_rounds_no_more_than_one_launch_per_diagonal(ctx, H, mb):
+    """The two schedules' errors against 64 bits, each an average over T * H * mb values.  How they vary between draws of that
+    size is a few per cent; one chain of additions a wave was 1.25 (H = 512) to 1.6 times (1024) the other schedule's error."""
+    g, T, V = synth.rng(47, H + mb), 12, 300
+    c = dict(H=H, mb=mb, T=T, L=1, V=V, ids=g.integers(0, V, size=(T, mb)).astype(np.int32),
+             embed=synth.uniform(g, (H, V), -1, 1), layers=[_rough_layer(g, H)], h0=[np.zeros((H, mb), np.float32)],
+             c0=[np.zeros((H, mb), np.float32)])
+    M, W, b = [_wide(c["layers"][0], k) for k in ("M", "Wh", "b")]
+    want, hp, cp = [], np.zeros((H, mb)), np.zeros((H, mb))
+    for t in range(T):
+        hp, cp = _cell_in_64_bits(M @ c["embed"][:, c["ids"][t]].astype(np.float64) + W @ hp + b, cp)
+        want.append(hp)
+    error = {}
+    for option in (1, 3):
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, option)
+        try:
+            h, _, _, path, _ = _run(ctx, c, clip=0.0)
+        finally:
+            ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
+        assert (path == RESIDENT) == (option == 3)
+        error[option] = np.linalg.norm(h[0] - np.stack(want)) / np.linalg.norm(want)
+    assert error[3] < 1.1 * error[1]

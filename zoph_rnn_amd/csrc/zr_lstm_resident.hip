@@ -75,7 +75,19 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
   constexpr int COLS = NARROW ? 16 : 32 * TN;    // columns of the workgroup's tile
   constexpr int NPROD = NARROW ? 2 * NG : NG;    // producers of a wave's K slice
   constexpr int NOUT = (kRows * COLS + 511) / 512;  // (row, column) pairs a thread finishes
+  // A long chain of fp32 additions rounds more than the schedule with one launch per diagonal, which divides K further.  So
+  // the sums are taken in pieces: two accumulators, for even and odd k, in narrow tiles up to H = 256, whose registers
+  // allow it; else the sums of CHAIN k-groups go to LDS and the accumulators start from zero again (wide tiles of H <= 256
+  // have short chains as they are).  Error of h against 64 bits, one layer, 12 steps: H = 1024, 16 columns 3.9e-7 without, 2.2e-7
+  // (2.4e-7 with one launch per diagonal), 512 3.0e-7, 2.3e-7 (2.4e-7), 1000 at 40 columns 3.9e-7, 2.7e-7 (3.0e-7).  Costs 0 to 2 %
+  // of a sweep, 4 % at up to 4 columns of 256 < H <= 512.  (Two accumulators there: 12 %, for registers; the sums back from LDS
+  // before the last group: 1.5 %.)
+  constexpr int NACC = NARROW && NG <= 2 ? 2 : 1;
+  constexpr bool PIECES = NG >= (NARROW ? 4 : 8);
+  constexpr int CHAIN = NARROW ? 4 : 16;
+  constexpr bool SUMS_AHEAD = !NARROW || NG > 4;  // the sums come back from LDS before the last group
   __shared__ float red[kWaves * COLS * kRedLd + kRows];  // (the last rows: read, not used, by threads that publish zeros)
+  __shared__ float s_bias[4][kRows];  // (registers are short)
   __shared__ int s_abort, s_last;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -128,7 +140,8 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
     const int publishes = (NARROW && (P.j_tiles & 1) && jt == P.j_tiles - 1 ? 2 : 1) * kRows * COLS;
     int oj[NOUT], on[NOUT];
     bool ok[NOUT], tile_ok[NOUT];
-    float bi[NOUT], bf[NOUT], bc[NOUT], bo[NOUT], c_state[NOUT];
+    float c_state[NOUT];
+    if (tid < 4 * kRows) s_bias[tid / kRows][tid % kRows] = P.bias[l][tid / kRows * H + min(j0 + tid % kRows, H - 1)];
     unsigned hp_off[NOUT];  // element inside a slot
 #pragma unroll
     for (int u = 0; u < NOUT; ++u) {
@@ -139,7 +152,6 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
       tile_ok[u] = o < publishes && n < mb;
       ok[u] = tile_ok[u] && j < H;
       const int jc = j < H ? j : H - 1, nc = n < mb ? n : mb - 1;
-      bi[u] = P.bias[l][jc], bf[u] = P.bias[l][H + jc], bc[u] = P.bias[l][2 * H + jc], bo[u] = P.bias[l][3 * H + jc];
       c_state[u] = P.c0[l][(long long)nc * H + jc];
       hp_off[u] = zr_resident_at(j, n, P.mbp);
     }
@@ -235,30 +247,62 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
     typedef float acc16 __attribute__((ext_vector_type(16)));
     for (int t = 0; t < P.T; ++t) {
       acc16 acc[TN];
-      zr_f32x4 acc4[NB];
+      zr_f32x4 acc4[NACC][NB];
+      auto clear = [&]() {
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn)
+        for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[tn][r] = 0.0f;
+          for (int r = 0; r < 16; ++r) acc[tn][r] = 0.0f;
 #pragma unroll
-      for (int b = 0; b < NB; ++b) acc4[b] = {0.0f, 0.0f, 0.0f, 0.0f};
-
-      auto mma = [&](const zr_f32x4 (&x)[TN], const float (&wg)[NB][4]) {
+        for (int q = 0; q < NACC; ++q)
+#pragma unroll
+          for (int b = 0; b < NB; ++b) acc4[q][b] = {0.0f, 0.0f, 0.0f, 0.0f};
+      };
+      clear();
+      // Partial sum u of this lane, and its place in LDS (the wave's own; free since the barrier behind the last cell).
+      constexpr int NE = NARROW ? 4 * NB : 16 * TN;
+      auto element = [&](int u) -> float {
+        if constexpr (!NARROW)
+          return acc[u >> 4][u & 15];
+        else if constexpr (NACC == 2)
+          return acc4[0][u >> 2][u & 3] + acc4[1][u >> 2][u & 3];
+        else
+          return acc4[0][u >> 2][u & 3];
+      };
+      float* mine = red + kslice * (COLS * kRedLd) + 4 * kq * kRedLd + cl;
+      auto place = [&](int u) -> float& {
+        return NARROW ? mine[(u & 3) * kRedLd + 16 * (u >> 2)] : mine[((u >> 4) * 32 + 8 * ((u >> 2) & 3) + (u & 3)) * kRedLd];
+      };
+      float before[PIECES ? NE : 1];  // the sums of all but the last chain
+      auto mma = [&](int seg, int i, const zr_f32x4 (&x)[TN], const float (&wg)[NB][4]) {
+        if (PIECES && SUMS_AHEAD && seg == 1 && i == NG - 1) {  // on their way while the last group is multiplied
+#pragma unroll
+          for (int u = 0; u < NE; ++u) before[PIECES ? u : 0] = place(u);
+          __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if constexpr (NARROW) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b) acc4[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0][e], wg[b][e], acc4[b], 0, 0, 0);
+            for (int b = 0; b < NB; ++b) {
+              zr_f32x4& a = acc4[e & (NACC - 1)][b];
+              a = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0][e], wg[b][e], a, 0, 0, 0);
+            }
           } else {
 #pragma unroll
             for (int tn = 0; tn < TN; ++tn)
               acc[tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[tn][e], wg[0][e], acc[tn], 0, 0, 0);
           }
         }
+        if (PIECES && ((i + 1) % CHAIN == 0 || i == NG - 1) && !(seg == 1 && i == NG - 1)) {
+#pragma unroll
+          for (int u = 0; u < NE; ++u) place(u) = seg == 0 && i < CHAIN ? element(u) : place(u) + element(u);
+          clear();
+        }
       };
       // One segment.  All of a wave's activations are in flight at once where the registers allow it, else a few groups
       // ahead of the ones being multiplied.
-      auto segment = [&](const float (&ws)[NG][NB][4], auto load) {
+      auto segment = [&](int seg, auto load) {
         constexpr int CH = NG <= 8 ? NG : (TN == 1 ? 4 : 2);
         constexpr int NC = NG / CH;
         zr_f32x4 x[NC > 1 ? 2 : 1][CH][TN];
@@ -272,7 +316,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
           }
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int i = 0; i < CH; ++i) mma(x[c & (NC > 1 ? 1 : 0)][i], ws[c * CH + i]);
+          for (int i = 0; i < CH; ++i) mma(seg, c * CH + i, x[c & (NC > 1 ? 1 : 0)][i], w[seg][c * CH + i]);
         }
       };
       auto load_packed = [&](const float* base) {
@@ -292,20 +336,20 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
       if (from_embed) {
         if constexpr (AHEAD) {
 #pragma unroll
-          for (int i = 0; i < NG; ++i) mma(x_ahead[i], w[0][i]);
+          for (int i = 0; i < NG; ++i) mma(0, i, x_ahead[i], w[0][i]);
         } else {
-          segment(w[0], load_embed);
+          segment(0, load_embed);
         }
       } else {
         if (l > P.l_begin) wait_for(flags_below, t + 2);
-        segment(w[0], load_packed(hp_below + (long long)(t + 1) * P.slot));
+        segment(0, load_packed(hp_below + (long long)(t + 1) * P.slot));
       }
       float mask_v[NOUT];
 #pragma unroll
       for (int u = 0; u < NOUT; ++u) mask_v[u] = tile_ok[u] ? (float)P.mask01[(long long)t * mb + n0 + on[u]] : 0.0f;
       // the layer's own previous step
       wait_for(flags_here, t + 1);
-      segment(w[1], load_packed(hp_mine + (long long)t * P.slot));
+      segment(1, load_packed(hp_mine + (long long)t * P.slot));
 
       // what the next step reads from below: asked for now, in flight while this step is finished
       if (t + 1 < P.T) {
@@ -319,18 +363,8 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
       }
 
       // partial sums of the 8 K slices through LDS, then the cell
-      float* mine = red + kslice * (COLS * kRedLd);
-      if constexpr (NARROW) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) mine[(4 * kq + r) * kRedLd + cl + 16 * b] = acc4[b][r];
-      } else {
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) mine[(tn * 32 + 8 * (r >> 2) + 4 * kq + (r & 3)) * kRedLd + cl] = acc[tn][r];
-      }
+      for (int u = 0; u < NE; ++u) place(u) = !PIECES ? element(u) : (SUMS_AHEAD ? before[PIECES ? u : 0] : place(u)) + element(u);
       __syncthreads();
       if (s_abort) {  // every wave of the workgroup sees the same value: waits come before this barrier
         if (tid == 0) __hip_atomic_store(my_flag, kResidentGaveUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -346,13 +380,14 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const float* p = red + on[u] * kRedLd + g * 8 + oj[u];
-          float sum = 0.0f;
+          float part[kWaves];
 #pragma unroll
-          for (int q = 0; q < kWaves; ++q) sum += p[q * (COLS * kRedLd)];
-          z[g] = sum;
+          for (int q = 0; q < kWaves; ++q) part[q] = p[q * (COLS * kRedLd)];
+          z[g] = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
         }
         float c;
-        zr_lstm_cell(z[0] + bi[u], z[1] + bf[u], z[2] + bc[u], z[3] + bo[u], c_state[u], mask_v[u], P.clip, g_v[u][0],
+        const int row = oj[u] % kRows;  // (a tile of zeros has rows past the tile)
+        zr_lstm_cell(z[0] + s_bias[0][row], z[1] + s_bias[1][row], z[2] + s_bias[2][row], z[3] + s_bias[3][row], c_state[u], mask_v[u], P.clip, g_v[u][0],
                      g_v[u][1], g_v[u][2], g_v[u][3], c, h_v[u]);
         c_state[u] = c;
         __hip_atomic_store(hp_out + hp_off[u], ok[u] ? h_v[u] : 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
