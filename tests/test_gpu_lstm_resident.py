@@ -279,3 +279,40 @@ def test_sweep_rounds_no_more_than_one_launch_per_diagonal(ctx, H, mb):
         assert (path == RESIDENT) == (option == 3)
         error[option] = np.linalg.norm(h[0] - np.stack(want)) / np.linalg.norm(want)
     assert error[3] < 1.1 * error[1]
+
+
+# 4 x 16, 8 x 16, 8 x 32 and 8 x 64 tiles with and without feed-input
+@pytest.mark.parametrize("H,mb", [(500, 37), (512, 8), (1000, 16), (1024, 1), (1024, 40), (1200, 8), (500, 128)])
+@pytest.mark.parametrize("feed", [False, True])
+def test_node_is_rounded_in_short_chains(ctx, H, mb, feed):
+    """Error of the pre-activations against 64 bits, from c' = f c + i u with c = 0 and i near 1 (a bias of 20): u = tanh(z_c), z_c
+    small, carries z_c's.  An addition rounds its result by a relative 2.5e-8 in the 2-norm, a chain of n by sqrt(n / 2) of
+    that; each wave's K / 8 products are four chains in narrow tiles, two in wide ones, then the chains and the
+    waves' sums are added pairwise (five additions of at most the final size).  A third above that passes: i, u and c' round too."""
+    g = synth.rng(48, H + mb)
+    layer = _rough_layer(g, H, feed_input=feed)
+    layer["M"][2], layer["Wh"][2] = layer["M"][2] * 0.02, layer["Wh"][2] * 0.02
+    if feed:
+        layer["Q"][2] = layer["Q"][2] * 0.02
+    layer["b"][0][:], layer["b"][2][:] = 20.0, 0.0
+    ly = Layer(ctx, layer)
+    x, hp, ht = [synth.uniform(g, (H, mb), -1, 1) for _ in range(3)]
+    d_h, d_c, ones = ctx.empty((H, mb)), ctx.empty((H, mb)), ctx.array(np.ones(mb, np.int32))
+    try:
+        if feed:
+            ids = ctx.array(np.arange(mb, dtype=np.int32))
+            ctx.lstm_step_embed(ly.w, ctx.array(x), mb, ids, ctx.array(hp), ctx.zeros((H, mb)), ones, mb, d_h, d_c, d_htild=ctx.array(ht))
+        else:
+            ctx.lstm_step(ly.w, ctx.array(x), ctx.array(hp), ctx.zeros((H, mb)), ones, mb, d_h, d_c)
+        ctx.sync()
+    finally:
+        ly.close()
+    z = np.asarray(layer["M"][2], np.float64) @ x + np.asarray(layer["Wh"][2], np.float64) @ hp
+    if feed:
+        z += np.asarray(layer["Q"][2], np.float64) @ ht
+    want = np.tanh(z)
+    K = (3 if feed else 2) * H
+    narrow = mb <= 16 or H <= 512 and (H + 3) // 4 * ((mb + 15) // 16) <= 256 or (H + 7) // 8 * ((mb + 15) // 16) <= 256
+    n = K / 8 / (4 if narrow else 2)
+    error = np.linalg.norm(d_c.get() - want) / np.linalg.norm(want)
+    assert error < 1.33 * 2.5e-8 * np.sqrt(n / 2 + 5)

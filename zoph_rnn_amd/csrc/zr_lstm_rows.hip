@@ -126,14 +126,20 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
     }
   };
   typedef float acc16 __attribute__((ext_vector_type(16)));
-  acc16 acc[TN];
-  zr_f32x4 acc4[NB];
+  // Several accumulators, for k of one remainder each: a chain of additions rounds the less the shorter it is, and the older
+  // kernels divide K further.  Error of h against 64 bits at H = 1024, one column 2.6e-7 with one accumulator, 1.7e-7 with four
+  // (K split across workgroups 1.7e-7), with feed-input 3.3e-7, 1.9e-7 (1.9e-7); H = 500 at 128 columns 2.0e-7, 1.6e-7 with
+  // two (1.6e-7).  782 nodes of H = 20 to 2000 take 0.6 % more time on average.
+  acc16 acc[2][TN];
+  zr_f32x4 acc4[4][NB];
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[tn][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[0][tn][r] = acc[1][tn][r] = 0.0f;
 #pragma unroll
-  for (int b = 0; b < NB; ++b) acc4[b] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc4[e][b] = {0.0f, 0.0f, 0.0f, 0.0f};
   int mg = kslice % G;  // the group (inside its segment) multiplied next
   auto mma = [&](Frag& q) {
     if (4 * KB * (mg + 1) > H) {  // the column ends inside this group: shift the moved loads back, zero what lies behind
@@ -158,11 +164,11 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
     for (int e = 0; e < 4; ++e) {
       if constexpr (NARROW) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) acc4[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x[0][e], q.w[b][e], acc4[b], 0, 0, 0);
+        for (int b = 0; b < NB; ++b) acc4[e][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x[0][e], q.w[b][e], acc4[e][b], 0, 0, 0);
       } else {
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
-          acc[tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(q.x[tn][e], q.w[0][e], acc[tn], 0, 0, 0);
+          acc[e & 1][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(q.x[tn][e], q.w[0][e], acc[e & 1][tn], 0, 0, 0);
       }
     }
   };
@@ -190,12 +196,12 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) mine[(4 * kq + r) * kRedLd + cl + 16 * b] = acc4[b][r];
+      for (int r = 0; r < 4; ++r) mine[(4 * kq + r) * kRedLd + cl + 16 * b] = (acc4[0][b][r] + acc4[1][b][r]) + (acc4[2][b][r] + acc4[3][b][r]);
   } else {
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mine[(tn * 32 + 8 * (r >> 2) + 4 * kq + (r & 3)) * kRedLd + cl] = acc[tn][r];
+      for (int r = 0; r < 16; ++r) mine[(tn * 32 + 8 * (r >> 2) + 4 * kq + (r & 3)) * kRedLd + cl] = acc[0][tn][r] + acc[1][tn][r];
   }
   __syncthreads();
 #pragma unroll
@@ -205,10 +211,10 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const float* p = red + on[u] * kRedLd + g * ROWS + oj[u];
-      float sum = 0.0f;
+      float part[kWaves];
 #pragma unroll
-      for (int q = 0; q < kWaves; ++q) sum += p[q * (COLS * kRedLd)];
-      z[g] = sum;
+      for (int q = 0; q < kWaves; ++q) part[q] = p[q * (COLS * kRedLd)];
+      z[g] = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
     }
     float gi, gf, gc, go, c, h;
     zr_lstm_cell(z[0] + bi[u], z[1] + bf[u], z[2] + bc[u], z[3] + bo[u], cprev_v[u], mask_v[u], P.clip, gi, gf, gc, go, c, h);
