@@ -142,3 +142,28 @@ def test_lstm_weight_gradients(ctx, H, T, mb):
     assert rel(dM.get(), d @ x.T.astype(np.float64)) < bound(K)
     assert rel(dWh.get(), d @ prev.T) < bound(K)
     assert rel(db.get(), d.sum(1)) < bound(K)
+
+
+@pytest.mark.parametrize("V,H,n", [(20000, 500, 257), (20001, 503, 512), (10001, 1000, 400), (12000, 1000, 1024)])
+def test_prepared_output_layer_is_rounded_in_short_chains(ctx, V, H, n):
+    """A probability is off by its logit's error, in proportion.  The logit of a large one is a sum that grows steadily, so the
+    partial sums have a third of the final square on average: K / 16 additions, each a relative 2.5e-8 in the 2-norm (mantissas
+    spread evenly in their logarithm), and the bias.  The exponential, its argument, the sum and the division add a part in
+    10^7.  (Measured: two thirds of that.  With the six products of 16 k added one by one twice to three times as much.)"""
+    g = synth.rng(46, V + n)
+    D = g.standard_normal((V, H)).astype(np.float32) / np.float32(H ** 0.5 / 3)
+    b = g.standard_normal(V).astype(np.float32)
+    h = g.standard_normal((H, n)).astype(np.float32)
+    dD, db, dh, out = ctx.array(np.asfortranarray(D)), ctx.array(b), ctx.array(np.asfortranarray(h)), ctx.empty((V, n))
+    ctx.softmax_prepare(dD, V, H)
+    try:
+        ctx.softmax_forward(dD, db, V, H, dh, n, capi.ZR_SOFTMAX_PROB, out)
+        ctx.sync()
+    finally:
+        ctx.softmax_release(dD)
+    z = D.astype(np.float64) @ h + b[:, None]
+    p = np.exp(z - z.max(0))
+    p /= p.sum(0)
+    size = np.sqrt((p * p * z * z).sum() / (p * p).sum())  # of the logits that count
+    error = np.linalg.norm(out.get() - p) / np.linalg.norm(p)
+    assert error < size * 2.5e-8 * np.sqrt(H / 16 / 3) + 1e-7

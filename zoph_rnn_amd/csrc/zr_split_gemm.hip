@@ -219,6 +219,12 @@ __device__ __forceinline__ void plain_tile(const SplitArgs& a, zr_f32x16 (&acc)[
 template <int TNW, int AL, int BL, int EPI>
 __global__ void __launch_bounds__(256, TNW == 2 ? 3 : 2) split_gemm_kernel(SplitArgs a) {
   constexpr int TN = 64 * TNW;
+  // The six products of 16 k are added up from zero and their sum is added to the accumulator: one rounding at its size where
+  // the products one by one make six.  For the logits of a prepared output layer, whose fp32 kernel divides K over four waves.
+  // Error of the probabilities against 64 bits at V = 50000, H = 1000, 257 to 1024 columns 4.3e-7 there, 1.0e-6 without
+  // this, 3.4e-7 with it; H = 500 2.1e-7, 4.1e-7, 1.9e-7.  It costs up to 19 % (50000 x 1000, 400 columns 346 -> 413 us, 512 367 ->
+  // 425; the fp32 kernel 473 there).  The other fp32 kernels' sums are no shorter than those of the products one by one.
+  constexpr bool SHORT = AL == ZR_SPLIT_PACK4 && EPI == ZR_EPI_SOFTMAX_PARTIAL;
   typedef Oper<TM> OA;
   typedef Oper<TN> OB;
   __shared__ u32x4 s[OA::SIZE + OB::SIZE];
@@ -275,13 +281,24 @@ __global__ void __launch_bounds__(256, TNW == 2 ? 3 : 2) split_gemm_kernel(Split
 #pragma unroll
         for (int q = 0; q < 3; ++q) y[q] = __builtin_bit_cast(bf16x8, s[(rb[j] ^ (4 * st)) + q * OB::TERM + 2 * st * OB::KG]);
         constexpr int P[6] = {2, 0, 1, 1, 0, 0}, Q[6] = {0, 2, 1, 0, 1, 0};  // the smallest products first
+        if constexpr (SHORT) {
 #pragma unroll
-        for (int p = 0; p < 6; ++p)
+          for (int i = 0; i < 2; ++i) {
+            zr_f32x16 sum = {};
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
-            acc[i][j] = EPI == ZR_EPI_SOFTMAX_PARTIAL
-                            ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i][P[p]], y[Q[p]], acc[i][j], 0, 0, 0)
-                            : __builtin_amdgcn_mfma_f32_32x32x16_bf16(y[Q[p]], x[i][P[p]], acc[i][j], 0, 0, 0);
+            for (int p = 0; p < 6; ++p) sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i][P[p]], y[Q[p]], sum, 0, 0, 0);
+            acc[i][j] += sum;
+            asm volatile("" : "+v"(acc[i][j]));  // done before the next sum: the registers hold no second one
+          }
+        } else {
+#pragma unroll
+          for (int p = 0; p < 6; ++p)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+              acc[i][j] = EPI == ZR_EPI_SOFTMAX_PARTIAL
+                              ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i][P[p]], y[Q[p]], acc[i][j], 0, 0, 0)
+                              : __builtin_amdgcn_mfma_f32_32x32x16_bf16(y[Q[p]], x[i][P[p]], acc[i][j], 0, 0, 0);
+        }
       }
     }
   }
