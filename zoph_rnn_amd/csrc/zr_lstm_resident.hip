@@ -141,7 +141,8 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
     int oj[NOUT], on[NOUT];
     bool ok[NOUT], tile_ok[NOUT];
     float c_state[NOUT];
-    if (tid < 4 * kRows) s_bias[tid / kRows][tid % kRows] = P.bias[l][tid / kRows * H + min(j0 + tid % kRows, H - 1)];
+    if (tid < 4 * kRows)  // (shifts and masks: a remainder of a signed index costs two registers, and those a tenth of a step)
+      (&s_bias[0][0])[tid] = P.bias[l][(tid >> 3) * H + (j0 + (tid & 7) < H ? j0 + (tid & 7) : H - 1)];
     unsigned hp_off[NOUT];  // element inside a slot
 #pragma unroll
     for (int u = 0; u < NOUT; ++u) {
@@ -386,7 +387,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG * TN <= 4 ? 4 : 2) lstm_reside
           z[g] = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
         }
         float c;
-        const int row = oj[u] % kRows;  // (a tile of zeros has rows past the tile)
+        const int row = oj[u] & (kRows - 1);  // (a tile of zeros has rows past the tile)
         zr_lstm_cell(z[0] + s_bias[0][row], z[1] + s_bias[1][row], z[2] + s_bias[2][row], z[3] + s_bias[3][row], c_state[u], mask_v[u], P.clip, g_v[u][0],
                      g_v[u][1], g_v[u][2], g_v[u][3], c, h_v[u]);
         c_state[u] = c;
