@@ -287,7 +287,7 @@ def test_sweep_rounds_no_more_than_one_launch_per_diagonal(ctx, H, mb):
 def test_node_is_rounded_in_short_chains(ctx, H, mb, feed):
     """Error of the pre-activations against 64 bits, from c' = f c + i u with c = 0 and i near 1 (a bias of 20): u = tanh(z_c), z_c
     small, carries z_c's.  An addition rounds its result by a relative 2.5e-8 in the 2-norm, a chain of n by sqrt(n / 2) of
-    that; each wave's K / 8 products are four chains in narrow tiles, two in wide ones, then the chains and the
+    that; each wave's K / 8 products are four chains in 8 x 16 tiles, else two; then the chains and the
     waves' sums are added pairwise (five additions of at most the final size).  A third above that passes: i, u and c' round too."""
     g = synth.rng(48, H + mb)
     layer = _rough_layer(g, H, feed_input=feed)
@@ -312,7 +312,6 @@ def test_node_is_rounded_in_short_chains(ctx, H, mb, feed):
         z += np.asarray(layer["Q"][2], np.float64) @ ht
     want = np.tanh(z)
     K = (3 if feed else 2) * H
-    narrow = mb <= 16 or H <= 512 and (H + 3) // 4 * ((mb + 15) // 16) <= 256 or (H + 7) // 8 * ((mb + 15) // 16) <= 256
-    n = K / 8 / (4 if narrow else 2)
+    n = K / 8 / (4 if H > 512 and (mb <= 16 or (H + 7) // 8 * ((mb + 15) // 16) <= 256) else 2)
     error = np.linalg.norm(d_c.get() - want) / np.linalg.norm(want)
     assert error < 1.33 * 2.5e-8 * np.sqrt(n / 2 + 5)

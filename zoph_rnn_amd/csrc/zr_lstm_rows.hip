@@ -36,14 +36,14 @@ struct LstmRows {
 typedef zr_f32x4 zr_f32x4_u __attribute__((aligned(4)));
 
 // NARROW: 16 columns on the 16 x 16 x 4 instruction; else TN tiles of 32 columns on the 32 x 32 x 2 one (ROWS = 8).
-template <int ROWS, int TN, bool NARROW>
+// PF: k-groups in flight.
+template <int ROWS, int TN, bool NARROW, int PF>
 __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
   static_assert(NARROW ? TN == 1 : ROWS == 8, "tile shape");
   constexpr int KB = NARROW ? 4 : 2;            // k-blocks of 4 per k-group
   constexpr int NB = NARROW ? ROWS / 4 : 1;     // weight sub-tiles
   constexpr int COLS = NARROW ? 16 : 32 * TN;
   constexpr int NOUT = (ROWS * COLS + 511) / 512;
-  constexpr int PF = NARROW || TN == 2 ? 8 : 10;  // k-groups in flight
   constexpr int NS = PF + 1;
   __shared__ float red[kWaves * COLS * kRedLd];
   // Workgroup ids congruent mod 8 share a die: the column tiles of a row tile, which read the same weights, go together.
@@ -129,15 +129,16 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
   // Several accumulators, for k of one remainder each: a chain of additions rounds the less the shorter it is, and the older
   // kernels divide K further.  Error of h against 64 bits at H = 1024, one column 2.6e-7 with one accumulator, 1.7e-7 with four
   // (K split across workgroups 1.7e-7), with feed-input 3.3e-7, 1.9e-7 (1.9e-7); H = 500 at 128 columns 2.0e-7, 1.6e-7 with
-  // two (1.6e-7).  782 nodes of H = 20 to 2000 take 0.6 % more time on average.
+  // two (1.6e-7).  Costs 0 to 1.5 %.
+  constexpr int NACC = NARROW && ROWS == 8 ? 4 : 2;
   acc16 acc[2][TN];
-  zr_f32x4 acc4[4][NB];
+  zr_f32x4 acc4[NACC][NB];
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[0][tn][r] = acc[1][tn][r] = 0.0f;
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
+  for (int e = 0; e < NACC; ++e)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc4[e][b] = {0.0f, 0.0f, 0.0f, 0.0f};
   int mg = kslice % G;  // the group (inside its segment) multiplied next
@@ -164,7 +165,10 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
     for (int e = 0; e < 4; ++e) {
       if constexpr (NARROW) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) acc4[e][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x[0][e], q.w[b][e], acc4[e][b], 0, 0, 0);
+        for (int b = 0; b < NB; ++b) {
+          zr_f32x4& a = acc4[e & (NACC - 1)][b];
+          a = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x[0][e], q.w[b][e], a, 0, 0, 0);
+        }
       } else {
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
@@ -196,7 +200,8 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) mine[(4 * kq + r) * kRedLd + cl + 16 * b] = (acc4[0][b][r] + acc4[1][b][r]) + (acc4[2][b][r] + acc4[3][b][r]);
+      for (int r = 0; r < 4; ++r) mine[(4 * kq + r) * kRedLd + cl + 16 * b] =
+            NACC == 4 ? (acc4[0][b][r] + acc4[1][b][r]) + (acc4[NACC - 2][b][r] + acc4[NACC - 1][b][r]) : acc4[0][b][r] + acc4[1][b][r];
   } else {
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn)
@@ -255,13 +260,18 @@ int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const flo
   P.n_tiles = (mb + cols - 1) / cols;
   const unsigned grid = (unsigned)((P.j_tiles + 7) / 8 * 8 * P.n_tiles);
   if (shape == 0)
-    lstm_rows_kernel<4, 1, true><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+    lstm_rows_kernel<4, 1, true, 8><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
   else if (shape == 1)
-    lstm_rows_kernel<8, 1, true><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+    lstm_rows_kernel<8, 1, true, 8><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+  // 8 x 32 tiles: all of a wave's k-groups in flight at once where ten are enough; else eight, for 128 registers a thread and so two
+  // workgroups on a compute unit (160 columns of H = 400 are 280 workgroups with those that leave at once: 15.8 us with ten,
+  // 13.3; 128 columns of H = 500 10.3, 9.6; but 128 of H = 300, ten groups a wave, 7.2, 8.1).
+  else if (shape == 2 && P.nseg * ((P.kp + 7) / 8) <= 10 * kWaves)
+    lstm_rows_kernel<8, 1, false, 10><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
   else if (shape == 2)
-    lstm_rows_kernel<8, 1, false><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+    lstm_rows_kernel<8, 1, false, 8><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
   else
-    lstm_rows_kernel<8, 2, false><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
+    lstm_rows_kernel<8, 2, false, 8><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
   ZR_LAUNCH_CHECK("lstm_rows_kernel");
   return ZR_OK;
 }
