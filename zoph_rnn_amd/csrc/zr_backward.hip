@@ -1135,13 +1135,14 @@ int zr_lstm_feed_backward(zr_ctx* ctx, const float* const d_Q[4], int H, int mb,
   ZR_CHECK_ARG(d_Q && d_dgates && d_htild && d_err_htild && d_dQ_stack, "zr_lstm_feed_backward: null pointer");
   for (int g = 0; g < 4; ++g) ZR_CHECK_ARG(d_Q[g] != nullptr, "zr_lstm_feed_backward: Q matrix %d is null", g);
   // error of h~ = sum_g Q_g^T d_g (src/LSTM.hpp:804-857: four products and add_four_matrices_kernel)
-  for (int half = 0; half < 2; ++half) {
+  const int per_launch = ctx->gemm_cfg == 0 && zr_small_gemm_shape(H, mb, H, 4, 1, 0, true, ctx->cu_count) >= 0 ? 4 : 2;
+  for (int first = 0; first < 4; first += per_launch) {
     ZrGemmDesc g = {};
     g.M = H;
     g.N = mb;
-    g.nseg = 2;
-    for (int s = 0; s < 2; ++s) {
-      const int gate = 2 * half + s;
+    g.nseg = per_launch;
+    for (int s = 0; s < per_launch; ++s) {
+      const int gate = first + s;
       g.K[s] = H;
       g.A[s] = d_Q[gate];
       g.lda[s] = H;
@@ -1153,7 +1154,7 @@ int zr_lstm_feed_backward(zr_ctx* ctx, const float* const d_Q[4], int H, int mb,
     g.ldc = H;
     g.batch = 1;
     g.epilogue = ZR_EPI_STORE;
-    g.accumulate = half;
+    g.accumulate = first > 0;
     rc = zr_gemm_launch(ctx, g);
     if (rc) return rc;
   }

@@ -10,11 +10,11 @@ namespace {
 
 struct GemmArgs {
   int M, N, nseg;
-  int K[3];
-  const float* A[3];
-  long long lda[3];
-  const float* B[3];
-  int ldb[3];
+  int K[4];
+  const float* A[4];
+  long long lda[4];
+  const float* B[4];
+  int ldb[4];
   float* C;
   int ldc;
   long long strideA, strideC, strideBias;
@@ -28,7 +28,7 @@ struct GemmArgs {
   int b_pack4;           // B segments are k-interleaved copies: element (k, n) at ((k/4)*N + n)*4 + k%4
   // bf16 weights: B[s] is the bf16 "hi" array and Blo[s] the "lo" array of the split activations, both
   // k-interleaved by 8 ([K/8][N][8]); see zr_split_pack_multi_kernel
-  const unsigned short* Blo[3];
+  const unsigned short* Blo[4];
   int accum;  // ZR_EPI_STORE only: C += result instead of C = result
   int stream_a;  // the weights are fetched with the streaming hint (ZrGemmDesc::stream_a)
   // groups > 0: blockIdx.z = group * batch + batch index; the group picks A, B and C from these tables
@@ -1187,7 +1187,14 @@ int zr_pack4_trans_launch(zr_ctx* ctx, const float* src, int M, int K, long long
 
 int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
   ZR_CHECK_ARG(d.M > 0 && d.N > 0, "gemm: M = %d, N = %d", d.M, d.N);
-  ZR_CHECK_ARG(d.nseg >= 1 && d.nseg <= 3, "gemm: nseg = %d", d.nseg);
+  // small products: narrow tiles
+  int small = -1;
+  if (ctx->gemm_cfg == 0 && d.epilogue != ZR_EPI_SOFTMAX_PARTIAL && d.nseg >= 1 && d.nseg <= 4) {
+    bool same = true;
+    for (int s = 1; s < d.nseg; ++s) same = same && d.K[s] == d.K[0];
+    if (same) small = zr_small_gemm_shape(d.M, d.N, d.K[0], d.nseg, d.batch * (d.groups > 0 ? d.groups : 1), d.a_pack, d.trans_a != 0, ctx->cu_count);
+  }
+  ZR_CHECK_ARG(d.nseg >= 1 && d.nseg <= (small >= 0 ? 4 : 3), "gemm: nseg = %d", d.nseg);
   ZR_CHECK_ARG((d.groups > 0 || d.C != nullptr) && d.ldc >= d.M, "gemm: C null or ldc %d < M %d", d.ldc, d.M);
   ZR_CHECK_ARG(d.batch >= 1 && d.batch <= 65535, "gemm: batch = %d", d.batch);
   ZR_CHECK_ARG(d.groups >= 0 && d.groups <= 8, "gemm: groups = %d", d.groups);
@@ -1211,7 +1218,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
   ga.nseg = d.nseg;
   bool vec = true;
   long long flops = 0;
-  for (int s = 0; s < 3; ++s) {
+  for (int s = 0; s < 4; ++s) {
     if (s < d.nseg) {
       ZR_CHECK_ARG(d.K[s] > 0, "gemm: K[%d] = %d", s, d.K[s]);
       ZR_CHECK_ARG(d.groups > 0 || (d.A[s] && d.B[s]), "gemm: null operand in segment %d", s);
@@ -1270,7 +1277,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
   if (d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) ZR_CHECK_ARG(d.bias && d.partials, "gemm: bias/partials required");
 
   ga.b_pack4 = 0;
-  for (int s = 0; s < 3; ++s) ga.Blo[s] = nullptr;
+  for (int s = 0; s < 4; ++s) ga.Blo[s] = nullptr;
   if (d.a_pack == 2) {
     ZR_CHECK_ARG(vec, "gemm: bf16 operand A needs 16-byte aligned activations with ldb %% 4 == 0");
     const bool one_term = ctx->bf16_terms == 1;
@@ -1297,6 +1304,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
         hi += 2 * e;
       }
     }
+    if (small >= 0) return zr_small_gemm(ctx, d, (const unsigned short* const*)ga.B, ga.Blo, small);
     if (d.nseg == 1 && d.M >= 8192 && d.N > 32 && d.N <= 1024 &&
         (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL)) {
       const int n32 = (d.N + 31) / 32;
@@ -1341,6 +1349,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
         ZR_CHECK_ARG(d.K[s] % 8 == 0, "gemm: a k-interleaved B needs K %% 8 == 0 (K[%d] = %d)", s, d.K[s]);
       ga.b_pack4 = 1;
     }
+    if (small >= 0) return zr_small_gemm(ctx, d, nullptr, nullptr, small);
     // Wide batches: the tall and row-range kernels serve up to 256 columns as well or better (50000 x 192 x 1000: 167
     // against 175 us), beyond that the split product does (33333 x 700 x 500: 174 against 602 us).  With fixed scratch
     // buffers only the statistics form, which needs none of them, and only where the fp32 kernels' copy of B would fit: the
@@ -1430,6 +1439,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
     if (d.N <= 32) return launch_pack4<2, 1, 2>(ctx, ga, d.epilogue, vec, zcount);
     return launch_pack4<2, 2, 2>(ctx, ga, d.epilogue, vec, zcount);
   }
+  if (small >= 0) return zr_small_gemm(ctx, d, nullptr, nullptr, small);
   if (d.nseg == 1 && zcount == 1 && d.groups == 0 && ctx->gemm_cfg == 0 &&
       ((d.epilogue == ZR_EPI_STORE && !ctx->fixed_scratch) || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) &&
       zr_split_gemm_takes_product(d.M, d.N, d.K[0], d.trans_a != 0, d.epilogue == ZR_EPI_SOFTMAX_PARTIAL, ctx->cu_count))

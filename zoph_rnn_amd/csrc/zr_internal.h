@@ -110,10 +110,10 @@ enum ZrEpilogue {
 
 struct ZrGemmDesc {
   int M, N;
-  int nseg;
-  int K[3];
-  const float* A[3];
-  int lda[3];
+  int nseg;  // up to 3 (4 where zr_small_gemm takes the product)
+  int K[4];
+  const float* A[4];
+  int lda[4];
   int trans_a;  // applies to every segment
   // 1: A is k-interleaved fp32: element (m, k) at ((k/4)*lda + m)*4 + k%4, lda = M rounded up to 32, K padded to
   //    a multiple of 8, pads zero (ZR_A_PACK4 in zr_mfma_core.h).
@@ -121,8 +121,8 @@ struct ZrGemmDesc {
   //    ((k/8)*lda + m)*8 + k%8, K a multiple of 16 (ZR_A_PACK8_BF16).
   // Single batch, no transpose.
   int a_pack;
-  const float* B[3];
-  int ldb[3];
+  const float* B[4];
+  int ldb[4];
   float* C;
   int ldc;
   // batch (blockIdx.z): A/C/bias advance by these strides (elements; bf16 elements for a bf16 A); B is shared
@@ -147,8 +147,8 @@ struct ZrGemmDesc {
   // (instead of C); lda/ldb/ldc, the batch count and its strides apply inside every problem.
   // a_pack == 2: segment s's activations already split and k-interleaved by 8 (zr_split_pack_x_launch's layout): the
   // bf16 "hi" array, and the "lo" array in two-term mode (null entries: the launch splits B[s] itself)
-  const unsigned short* Bhi[3];
-  const unsigned short* Blo[3];
+  const unsigned short* Bhi[4];
+  const unsigned short* Blo[4];
   int b_packed;  // with a_pack == 1: B (and every gB) is already k-interleaved, element (k, n) at ((k/4)*N + n)*4 + k%4
                  // (K a multiple of 8, 16-byte aligned); ldb is ignored
   int groups;
@@ -158,6 +158,9 @@ struct ZrGemmDesc {
 };
 
 int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d);
+// Small products on narrow tiles (zr_small_gemm.hip), every segment with the same K, any epilogue but the soft-max partials;
+// shape: as zr_small_gemm_shape has it (zr_rules.h).  Bhi / Blo: the activations' bf16 terms where d.a_pack == 2 (Blo[0] null: one term).
+int zr_small_gemm(zr_ctx* ctx, const ZrGemmDesc& d, const unsigned short* const Bhi[4], const unsigned short* const Blo[4], int shape);
 // Packs one M x K column-major matrix (leading dimension ld) into the k-interleaved layout [kp/4][ldp][4] with
 // zero padding (ldp >= M a multiple of 32, kp >= K a multiple of 8).  dst holds kp*ldp floats.
 int zr_pack4_launch(zr_ctx* ctx, const float* src, int M, int K, long long ld, int ldp, int kp, float* dst);

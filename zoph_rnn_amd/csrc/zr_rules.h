@@ -211,3 +211,33 @@ inline bool zr_outer_takes(int count, int M, int N, int K) {
 inline bool zr_grouped_small_tiles(long long tiles, int columns, int cus) {
   return tiles <= cus || (columns > 32 && 2 * tiles <= 3LL * cus);
 }
+
+// ---- small products (zr_small_gemm.hip): narrow tiles whose waves have all their operands in flight
+
+// Shape: 0 = 16 rows x 16 columns, 1 = 16 x 32, 2 = 32 x 32, -1 = the other kernels.  z: independent products of one launch.  a_pack,
+// trans_a: the left operand's layout as ZrGemmDesc has it.  Estimates of a launch in us (within 16 % of 330 sizes on each shape): a
+// trip to memory and the launch, and the K range of a workgroup, alone on its compute unit or beside a second one; beyond two a
+// compute unit the wider tiles of the other kernels win, and so they do where 32 x 32 tiles are the best choice here and the
+// matrix is read 4 bytes a lane (column-major), or row-major up to K = 1500: 1000 x 256 x 1000 11.8 / 10.2 and 11.4 / 10.8.
+// This one / the others, us: 500 x 64 x 500 4.5 / 6.3 row-major, 4.6 / 7.0 column-major; 1000 x 64 x 1000 6.2 / 9.8; 2 products of
+// 500 x 64 x 2000 13.0 / 18.6 (the whole node), 1000 x 64 x 4000 26.1 / 33.4; 100 x 20 x 100 3.6 / 4.1; an attention step on prepared matrices,
+// H = 500, 37 columns 19.6 / 35.2; bf16 matrices, H = 1024, 64 columns 24.0 / 30.4; sweeps back through 12 steps, 2 x 100, 128 columns 136 /
+// 242, 2 x 500, 64 columns 243 / 293, 2 x 1000, 128 columns 771 / 966.  Of 200 sizes five are slower than with the others, by 2 to 10 %.
+inline int zr_small_gemm_shape(int M, int N, int K, int nseg, int z, int a_pack, bool trans_a, int cus) {
+  if (K < 16) return -1;
+  const double slope[3] = {0.0036, 0.0052, 0.0078}, second[3] = {1.55, 1.8, 1.9};
+  const double k = (double)K * nseg * (a_pack == 2 ? 0.5 : 1.0);  // bf16 weights: twice the k for the same bytes and instructions
+  int best = -1;
+  double us = 0.0;
+  for (int s = 0; s < 3; ++s) {
+    const int rows = s == 2 ? 32 : 16, cols = s == 0 ? 16 : 32;
+    const long long wgs = (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * z;
+    if (wgs > 2LL * cus) continue;
+    const double t = 3.4 + slope[s] * k * (wgs > cus ? second[s] : 1.0);
+    if (best < 0 || t < us) {
+      best = s, us = t;
+      if (s == 2 && (a_pack == 0 ? !trans_a || k < 1500.0 : a_pack == 2 && wgs > cus && k > 512.0)) best = -1;
+    }
+  }
+  return best;
+}
