@@ -199,6 +199,11 @@ enum ZrSplitLayout {
 int zr_split_gemm(zr_ctx* ctx, int M, int N, int K, const float* A, long long lda, int a_layout, const float* B,
                   long long ldb, int b_layout, float* C, long long ldc, const float* bias, float* partials, int accumulate);
 
+// The output layer's product on a prepared fp32 matrix (k-interleaved, ldp = rows rounded up to 32), with the soft-max partials
+// (zr_logits.hip).  tn 32-column blocks a tile, `waves` 32-row blocks: as zr_logits_plan has it (zr_rules.h).  No scratch.
+int zr_logits_split(zr_ctx* ctx, int V, int cols, int H, const float* packed, int ldp, const float* h, long long ldh, float* C,
+                    long long ldc, const float* bias, float* partials, bool stream, int tn, int waves);
+
 struct zr_lstm_weights {
   int H;
   int nseg;        // 2 (M, Wh) or 3 (+Q)

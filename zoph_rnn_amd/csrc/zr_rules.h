@@ -241,3 +241,46 @@ inline int zr_small_gemm_shape(int M, int N, int K, int nseg, int z, int a_pack,
   }
   return best;
 }
+
+// ---- the output layer's product on a prepared fp32 matrix (zr_logits.hip)
+
+// tn: 32-column blocks of a tile, waves: 32-row blocks of a workgroup; tn = 0: the other kernels.
+// Estimated time, us: (steps of 32 k + what filling and the epilogue take) * a step of the workgroups that share a compute unit (one of four
+// waves alone; two of four or one of eight, whose matrix instructions fill it), times the rounds: within 11 % of 2700 measured
+// launches (V = 1000 .. 50000, H = 64 .. 1000, 33 to 1000 columns), and the choice is 4 % from the best tile on average.
+// Against the kernels before, the product alone, us: 50000 x 128 x 1000 123 -> 98, 192 columns 173 -> 125 (in turn with other kernels), 30011 x 33 x 500 30 ->
+// 21, 33333 x 700 x 500 206 -> 171, 50000 x 128 x 333 79 -> 39, 16000 x 700 x 200 172 -> 53, 1000 x 64 x 64 8.9 -> 5.1.  Beyond 1024 columns the split product on the
+// plain matrix keeps what it takes, but for half-empty tiles: it has 256-column tiles and fewer conversions, and the estimate above does not know
+// the clock a launch of milliseconds runs at (50000 x 6400 x 1000 3.93 ms there, 4.09 here and 1.4 ms more inside a training
+// step; 20000 x 1280 x 500 208 us, 204; but 3000 x 3000 x 1000 171, 126).
+// Not where up to three 32 x 32 blocks a compute unit with K over eight waves are all there is to do and K is long: 1000 x 64 x 1000 10.3
+// against 24.2, 4000 x 128 x 777 17.3 / 20.5; but 4000 x 192 x 777 24.4 / 20.7, 8000 x 128 x 1000 28.2 / 25.3, 4000 x 192 x 500 18.0 / 14.9.
+struct ZrLogitsPlan {
+  int tn, waves;
+};
+inline ZrLogitsPlan zr_logits_plan(int V, int cols, int H, int cus) {
+  ZrLogitsPlan plan = {0, 0};
+  const long long blocks = (V + 31) / 32, n32 = (cols + 31) / 32;
+  // 32-bit offsets into the matrix, and a few steps past it
+  if (cols <= 32 || (((long long)H + 7) / 8 * 8 + 160) * blocks * 32 * 4 >= 1LL << 32) return plan;
+  const int steps = (H + 31) / 32;
+  double best = 0.0;
+  for (int tn = 1; tn <= 6; ++tn)
+    for (int waves = 8; waves >= 4; waves -= 4) {
+      const long long n_tiles = (n32 + tn - 1) / tn, rounds = ((blocks + waves - 1) / waves * n_tiles + cus - 1) / cus;
+      const double full = 0.4 + 0.456 * tn, alone = 0.306 + 0.334 * tn;
+      // (the matrix is fetched and split once for every column tile)
+      const double us = (1.0 + 0.02 * (n_tiles - 1)) * (steps + 3.7) * (waves == 8 ? rounds * full : (double)(rounds / 2) * full + (rounds & 1) * alone);
+      if (!plan.tn || us < best) best = us, plan.tn = tn, plan.waves = waves;
+    }
+  double other = -1.0;
+  if (cols > 1024 && zr_split_gemm_takes_product(V, cols, H, false, true, cus)) {
+    const long long m = (V + 127) / 128;
+    const double narrow = zr_split_launch_us(2, m * ((cols + 127) / 128), steps, cus), wide = zr_split_launch_us(4, m * ((cols + 255) / 256), steps, cus);
+    other = (narrow < wide ? narrow : wide) / 1.5;
+  } else if (H >= 512 && V < 8192 && blocks * n32 <= 3LL * cus) {
+    other = 2.0 + 0.0095 * H * ((blocks * n32 + cus - 1) / cus);
+  }
+  if (other > 0.0 && other <= best) plan.tn = plan.waves = 0;
+  return plan;
+}

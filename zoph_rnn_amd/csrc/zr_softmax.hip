@@ -183,18 +183,34 @@ int logits_with_partials(zr_ctx* ctx, const float* d_D, const float* d_b_d, int 
   d.K[0] = H;
   d.A[0] = d_D;
   d.lda[0] = V;
+  ZrLogitsPlan plan = {0, 0};
   for (int i = 0; i < ZR_MAX_PACKED_D; ++i) {
     const zr_ctx::PackedD& e = ctx->packed_d[i];
     if (e.key == d_D && e.V == V && e.H == H) {  // registered with zr_softmax_prepare: use the MFMA-layout copy
-      // ... unless the batch is thousands of columns wide (all time steps of a training minibatch at once) and too small a
-      // product for the split terms, which read either form: there the LDS-staged kernel on the plain matrix is faster than
+      if (!e.bf16 && ctx->gemm_cfg == 0) plan = zr_logits_plan(V, mb, H, ctx->cu_count);
+      // ... unless the batch is thousands of columns wide (all time steps of a training minibatch at once) and that kernel does
+      // not take it: there the split terms, which read either form, or the LDS-staged kernel on the plain matrix are faster than
       // the register-streaming one on the fp32 copy
-      if (!e.bf16 && mb > 1024) break;
+      if (!e.bf16 && mb > 1024 && !plan.tn) break;
       d.A[0] = (const float*)e.d_pack;
       d.lda[0] = e.ldp;
       d.a_pack = e.bf16 ? 2 : 1;
       break;
     }
+  }
+  const bool stream = (size_t)V * H * (d.a_pack == 2 ? 2 : 4) >= ((size_t)64 << 20);
+  if (plan.tn) {
+    if (ctx->fixed_scratch && mb <= 1024 && V >= 2048 && H % 8 == 0 && ((uintptr_t)d_h & 15u) == 0) {
+      // nothing of it is used here; the limit of the entry point does not follow the kernel
+      void* p = nullptr;
+      rc = zr_ctx_scratch(ctx, 0, sizeof(float) * (size_t)H * mb, &p);
+      if (rc) return rc;
+    }
+    rc = zr_logits_split(ctx, V, mb, H, d.A[0], d.lda[0], d_h, H, d_logits, V, d_b_d, (float*)scratch, stream, plan.tn, plan.waves);
+    if (rc) return rc;
+    *partials_out = (float*)scratch;
+    *nblocks_out = nblocks;
+    return ZR_OK;
   }
   d.B[0] = d_h;
   d.ldb[0] = H;
@@ -212,7 +228,7 @@ int logits_with_partials(zr_ctx* ctx, const float* d_D, const float* d_b_d, int 
   d.batch = 1;
   d.bias = d_b_d;
   d.epilogue = ZR_EPI_SOFTMAX_PARTIAL;
-  d.stream_a = (size_t)V * H * (d.a_pack == 2 ? 2 : 4) >= ((size_t)64 << 20) ? 1 : 0;
+  d.stream_a = stream ? 1 : 0;
   d.partials = (float*)scratch;
   rc = zr_gemm_launch(ctx, d);
   if (rc) return rc;
