@@ -11,12 +11,11 @@
 // split K; weights stream from HBM/L2 straight into MFMA operand registers (full 128-byte lines), the
 // activations are fetched with 16-byte loads along K.  See zr_mfma_core.h.
 #include "zr_internal.h"
+#include "zr_lstm_sweep.h"
 #include "zr_math.h"
 #include "zr_mfma_core.h"
 
 namespace {
-
-constexpr int kMaxUnits = 8;
 
 struct LstmUnit {
   const void* W;            // [nseg][4] packed matrices: fp32 [kp/4][ldw][4] or bf16 [kp/8][ldw][8] each
@@ -583,250 +582,6 @@ __global__ void __launch_bounds__(64 * NWV) lstm_lds_kernel(LstmLaunch2 P) {
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Whole-sweep kernel: ONE launch runs every (layer, time step) node of a stacked forward pass.
-//
-// A workgroup owns the same tile -- 32 hidden rows x 32*TN batch columns of one layer -- at every time step and loops
-// over t itself.  Node (l, t) needs h of (l-1, t) and of (l, t-1), each produced by the j_tiles workgroups that own
-// the same batch columns of that layer: every (layer, column tile) has an arrival counter in device memory that its
-// producers bump once per time step, and a consumer waits until the counter reaches (steps needed) * j_tiles.  The
-// layers settle into a skewed pipeline: a layer above the first consumes its recurrent input first and the input from
-// below second, so it trails the layer below by half a step and that hand-over hides behind half a K loop; a layer
-// never waits for the layer above it.
-// Compared with one launch per diagonal this removes, per step, the launch, the drain of the slowest tile and the
-// refill of the operand pipeline from a cold start; the cell state never leaves registers.
-//
-// Hand-over through memory: h is written twice, to the caller's array (plain stores, visible at kernel end) and to a
-// k-interleaved copy [H/4][mb][4] per (layer, t) that the consumers read.  The chip's eight dies have one L2 each.
-// The copy is written with device-scope stores (written through to memory); every wave waits for its stores to
-// complete, then a workgroup barrier, then one thread bumps the counter.  A consumer polls the counter with
-// device-scope loads and reads the copy with ordinary loads.  Those cannot hit a stale line as long as no line is
-// cached before it was written: caches are clean when the kernel starts, every line of a copy is read only after
-// the wait for its producers, and with mb % 8 == 0 a 128-byte line (8 columns x 4 rows) has one producer.  For other
-// minibatch sizes lines straddle producers, and the consumers invalidate their caches after every wait instead
-// (device-scope acquire), which costs about 4 % at the benchmark shape.
-//
-// Operand fetch: buffer loads (descriptor base + scalar offset advancing with k + fixed 32-bit lane offset), so the K
-// loop holds no vector instruction other than the MFMAs; see zr_mma_segment_u.
-//
-// Progress: the launch must be wholly resident (the host checks grid <= CUs x resident workgroups per CU), then the
-// dependency graph is acyclic and every wait ends.  Every wait is bounded all the same: a workgroup that runs out of
-// polls marks every counter, which releases all other waiters, raises the status flag and leaves; the others leave
-// at their next wait.
-// ---------------------------------------------------------------------------------------------------------
-constexpr int kSweepGaveUp = 1 << 28;  // bit set in every counter by a workgroup that stopped waiting
-constexpr int kSweepCtrStride = 32;    // ints between counters: one 128-byte line each
-
-struct LstmSweep {
-  const float* W[kMaxUnits];     // per layer: [2][4] packed fp32 matrices
-  const float* bias[kMaxUnits];  // per layer: [4][H]
-  const float* h0[kMaxUnits];
-  const float* c0[kMaxUnits];
-  float* h_all[kMaxUnits];
-  float* c_all[kMaxUnits];
-  float* gates_all[kMaxUnits];   // null: gates not kept
-  const float* embed;
-  const int* ids;                // [T][mb], already non-negative
-  const int* mask01;             // [T][mb]
-  float* hp;                     // [nl][T] k-interleaved copies of h, H*mb floats each
-  int* counters;                 // [nl][n_tiles] at kSweepCtrStride, zero at launch
-  int* status;                   // set to 1 when a wait was abandoned
-  int nl, T, V, H, mb, ldw, kp, j_tiles, n_tiles;
-  float clip;
-  int spin_limit;
-  int fence;   // 1: consumers invalidate their caches after every wait (see lstm_sweep_kernel)
-};
-
-// All threads of the workgroup call this.  False: leave the kernel.
-__device__ __forceinline__ bool sweep_wait(const LstmSweep& P, int* ctr, int target, int* s_go) {
-  if (threadIdx.x == 0) {
-    int v = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int spins = 0; v < target && spins < P.spin_limit; ++spins) {
-      __builtin_amdgcn_s_sleep(8);
-      v = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    const bool ok = v >= target && !(v & kSweepGaveUp);
-    if (!ok) {
-      if (!(v & kSweepGaveUp)) {
-        const int n = P.nl * P.n_tiles;
-        for (int i = 0; i < n; ++i) atomicOr(P.counters + i * kSweepCtrStride, kSweepGaveUp);
-      }
-      __hip_atomic_store(P.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    *s_go = ok ? 1 : 0;
-  }
-  __syncthreads();
-  const bool go = *s_go != 0;
-  if (go && P.fence) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  return go;
-}
-
-template <int TN>
-__global__ void __launch_bounds__(256) lstm_sweep_kernel(LstmSweep P) {
-  constexpr int KS = 4;
-  __shared__ __align__(16) float red[KS * 4 * TN * 16 * 64];  // all partial tiles of the workgroup at once
-  __shared__ int s_go[2];
-  // same die-aware placement as lstm_fused_kernel, with one unit per layer.  (Two workgroups per CU on 32-column tiles
-  // -- 512 workgroups for four layers of H = 1000 at 128 columns -- measured 2 % slower than one on 64-column tiles.)
-  const int id = blockIdx.x;
-  const int r8 = id & 7;
-  const int q = id >> 3;
-  const int nt = q % P.n_tiles;
-  const int groups = P.nl * P.j_tiles;
-  const int group = r8 * ((groups + 7) >> 3) + q / P.n_tiles;
-  if (q / P.n_tiles >= ((groups + 7) >> 3) || group >= groups) return;
-  const int l = group / P.j_tiles;
-  const int jt = group % P.j_tiles;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int kslice = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int H = P.H, mb = P.mb;
-  const int j0 = jt * 32;
-  const int n0 = nt * 32 * TN;
-  const long long n_el = (long long)H * mb;
-  constexpr int NV = zr_visit_count<TN, KS>();
-  // batch column of visit i of a lane in half-wave `half`, clamped
-  auto visit_col = [&](int i, int half) {
-    const int slot = zr_wide_visit_slot<KS>(kslice, i);
-    const int tn = slot >> 4, r = slot & 15;
-    const int n = n0 + tn * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-    return n < mb ? n : mb - 1;
-  };
-  auto clamp_col = [&](int c) { return c < mb ? c : mb - 1; };
-  auto clamp_id = [&](int v) { return v < 0 ? 0 : (v >= P.V ? P.V - 1 : v); };
-
-  const float* bias = P.bias[l];
-  float bi, bf, bc, bo;
-  float c_state[NV];  // cell state of this thread's outputs, carried from step to step
-  int idv[TN];        // layer 0: embedding column of each batch column, fetched one step ahead
-  {
-    const int jl = lane & 31, half = lane >> 5;
-    const int jc = j0 + jl < H ? j0 + jl : H - 1;
-    bi = bias[jc], bf = bias[H + jc], bc = bias[2 * H + jc], bo = bias[3 * H + jc];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) c_state[i] = P.c0[l][(long long)visit_col(i, half) * H + jc];
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) idv[tn] = (l == 0) ? clamp_id(P.ids[clamp_col(n0 + tn * 32 + jl)]) : 0;
-  }
-
-  const long long HH = (long long)P.kp * P.ldw;
-  const float* Wl = P.W[l];
-  int* my_ctr = P.counters + (l * P.n_tiles + nt) * kSweepCtrStride;
-  int* below_ctr = P.counters + ((l > 0 ? l - 1 : 0) * P.n_tiles + nt) * kSweepCtrStride;
-  float* hp_mine = P.hp + (long long)l * P.T * n_el;
-  const float* hp_below = P.hp + (long long)(l > 0 ? l - 1 : 0) * P.T * n_el;
-  float* gates = P.gates_all[l];
-
-  for (int t = 0; t < P.T; ++t) {
-    // Everything that depends on the lane is derived afresh in each time step from a lane index the compiler cannot
-    // see through: hoisted out of the loop, the per-lane addresses of both K loops would have to stay in registers
-    // through all of it, and the kernel has none to spare.
-    int lane_t = lane;
-    asm volatile("" : "+v"(lane_t));
-    const int jl = lane_t & 31, half = lane_t >> 5;
-    const int j = j0 + jl;
-    const bool j_ok = j < H;
-    int cols[TN];
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) cols[tn] = clamp_col(n0 + tn * 32 + jl);
-    const unsigned woffb = 16u * (unsigned)(j + half * P.ldw);
-    int idn[TN];
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const int tt = t + 1 < P.T ? t + 1 : t;
-      idn[tn] = (l == 0) ? clamp_id(P.ids[(long long)tt * mb + cols[tn]]) : 0;
-    }
-
-    zr_f32x16 acc[4][TN];
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[g][tn][r] = 0.0f;
-
-    for (int q = 0; q < 2; ++q) {
-      // segment 0: input from below (h of (l-1, t), or the embedding columns); segment 1: h of (l, t-1).  Layers above
-      // the first take the recurrent segment first: it only needs the layer's own previous step, so a layer can trail
-      // the one below it by half a step instead of a whole one (the pipeline of layers fills and drains in half the
-      // time) and the wait for the layer below hides behind half a K loop.  The order is fixed per layer, so the
-      // summation order, and with it every bit of the result, does not depend on timing.
-      const int s = (l > 0) ? 1 - q : q;
-      const bool packed = (s == 0) ? (l > 0) : (t > 0);
-      // The weights of the first ring stages go out before the wait for the activations: they depend on nothing, so
-      // their latency overlaps the poll (and the wait, when there is one): -2.8 % per sweep.  (Sending those of a
-      // step's first segment out even earlier, before the previous step's epilogue, keeps 96 more registers live
-      // through it and came out 0.3 % slower.)
-      unsigned wsoff[4];
-#pragma unroll
-      for (int g = 0; g < 4; ++g) wsoff[g] = (unsigned)(((long long)s * 4 + g) * HH * 4);
-      constexpr int PF = lstm_prefetch_depth(TN, KS);
-      ZrFrag<4, TN> ring[PF + 1];
-      const __amdgpu_buffer_rsrc_t wrsrc = zr_make_rsrc(Wl);
-      zr_preload_w<4, TN, KS, PF>(ring, wrsrc, wsoff, woffb, 32u * (unsigned)P.ldw, H, kslice);
-      if (packed) {
-        int* ctr = (s == 0) ? below_ctr : my_ctr;
-        const int target = ((s == 0) ? t + 1 : t) * P.j_tiles;
-        if (!sweep_wait(P, ctr, target, &s_go[s])) return;
-      }
-      const float* xp = (s == 0) ? hp_below + (long long)t * n_el : hp_mine + (long long)(t > 0 ? t - 1 : 0) * n_el;
-      const float* xu = (s == 0) ? P.embed : P.h0[l];
-      unsigned xoffb[TN];
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) {
-        const unsigned c = (s == 0) ? (unsigned)idv[tn] : (unsigned)cols[tn];
-        xoffb[tn] = packed ? 16u * ((unsigned)cols[tn] + (unsigned)(half * mb)) : 4u * (c * (unsigned)H + 4u * half);
-      }
-      zr_mma_segment_u<4, TN, KS, PF, true>(acc, wrsrc, wsoff, woffb, 32u * (unsigned)P.ldw,
-                                            zr_make_rsrc(packed ? xp : xu), xoffb, packed ? 32u * (unsigned)mb : 32u, H,
-                                            kslice, ring);
-    }
-
-    // the column masks are fetched here, behind the K loops, and arrive while the partial tiles are being summed
-    float mask_v[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) mask_v[i] = (float)P.mask01[(long long)t * mb + visit_col(i, half)];
-    float* h_out = P.h_all[l] + (long long)t * n_el;
-    float* c_out = P.c_all[l] + (long long)t * n_el;
-    float* hp_out = hp_mine + (long long)t * n_el;
-    // Only the k-interleaved copy of h, which the waiting workgroups read, goes out before the arrival is published;
-    // the outputs nobody waits for (h, c and the gate values kept for training) are held in registers and stored
-    // after it, so that their write latency overlaps the next step instead of sitting in front of the publish.
-    float h_v[NV], g_v[4][NV];
-    zr_reduce_visit_wide<4, TN, KS>(acc, red, kslice, lane, [&](const float(&z)[4], int tn, int r, int vi) {
-      const int n = n0 + tn * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-      float c;
-      zr_lstm_cell(z[0] + bi, z[1] + bf, z[2] + bc, z[3] + bo, c_state[vi], mask_v[vi], P.clip, g_v[0][vi], g_v[1][vi],
-                   g_v[2][vi], g_v[3][vi], c, h_v[vi]);
-      c_state[vi] = c;
-      if (j_ok && n < mb)
-        __hip_atomic_store(hp_out + ((long long)(j >> 2) * mb + n) * 4 + (j & 3), h_v[vi], __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    });
-    // publish this step: every wave's stores have completed before the barrier, then one arrival per workgroup
-    zr_publish_barrier();
-    if (tid == 0) atomicAdd(my_ctr, 1);
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int slot = zr_wide_visit_slot<KS>(kslice, i);
-      const int n = n0 + (slot >> 4) * 32 + 8 * ((slot & 15) >> 2) + 4 * half + (slot & 3);
-      if (j_ok && n < mb) {
-        const long long ix = (long long)n * H + j;
-        c_out[ix] = c_state[i];
-        h_out[ix] = h_v[i];
-        if (gates) {
-          float* gt = gates + (long long)t * 4 * n_el + ix;
-#pragma unroll
-          for (int g = 0; g < 4; ++g) gt[g * n_el] = g_v[g][i];
-        }
-      }
-    }
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) idv[tn] = idn[tn];
-  }
-}
-
-// ---------------------------------------------------------------------------------------------------------
 // One decoder time step through ALL layers in one launch (the LSTM part of neuralMT_model::forward_prop_target,
 // src/model.hpp:2573-2640: layer 0 on the embedding column of the current word, the previous step's attention output
 // through Q when feed-input is on, layer l > 0 on h_t of layer l-1).
@@ -1315,24 +1070,6 @@ int launch_fused(zr_ctx* ctx, LstmLaunch& L, bool vec) {
 }
 
 
-// Resident workgroups of lstm_sweep_kernel<TN> the device can hold at once (0: unknown / query failed).
-template <int TN>
-int sweep_capacity(zr_ctx* ctx) {
-  int& cached = ctx->sweep_capacity[TN];
-  if (cached == 0) {
-    int cus = 0, per_cu = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lstm_sweep_kernel<TN>, 256, 0) != hipSuccess) {
-      (void)hipGetLastError();
-      cached = -1;
-    } else {
-      ctx->cu_count = cus;
-      cached = cus * per_cu > 0 ? cus * per_cu : -1;
-    }
-  }
-  return cached > 0 ? cached : 0;
-}
-
 // Runs right behind lstm_sweep_kernel.  A sweep whose workgroups gave up a wait leaves part of h_all / c_all
 // unwritten; whatever is queued behind it on the stream would read stale memory.  When the status flag is up this
 // kernel overwrites every output of the sweep with NaN, so that nothing downstream can pass for a result; when it
@@ -1367,13 +1104,6 @@ int poison_if_abandoned(zr_ctx* ctx, int nl, int T, int H, int mb, float* const 
   lstm_sweep_poison_kernel<<<(unsigned)(blocks < 512 ? blocks : 512), 256, 0, ctx->stream>>>(Q);
   ZR_LAUNCH_CHECK("lstm_sweep_poison_kernel");
   return ZR_OK;
-}
-
-template <int TN>
-int launch_sweep_v(zr_ctx* ctx, LstmSweep& P, int grid) {
-  lstm_sweep_kernel<TN><<<grid, 256, 0, ctx->stream>>>(P);
-  ZR_LAUNCH_CHECK("lstm_sweep_kernel");
-  return poison_if_abandoned(ctx, P.nl, P.T, P.H, P.mb, P.h_all, P.c_all, P.gates_all);
 }
 
 // Resident workgroups of lstm_decoder_stack_kernel (either tile width) the device can hold at once (0: unknown /
@@ -1833,16 +1563,16 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
   const bool single_ok = !layers[0]->bf16 && ctx->lstm_fused && (ctx->lstm_sweep >= 2 || (ctx->lstm_sweep == 0 && alone));
   // Whole-sweep kernel with streamed weights: when its workgroups -- one tile of one layer each, kept for all T steps --
   // fit on the chip together.
-  const int j_tiles = (H + 31) / 32, n32 = (mb + 31) / 32;
+  const int j_tiles = (H + 31) / 32, n32 = (mb + 31) / 32, columns = (mb + 7) & ~7;
   const int groups = nl * j_tiles;
   const int padded = (groups + 7) / 8 * 8;
   int tn = 0;
   if (single_ok && vec && H % 8 == 0 && nl <= kMaxUnits) {
-    if ((long long)padded * n32 <= sweep_capacity<1>(ctx)) tn = 1;
-    else if ((long long)padded * ((n32 + 1) / 2) <= sweep_capacity<2>(ctx)) tn = 2;
+    if ((long long)padded * n32 <= zr_sweep_capacity(ctx, 1)) tn = 1;
+    else if ((long long)padded * ((n32 + 1) / 2) <= zr_sweep_capacity(ctx, 2)) tn = 2;
     // the kernel addresses its operands as descriptor base + 32-bit byte offsets
     const long long lim = 1LL << 32;
-    const bool offsets_fit = (long long)V * H * 4 < lim && (long long)n * 4 < lim &&
+    const bool offsets_fit = (long long)V * H * 4 < lim && 6LL * H * columns < lim &&
                              8LL * layers[0]->kp * layers[0]->ldw * 4 < lim;
     if (!offsets_fit || (tn && nl * ((n32 + tn - 1) / tn) > 512) || (long long)T * j_tiles >= kSweepGaveUp) tn = 0;
   }
@@ -1867,15 +1597,21 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
       return poison_if_abandoned(ctx, nl, T, H, mb, d_h_all, d_c_all, d_gates_all);
     }
   }
+  const size_t ctr_bytes = sizeof(int) * 512 * kSweepCtrStride;
+  void* p = nullptr;
+  if (tn) {
+    // h of every node as three bf16 terms, and the embedding columns; without the memory for that, one launch per diagonal
+    rc = zr_ctx_scratch(ctx, 1, ctr_bytes + 6 * ((size_t)nl * (T + 1) + T) * H * columns, &p);
+    if (rc == ZR_ENOMEM) tn = 0;
+    else if (rc) return rc;
+  }
   if (tn) {
     const int n_tiles = (n32 + tn - 1) / tn;
     LstmSweep P = {};
-    const size_t ctr_bytes = sizeof(int) * 512 * kSweepCtrStride;
-    void* p = nullptr;
-    rc = zr_ctx_scratch(ctx, 1, ctr_bytes + sizeof(float) * (size_t)nl * T * n, &p);
-    if (rc) return rc;
     P.counters = (int*)p;
-    P.hp = (float*)((char*)p + ctr_bytes);
+    P.hp = (unsigned short*)((char*)p + ctr_bytes);
+    P.xp = P.hp + 3 * (size_t)nl * (T + 1) * H * columns;
+    P.columns = columns;
     rc = zr_memset_zero(ctx, P.counters, sizeof(int) * (size_t)nl * n_tiles * kSweepCtrStride);
     if (rc) return rc;
     for (int l = 0; l < nl; ++l) {
@@ -1902,12 +1638,10 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
     P.n_tiles = n_tiles;
     P.clip = clip_threshold;
     P.spin_limit = ctx->sweep_spin > 0 ? ctx->sweep_spin : (1 << 20);
-    // Without the invalidation a consumer relies on never having cached a line before its producer wrote it: true
-    // when no 128-byte line of the k-interleaved copies is shared between two producers, i.e. mb % 8 == 0.
-    P.fence = (mb % 8 == 0) ? 0 : 1;
     ctx->last_stack_path = ZR_LSTM_STACK_PATH_SWEEP;
     ctx->last_sweep_kernel = ZR_LSTM_SWEEP_STREAMED;
-    return tn == 1 ? launch_sweep_v<1>(ctx, P, padded * n_tiles) : launch_sweep_v<2>(ctx, P, padded * n_tiles);
+    rc = zr_sweep_launch(ctx, P, tn);
+    return rc ? rc : poison_if_abandoned(ctx, nl, T, H, mb, d_h_all, d_c_all, d_gates_all);
   }
   // Every h is also written in a k-interleaved layout ([H/4][mb][4]) into a small ping-pong buffer per layer: its
   // two consumers on the next diagonal, (l+1, t) and (l, t+1), then fetch activations with contiguous 16-byte

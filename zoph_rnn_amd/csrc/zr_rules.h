@@ -80,12 +80,13 @@ inline double zr_sweep_diagonals_us(int nl, int H, int mb, int T, bool vec, int 
   return us;
 }
 
-// Streamed weights on tiles of 32 * tn columns: a hand-over of 5 us, a little more with every layer, and the K loop of a workgroup (the groups of 8 k of both
-// segments over 4 waves, 16 tn instructions of 64 cycles each at 2.3 GHz), or the weights at 6 TB/s where they outgrow the
-// caches (4 layers of H = 2000 87 us a step, 61 by the K loop); half a step more per layer to fill.
+// Streamed weights on tiles of 32 * tn columns: a hand-over, a little more with every layer, and the steps of 64 k of both segments (an even number of
+// each) at 0.74 us of 32 columns and 1.18 of 64, or the weights at 6 TB/s where they outgrow the caches (4 layers of H = 2000 85 us a
+// step); half a step more per layer to fill.  Within 17 % of 297 sizes (H = 128 .. 2000, 12 to 256 columns), 4 % on average.
 inline double zr_sweep_streamed_us(int nl, int H, int T, int tn) {
-  const double k_loop = 2.0 * ((H + 7) / 8) / 4 * 16 * 64 / 2300.0 * tn, weights = 32.0 * nl * H * H / 6.0e6;
-  return (T + 0.5 * nl) * (4.9 + 0.25 * nl + (k_loop > weights ? k_loop : weights));
+  const double steps = (H + 127) / 128 * 4.0, weights = 32.0 * nl * H * H / 6.0e6 + 3.5;
+  const double k_loop = tn == 1 ? 3.6 + 0.42 * nl + 0.74 * steps : 1.5 + 1.6 * nl + 1.18 * steps;
+  return (T + 0.5 * nl) * (k_loop > weights ? k_loop : weights);
 }
 
 // Resident weights, one launch of `layers` layers (the sweep's first or a later one): classes by H up to 128, 256, 512, 1024 and
