@@ -30,15 +30,20 @@ struct zr_lstm_train {
 namespace {
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+// Floats from one address of device memory to another, which need not be of the same allocation.
+inline long long float_offset(const float* from, const float* to) {
+  return (long long)((intptr_t)to - (intptr_t)from) / (long long)sizeof(float);
+}
 
-__global__ void __launch_bounds__(256) stack_gates_kernel(const float* __restrict__ g0, const float* __restrict__ g1,
-                                                          const float* __restrict__ g2, const float* __restrict__ g3,
-                                                          int H, float* __restrict__ dst) {
-  // dst: H x 4H column-major, dst[k + (g*H + j)*H] = W_g[j + k*H]; 32 x 32 tiles through LDS
+struct StackGates {
+  const float* src[8];
+};
+__global__ void __launch_bounds__(256) stack_gates_kernel(StackGates P, int H, float* __restrict__ dst) {
+  // two stacks of four gates, H x 4H column-major each: dst[k + (g*H + j)*H] = W_g[j + k*H]; 32 x 32 tiles through LDS
   __shared__ float tile[32][33];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int g = blockIdx.z;
-  const float* src = g == 0 ? g0 : (g == 1 ? g1 : (g == 2 ? g2 : g3));
+  const float* src = P.src[g];
   const int j0 = blockIdx.x * 32, k0 = blockIdx.y * 32;
   for (int i = ty; i < 32; i += 8) {
     const int j = j0 + tx, k = k0 + i;
@@ -415,6 +420,52 @@ __global__ void __launch_bounds__(256) sgd_apply_kernel(float* __restrict__ W, c
 }
 
 
+// The update of a small matrix (ZR_CLIP_MATRIX_NORM) in one launch: every workgroup adds up the squares of the whole gradient, in the same
+// order, and updates its own part of W.  vec: W and g 16-byte aligned.  W and g do not overlap.
+__global__ void __launch_bounds__(1024) sgd_small_kernel(float* __restrict__ W, const float* __restrict__ g, int n, int vec, float scale,
+                                                         float threshold, float lr) {
+  __shared__ double s[16];
+  const int tid = threadIdx.x, n4 = vec ? n >> 2 : 0;
+  const zr_f32x4* g4 = (const zr_f32x4*)g;
+  double acc[4] = {};
+  int i = tid;
+  for (; i + 3 * 1024 < n4; i += 4 * 1024) {
+    zr_f32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = g4[i + 1024 * u];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[u] += (double)v[u][c] * (double)v[u][c];
+  }
+  for (; i < n4; i += 1024) {
+    const zr_f32x4 v = g4[i];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] += (double)v[c] * (double)v[c];
+  }
+  for (i = 4 * n4 + tid; i < n; i += 1024) acc[0] += (double)g[i] * (double)g[i];
+  double ss = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+  if ((tid & 63) == 0) s[tid >> 6] = ss;
+  __syncthreads();
+  ss = 0.0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) ss += s[w];
+  const float norm = (float)sqrt(ss) * fabsf(scale);
+  const float f = lr * (norm > threshold ? threshold / norm : 1.0f) * scale;
+  const int first = blockIdx.x * 1024 + tid, stride = gridDim.x * 1024;
+  for (i = first; i < n4; i += stride) {
+    const zr_f32x4 x = g4[i];
+    zr_f32x4 w = ((zr_f32x4*)W)[i];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) w[c] += f * x[c];
+    ((zr_f32x4*)W)[i] = w;
+  }
+  for (i = 4 * n4 + first; i < n; i += stride) W[i] += f * g[i];
+}
+
+
 // ---- attention backward (attention_node::back_prop, src/attention_node.hpp:398-669) --------------------------------
 
 __device__ __forceinline__ float bwd_wave_sum(float v) {
@@ -431,14 +482,39 @@ __device__ __forceinline__ float bwd_block_sum(float v, float* red) {
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// zero_h_t + tanh_grad_kernel (src/custom_kernels.h:2212, :1835): e = err * mask * (1 - h~^2)
-__global__ void __launch_bounds__(256) attn_bwd_e_kernel(const float* __restrict__ err, const float* __restrict__ htild,
-                                                         const int* __restrict__ mask01, int H, long long n,
-                                                         float* __restrict__ e) {
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-    const float t = htild[i];
-    e[i] = err[i] * (float)mask01[i / H] * (1.0f - t * t);
+// What a workgroup of 1024 threads does that writes 32 rows of an H x mb matrix and adds the sum of other values over the columns to a
+// vector: thread (x, y) has row x of the block and every 32nd column.  f(i, column, row) stores element i and returns what is summed.
+// One launch where an element-wise kernel and a sum over its result were two (H = 500, 64 columns: 2.6 and 3.3 us).
+template <typename F>
+__device__ __forceinline__ void rows_with_sum(F f, int H, int mb, float* __restrict__ sum) {
+  __shared__ float part[32][32];
+  const int x = threadIdx.x & 31, y = threadIdx.x >> 5, row = blockIdx.x * 32 + x;
+  float s = 0.0f;
+  if (row < H) {
+#pragma unroll 4
+    for (int b = y; b < mb; b += 32) s += f((size_t)b * H + row, b, row);
   }
+  part[y][x] = s;
+  __syncthreads();
+  if (y == 0 && row < H) {
+#pragma unroll
+    for (int i = 1; i < 32; ++i) s += part[i][x];
+    sum[row] += s;
+  }
+}
+
+// zero_h_t + tanh_grad_kernel (src/custom_kernels.h:2212, :1835): e = err * mask * (1 - h~^2); its sum over the columns is the gradient of
+// the output bias
+__global__ void __launch_bounds__(1024) attn_bwd_e_kernel(const float* __restrict__ err, const float* __restrict__ htild,
+                                                          const int* __restrict__ mask01, int H, int mb,
+                                                          float* __restrict__ e, float* __restrict__ d_bias) {
+  rows_with_sum(
+      [&](size_t i, int b, int) {
+        const float t = htild[i], v = err[i] * (float)mask01[b] * (1.0f - t * t);
+        e[i] = v;
+        return v;
+      },
+      H, mb, d_bias);
 }
 
 // error_alignments_kernel_large + error_hs_ct_kernel_large (:1968, :2179), one workgroup per (window slot, column):
@@ -523,20 +599,22 @@ __global__ void __launch_bounds__(64) attn_bwd_column_kernel(const float* __rest
 }
 
 // att_vp_error and grad_W_p_kernel (:2040, :2051) in one pass over tanh_1
-__global__ void __launch_bounds__(256) attn_bwd_vp_wp_kernel(const float* __restrict__ tanh1,
-                                                             const float* __restrict__ v_p,
-                                                             const float* __restrict__ col, int H, int mb, long long n,
-                                                             float* __restrict__ tv, float* __restrict__ tw) {
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-    const int b = (int)(i / H), k = (int)(i % H);
-    const float t = tanh1[i], sig = col[2 * mb + b];
-    tv[i] = col[b] * t;
-    tw[i] = col[mb + b] * v_p[k] * sig * (1.0f - sig) * (1.0f - t * t);
-  }
+__global__ void __launch_bounds__(1024) attn_bwd_vp_wp_kernel(const float* __restrict__ tanh1,
+                                                              const float* __restrict__ v_p,
+                                                              const float* __restrict__ col, int H, int mb,
+                                                              float* __restrict__ tw, float* __restrict__ d_vp) {
+  rows_with_sum(
+      [&](size_t i, int b, int k) {
+        const float t = tanh1[i], sig = col[2 * mb + b];
+        tw[i] = col[mb + b] * v_p[k] * sig * (1.0f - sig) * (1.0f - t * t);
+        return col[b] * t;
+      },
+      H, mb, d_vp);
 }
 
-// The loop of src/attention_node.hpp:580-601 for one column per workgroup: h_s_sum[:, b] = sum_j scaling_j h_s_j
-// (scale_ht_kernel + add_two_mats_kernel) and the error of h_s_j += scaling_j * (W_a^T h)[:, b] (copy_errors_source).
+// The loop of src/attention_node.hpp:580-601, 256 rows of one column per workgroup: h_s_sum[:, b] = sum_j scaling_j h_s_j
+// (scale_ht_kernel + add_two_mats_kernel) and the error of h_s_j += scaling_j * (W_a^T h)[:, b] (copy_errors_source).  Eight source states on their
+// way at once: one after another, with 64 workgroups for 64 columns, took 15.8 us at H = 500.
 __global__ void __launch_bounds__(256) attn_bwd_hs_kernel(const float* __restrict__ q,
                                                           const float* const* __restrict__ table,
                                                           float* const* __restrict__ err_table,
@@ -544,26 +622,35 @@ __global__ void __launch_bounds__(256) attn_bwd_hs_kernel(const float* __restric
                                                           const int* __restrict__ indices,
                                                           const float* __restrict__ scal, int H, int mb, int W,
                                                           int longest, float* __restrict__ hs_sum) {
-  const int b = blockIdx.x;
+  const int b = blockIdx.x, i = blockIdx.y * 256 + threadIdx.x;
+  if (i >= H) return;
   const int len = batch_info[b], off = batch_info[mb + b];
-  for (int i0 = 0; i0 < H; i0 += 256) {
-    const int i = i0 + threadIdx.x;
-    const bool ok = i < H;
-    const float qv = ok ? q[(size_t)b * H + i] : 0.0f;
-    float acc = 0.0f;
-    for (int j = 0; j < W; ++j) {
-      const int s = indices[b + (size_t)mb * j];
-      if (s == -1) continue;
+  const size_t at = (size_t)b * H + i;
+  const float qv = q[at];
+  float acc = 0.0f;
+  for (int j0 = 0; j0 < W; j0 += 8) {
+    float hs[8], err[8], sc[8];
+    float* to[8];
+    bool on[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {  // the same in every thread
+      const int j = j0 + u < W ? j0 + u : W - 1, s = indices[b + (size_t)mb * j];
+      on[u] = j0 + u < W && s != -1;
       int t = len - 1 - s + off;
       t = t < 0 ? 0 : (t >= longest ? longest - 1 : t);
-      const float sc = scal[j + (size_t)W * b];
-      if (ok) {
-        acc += table[t][(size_t)b * H + i] * sc;
-        err_table[t][(size_t)b * H + i] += qv * sc;
-      }
+      sc[u] = scal[j + (size_t)W * b];
+      to[u] = err_table[t] + at;
+      hs[u] = on[u] ? table[t][at] : 0.0f;
+      err[u] = on[u] ? *to[u] : 0.0f;
     }
-    if (ok) hs_sum[(size_t)b * H + i] = acc;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (on[u]) {
+        acc += hs[u] * sc[u];
+        *to[u] = err[u] + qv * sc[u];
+      }
   }
+  hs_sum[at] = acc;
 }
 
 // dropout_kernel (src/custom_kernels.h:1556-1560)
@@ -669,17 +756,12 @@ int zr_lstm_train_refresh(zr_ctx* ctx, zr_lstm_train* w, const float* const d_M[
   ZR_CHECK_ARG(w && d_M && d_Wh, "zr_lstm_train_refresh: null pointer");
   const int H = w->H;
   const size_t per = 4 * (size_t)H * H;
-  dim3 grid((H + 31) / 32, (H + 31) / 32, 4);
-  stack_gates_kernel<<<grid, 256, 0, ctx->stream>>>(d_Wh[0], d_Wh[1], d_Wh[2], d_Wh[3], H, w->d_stack);
+  StackGates P;
+  for (int g = 0; g < 4; ++g) P.src[g] = d_Wh[g], P.src[4 + g] = d_M[g];
+  stack_gates_kernel<<<dim3((H + 31) / 32, (H + 31) / 32, 8), 256, 0, ctx->stream>>>(P, H, w->d_stack);
   ZR_LAUNCH_CHECK("stack_gates_kernel");
-  stack_gates_kernel<<<grid, 256, 0, ctx->stream>>>(d_M[0], d_M[1], d_M[2], d_M[3], H, w->d_stack + per);
-  ZR_LAUNCH_CHECK("stack_gates_kernel");
-  for (int z = 0; z < 2; ++z) {
-    rc = zr_pack4_launch(ctx, w->d_stack + z * per, H, 4 * H, H, w->ldp, w->kp,
-                         w->d_stack_pack + (size_t)z * w->kp * w->ldp);
-    if (rc) return rc;
-  }
-  return ZR_OK;
+  const float* stacks[2] = {w->d_stack, w->d_stack + per};
+  return zr_pack4_multi_launch(ctx, 2, stacks, H, 4 * H, H, w->ldp, w->kp, w->d_stack_pack, 0, nullptr, nullptr);
 }
 
 int zr_lstm_train_destroy(zr_ctx* ctx, zr_lstm_train* w) {
@@ -786,6 +868,8 @@ int zr_lstm_stack_backward_clamped(zr_ctx* ctx, int nl, const zr_lstm_train* con
         g.gA[nu] = packed_ok ? layers[l]->d_stack_pack : layers[l]->d_stack;
         g.gB[nu] = bpack ? G.dgp[nu] : G.dg[nu];
         g.gC[nu] = w_l;
+        // layer 0's error to below goes where the caller wants it
+        if (l == 0 && d_err_below0) g.gStrideC[nu] = float_offset(w_l, d_err_below0 + (size_t)t * n);
         ++nu;
       }
       if (nu == 0) continue;
@@ -815,10 +899,6 @@ int zr_lstm_stack_backward_clamped(zr_ctx* ctx, int nl, const zr_lstm_train* con
       rc = zr_gemm_launch(ctx, g);
       if (rc) return rc;
     }
-    const int t0 = d;  // layer 0's node on this diagonal
-    if (d_err_below0 && t0 < T)
-      ZR_HIP(hipMemcpyAsync(d_err_below0 + (size_t)t0 * n, wk(d, 0) + n, sizeof(float) * n, hipMemcpyDeviceToDevice,
-                            ctx->stream));
   }
   // node (l, 0) is on diagonal l
   for (int l = 0; l < nl; ++l) {
@@ -918,22 +998,12 @@ int zr_lstm_node_backward(zr_ctx* ctx, const zr_lstm_train* layer, int mb, const
                    d_dgates && d_err_h_prev && d_err_c_prev,
                "zr_lstm_node_backward: null pointer");
   const int H = layer->H;
-  const size_t n = (size_t)H * mb;
   dim3 egrid((H + 255) / 256, mb);
   lstm_node_backward_kernel<<<egrid, 256, 0, ctx->stream>>>(d_gates[0], d_gates[1], d_gates[2], d_gates[3], d_c,
                                                             d_c_prev, d_mask01, d_err_above, d_err_h_next,
                                                             d_err_c_next, d_err_c_prev, H, mb, d_dgates);
   ZR_LAUNCH_CHECK("lstm_node_backward_kernel");
-  // the two error products share their right-hand side: one batched launch when the outputs are adjacent
-  // (d_err_below == d_err_h_prev + H*mb), else through a scratch pair and two copies
-  float* out = d_err_h_prev;
-  const bool adjacent = d_err_below == d_err_h_prev + n;
-  if (!adjacent) {
-    void* scratch = nullptr;
-    rc = zr_ctx_scratch(ctx, 1, sizeof(float) * 2 * n, &scratch);
-    if (rc) return rc;
-    out = (float*)scratch;
-  }
+  // the two error products share their right-hand side: one batched launch
   ZrGemmDesc g = {};
   g.M = H;
   g.N = mb;
@@ -946,19 +1016,12 @@ int zr_lstm_node_backward(zr_ctx* ctx, const zr_lstm_train* layer, int mb, const
   g.strideA = 4LL * H * H;
   g.B[0] = d_dgates;
   g.ldb[0] = 4 * H;
-  g.C = out;
+  g.C = d_err_h_prev;
   g.ldc = H;
   g.batch = d_err_below ? 2 : 1;
-  g.strideC = (long long)n;
+  g.strideC = d_err_below ? float_offset(d_err_h_prev, d_err_below) : 0;
   g.epilogue = ZR_EPI_STORE;
-  rc = zr_gemm_launch(ctx, g);
-  if (rc) return rc;
-  if (!adjacent) {
-    ZR_HIP(hipMemcpyAsync(d_err_h_prev, out, sizeof(float) * n, hipMemcpyDeviceToDevice, ctx->stream));
-    if (d_err_below)
-      ZR_HIP(hipMemcpyAsync(d_err_below, out + n, sizeof(float) * n, hipMemcpyDeviceToDevice, ctx->stream));
-  }
-  return ZR_OK;
+  return zr_gemm_launch(ctx, g);
 }
 
 int zr_attn_set_error_tables(zr_ctx* ctx, zr_attn* a, float* const* h_err_tables, int n) {
@@ -997,18 +1060,17 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   const size_t n = (size_t)H * mb;
   const float sigma_sq = (float)((a->D * a->D) / 4.0);  // src/attention_node.hpp:50
   void* scratch = nullptr;
-  rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (6 * n + 2 * (size_t)W * mb + 3 * (size_t)mb), &scratch);
+  rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (5 * n + 2 * (size_t)W * mb + 3 * (size_t)mb), &scratch);
   if (rc) return rc;
   float* e = (float*)scratch;
   float* err_ct = e + n;
-  float* tv = e + 2 * n;
-  float* tw = e + 3 * n;
-  float* hs_sum = e + 4 * n;
-  float* tr = e + 5 * n;  // a transposed right-hand side, mb x H
-  float* err_as = e + 6 * n;
+  float* tw = e + 2 * n;
+  float* hs_sum = e + 3 * n;
+  float* tr = e + 4 * n;  // a transposed right-hand side, mb x H
+  float* err_as = e + 5 * n;
   float* scal = err_as + (size_t)W * mb;
   float* col = scal + (size_t)W * mb;
-  const int eg = (int)((n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048);
+  const int row_blocks = (H + 31) / 32;
 
   // C (H x H) += A (H x mb) * B^T for B H x mb (cuBLAS gemm N, T with beta = 1 in the reference)
   auto outer_acc = [&](const float* A, const float* B, float* C) -> int {
@@ -1050,7 +1112,7 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
     return zr_gemm_launch(ctx, g);
   };
 
-  attn_bwd_e_kernel<<<eg, 256, 0, ctx->stream>>>(d_err_htild, d_h_tild, d_mask01, H, (long long)n, e);
+  attn_bwd_e_kernel<<<row_blocks, 1024, 0, ctx->stream>>>(d_err_htild, d_h_tild, d_mask01, H, mb, e, grads->d_out_bias);  // :456
   ZR_LAUNCH_CHECK("attn_bwd_e_kernel");
   const bool outer = zr_outer_takes(2, H, H, mb);
   if (outer) {
@@ -1060,7 +1122,6 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
     if ((rc = outer_acc(e, d_c_t, grads->d_W_c1))) return rc;                   // :437
     if ((rc = outer_acc(e, d_h_t, grads->d_W_c2))) return rc;                   // :443
   }
-  if ((rc = row_sum_launch(ctx, e, H, mb, grads->d_out_bias, 1))) return rc;    // :456
   {
     // W_c1^T e and W_c2^T e (:464, :476), one launch
     ZrGemmDesc g = {};
@@ -1087,13 +1148,12 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   attn_bwd_column_kernel<<<mb, 64, 0, ctx->stream>>>(a->d_tanh1, a->v_p, d_batch_info, d_indices, d_alignments, d_p_t,
                                                      err_as, H, mb, W, sigma_sq, col, scal);
   ZR_LAUNCH_CHECK("attn_bwd_column_kernel");
-  attn_bwd_vp_wp_kernel<<<eg, 256, 0, ctx->stream>>>(a->d_tanh1, a->v_p, col, H, mb, (long long)n, tv, tw);
+  attn_bwd_vp_wp_kernel<<<row_blocks, 1024, 0, ctx->stream>>>(a->d_tanh1, a->v_p, col, H, mb, tw, grads->d_v_p);  // :536
   ZR_LAUNCH_CHECK("attn_bwd_vp_wp_kernel");
-  if ((rc = row_sum_launch(ctx, tv, H, mb, grads->d_v_p, 1))) return rc;        // :536
   if (!outer && (rc = outer_acc(tw, d_h_t, grads->d_W_p))) return rc;           // :545
   if ((rc = product(a->W_p, 1, tw, d_err_h_t, 1, ZR_EPI_STORE))) return rc;     // :551
   if ((rc = product(a->W_a, 1, d_h_t, a->d_q, 0, ZR_EPI_STORE))) return rc;     // W_a^T h of the forward pass again
-  attn_bwd_hs_kernel<<<mb, 256, 0, ctx->stream>>>(a->d_q, a->d_table, a->d_err_table, d_batch_info, d_indices, scal, H, mb,
+  attn_bwd_hs_kernel<<<dim3(mb, (H + 255) / 256), 256, 0, ctx->stream>>>(a->d_q, a->d_table, a->d_err_table, d_batch_info, d_indices, scal, H, mb,
                                                   W, a->longest_sent, hs_sum);
   ZR_LAUNCH_CHECK("attn_bwd_hs_kernel");
   if (outer)
@@ -1355,6 +1415,13 @@ int zr_sgd_update_clipped(zr_ctx* ctx, float* d_W, const float* d_grad, long lon
   ZR_CHECK_ARG(clip_mode == ZR_CLIP_NONE || threshold > 0.0f, "zr_sgd_update_clipped: threshold = %g", (double)threshold);
   ZR_CHECK_ARG(clip_mode != ZR_CLIP_WHOLE_NORM || d_sumsq, "zr_sgd_update_clipped: whole-model clipping without d_sumsq");
   if (n == 0) return ZR_OK;
+  const int vec = aligned16(d_W) && aligned16(d_grad) ? 1 : 0;
+  const bool apart = (uintptr_t)(d_W + n) <= (uintptr_t)d_grad || (uintptr_t)(d_grad + n) <= (uintptr_t)d_W;
+  if (clip_mode == ZR_CLIP_MATRIX_NORM && apart && zr_sgd_small(n, vec)) {
+    sgd_small_kernel<<<(unsigned)(((vec ? (n + 3) / 4 : n) + 1023) / 1024), 1024, 0, ctx->stream>>>(d_W, d_grad, (int)n, vec, scale, threshold, learning_rate);
+    ZR_LAUNCH_CHECK("sgd_small_kernel");
+    return ZR_OK;
+  }
   const int n_partial = 256;
   void* scratch = nullptr;
   rc = zr_ctx_scratch(ctx, 1, sizeof(double) * n_partial, &scratch);
@@ -1363,7 +1430,6 @@ int zr_sgd_update_clipped(zr_ctx* ctx, float* d_W, const float* d_grad, long lon
     sumsq_partial_kernel<<<n_partial, 1024, 0, ctx->stream>>>(d_grad, n, aligned16(d_grad) ? 1 : 0, (double*)scratch);
     ZR_LAUNCH_CHECK("sumsq_partial_kernel");
   }
-  const int vec = aligned16(d_W) && aligned16(d_grad) ? 1 : 0;
   const long long blocks = ((vec ? (n + 3) / 4 : n) + 255) / 256;
   sgd_apply_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, ctx->stream>>>(
       d_W, d_grad, n, vec, scale, clip_mode, threshold, learning_rate, (const double*)scratch, n_partial, d_sumsq);

@@ -155,6 +155,7 @@ struct ZrGemmDesc {
   const float* gA[8];
   const float* gB[8];
   float* gC[8];
+  long long gStrideC[8];  // where a group's second result lies against its first (0: strideC)
 };
 
 int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d);
@@ -164,6 +165,9 @@ int zr_small_gemm(zr_ctx* ctx, const ZrGemmDesc& d, const unsigned short* const 
 // Packs one M x K column-major matrix (leading dimension ld) into the k-interleaved layout [kp/4][ldp][4] with
 // zero padding (ldp >= M a multiple of 32, kp >= K a multiple of 8).  dst holds kp*ldp floats.
 int zr_pack4_launch(zr_ctx* ctx, const float* src, int M, int K, long long ld, int ldp, int kp, float* dst);
+// The same for n (at most 12) matrices of one shape, matrix i to dst + i*kp*ldp, and n_vec (at most 4) vectors of M floats to vec_dst + i*M.
+int zr_pack4_multi_launch(zr_ctx* ctx, int n, const float* const* src, int M, int K, long long ld, int ldp, int kp, float* dst, int n_vec,
+                          const float* const* vec, float* vec_dst);
 // Activations X (K x N fp32, column n at src + n*ld, K % 4 == 0, 16-byte aligned) into the k-interleaved layout
 // [K/4][N][4] (element (k, n) at ((k/4)*N + n)*4 + k%4).
 int zr_pack4_x_launch(zr_ctx* ctx, const float* src, int K, int N, int ld, float* dst);

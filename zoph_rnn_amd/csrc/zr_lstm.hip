@@ -1166,27 +1166,25 @@ static int pack_weights(zr_ctx* ctx, const char* who, bool bf16, const float* co
     delete w;
     return zr_set_error(ZR_ENOMEM, "%s: allocation failed (H = %d, nseg = %d)", who, H, nseg);
   }
-  for (int g = 0; g < 4; ++g) {
-    const float* segs[3] = {d_M[g], d_Wh[g], d_Q ? d_Q[g] : nullptr};
-    for (int s = 0; s < nseg; ++s) {
-      const size_t off = ((size_t)s * 4 + g) * HH;
-      rc = bf16 ? zr_pack8_bf16_launch(ctx, segs[s], H, H, H, ldw, kp, (unsigned short*)w->d_W + off)
-                : zr_pack4_launch(ctx, segs[s], H, H, H, ldw, kp, (float*)w->d_W + off);
-      if (rc != ZR_OK) {
-        (void)hipFree(w->d_W);
-        (void)hipFree(w->d_bias);
-        delete w;
-        return ZR_EHIP;
-      }
+  const float* mats[12];
+  for (int s = 0; s < nseg; ++s)
+    for (int g = 0; g < 4; ++g) mats[4 * s + g] = s == 0 ? d_M[g] : (s == 1 ? d_Wh[g] : d_Q[g]);
+  rc = ZR_OK;
+  if (bf16) {
+    for (int i = 0; i < 4 * nseg && rc == ZR_OK; ++i)
+      rc = zr_pack8_bf16_launch(ctx, mats[i], H, H, H, ldw, kp, (unsigned short*)w->d_W + i * HH);
+    for (int g = 0; g < 4 && rc == ZR_OK; ++g) {
+      hipError_t e = hipMemcpyAsync(w->d_bias + (size_t)g * H, d_b[g], sizeof(float) * H, hipMemcpyDeviceToDevice, ctx->stream);
+      if (e != hipSuccess) rc = zr_set_error(ZR_EHIP, "%s: bias copy failed: %s", who, hipGetErrorString(e));
     }
-    hipError_t e = hipMemcpyAsync(w->d_bias + (size_t)g * H, d_b[g], sizeof(float) * H, hipMemcpyDeviceToDevice,
-                                  ctx->stream);
-    if (e != hipSuccess) {
-      (void)hipFree(w->d_W);
-      (void)hipFree(w->d_bias);
-      delete w;
-      return zr_set_error(ZR_EHIP, "%s: bias copy failed: %s", who, hipGetErrorString(e));
-    }
+  } else {
+    rc = zr_pack4_multi_launch(ctx, 4 * nseg, mats, H, H, H, ldw, kp, (float*)w->d_W, 4, d_b, w->d_bias);
+  }
+  if (rc != ZR_OK) {
+    (void)hipFree(w->d_W);
+    (void)hipFree(w->d_bias);
+    delete w;
+    return ZR_EHIP;
   }
   *out = w;
   return ZR_OK;

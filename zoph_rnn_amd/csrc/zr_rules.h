@@ -285,3 +285,10 @@ inline ZrLogitsPlan zr_logits_plan(int V, int cols, int H, int cus) {
   if (other > 0.0 && other <= best) plan.tn = plan.waves = 0;
   return plan;
 }
+
+// ---- the clipped update of one matrix (zr_sgd_update): one launch whose workgroups each read the whole gradient, or a launch for the
+// norm and one for the update
+
+// us of a call, one launch / two (the second is the time to launch them): 300 values 4.2 / 7.0, 40000 4.2 / 7.0, 90000 5.6 / 7.0, 131072 6.6 / 7.0,
+// 160000 7.6 / 7.0, 250000 10.0 / 6.9.  A quarter of that with four bytes a load.
+inline bool zr_sgd_small(long long n, bool vec) { return n <= (vec ? 112000 : 28000); }

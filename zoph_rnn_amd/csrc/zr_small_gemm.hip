@@ -34,6 +34,7 @@ struct SmallArgs {
   const float* gA[8];
   const float* gB[8];
   float* gC[8];
+  long long gStrideC[8];
 };
 
 typedef zr_f32x4 zr_f32x4_u __attribute__((aligned(4)));
@@ -67,7 +68,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a)
   const int tid = threadIdx.x, lane = tid & 63, cl = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = 16 * TM * mt, n0 = 16 * TN * nt;
-  float* C = (a.groups ? a.gC[group] : a.C) + zb * a.strideC;
+  float* C = a.groups ? a.gC[group] + zb * a.gStrideC[group] : a.C + zb * a.strideC;
   const float* bias = a.bias ? a.bias + zb * a.strideBias : nullptr;
 
   // the outputs this thread finishes: what is added to them is fetched ahead of the K loop
@@ -281,7 +282,7 @@ int zr_small_gemm(zr_ctx* ctx, const ZrGemmDesc& d, const unsigned short* const 
   a.strideA = d.strideA, a.strideC = d.strideC, a.strideBias = d.strideBias;
   a.bias = d.bias, a.mask = d.mask, a.Cpack = d.Cpack, a.Chi = d.Chi, a.Clo = d.Clo;
   a.groups = d.groups;
-  for (int g = 0; g < d.groups; ++g) a.gA[g] = d.gA[g], a.gB[g] = d.gB[g], a.gC[g] = d.gC[g];
+  for (int g = 0; g < d.groups; ++g) a.gA[g] = d.gA[g], a.gB[g] = d.gB[g], a.gC[g] = d.gC[g], a.gStrideC[g] = d.gStrideC[g] ? d.gStrideC[g] : d.strideC;
   const int tm = shape == 2 ? 32 : 16, tn = shape == 0 ? 16 : 32;
   a.m_tiles = (d.M + tm - 1) / tm;
   a.n_tiles = (d.N + tn - 1) / tn;
