@@ -1371,6 +1371,10 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
         ZR_CHECK_ARG(d.K[s] % 8 == 0, "gemm: a k-interleaved B needs K %% 8 == 0 (K[%d] = %d)", s, d.K[s]);
       ga.b_pack4 = 1;
     }
+    if (d.groups > 0 && ga.b_pack4 && vec && d.K[0] % 8 == 0 && d.epilogue == ZR_EPI_STORE && !d.accumulate && ctx->gemm_cfg == 0 &&
+        (long long)d.K[0] * (d.lda[0] > d.N ? d.lda[0] : d.N) * 4 < (1LL << 32) &&
+        zr_error_products_takes((long long)((d.M + 31) / 32) * ((d.N + 31) / 32) * zcount, d.N, ctx->cu_count))
+      return zr_error_products(ctx, d);
     if (small >= 0) return zr_small_gemm(ctx, d, nullptr, nullptr, small);
     // Wide batches: the tall and row-range kernels serve up to 256 columns as well or better (50000 x 192 x 1000: 167
     // against 175 us), beyond that the split product does (33333 x 700 x 500: 174 against 602 us).  With fixed scratch

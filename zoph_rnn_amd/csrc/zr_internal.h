@@ -162,6 +162,8 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d);
 // Small products on narrow tiles (zr_small_gemm.hip), every segment with the same K, any epilogue but the soft-max partials;
 // shape: as zr_small_gemm_shape has it (zr_rules.h).  Bhi / Blo: the activations' bf16 terms where d.a_pack == 2 (Blo[0] null: one term).
 int zr_small_gemm(zr_ctx* ctx, const ZrGemmDesc& d, const unsigned short* const Bhi[4], const unsigned short* const Blo[4], int shape);
+// Grouped products on k-interleaved operands of K % 8 == 0 (d.b_packed), plain stores, as three bf16 terms an operand (zr_error_products.hip).
+int zr_error_products(zr_ctx* ctx, const ZrGemmDesc& d);
 // Packs one M x K column-major matrix (leading dimension ld) into the k-interleaved layout [kp/4][ldp][4] with
 // zero padding (ldp >= M a multiple of 32, kp >= K a multiple of 8).  dst holds kp*ldp floats.
 int zr_pack4_launch(zr_ctx* ctx, const float* src, int M, int K, long long ld, int ldp, int kp, float* dst);

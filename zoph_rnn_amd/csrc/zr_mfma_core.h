@@ -212,8 +212,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t zr_make_rsrc(const void* base)
 // The weight halves of the first PF ring stages of a segment, issued ahead of time (zr_mma_segment_u with WPRE then
 // fetches only the activation halves in its prologue): weights depend on nothing, so a caller that must wait for its
 // activations can have them in flight during the wait.
-template <int TM, int TN, int KS, int PF, int WAUX = 0>
-__device__ __forceinline__ void zr_preload_w(ZrFrag<TM, TN> (&f)[PF + 1], __amdgpu_buffer_rsrc_t wrsrc,
+template <int TM, int TN, int KS, int PF, int WAUX = 0, int NS = PF + 1>
+__device__ __forceinline__ void zr_preload_w(ZrFrag<TM, TN> (&f)[NS], __amdgpu_buffer_rsrc_t wrsrc,
                                              const unsigned (&wsoff)[TM], unsigned woffb, unsigned wstep, int K,
                                              int kslice) {
   const int last = (K >> 3) - 1;
@@ -308,6 +308,161 @@ __device__ __forceinline__ void zr_mma_segment_u(zr_f32x16 (&acc)[TM][TN], __amd
     for (int s = 0; s < PF; ++s)
       if (it + s < n_mine) mma(f[s]);
   }
+}
+
+// zr_mma_segment_u on the bf16 matrix cores: every fp32 operand as three exact bf16 terms, six products, the same loads.  Two k-groups make
+// one step: a lane's eight k are its four of the one and its four of the other, for both operands.  The terms of a step are made beside
+// the products of the step before, and a revolution's products are summed from zero before they reach the accumulator.  R: slots of the ring (a multiple of 4), R - 2 groups ahead; WPRE: the weight halves of those are on
+// their way (zr_preload_w).  Terms of an infinite operand are infinity and NaN: where a sum comes out infinite or NaN the caller
+// computes it again with zr_mma_segment_u.
+typedef __bf16 zr_bf16x8_s __attribute__((ext_vector_type(8)));
+typedef __bf16 zr_bf16x2_s __attribute__((ext_vector_type(2)));
+// Two values' leading bf16 terms (rounded to nearest) in one register; the values become what is left of them.
+__device__ __forceinline__ unsigned zr_next_terms(float& a, float& b) {
+  unsigned t = __builtin_bit_cast(unsigned, zr_bf16x2_s{(__bf16)a, (__bf16)b});
+  asm("" : "+v"(t));  // one conversion for both values
+  a -= __uint_as_float(t << 16);
+  b -= __uint_as_float(t & 0xffff0000u);
+  return t;
+}
+__device__ __forceinline__ void zr_split8(const float (&lo)[4], const float (&hi)[4], zr_bf16x8_s (&term)[3]) {
+  zr_u32x4v t[3];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    float a = p < 2 ? lo[2 * p] : hi[2 * p - 4], b = p < 2 ? lo[2 * p + 1] : hi[2 * p - 3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) t[q][p] = zr_next_terms(a, b);
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) term[q] = __builtin_bit_cast(zr_bf16x8_s, t[q]);
+}
+
+template <int TM, int TN>
+struct ZrTerms {
+  zr_bf16x8_s x[TN][3], w[TM][3];
+};
+
+template <int TM, int TN, int KS, int R, bool WPRE>
+__device__ __forceinline__ void zr_mma_segment_split(zr_f32x16 (&acc)[TM][TN], __amdgpu_buffer_rsrc_t wrsrc,
+                                                     const unsigned (&wsoff)[TM], unsigned woffb, unsigned wstep,
+                                                     __amdgpu_buffer_rsrc_t xrsrc, const unsigned (&xoffb)[TN],
+                                                     unsigned xstep, int K, int kslice, ZrFrag<TM, TN> (&f)[R]) {
+  static_assert(R % 4 == 0, "pairs of slots, and an even number of pairs a revolution");
+  const int nfull = K >> 3;  // K % 8 == 0
+  constexpr int AHEAD = R - 2;
+  auto load_x = [&](ZrFrag<TM, TN>& f, int g) {
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) {
+      const zr_u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)xoffb[tn], (int)((unsigned)g * xstep), 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f.x[tn][i] = __uint_as_float(v[i]);
+    }
+  };
+  auto load_full = [&](ZrFrag<TM, TN>& f, int g) {
+    load_x(f, g);
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+      const zr_u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + (unsigned)g * wstep), 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f.w[tm][i] = __uint_as_float(v[i]);
+    }
+  };
+  auto split = [&](const ZrFrag<TM, TN>& a, const ZrFrag<TM, TN>& b, ZrTerms<TM, TN>& t) {
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) zr_split8(a.x[tn], b.x[tn], t.x[tn]);
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) zr_split8(a.w[tm], b.w[tm], t.w[tm]);
+  };
+  zr_f32x16 sum[TM][TN];
+  auto clear = [&] {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[tm][tn][r] = 0.0f;
+  };
+  auto add = [&] {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) acc[tm][tn] += sum[tm][tn];
+  };
+  auto mma = [&](const ZrTerms<TM, TN>& t) {
+    constexpr int X[6] = {2, 0, 1, 1, 0, 0}, W[6] = {0, 2, 1, 0, 1, 0};  // the smallest products first
+#pragma unroll
+    for (int p = 0; p < 6; ++p)
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+          sum[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.x[tn][X[p]], t.w[tm][W[p]], sum[tm][tn], 0, 0, 0);
+  };
+  if (kslice >= nfull) return;
+  const int last = nfull - 1;
+  const int n_mine = (nfull - kslice + KS - 1) / KS;
+  auto group = [&](int i) {
+    const int gl = kslice + i * KS;
+    return gl < last ? gl : last;
+  };
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) {
+    if (WPRE)
+      load_x(f[s], group(s));
+    else
+      load_full(f[s], group(s));
+  }
+  // the group behind the last is nothing, in either operand
+  auto single = [&](ZrFrag<TM, TN>& f, bool there) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) f.x[tn][i] = there ? f.x[tn][i] : 0.0f;
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) f.w[tm][i] = there ? f.w[tm][i] : 0.0f;
+    }
+  };
+  ZrTerms<TM, TN> t[2];
+  if (n_mine == 1) single(f[1], false);
+  split(f[0], f[1], t[0]);
+  int it = 0;
+  // a revolution whose pairs and the one after them are whole
+  for (; it + R + 2 <= n_mine; it += R) {
+    clear();
+#pragma unroll
+    for (int s = 0; s < R; s += 2) {
+      load_full(f[(s + AHEAD) % R], group(it + s + AHEAD));
+      load_full(f[(s + AHEAD + 1) % R], group(it + s + AHEAD + 1));
+      mma(t[(s >> 1) & 1]);
+      split(f[(s + 2) % R], f[(s + 3) % R], t[((s >> 1) + 1) & 1]);
+      // matrix instructions, conversions and loads in turn
+      constexpr int NL = 2 * (TM + TN), NM = 6 * TM * TN, PER = (44 * (TM + TN) + NM - 1) / NM;
+#pragma unroll
+      for (int i = 0; i < NM; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);
+        if (i < NL) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    add();
+  }
+  clear();
+  // at most R + 1 groups are left, the first AHEAD of them loaded
+#pragma unroll
+  for (int s = 0; s < R + 2; s += 2) {
+    if (it + s >= n_mine) break;
+    if (s + AHEAD < R + 2) {
+      load_full(f[(s + AHEAD) % R], group(it + s + AHEAD));
+      load_full(f[(s + AHEAD + 1) % R], group(it + s + AHEAD + 1));
+    }
+    mma(t[(s >> 1) & 1]);
+    if (it + s + 2 < n_mine) {
+      if (it + s + 3 >= n_mine) single(f[(s + 3) % R], false);
+      split(f[(s + 2) % R], f[(s + 3) % R], t[((s >> 1) + 1) & 1]);
+    }
+  }
+  add();
 }
 
 // The same with a ring of its own (no weights fetched ahead).

@@ -213,6 +213,12 @@ inline bool zr_grouped_small_tiles(long long tiles, int columns, int cus) {
   return tiles <= cus || (columns > 32 && 2 * tiles <= 3LL * cus);
 }
 
+// The same products on k-interleaved operands as three bf16 terms, 64 x 64 tiles (zr_error_products.hip): faster as soon as there are more 32 x 32
+// tiles than compute units, beyond 32 columns.  us of a sweep of 12 steps on the kernels above / on this one: 4 x 300, 100 columns (320 tiles)
+// 388 / 343, 1 x 768, 192 columns (288) 626 / 505, 4 x 1000, 128 columns (1024) 1190 / 922, 2 x 1200, 192 columns (912) 3041 / 912; but 2 x
+// 500, 128 columns (256) 313 / 411, and 4 x 2000, 20 columns (504) 1499 / 1546.
+inline bool zr_error_products_takes(long long tiles, int columns, int cus) { return tiles > cus && columns > 32; }
+
 // ---- small products (zr_small_gemm.hip): narrow tiles whose waves have all their operands in flight
 
 // Shape: 0 = 16 rows x 16 columns, 1 = 16 x 32, 2 = 32 x 32, -1 = the other kernels.  z: independent products of one launch.  a_pack,
