@@ -635,7 +635,7 @@ struct LstmDecStack {
   int nl, V, H, mb, ldw, kp, j_tiles, n_tiles;
   float clip;
   int spin_limit;
-  int fence;                      // as in LstmSweep
+  int fence;                      // 1: consumers invalidate their caches after every wait (mb % 8 != 0: lines with two producers)
   int wait_extra;                 // arrivals a layer's wait for the layer below expects beyond the real ones (tests)
   int helpers;                    // 0: every tile has a role-1 workgroup of its own (grid.y = 2); else the number of
                                   // role-1 workgroups behind the chain slots of a one-dimensional grid
@@ -719,7 +719,7 @@ __global__ void __launch_bounds__(256) lstm_decoder_stack_kernel(LstmDecStack P)
       const int tile = jt * P.n_tiles + nt;
       const bool covered = l >= P.l_split;  // role 1 (or a helper) delivers this layer's independent products
 
-      // per-lane values are derived afresh in every job (see lstm_sweep_kernel)
+      // per-lane values are derived afresh in every job: hoisted out of the loop, they would stay in registers through all of it
       int lane_t = lane;
       asm volatile("" : "+v"(lane_t));
       const int jl = lane_t & 31, half = lane_t >> 5;
