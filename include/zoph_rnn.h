@@ -129,6 +129,10 @@ const char* zr_version(void);
                                         device): 0 auto (taken whenever it applies; ZR_OPT_LSTM_SWEEP = 1 also
                                         switches it off), 1 never (three launches).  Its waits are bounded like the
                                         single-launch LSTM schedules' and reported the same way */
+#define ZR_OPT_LSTM_SWEEP_SCRATCH 12 /* KiB of scratch memory that a sweep as one launch may use (0 = what the device has
+                                        left).  The streamed sweep needs 6 * (L * (T + 1) + T) * H bytes a column (columns in
+                                        eights), the resident one 4 * L * (T + 1) * H; a schedule there is no memory for
+                                        is passed over, with ZR_OPT_LSTM_SWEEP = 2 and 3 too */
 
 /* full_matrix_setup / cudaMalloc / cudaMemcpy / cudaMemset call sites (src/BZ_CUDA_UTIL.h:358-399 and the
  * layer constructors, e.g. src/LSTM.hpp:23-42). */

@@ -80,3 +80,32 @@ def test_rounds_no_more_than_one_launch_per_diagonal(ctx, H, mb):
         error[option] = np.linalg.norm(h[0] - np.stack(want)) / np.linalg.norm(want)
     print(H, mb, error)
     assert error[2] < 1.1 * error[1]
+
+
+def test_next_best_schedule_where_there_is_no_memory(ctx):
+    """Estimated us of this size: streamed 305, resident 433, one launch per diagonal 516.  What a schedule may not have is not taken from the
+    scratch buffer either, whose size the query tells."""
+    H, mb, T, L = 704, 64, 12, 3
+    c = r._case(H, mb, T, L)
+    resident_kib = 4 * L * (T + 1) * H * mb // 1024 + 1  # the streamed sweep needs half as much again and the embedding columns
+    want, paths, held = {}, {}, []
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 1)
+    want["diagonals"] = r._run(ctx, c)[0]
+    for option in (0, 2, 3):
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, option)
+        for limit in (0, resident_kib, 1, 0):
+            ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SCRATCH, limit)
+            try:
+                h, _, _, path, abandoned = r._run(ctx, c)
+            finally:
+                ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SCRATCH, 0)
+            held.append(ctx.query(capi.ZR_QUERY_SCRATCH_KIB))
+            assert not abandoned
+            paths.setdefault((option, limit), []).append(path)
+            assert np.array_equal(want.setdefault(path, h), h)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 2)
+    diagonals = (capi.ZR_LSTM_STACK_PATH_DIAGONALS, 0)
+    for option, first in ((0, STREAMED), (2, STREAMED), (3, r.RESIDENT)):
+        assert paths[option, 0] == [first] * 2 and paths[option, resident_kib] == [r.RESIDENT] and paths[option, 1] == [diagonals], paths
+    assert np.array_equal(want[diagonals], want["diagonals"])
+    assert held == sorted(held), held

@@ -29,6 +29,7 @@ struct zr_ctx {
   int* d_step_flags; // ZR_MAX_STEP_FLAGS flags of lstm_resident_kernel (the first 32 hold its departure count), zero between launches
   int lstm_sweep;    // whole-sweep LSTM kernels: 0 auto, 1 never, 2 / 3 streamed / resident weights whenever the launch fits
   int sweep_spin;    // polls before a waiting workgroup of that kernel gives up (0: default)
+  int sweep_scratch_kib;  // ZR_OPT_LSTM_SWEEP_SCRATCH
   int step_wait_extra;  // arrivals the decoder step's layer waits expect beyond the real ones (tests of giving up)
   int stack_helpers;    // 1 (default): the decoder step may run 32-column tiles with helper workgroups (zr_lstm.hip)
   int cu_count;      // compute units of the device
@@ -91,6 +92,9 @@ int zr_bind_device(zr_ctx* ctx);
 int zr_live_contexts(int device);
 // Returns a context-owned scratch buffer of at least `bytes` (slot 0 or 1).
 int zr_ctx_scratch(zr_ctx* ctx, int slot, size_t bytes, void** out);
+// The same for a call that has a way without it: ZR_ENOMEM, with the buffer there is left as it is, where the device has no
+// room for it or ZR_OPT_LSTM_SWEEP_SCRATCH allows less.
+int zr_ctx_scratch_if_room(zr_ctx* ctx, int slot, size_t bytes, void** out);
 // Size of the statically allocated device scratch array every GPU holds for the allocation-free entry point, and
 // how that entry point divides it between the two scratch slots.
 #define ZR_STATIC_SCRATCH_BYTES (32u << 20)

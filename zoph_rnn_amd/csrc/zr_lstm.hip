@@ -1574,34 +1574,43 @@ int zr_lstm_stack_forward_train(zr_ctx* ctx, int nl, const zr_lstm_weights* cons
                              8LL * layers[0]->kp * layers[0]->ldw * 4 < lim;
     if (!offsets_fit || (tn && nl * ((n32 + tn - 1) / tn) > 512) || (long long)T * j_tiles >= kSweepGaveUp) tn = 0;
   }
-  // Which schedule: the least estimated time (zr_rules.h).
-  if (single_ok) {
-    const double diag_us = zr_sweep_diagonals_us(nl, H, mb, T, vec, ctx->cu_count);
-    const double sweep_us = tn ? zr_sweep_streamed_us(nl, H, T, tn) : -1.0;
-    if (tn && !ctx->lstm_sweep && diag_us < sweep_us) tn = 0;
-    const double other_us = tn ? sweep_us : diag_us;
-    ZrResidentPlan plan = {};
-    // option 2: the streamed sweep where it fits, 3: the one with resident weights where that fits
-    if (ctx->lstm_sweep == 2 ? !tn : ctx->lstm_sweep == 3 || (!ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts)) {
-      plan = zr_lstm_resident_plan(ctx, nl, H, mb, T);
-      if (plan.us < 0.0 || (!ctx->lstm_sweep && other_us <= plan.us)) plan.at_once = 0;
-    }
-    if (plan.at_once) {
-      rc = zr_lstm_resident_sweep(ctx, plan, nl, layers, d_embed, V, d_ids_nonneg, d_mask01, T, mb, d_h0, d_c0,
-                                  clip_threshold, d_h_all, d_c_all, d_gates_all);
-      if (rc) return rc;
-      ctx->last_stack_path = ZR_LSTM_STACK_PATH_SWEEP;
-      ctx->last_sweep_kernel = ZR_LSTM_SWEEP_RESIDENT;
-      return poison_if_abandoned(ctx, nl, T, H, mb, d_h_all, d_c_all, d_gates_all);
-    }
-  }
+  // h of every node as three bf16 terms, and the embedding columns
   const size_t ctr_bytes = sizeof(int) * 512 * kSweepCtrStride;
+  const size_t sweep_bytes = ctr_bytes + 6 * ((size_t)nl * (T + 1) + T) * H * columns;
   void* p = nullptr;
-  if (tn) {
-    // h of every node as three bf16 terms, and the embedding columns; without the memory for that, one launch per diagonal
-    rc = zr_ctx_scratch(ctx, 1, ctr_bytes + 6 * ((size_t)nl * (T + 1) + T) * H * columns, &p);
-    if (rc == ZR_ENOMEM) tn = 0;
-    else if (rc) return rc;
+  // Which schedule: the least estimated time (zr_rules.h) of those that there is memory for.
+  const int fits = tn;
+  for (bool room_streamed = true, room_resident = true;;) {
+    tn = room_streamed ? fits : 0;
+    if (single_ok) {
+      const double diag_us = zr_sweep_diagonals_us(nl, H, mb, T, vec, ctx->cu_count);
+      const double sweep_us = tn ? zr_sweep_streamed_us(nl, H, T, tn) : -1.0;
+      if (tn && !ctx->lstm_sweep && diag_us < sweep_us) tn = 0;
+      const double other_us = tn ? sweep_us : diag_us;
+      ZrResidentPlan plan = {};
+      // option 2: the streamed sweep where it fits, 3: the one with resident weights where that fits
+      if (room_resident && (ctx->lstm_sweep == 2 ? !tn : ctx->lstm_sweep == 3 || (!ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts))) {
+        plan = zr_lstm_resident_plan(ctx, nl, H, mb, T);
+        if (plan.us < 0.0 || (!ctx->lstm_sweep && other_us <= plan.us)) plan.at_once = 0;
+      }
+      if (plan.at_once) {
+        rc = zr_lstm_resident_sweep(ctx, plan, nl, layers, d_embed, V, d_ids_nonneg, d_mask01, T, mb, d_h0, d_c0,
+                                    clip_threshold, d_h_all, d_c_all, d_gates_all);
+        if (rc == ZR_ENOMEM) {  // nothing is queued
+          room_resident = false;
+          continue;
+        }
+        if (rc) return rc;
+        ctx->last_stack_path = ZR_LSTM_STACK_PATH_SWEEP;
+        ctx->last_sweep_kernel = ZR_LSTM_SWEEP_RESIDENT;
+        return poison_if_abandoned(ctx, nl, T, H, mb, d_h_all, d_c_all, d_gates_all);
+      }
+    }
+    if (!tn) break;
+    rc = zr_ctx_scratch_if_room(ctx, 1, sweep_bytes, &p);
+    if (rc == ZR_OK) break;
+    if (rc != ZR_ENOMEM) return rc;
+    room_streamed = false;
   }
   if (tn) {
     const int n_tiles = (n32 + tn - 1) / tn;

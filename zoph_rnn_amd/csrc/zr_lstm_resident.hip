@@ -474,7 +474,7 @@ int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, cons
   const int per_layer = j_tiles * plan.n_tiles;
   const long long slot = zr_resident_slot(H, mb);
   void* p = nullptr;
-  int rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (size_t)(nl * (long long)(T + 1) * slot), &p);
+  int rc = zr_ctx_scratch_if_room(ctx, 1, sizeof(float) * (size_t)(nl * (long long)(T + 1) * slot), &p);
   if (rc) return rc;
   LstmResident P = {};
   for (int l = 0; l < nl; ++l) {

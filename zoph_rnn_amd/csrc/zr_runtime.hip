@@ -80,6 +80,17 @@ int zr_ctx_scratch(zr_ctx* ctx, int slot, size_t bytes, void** out) {
   return ZR_OK;
 }
 
+int zr_ctx_scratch_if_room(zr_ctx* ctx, int slot, size_t bytes, void** out) {
+  if (ctx->sweep_scratch_kib && bytes > (size_t)ctx->sweep_scratch_kib << 10)
+    return zr_set_error(ZR_ENOMEM, "%zu bytes of scratch memory are more than ZR_OPT_LSTM_SWEEP_SCRATCH", bytes);
+  const size_t cap = slot == 0 ? ctx->scratch_bytes : ctx->scratch2_bytes;
+  size_t free_bytes = 0, total = 0;
+  if (cap < bytes && hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes + cap < bytes + bytes / 4)
+    return zr_set_error(ZR_ENOMEM, "no room for %zu bytes of scratch memory", bytes);
+  (void)hipGetLastError();
+  return zr_ctx_scratch(ctx, slot, bytes, out);
+}
+
 extern "C" {
 
 const char* zr_last_error(void) { return g_err; }
@@ -256,6 +267,10 @@ int zr_ctx_set_option(zr_ctx* ctx, int option, int value) {
     case ZR_OPT_LSTM_SWEEP_SPIN:
       ZR_CHECK_ARG(value >= 0, "ZR_OPT_LSTM_SWEEP_SPIN must not be negative");
       ctx->sweep_spin = value;
+      return ZR_OK;
+    case ZR_OPT_LSTM_SWEEP_SCRATCH:
+      ZR_CHECK_ARG(value >= 0, "ZR_OPT_LSTM_SWEEP_SCRATCH must not be negative");
+      ctx->sweep_scratch_kib = value;
       return ZR_OK;
     case ZR_OPT_LSTM_STEP_WAIT_EXTRA:
       ZR_CHECK_ARG(value >= 0 && value <= 1024, "ZR_OPT_LSTM_STEP_WAIT_EXTRA must be in [0, 1024]");
