@@ -2,6 +2,7 @@
 // Serves the softmax logits (with per-block max / sum-exp partials), the attention projections (tanh, bias,
 // mask fused) and the plain cublasSgemm replacement.  See zr_mfma_core.h for the operand mapping.
 #include <math.h>
+#include <stddef.h>
 
 #include "zr_internal.h"
 #include "zr_mfma_core.h"
@@ -10,11 +11,11 @@ namespace {
 
 struct GemmArgs {
   int M, N, nseg;
-  int K[4];
-  const float* A[4];
-  long long lda[4];
-  const float* B[4];
-  int ldb[4];
+  int K[3];
+  const float* A[3];
+  long long lda[3];
+  const float* B[3];
+  int ldb[3];
   float* C;
   int ldc;
   long long strideA, strideC, strideBias;
@@ -28,7 +29,7 @@ struct GemmArgs {
   int b_pack4;           // B segments are k-interleaved copies: element (k, n) at ((k/4)*N + n)*4 + k%4
   // bf16 weights: B[s] is the bf16 "hi" array and Blo[s] the "lo" array of the split activations, both
   // k-interleaved by 8 ([K/8][N][8]); see zr_split_pack_multi_kernel
-  const unsigned short* Blo[4];
+  const unsigned short* Blo[3];
   int accum;  // ZR_EPI_STORE only: C += result instead of C = result
   int stream_a;  // the weights are fetched with the streaming hint (ZrGemmDesc::stream_a)
   // groups > 0: blockIdx.z = group * batch + batch index; the group picks A, B and C from these tables
@@ -38,6 +39,9 @@ struct GemmArgs {
   float* gC[8];
   long long gStrideC[8];
 };
+// What an ungrouped product reads is four 64-byte lines of arguments.  With room for the four segments of zr_small_gemm it was five, and every
+// launch of these kernels took 0.3 us longer (775 x 230 x 38 4.47 -> 4.80).
+static_assert(offsetof(GemmArgs, gA) <= 256, "the arguments of an ungrouped product");
 
 template <int... I>
 struct zr_int_seq {};
@@ -1215,7 +1219,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
     for (int s = 1; s < d.nseg; ++s) same = same && d.K[s] == d.K[0];
     if (same) small = zr_small_gemm_shape(d.M, d.N, d.K[0], d.nseg, d.batch * (d.groups > 0 ? d.groups : 1), d.a_pack, d.trans_a != 0, ctx->cu_count);
   }
-  ZR_CHECK_ARG(d.nseg >= 1 && d.nseg <= (small >= 0 ? 4 : 3), "gemm: nseg = %d", d.nseg);
+  ZR_CHECK_ARG(d.nseg >= 1 && d.nseg <= (small >= 0 && !d.a_pack ? 4 : 3), "gemm: nseg = %d", d.nseg);
   ZR_CHECK_ARG((d.groups > 0 || d.C != nullptr) && d.ldc >= d.M, "gemm: C null or ldc %d < M %d", d.ldc, d.M);
   ZR_CHECK_ARG(d.batch >= 1 && d.batch <= 65535, "gemm: batch = %d", d.batch);
   ZR_CHECK_ARG(d.groups >= 0 && d.groups <= 8, "gemm: groups = %d", d.groups);
@@ -1256,11 +1260,13 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
       // per-lane weight offsets are 32-bit element indices
       ZR_CHECK_ARG(d.trans_a ? ((long long)d.M * d.lda[s] + 8 < (1LL << 31)) : (d.M + 8LL * d.lda[s] < (1LL << 31)),
                    "gemm: operand A of segment %d is too large for 32-bit offsets", s);
-      ga.K[s] = d.K[s];
-      ga.A[s] = d.A[s];
-      ga.lda[s] = d.lda[s];
-      ga.B[s] = d.B[s];
-      ga.ldb[s] = d.ldb[s];
+      if (s < 3) {  // (a fourth one is zr_small_gemm's)
+        ga.K[s] = d.K[s];
+        ga.A[s] = d.A[s];
+        ga.lda[s] = d.lda[s];
+        ga.B[s] = d.B[s];
+        ga.ldb[s] = d.ldb[s];
+      }
       vec = vec && (d.ldb[s] % 4 == 0) && (((uintptr_t)d.B[s] & 15u) == 0);
       for (int g = 0; g < d.groups; ++g) vec = vec && (((uintptr_t)d.gB[g] & 15u) == 0);
       if (d.trans_a) {
@@ -1268,7 +1274,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
         for (int g = 0; g < d.groups; ++g) vec = vec && (((uintptr_t)d.gA[g] & 15u) == 0);
       }
       flops += 2LL * d.M * d.N * d.K[s];
-    } else {
+    } else if (s < 3) {
       ga.K[s] = 0;
       ga.A[s] = nullptr;
       ga.lda[s] = 0;
@@ -1299,7 +1305,7 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
   if (d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) ZR_CHECK_ARG(d.bias && d.partials, "gemm: bias/partials required");
 
   ga.b_pack4 = 0;
-  for (int s = 0; s < 4; ++s) ga.Blo[s] = nullptr;
+  for (int s = 0; s < 3; ++s) ga.Blo[s] = nullptr;
   if (d.a_pack == 2) {
     ZR_CHECK_ARG(vec, "gemm: bf16 operand A needs 16-byte aligned activations with ldb %% 4 == 0");
     const bool one_term = ctx->bf16_terms == 1;
