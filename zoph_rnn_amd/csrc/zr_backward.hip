@@ -485,21 +485,31 @@ __device__ __forceinline__ float bwd_block_sum(float v, float* red) {
 // What a workgroup of 1024 threads does that writes 32 rows of an H x mb matrix and adds the sum of other values over the columns to a
 // vector: thread (x, y) has row x of the block and every 32nd column.  f(i, column, row) stores element i and returns what is summed.
 // One launch where an element-wise kernel and a sum over its result were two (H = 500, 64 columns: 2.6 and 3.3 us).
+// gridDim.y > 1: that many workgroups share the columns; their sums go to a row of `sum` each, H values apart.
 template <typename F>
 __device__ __forceinline__ void rows_with_sum(F f, int H, int mb, float* __restrict__ sum) {
   __shared__ float part[32][32];
   const int x = threadIdx.x & 31, y = threadIdx.x >> 5, row = blockIdx.x * 32 + x;
+  int first = 0, end = mb;
+  if (gridDim.y > 1) {
+    const int per = (mb + gridDim.y - 1) / gridDim.y;
+    first = blockIdx.y * per;
+    end = first + per < mb ? first + per : mb;
+  }
   float s = 0.0f;
   if (row < H) {
 #pragma unroll 4
-    for (int b = y; b < mb; b += 32) s += f((size_t)b * H + row, b, row);
+    for (int b = first + y; b < end; b += 32) s += f((size_t)b * H + row, b, row);
   }
   part[y][x] = s;
   __syncthreads();
   if (y == 0 && row < H) {
 #pragma unroll
     for (int i = 1; i < 32; ++i) s += part[i][x];
-    sum[row] += s;
+    if (gridDim.y == 1)
+      sum[row] += s;
+    else
+      sum[(size_t)blockIdx.y * H + row] = s;
   }
 }
 
@@ -1060,7 +1070,8 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   const size_t n = (size_t)H * mb;
   const float sigma_sq = (float)((a->D * a->D) / 4.0);  // src/attention_node.hpp:50
   void* scratch = nullptr;
-  rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (5 * n + 2 * (size_t)W * mb + 3 * (size_t)mb), &scratch);
+  const int parts = zr_attn_sum_parts(mb);
+  rc = zr_ctx_scratch(ctx, 1, sizeof(float) * (5 * n + 2 * (size_t)W * mb + 3 * (size_t)mb + (parts > 1 ? (size_t)parts * H : 0)), &scratch);
   if (rc) return rc;
   float* e = (float*)scratch;
   float* err_ct = e + n;
@@ -1070,7 +1081,13 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   float* err_as = e + 5 * n;
   float* scal = err_as + (size_t)W * mb;
   float* col = scal + (size_t)W * mb;
-  const int row_blocks = (H + 31) / 32;
+  float* sums = col + 3 * (size_t)mb;  // parts x H
+  const dim3 row_blocks((H + 31) / 32, parts);
+  auto add_sums = [&](float* to) -> int {  // of rows_with_sum in parts
+    if (parts > 1) row_sum_pass(ctx, sums, H, parts, parts, to, 1);
+    ZR_LAUNCH_CHECK("row_sum_kernel");
+    return ZR_OK;
+  };
 
   // C (H x H) += A (H x mb) * B^T for B H x mb (cuBLAS gemm N, T with beta = 1 in the reference)
   auto outer_acc = [&](const float* A, const float* B, float* C) -> int {
@@ -1112,8 +1129,9 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
     return zr_gemm_launch(ctx, g);
   };
 
-  attn_bwd_e_kernel<<<row_blocks, 1024, 0, ctx->stream>>>(d_err_htild, d_h_tild, d_mask01, H, mb, e, grads->d_out_bias);  // :456
+  attn_bwd_e_kernel<<<row_blocks, 1024, 0, ctx->stream>>>(d_err_htild, d_h_tild, d_mask01, H, mb, e, parts > 1 ? sums : grads->d_out_bias);  // :456
   ZR_LAUNCH_CHECK("attn_bwd_e_kernel");
+  if ((rc = add_sums(grads->d_out_bias))) return rc;
   const bool outer = zr_outer_takes(2, H, H, mb);
   if (outer) {
     rc = outer_launch(ctx, OuterProducts{{e, e}, {d_c_t, d_h_t}, {grads->d_W_c1, grads->d_W_c2}}, 2, H, H, mb);
@@ -1148,8 +1166,9 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   attn_bwd_column_kernel<<<mb, 64, 0, ctx->stream>>>(a->d_tanh1, a->v_p, d_batch_info, d_indices, d_alignments, d_p_t,
                                                      err_as, H, mb, W, sigma_sq, col, scal);
   ZR_LAUNCH_CHECK("attn_bwd_column_kernel");
-  attn_bwd_vp_wp_kernel<<<row_blocks, 1024, 0, ctx->stream>>>(a->d_tanh1, a->v_p, col, H, mb, tw, grads->d_v_p);  // :536
+  attn_bwd_vp_wp_kernel<<<row_blocks, 1024, 0, ctx->stream>>>(a->d_tanh1, a->v_p, col, H, mb, tw, parts > 1 ? sums : grads->d_v_p);  // :536
   ZR_LAUNCH_CHECK("attn_bwd_vp_wp_kernel");
+  if ((rc = add_sums(grads->d_v_p))) return rc;
   if (!outer && (rc = outer_acc(tw, d_h_t, grads->d_W_p))) return rc;           // :545
   if ((rc = product(a->W_p, 1, tw, d_err_h_t, 1, ZR_EPI_STORE))) return rc;     // :551
   if ((rc = product(a->W_a, 1, d_h_t, a->d_q, 0, ZR_EPI_STORE))) return rc;     // W_a^T h of the forward pass again

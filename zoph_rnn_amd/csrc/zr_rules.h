@@ -249,6 +249,13 @@ inline int zr_small_gemm_shape(int M, int N, int K, int nseg, int z, int a_pack,
   return best;
 }
 
+// ---- sums over the columns of an attention node's backward pass (rows_with_sum): workgroups that share the columns of 32 rows
+
+// us of both sums' kernels, an element-wise one and a separate sum / one workgroup that walks all columns / in parts: H = 64, 64 columns 9.6 /
+// 5.6, 512 15.4 / 9.9, 1024 15.9 / 15.4 / 13.1, 2048 19.3 / 25.9 / 12.4; H = 1000, 64 14.7 / 6.6, 512 28.2 / 11.9, 1024 28.8 / 23.0 / 20.4, 2048
+// 32.0 / 47.2 / 24.9.
+inline int zr_attn_sum_parts(int mb) { return mb <= 512 ? 1 : (mb + 255) / 256; }
+
 // ---- the output layer's product on a prepared fp32 matrix (zr_logits.hip)
 
 // tn: 32-column blocks of a tile, waves: 32-row blocks of a workgroup; tn = 0: the other kernels.
