@@ -222,14 +222,15 @@ inline bool zr_error_products_takes(long long tiles, int columns, int cus) { ret
 // ---- small products (zr_small_gemm.hip): narrow tiles whose waves have all their operands in flight
 
 // Shape: 0 = 16 rows x 16 columns, 1 = 16 x 32, 2 = 32 x 32, -1 = the other kernels.  z: independent products of one launch.  a_pack,
-// trans_a: the left operand's layout as ZrGemmDesc has it.  Estimates of a launch in us (within 16 % of 330 sizes on each shape): a
-// trip to memory and the launch, and the K range of a workgroup, alone on its compute unit or beside a second one; beyond two a
-// compute unit the wider tiles of the other kernels win, and so they do where 32 x 32 tiles are the best choice here and the
-// matrix is read 4 bytes a lane (column-major), or row-major up to K = 1500: 1000 x 256 x 1000 11.8 / 10.2 and 11.4 / 10.8.
-// This one / the others, us: 500 x 64 x 500 4.5 / 6.3 row-major, 4.6 / 7.0 column-major; 1000 x 64 x 1000 6.2 / 9.8; 2 products of
-// 500 x 64 x 2000 13.0 / 18.6 (the whole node), 1000 x 64 x 4000 26.1 / 33.4; 100 x 20 x 100 3.6 / 4.1; an attention step on prepared matrices,
-// H = 500, 37 columns 19.6 / 35.2; bf16 matrices, H = 1024, 64 columns 24.0 / 30.4; sweeps back through 12 steps, 2 x 100, 128 columns 136 /
-// 242, 2 x 500, 64 columns 243 / 293, 2 x 1000, 128 columns 771 / 966.  Of 200 sizes five are slower than with the others, by 2 to 10 %.
+// trans_a: the left operand's layout as ZrGemmDesc has it.  Estimates of a launch in us: a trip to memory and the launch, and the K range of a
+// workgroup, alone on its compute unit or beside a second one; beyond two a compute unit the wider tiles of the other kernels win, and so they do
+// where 32 x 32 tiles are the best choice here and the matrix is read 4 bytes a lane (column-major), or row-major up to K = 1500: 1000 x 256 x 1000
+// 11.8 / 10.2 and 11.4 / 10.8; and on column-major matrices beyond one and three quarters: 1111 x 110 x 736 8.6 / 8.0.
+// This one / the others, us: 500 x 64 x 500 4.2 / 7.0 column-major; 1000 x 64 x 1000 6.2 / 9.5; 2 products of 500 x 128 x 2000 13.7 / 16.8, 1000 x 20 x
+// 4000 14.9 / 27.3; 100 x 20 x 100 row-major 3.2 / 4.1; an attention step on prepared matrices, H = 500, 37 columns 19.6 / 35.2; bf16 matrices, H = 1024,
+// 64 columns 24.0 / 30.4; sweeps back through 12 steps, 2 x 100, 128 columns 136 / 242, 2 x 500, 64 columns 243 / 293, 2 x 1000, 128 columns 771 /
+// 966.  Of 485 sizes of one and two products the choice is 1.7 % from the best shape on average, and slower than the others at two: 819 x 143 x 1176
+// row-major 13.2 / 11.4, 1156 x 193 x 20 4.1 / 3.9.
 inline int zr_small_gemm_shape(int M, int N, int K, int nseg, int z, int a_pack, bool trans_a, int cus) {
   if (K < 16) return -1;
   const double slope[3] = {0.0036, 0.0052, 0.0078}, second[3] = {1.55, 1.8, 1.9};
@@ -239,7 +240,7 @@ inline int zr_small_gemm_shape(int M, int N, int K, int nseg, int z, int a_pack,
   for (int s = 0; s < 3; ++s) {
     const int rows = s == 2 ? 32 : 16, cols = s == 0 ? 16 : 32;
     const long long wgs = (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * z;
-    if (wgs > 2LL * cus) continue;
+    if (wgs > 2LL * cus || (s == 0 && a_pack == 0 && !trans_a && 4 * wgs > 7LL * cus)) continue;
     const double t = 3.4 + slope[s] * k * (wgs > cus ? second[s] : 1.0);
     if (best < 0 || t < us) {
       best = s, us = t;

@@ -50,7 +50,10 @@ __device__ __forceinline__ zr_f32x4 shifted(zr_f32x4 v, int d) {
   return r;
 }
 
-template <int TM, int TN, int AMODE, int PF>
+// ONE: one segment, ungrouped.  No load then needs an entry of a table of arguments by a computed index, which took a second trip for arguments
+// ahead of the first loads and others inside the loop: 885 x 126 x 98 5.0 -> 4.5 us, 1026 x 105 x 1030 11.7 -> 9.8, 2535 x 34 x 1463
+// 15.7 -> 13.2.
+template <int TM, int TN, int AMODE, int PF, bool ONE>
 __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a) {
   constexpr bool BF16 = zr_is_bf16_mode(AMODE), LO = AMODE == ZR_A_PACK8_BF16;
   constexpr int KG = BF16 ? 32 : 16;        // k of a group
@@ -64,11 +67,11 @@ __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a)
   if (tile >= tiles) return;
   const int row_tile = tile / a.n_tiles, nt = tile - row_tile * a.n_tiles;
   const int z = row_tile / a.m_tiles, mt = row_tile - z * a.m_tiles;
-  const int group = z / a.batch, zb = z - group * a.batch;
+  const int group = ONE ? 0 : z / a.batch, zb = z - group * a.batch;
   const int tid = threadIdx.x, lane = tid & 63, cl = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = 16 * TM * mt, n0 = 16 * TN * nt;
-  float* C = a.groups ? a.gC[group] + zb * a.gStrideC[group] : a.C + zb * a.strideC;
+  float* C = !ONE && a.groups ? a.gC[group] + zb * a.gStrideC[group] : a.C + zb * a.strideC;
   const float* bias = a.bias ? a.bias + zb * a.strideBias : nullptr;
 
   // the outputs this thread finishes: what is added to them is fetched ahead of the K loop
@@ -92,16 +95,16 @@ __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a)
 #pragma unroll
   for (int j = 0; j < TN; ++j) col[j] = n0 + 16 * j + cl < a.N ? n0 + 16 * j + cl : a.N - 1;
 
-  const int K = a.K, G = (K + KG - 1) / KG, total = a.nseg * G;
+  const int K = a.K, G = (K + KG - 1) / KG, total = ONE ? G : a.nseg * G;
   struct Frag {
     zr_f32x4 w[TM], x[TN], xl[LO ? TN : 1];
   };
   Frag f[NS];
   // The k-groups of all segments in one row, dealt to the waves in turn: group r is (segment r / G, group r % G).
-  int ls = wave / G, lg = wave - ls * G, lr = wave;  // the next group to load
+  int ls = ONE ? 0 : wave / G, lg = wave - ls * G, lr = wave;  // the next group to load
   auto load = [&](Frag& q) {
-    const float* A = a.groups ? a.gA[group] : a.A[ls];
-    const float* B = a.groups ? a.gB[group] : a.B[ls];
+    const float* A = !ONE && a.groups ? a.gA[group] : a.A[ls];
+    const float* B = !ONE && a.groups ? a.gB[group] : a.B[ls];
     const long long lda = a.lda[ls], ldb = a.ldb[ls];
     if constexpr (BF16) {
       const int kb = 4 * lg + kq, last = (K >> 3) - 1, k8 = kb < last ? kb : last;
@@ -146,12 +149,13 @@ __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a)
     if (lr + kWaves < total) {
       lr += kWaves;
       lg += kWaves;
-      while (lg >= G) lg -= G, ++ls;
+      if (!ONE)
+        while (lg >= G) lg -= G, ++ls;
     }
   };
 
   zr_f32x4 acc[NACC][TM][TN] = {};
-  int mg = wave % G;  // the group (inside its segment) multiplied next
+  int mg = ONE ? wave : wave % G;  // the group (inside its segment) multiplied next
   auto mma = [&](Frag& q) {
     if (KG * (mg + 1) > K) {  // K ends inside this group: shift the moved loads back, zeros behind the end in both operands
       if constexpr (BF16) {
@@ -174,7 +178,8 @@ __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a)
       }
     }
     mg += kWaves;
-    while (mg >= G) mg -= G;
+    if (!ONE)
+      while (mg >= G) mg -= G;
     if constexpr (BF16) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -256,14 +261,22 @@ __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a)
   }
 }
 
+template <int TM, int TN, int AMODE, int PF>
+void launch_mode(const SmallArgs& a, unsigned grid, hipStream_t stream) {
+  if (a.nseg == 1 && !a.groups)
+    small_gemm_kernel<TM, TN, AMODE, PF, true><<<grid, 64 * kWaves, 0, stream>>>(a);
+  else
+    small_gemm_kernel<TM, TN, AMODE, PF, false><<<grid, 64 * kWaves, 0, stream>>>(a);
+}
+
 template <int TM, int TN, int PF>
 void launch(const SmallArgs& a, int amode, unsigned grid, hipStream_t stream) {
   switch (amode) {
-    case ZR_A_NN: small_gemm_kernel<TM, TN, ZR_A_NN, PF><<<grid, 64 * kWaves, 0, stream>>>(a); break;
-    case ZR_A_TRANS: small_gemm_kernel<TM, TN, ZR_A_TRANS, PF><<<grid, 64 * kWaves, 0, stream>>>(a); break;
-    case ZR_A_PACK4: small_gemm_kernel<TM, TN, ZR_A_PACK4, PF><<<grid, 64 * kWaves, 0, stream>>>(a); break;
-    case ZR_A_PACK8_BF16: small_gemm_kernel<TM, TN, ZR_A_PACK8_BF16, PF><<<grid, 64 * kWaves, 0, stream>>>(a); break;
-    default: small_gemm_kernel<TM, TN, ZR_A_PACK8_BF16_1T, PF><<<grid, 64 * kWaves, 0, stream>>>(a); break;
+    case ZR_A_NN: launch_mode<TM, TN, ZR_A_NN, PF>(a, grid, stream); break;
+    case ZR_A_TRANS: launch_mode<TM, TN, ZR_A_TRANS, PF>(a, grid, stream); break;
+    case ZR_A_PACK4: launch_mode<TM, TN, ZR_A_PACK4, PF>(a, grid, stream); break;
+    case ZR_A_PACK8_BF16: launch_mode<TM, TN, ZR_A_PACK8_BF16, PF>(a, grid, stream); break;
+    default: launch_mode<TM, TN, ZR_A_PACK8_BF16_1T, PF>(a, grid, stream); break;
   }
 }
 
