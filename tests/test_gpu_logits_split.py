@@ -6,6 +6,7 @@ a partial sum at most once for every product it adds -- and the steps' sums are 
 import numpy as np
 import pytest
 
+from test_gpu_backward import ctx_get
 from zoph_rnn_amd import capi
 
 pytestmark = pytest.mark.gpu
@@ -85,3 +86,28 @@ def test_decoder_width_is_the_same_with_and_without_static_scratch(ctx):
     ctx.softmax_forward(dD, db, V, H, dh, n, capi.ZR_SOFTMAX_PROB, y, static=True)
     ctx.sync()
     assert np.array_equal(x.get(), y.get())
+
+
+@pytest.mark.parametrize("n", [33, 64, 100, 257])
+def test_matrices_past_32_bit_offsets(ctx, n):
+    """From 4 GiB on the row-range kernel and, beyond 256 columns, the split product take a prepared matrix."""
+    V, H = 262177, 4104
+    r = np.random.default_rng(n)
+    dD, b = ctx.empty((V, H)), r.uniform(-1, 1, V).astype(np.float32)
+    ctx.uniform_fill(7, n, dD, V * H)
+    h = np.asfortranarray(r.uniform(-0.1, 0.1, (H, n)).astype(np.float32))
+    out = ctx.empty((V, n))
+    ctx.softmax_prepare(dD, V, H)
+    try:
+        ctx.softmax_forward(dD, ctx.array(b), V, H, ctx.array(h), n, capi.ZR_SOFTMAX_LOGPROB, out)
+        ctx.sync()
+    finally:
+        ctx.softmax_release(dD)
+    x = out.get()
+    rows = np.r_[0:24, V // 2:V // 2 + 24, V - 24:V]
+    D = np.stack([np.concatenate([ctx_get(ctx, dD.at(k * V + int(i)), (24,)) for i in rows[::24]]) for k in range(H)], axis=1)
+    want, most = D.astype(np.float64) @ h + b[rows, None], bound(D, b[rows], h)
+    # log-probabilities: the logits less one number a column, whose own rounding and the subtraction's are 2^-23 of it
+    less = np.median(want - x[rows], axis=0)
+    assert np.all(np.abs(want - x[rows] - less) <= 2 * most + 2.0 ** -23 * np.abs(less))
+    assert np.all(np.abs(np.exp(x.astype(np.float64)).sum(0) - 1.0) < 1e-3)

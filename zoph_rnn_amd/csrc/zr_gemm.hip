@@ -428,44 +428,6 @@ __global__ void __launch_bounds__(256, 2) gemm_stream_kernel(GemmArgs a) {
     gemm_tile<1, 1, 1, ZR_A_PACK4, true, EPI, PF, true, WAUX>(a, (blocks - 1) * 32, 0, true, 0, nullptr, 0, lane);
 }
 
-// Tall weight matrix (k-interleaved) times a minibatch that is a multiple of 128 columns wide, balanced over the
-// CUs without a persistent loop.  A workgroup takes one 64-row x 128-column tile; two workgroups share a CU (256
-// registers each: 128 accumulators and a two-deep operand ring), so that the epilogue of one tile -- cross-wave sum,
-// soft-max partials, stores: a fifth of a tile's time -- and the ramp-up of the next overlap the other workgroup's K
-// loop instead of leaving the matrix pipe idle.  The number of such tiles is rarely a multiple of the number of CUs,
-// and a last, mostly empty round costs as much as a full one.  So only as many
-// 64-row tiles as fill whole rounds are taken that way (workgroups [0, n_big)); the rows left over go to the
-// workgroups behind them as 32 x 32 tiles, which the hardware hands out as the CUs run dry, and whose round lasts an
-// eighth of a big one.  Workgroup ids congruent modulo 8 share an XCD: each XCD takes a contiguous range of big row
-// tiles and the column tiles of one row tile run side by side on it.
-// Big tile of gemm_tall_kernel: 32*TM rows x 32*TN columns, operand ring PF deep, OCC workgroups per CU.  Measured on the 50000 x 128 x 1000 logits product (kernel time, us): one workgroup per CU with a six-deep
-// ring (all 512 registers) 134-136; two per CU with a ring of two 119, of three 122, of one 122; 32 x 128 tiles at two
-// per CU 123; 64 x 64 tiles at three per CU 123.  Giving every resident workgroup the same share of the rows (512
-// workgroups of one 64-row and one 32-row tile each, all resident from start to end, instead of 768 tiles of which the
-// last 256 run one to a CU) changed nothing: 123.9 us for the whole output layer either way.
-// Minibatches that are a multiple of 64 but not of 128 columns wide (192 beam columns) take 64 x 64 tiles at three
-// workgroups per CU.
-template <int EPI, int TM, int TN, int PF, int OCC, int WAUX>
-__global__ void __launch_bounds__(256, OCC) gemm_tall_kernel(GemmArgs a, int big_rows, int n_col_tiles, int n_big) {
-  __shared__ float red[4 * TN * 16 * 64];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int kslice = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int bid = blockIdx.x;
-  if (bid < n_big) {
-    const int r8 = bid & 7, q = bid >> 3;
-    const int mpx = big_rows >> 3;  // big_rows is a multiple of 8
-    const int nt = q % n_col_tiles;
-    const int mt = r8 * mpx + q / n_col_tiles;
-    gemm_tile<TM, TN, 4, ZR_A_PACK4, true, EPI, PF, true, WAUX>(a, mt * 32 * TM, nt * 32 * TN, true, 0, red, kslice, lane);
-  } else {
-    const int idx = bid - n_big;
-    const int n32 = (a.N + 31) >> 5;
-    const int blk = big_rows * TM + idx / n32;
-    gemm_tile<1, 1, 4, ZR_A_PACK4, true, EPI, 8>(a, blk * 32, (idx % n32) * 32, true, 0, red, kslice, lane);
-  }
-}
-
 // Soft-max-partial epilogue for accumulators held the other way round: lane = column (n0 + 32*tn + lane % 32),
 // register r = row m0 + 32*tm + 8*(r/4) + 4*(lane/32) + r%4.  A 32-row block's maximum and sum of exponentials are then
 // 15 in-lane operations and one exchange between the half-waves each (against five cross-lane stages per VALUE when a
@@ -1003,48 +965,6 @@ int launch_bf16_lds(zr_ctx* ctx, GemmArgs& ga) {
   return ZR_OK;
 }
 
-// gemm_tall_kernel: N a multiple of 128, fp32 k-interleaved A.  Returns false when the shape is better served by the
-// row-range kernel (too many rows would be left to the small tiles).
-template <int TM, int TN, int PF, int OCC>
-bool launch_tall_v(zr_ctx* ctx, GemmArgs& ga, int epi, int* rc) {
-  const int blocks = (ga.M + 31) / 32;
-  const int n_col_tiles = ga.N / (32 * TN);
-  const int n32 = ga.N / 32;
-  const long long row_tiles = blocks / TM;  // whole big row tiles
-  // as many big row tiles as fill whole rounds of 256 workgroups, a multiple of 8 of them
-  long long big_rows = (row_tiles * n_col_tiles / 256) * 256 / n_col_tiles;
-  big_rows = big_rows / 8 * 8;
-  const long long small = (long long)(blocks - TM * big_rows) * n32;
-  const bool offsets_fit = (long long)ga.K[0] * ga.lda[0] * 4 + 4096 < (1LL << 32) && (long long)ga.K[0] * ga.N * 4 < (1LL << 32);
-  if (big_rows == 0 || small > 1024 || !offsets_fit) {
-    // the left-over rows would be more than four rounds of small tiles: leave the shape to the row-range kernel
-    return false;
-  }
-  ga.m_tiles = ga.n_tiles = 0;
-  const int n_big = (int)(big_rows * n_col_tiles);
-  const unsigned grid = (unsigned)(n_big + small);
-  if (epi == ZR_EPI_STORE)
-    gemm_tall_kernel<ZR_EPI_STORE, TM, TN, PF, OCC, 0><<<grid, 256, 0, ctx->stream>>>(ga, (int)big_rows, n_col_tiles, n_big);
-  else if (ga.stream_a)
-    gemm_tall_kernel<ZR_EPI_SOFTMAX_PARTIAL, TM, TN, PF, OCC, ZR_AUX_STREAM><<<grid, 256, 0, ctx->stream>>>(
-        ga, (int)big_rows, n_col_tiles, n_big);
-  else
-    gemm_tall_kernel<ZR_EPI_SOFTMAX_PARTIAL, TM, TN, PF, OCC, 0><<<grid, 256, 0, ctx->stream>>>(ga, (int)big_rows,
-                                                                                               n_col_tiles, n_big);
-  hipError_t e = hipGetLastError();
-  *rc = e == hipSuccess ? ZR_OK : zr_set_error(ZR_EHIP, "launch of gemm_tall_kernel failed: %s", hipGetErrorString(e));
-  return true;
-}
-
-// gemm_tall_kernel: N a multiple of 128, 96 or 64 (column tiles of that width: two workgroups per CU at 128, three
-// below), fp32 k-interleaved A.  Returns false when the shape is better served by the row-range kernel (too many rows
-// would be left to the small tiles).  Measured at 50000 x 192 x 1000: row ranges 201 us, 64 x 64 tiles 190, 64 x 96 182.
-bool launch_tall(zr_ctx* ctx, GemmArgs& ga, int epi, int* rc) {
-  if (ga.N % 128 == 0) return launch_tall_v<2, 4, 2, 2>(ctx, ga, epi, rc);
-  if (ga.N % 96 == 0) return launch_tall_v<2, 3, 2, 3>(ctx, ga, epi, rc);
-  return launch_tall_v<2, 2, 2, 3>(ctx, ga, epi, rc);
-}
-
 // Activations X (K x N fp32, column n at src + n*ld, K % 8 == 0) -> two bf16 arrays hi and lo with x = hi + lo up
 // to 2^-16 |x|, each k-interleaved by 8: element (k, n) at ((k/8)*N + n)*8 + k%8.
 // A workgroup takes 16 columns x 16 k-groups, one per thread, and turns them through LDS: it reads with 16 consecutive
@@ -1382,8 +1302,8 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
         zr_error_products_takes((long long)((d.M + 31) / 32) * ((d.N + 31) / 32) * zcount, d.N, ctx->cu_count))
       return zr_error_products(ctx, d);
     if (small >= 0) return zr_small_gemm(ctx, d, nullptr, nullptr, small);
-    // Wide batches: the tall and row-range kernels serve up to 256 columns as well or better (50000 x 192 x 1000: 167
-    // against 175 us), beyond that the split product does (33333 x 700 x 500: 174 against 602 us).  With fixed scratch
+    // The output layer's matrices that zr_logits_plan leaves, from 4 GiB on: the row-range kernel up to 256 columns, beyond that the split
+    // product (33333 x 700 x 500: 174 against 602 us).  With fixed scratch
     // buffers only the statistics form, which needs none of them, and only where the fp32 kernels' copy of B would fit: the
     // limit of the entry point does not follow the kernel.
     if (d.nseg == 1 && zcount == 1 && !d.b_packed && d.groups == 0 && ctx->gemm_cfg == 0 && d.N > 256 &&
@@ -1421,10 +1341,6 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
     if (vec && d.nseg == 1 && zcount == 1 && d.M >= 8192 && d.N <= 1024 && ctx->gemm_cfg != 11 &&
         (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL)) {
       const int n32 = (d.N + 31) / 32;
-      if ((d.N % 64 == 0 || d.N % 96 == 0) && ga.b_pack4 && ctx->gemm_cfg == 0) {
-        int rc = ZR_OK;
-        if (launch_tall(ctx, ga, d.epilogue, &rc)) return rc;
-      }
       if (d.N <= 32 && ga.b_pack4 && d.K[0] % 8 == 0 && ctx->gemm_cfg == 0 &&
           (long long)d.K[0] * ga.lda[0] * 4 + 4096 < (1LL << 32)) {
         // one 32-row block per wave while there are waves (three workgroups per compute unit), more beyond that

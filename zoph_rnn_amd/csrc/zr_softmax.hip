@@ -159,8 +159,8 @@ softmax_loss_kernel(const float* __restrict__ logits, int V, int mb, const doubl
 }
 
 // d_h_packed: optional k-interleaved copy of d_h ([H/4][mb][4]); used when the product runs on the registered fp32 copy
-// of D and H % 8 == 0 (the product then skips its own re-layout of d_h), but not where the split product takes the call,
-// which reads d_h as it lies: with and without the copy the same kernel runs.
+// of D and H % 8 == 0 (the product then skips its own re-layout of d_h), but not where zr_logits_plan or the split product
+// takes the call, which read d_h as it lies: with and without the copy the same kernel runs.
 // d_partials_ext: where the [mb][nblocks][2] pairs go instead of context scratch (ZR_SOFTMAX_LOGITS_BLOCKS: the caller's
 // buffer; no column statistics follow them there).
 int logits_with_partials(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, int H, const float* d_h, int mb,
