@@ -53,7 +53,7 @@ __global__ void __launch_bounds__(256, 1) error_products_kernel(ErrorProducts P)
   clear();
   {
     ZrFrag<2, 2> ring[RING];
-    zr_mma_segment_split<2, 2, KS, RING, false>(acc, wrsrc, wsoff, woffb, 32u * (unsigned)P.ldp, xrsrc, xoffb, 32u * (unsigned)P.N, P.K, wave, ring);
+    zr_mma_segment_split<2, 2, KS, RING>(acc, wrsrc, wsoff, woffb, 32u * (unsigned)P.ldp, xrsrc, xoffb, 32u * (unsigned)P.N, P.K, wave, ring);
   }
   bool finite = true;
 #pragma unroll

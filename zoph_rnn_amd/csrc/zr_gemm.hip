@@ -720,7 +720,7 @@ __global__ void __launch_bounds__(64 * NWV) gemm_lds_kernel(GemmArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[tm][r] = 0.0f;
 
-  zr_u32x4v wreg[WLD];
+  zr_u32x4 wreg[WLD];
   zr_f32x4 xf[2][4];
   // gload only issues loads (the values stay in registers while the current chunk is multiplied) so that several
   // loads stay in flight.
@@ -733,7 +733,7 @@ __global__ void __launch_bounds__(64 * NWV) gemm_lds_kernel(GemmArgs a) {
     for (int gq = 0; gq < 4; ++gq) {
       int kx = c * KC + 8 * gq;
       kx = kx + 8 <= K ? kx : K - 8;  // wave-uniform: the weights of the k values this replaces are zeros
-      const zr_u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)(xoffb + (unsigned)kx * 4u), 0, 0);
+      const zr_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)(xoffb + (unsigned)kx * 4u), 0, 0);
       xdst[gq].x = __uint_as_float(v.x);
       xdst[gq].y = __uint_as_float(v.y);
       xdst[gq].z = __uint_as_float(v.z);

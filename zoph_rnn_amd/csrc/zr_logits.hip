@@ -40,24 +40,6 @@ constexpr int KC = 32;  // k of a step
 // k-groups at a time) nor a store (all four) finds two of its items in the same banks.
 __device__ __forceinline__ int turned(int c, int kg) { return c ^ (8 * (kg & 1) + 4 * (kg >> 1)); }
 
-// Two values' leading bf16 terms (rounded to nearest) in one register; the values become what is left of them.
-__device__ __forceinline__ unsigned next_terms(float& a, float& b) {
-  unsigned t = __builtin_bit_cast(unsigned, zr_bf16x2{(__bf16)a, (__bf16)b});
-  asm("" : "+v"(t));  // one conversion for both values
-  a -= __uint_as_float(t << 16);
-  b -= __uint_as_float(t & 0xffff0000u);
-  return t;
-}
-// Eight consecutive k as three fragments.
-__device__ __forceinline__ void split_terms(const zr_f32x4& lo, const zr_f32x4& hi, zr_u32x4 (&term)[3]) {
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    float a = p < 2 ? lo[2 * p] : hi[2 * p - 4], b = p < 2 ? lo[2 * p + 1] : hi[2 * p - 3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) term[q][p] = next_terms(a, b);
-  }
-}
-
 template <int TN, int W, int PD, int WAUX>
 __global__ void __launch_bounds__(64 * W, 2) logits_split_kernel(LogitsArgs a) {
   constexpr int COLS = 32 * TN, KG = COLS, TERM = 4 * KG, BUF = 3 * TERM;
@@ -114,7 +96,7 @@ __global__ void __launch_bounds__(64 * W, 2) logits_split_kernel(LogitsArgs a) {
       const int item = tid + 64 * W * i, kg = item & 3;
       if (ITEMS % (64 * W) != 0 && item >= ITEMS) break;
       zr_u32x4 term[3];
-      split_terms(bv[i][0], bv[i][1], term);
+      zr_split_terms(bv[i][0], bv[i][1], term);
       zr_u32x4* d = s + buf * BUF + kg * KG + turned(item >> 2, kg);
 #pragma unroll
       for (int q = 0; q < 3; ++q) d[q * TERM] = term[q];
@@ -131,7 +113,7 @@ __global__ void __launch_bounds__(64 * W, 2) logits_split_kernel(LogitsArgs a) {
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       zr_u32x4 term[3];
-      split_terms(v[2 * st], v[2 * st + 1], term);
+      zr_split_terms(v[2 * st], v[2 * st + 1], term);
 #pragma unroll
       for (int q = 0; q < 3; ++q) x[st][q] = __builtin_bit_cast(zr_bf16x8, term[q]);
     }

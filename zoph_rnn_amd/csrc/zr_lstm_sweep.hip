@@ -44,24 +44,6 @@ namespace {
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at any multiple of 4
 typedef unsigned zr_u32x2 __attribute__((ext_vector_type(2)));
 
-// Two values' leading bf16 terms (rounded to nearest) in one register; the values become what is left of them.
-__device__ __forceinline__ unsigned next_terms(float& a, float& b) {
-  unsigned t = __builtin_bit_cast(unsigned, zr_bf16x2{(__bf16)a, (__bf16)b});
-  asm("" : "+v"(t));  // one conversion for both values
-  a -= __uint_as_float(t << 16);
-  b -= __uint_as_float(t & 0xffff0000u);
-  return t;
-}
-// Eight consecutive k as three fragments.
-__device__ __forceinline__ void split_terms(const zr_f32x4& lo, const zr_f32x4& hi, zr_u32x4 (&term)[3]) {
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    float a = p < 2 ? lo[2 * p] : hi[2 * p - 4], b = p < 2 ? lo[2 * p + 1] : hi[2 * p - 3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) term[q][p] = next_terms(a, b);
-  }
-}
-
 // All threads of the workgroup call this.  False: leave the kernel.
 __device__ __forceinline__ bool sweep_wait(const LstmSweep& P, int* ctr, int target, int* s_go) {
   if (threadIdx.x == 0) {
@@ -96,7 +78,7 @@ __global__ void __launch_bounds__(256) lstm_sweep_terms_kernel(LstmSweep P) {
   unsigned short* d = (which ? P.hp + (long long)(which - 1) * (P.T + 1) * slot : P.xp + t * slot) + ((long long)kg * P.columns + n) * 8;
   zr_u32x4 term[3];
   const zr_f32x4 lo = *(const f32x4u*)(x + 8 * kg), hi = *(const f32x4u*)(x + 8 * kg + 4);
-  split_terms(lo, hi, term);
+  zr_split_terms(lo, hi, term);
 #pragma unroll
   for (int q = 0; q < 3; ++q) *(zr_u32x4*)(d + q * n_el) = term[q];
 }
@@ -171,7 +153,7 @@ __global__ void __launch_bounds__(512, 2) lstm_sweep_kernel(LstmSweep P) {
   zr_bf16x8 x[2][3];  // the weights of 16 k in use, and the next 16 k's, split beside the products of these
   auto split_a = [&](const zr_f32x4& lo, const zr_f32x4& hi, zr_bf16x8 (&x)[3]) {
     zr_u32x4 term[3];
-    split_terms(lo, hi, term);
+    zr_split_terms(lo, hi, term);
 #pragma unroll
     for (int q = 0; q < 3; ++q) x[q] = __builtin_bit_cast(zr_bf16x8, term[q]);
   };
@@ -336,10 +318,10 @@ __global__ void __launch_bounds__(512, 2) lstm_sweep_kernel(LstmSweep P) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         if constexpr (TN == 2) {
-          const unsigned lo = next_terms(left[0], left[1]), hi = next_terms(left[2], left[3]);
+          const unsigned lo = zr_next_terms(left[0], left[1]), hi = zr_next_terms(left[2], left[3]);
           __hip_atomic_store((unsigned long long*)(d + q * n_el), lo | (unsigned long long)hi << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-          __hip_atomic_store((unsigned*)(d + q * n_el), next_terms(left[0], left[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store((unsigned*)(d + q * n_el), zr_next_terms(left[0], left[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
       }
     }

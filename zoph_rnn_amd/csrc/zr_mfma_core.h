@@ -198,7 +198,28 @@ __device__ __forceinline__ void zr_mma_segment(zr_f32x16 (&acc)[TM][TN], const f
 //   xoffb[tn]: this lane's byte offset of its column, 4*half included
 //   wstep / xstep: bytes per k-group of 8 (weights: 32*lda; activations: 32 for a plain column, 32*mb k-interleaved)
 // Every offset sum must stay below 4 GiB (the host checks the extents).
-typedef unsigned zr_u32x4v __attribute__((ext_vector_type(4)));
+typedef unsigned zr_u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 zr_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 zr_bf16x2 __attribute__((ext_vector_type(2)));
+
+// Two values' leading bf16 terms (rounded to nearest) in one register; the values become what is left of them.
+__device__ __forceinline__ unsigned zr_next_terms(float& a, float& b) {
+  unsigned t = __builtin_bit_cast(unsigned, zr_bf16x2{(__bf16)a, (__bf16)b});
+  asm("" : "+v"(t));  // one conversion for both values: without this the compiler converts one of them a second time
+  a -= __uint_as_float(t << 16);
+  b -= __uint_as_float(t & 0xffff0000u);
+  return t;
+}
+// Eight consecutive k, four and four, as three fragments of exact terms (zr_split_gemm.hip says why that loses nothing).
+template <typename Four>
+__device__ __forceinline__ void zr_split_terms(const Four& lo, const Four& hi, zr_u32x4 (&term)[3]) {
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    float a = p < 2 ? lo[2 * p] : hi[2 * p - 4], b = p < 2 ? lo[2 * p + 1] : hi[2 * p - 3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) term[q][p] = zr_next_terms(a, b);
+  }
+}
 // Cache policy operand of the weight fetches (the buffer-load builtin's last argument): 0 = default, ZR_AUX_STREAM =
 // the non-temporal hint.  A matrix that is read once per step and is a large part of the memory-side cache (the output
 // layer's: 200 MB of its 256 MB at 50 000 x 1000) otherwise pushes out everything the rest of the step re-reads -- the
@@ -212,8 +233,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t zr_make_rsrc(const void* base)
 // The weight halves of the first PF ring stages of a segment, issued ahead of time (zr_mma_segment_u with WPRE then
 // fetches only the activation halves in its prologue): weights depend on nothing, so a caller that must wait for its
 // activations can have them in flight during the wait.
-template <int TM, int TN, int KS, int PF, int WAUX = 0, int NS = PF + 1>
-__device__ __forceinline__ void zr_preload_w(ZrFrag<TM, TN> (&f)[NS], __amdgpu_buffer_rsrc_t wrsrc,
+template <int TM, int TN, int KS, int PF, int WAUX = 0>
+__device__ __forceinline__ void zr_preload_w(ZrFrag<TM, TN> (&f)[PF + 1], __amdgpu_buffer_rsrc_t wrsrc,
                                              const unsigned (&wsoff)[TM], unsigned woffb, unsigned wstep, int K,
                                              int kslice) {
   const int last = (K >> 3) - 1;
@@ -223,7 +244,7 @@ __device__ __forceinline__ void zr_preload_w(ZrFrag<TM, TN> (&f)[NS], __amdgpu_b
     gl = gl < last ? gl : last;
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
-      const zr_u32x4v v =
+      const zr_u32x4 v =
           __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + (unsigned)gl * wstep), WAUX);
       f[s].w[tm][0] = __uint_as_float(v.x);
       f[s].w[tm][1] = __uint_as_float(v.y);
@@ -244,7 +265,7 @@ __device__ __forceinline__ void zr_mma_segment_u(zr_f32x16 (&acc)[TM][TN], __amd
     const unsigned ug = (unsigned)g;  // wave-uniform
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) {
-      const zr_u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)xoffb[tn], (int)(ug * xstep), 0);
+      const zr_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)xoffb[tn], (int)(ug * xstep), 0);
       f.x[tn][0] = __uint_as_float(v.x);
       f.x[tn][1] = __uint_as_float(v.y);
       f.x[tn][2] = __uint_as_float(v.z);
@@ -256,7 +277,7 @@ __device__ __forceinline__ void zr_mma_segment_u(zr_f32x16 (&acc)[TM][TN], __amd
     load_x(f, g);
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
-      const zr_u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + ug * wstep), WAUX);
+      const zr_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + ug * wstep), WAUX);
       f.w[tm][0] = __uint_as_float(v.x);
       f.w[tm][1] = __uint_as_float(v.y);
       f.w[tm][2] = __uint_as_float(v.z);
@@ -312,37 +333,15 @@ __device__ __forceinline__ void zr_mma_segment_u(zr_f32x16 (&acc)[TM][TN], __amd
 
 // zr_mma_segment_u on the bf16 matrix cores: every fp32 operand as three exact bf16 terms, six products, the same loads.  Two k-groups make
 // one step: a lane's eight k are its four of the one and its four of the other, for both operands.  The terms of a step are made beside
-// the products of the step before, and a revolution's products are summed from zero before they reach the accumulator.  R: slots of the ring (a multiple of 4), R - 2 groups ahead; WPRE: the weight halves of those are on
-// their way (zr_preload_w).  Terms of an infinite operand are infinity and NaN: where a sum comes out infinite or NaN the caller
-// computes it again with zr_mma_segment_u.
-typedef __bf16 zr_bf16x8_s __attribute__((ext_vector_type(8)));
-typedef __bf16 zr_bf16x2_s __attribute__((ext_vector_type(2)));
-// Two values' leading bf16 terms (rounded to nearest) in one register; the values become what is left of them.
-__device__ __forceinline__ unsigned zr_next_terms(float& a, float& b) {
-  unsigned t = __builtin_bit_cast(unsigned, zr_bf16x2_s{(__bf16)a, (__bf16)b});
-  asm("" : "+v"(t));  // one conversion for both values
-  a -= __uint_as_float(t << 16);
-  b -= __uint_as_float(t & 0xffff0000u);
-  return t;
-}
-__device__ __forceinline__ void zr_split8(const float (&lo)[4], const float (&hi)[4], zr_bf16x8_s (&term)[3]) {
-  zr_u32x4v t[3];
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    float a = p < 2 ? lo[2 * p] : hi[2 * p - 4], b = p < 2 ? lo[2 * p + 1] : hi[2 * p - 3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) t[q][p] = zr_next_terms(a, b);
-  }
-#pragma unroll
-  for (int q = 0; q < 3; ++q) term[q] = __builtin_bit_cast(zr_bf16x8_s, t[q]);
-}
-
+// the products of the step before, and a revolution's products are summed from zero before they reach the accumulator.  R: slots of the ring (a multiple of 4), R - 2
+// groups ahead.  Terms of an infinite operand are infinity and NaN: where a sum comes out infinite or NaN the caller computes it again with
+// zr_mma_segment_u.
 template <int TM, int TN>
 struct ZrTerms {
-  zr_bf16x8_s x[TN][3], w[TM][3];
+  zr_bf16x8 x[TN][3], w[TM][3];
 };
 
-template <int TM, int TN, int KS, int R, bool WPRE>
+template <int TM, int TN, int KS, int R>
 __device__ __forceinline__ void zr_mma_segment_split(zr_f32x16 (&acc)[TM][TN], __amdgpu_buffer_rsrc_t wrsrc,
                                                      const unsigned (&wsoff)[TM], unsigned woffb, unsigned wstep,
                                                      __amdgpu_buffer_rsrc_t xrsrc, const unsigned (&xoffb)[TN],
@@ -350,28 +349,31 @@ __device__ __forceinline__ void zr_mma_segment_split(zr_f32x16 (&acc)[TM][TN], _
   static_assert(R % 4 == 0, "pairs of slots, and an even number of pairs a revolution");
   const int nfull = K >> 3;  // K % 8 == 0
   constexpr int AHEAD = R - 2;
-  auto load_x = [&](ZrFrag<TM, TN>& f, int g) {
+  auto load_full = [&](ZrFrag<TM, TN>& f, int g) {
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) {
-      const zr_u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)xoffb[tn], (int)((unsigned)g * xstep), 0);
+      const zr_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)xoffb[tn], (int)((unsigned)g * xstep), 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) f.x[tn][i] = __uint_as_float(v[i]);
     }
-  };
-  auto load_full = [&](ZrFrag<TM, TN>& f, int g) {
-    load_x(f, g);
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
-      const zr_u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + (unsigned)g * wstep), 0);
+      const zr_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + (unsigned)g * wstep), 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) f.w[tm][i] = __uint_as_float(v[i]);
     }
   };
+  auto split8 = [](const float (&lo)[4], const float (&hi)[4], zr_bf16x8 (&t)[3]) {
+    zr_u32x4 term[3];
+    zr_split_terms(lo, hi, term);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) t[q] = __builtin_bit_cast(zr_bf16x8, term[q]);
+  };
   auto split = [&](const ZrFrag<TM, TN>& a, const ZrFrag<TM, TN>& b, ZrTerms<TM, TN>& t) {
 #pragma unroll
-    for (int tn = 0; tn < TN; ++tn) zr_split8(a.x[tn], b.x[tn], t.x[tn]);
+    for (int tn = 0; tn < TN; ++tn) split8(a.x[tn], b.x[tn], t.x[tn]);
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm) zr_split8(a.w[tm], b.w[tm], t.w[tm]);
+    for (int tm = 0; tm < TM; ++tm) split8(a.w[tm], b.w[tm], t.w[tm]);
   };
   zr_f32x16 sum[TM][TN];
   auto clear = [&] {
@@ -406,12 +408,7 @@ __device__ __forceinline__ void zr_mma_segment_split(zr_f32x16 (&acc)[TM][TN], _
     return gl < last ? gl : last;
   };
 #pragma unroll
-  for (int s = 0; s < AHEAD; ++s) {
-    if (WPRE)
-      load_x(f[s], group(s));
-    else
-      load_full(f[s], group(s));
-  }
+  for (int s = 0; s < AHEAD; ++s) load_full(f[s], group(s));
   // the group behind the last is nothing, in either operand
   auto single = [&](ZrFrag<TM, TN>& f, bool there) {
 #pragma unroll
@@ -665,9 +662,6 @@ __device__ __forceinline__ void zr_half_wave_softmax_stats(const float (&v)[G], 
 // ZR_A_PACK8_BF16_1T: the same weight layout in single-term mode (activations rounded to bf16 once, no lo array)
 enum { ZR_A_PACK8_BF16 = 3, ZR_A_PACK8_BF16_1T = 4 };
 constexpr bool zr_is_bf16_mode(int amode) { return amode == ZR_A_PACK8_BF16 || amode == ZR_A_PACK8_BF16_1T; }
-typedef __bf16 zr_bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 zr_bf16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned zr_u32x4 __attribute__((ext_vector_type(4)));
 
 // (x0, x1) -> packed bf16 pairs hi and lo with x = hi + lo up to 2^-17 |x|
 __device__ __forceinline__ void zr_split_bf16_pair(float x0, float x1, unsigned& hi, unsigned& lo) {

@@ -19,11 +19,12 @@
 // each other's conversions and barriers.  50000 x 6400 x 1000: 128 x 128 tiles 3.94 ms, 128 x 256 3.49 (184 TFLOP/s of fp32 work;
 // the fp32 instructions' kernel 5.70); 4000 x 1000 x 6400 0.47 -> 0.31; 33333 x 700 x 500 0.60 -> 0.16.
 #include "zr_internal.h"
+#include "zr_mfma_core.h"
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef zr_bf16x8 bf16x8;
+typedef zr_u32x4 u32x4;
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at any multiple of 4
 
@@ -125,16 +126,6 @@ __device__ __forceinline__ void load_operand(f32x4u (&v)[ROWS / 32], const float
   }
 }
 
-// Two values' leading bf16 terms (rounded to nearest) in one register; the values become what is left of them.
-__device__ __forceinline__ unsigned next_terms(float& a, float& b) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  unsigned t = __builtin_bit_cast(unsigned, bf16x2{(__bf16)a, (__bf16)b});
-  asm("" : "+v"(t));  // one conversion for both values: without this the compiler converts one of them a second time
-  a -= __uint_as_float(t << 16);
-  b -= __uint_as_float(t & 0xffff0000u);
-  return t;
-}
-
 template <int ROWS, int LAYOUT>
 __device__ __forceinline__ void store_operand(u32x4* s, const f32x4u (&v)[ROWS / 32], int t) {
   typedef Oper<ROWS> O;
@@ -144,12 +135,8 @@ __device__ __forceinline__ void store_operand(u32x4* s, const f32x4u (&v)[ROWS /
       u32x4* d = LAYOUT == ZR_SPLIT_PACK4 ? s + (t >> 6) * O::KG + lds_row((t & 63) + 64 * i, t >> 6)
                                           : s + (t & 3) * O::KG + lds_row((t >> 2) + 64 * i, t & 3);
       u32x4 term[3];
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        float a = v[2 * i + p / 2][2 * (p & 1)], b = v[2 * i + p / 2][2 * (p & 1) + 1];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) term[q][p] = next_terms(a, b);
-      }
+      const zr_f32x4 lo = v[2 * i], hi = v[2 * i + 1];
+      zr_split_terms(lo, hi, term);
 #pragma unroll
       for (int q = 0; q < 3; ++q) d[q * O::TERM] = term[q];
     }
@@ -164,7 +151,7 @@ __device__ __forceinline__ void store_operand(u32x4* s, const f32x4u (&v)[ROWS /
         for (int p = 0; p < 2; ++p) {
           float a = v[4 * i + 2 * p][e], b = v[4 * i + 2 * p + 1][e];
 #pragma unroll
-          for (int q = 0; q < 3; ++q) term[q][p] = next_terms(a, b);
+          for (int q = 0; q < 3; ++q) term[q][p] = zr_next_terms(a, b);
         }
 #pragma unroll
         for (int q = 0; q < 3; ++q) d[q * O::TERM * 2] = term[q];
