@@ -778,8 +778,10 @@ int zr_decoder_step(zr_ctx* ctx, int nl, const zr_lstm_weights* const layers[], 
   if (rc) return rc;
   if (!attn)
     return zr_softmax_forward_packed(ctx, d_D, d_b_d, V_out, layers[0]->H, top, nullptr, mb, mode, d_out, nullptr);
+  // h~ k-interleaved only for an output product that reads it so (zr_logits_plan's reads it as it lies)
+  const bool htpack = packed && (ctx->gemm_cfg != 0 || !zr_logits_plan(V_out, mb, attn->H, ctx->cu_count).tn);
   rc = attn_step_impl(ctx, attn, d_batch_info, top, d_mask01, d_htild, d_alignments, d_indices, d_p_t, d_c_ctx,
-                      (pack32 || split16) && wrote, packed ? attn->d_htpack : nullptr);
+                      (pack32 || split16) && wrote, htpack ? attn->d_htpack : nullptr);
   if (rc) return rc;
   // (the k-interleaved h~ only if the attention step says it wrote it)
   return zr_softmax_forward_packed(ctx, d_D, d_b_d, V_out, attn->H, d_htild,
