@@ -1,5 +1,5 @@
 """The output layer's product on a prepared fp32 matrix beyond 32 columns (csrc/zr_logits.hip): edges of its 32-row blocks, its tiles
-of one to six 32-column blocks with four or eight waves, and its steps of 32 k.
+of one to six 32-column blocks with four or eight waves (test_rules_cpu.py holds that the sizes here take each), and its steps of 32 k.
 Tolerance: the products of 32 k are six exact terms each, added one after another in fp32 -- twelve instructions, each rounding
 a partial sum at most once for every product it adds -- and the steps' sums are added in turn: at most K + 12 roundings of
 2^-24 of the sum of the terms' magnitudes; the three terms left out are below one more."""
@@ -43,8 +43,13 @@ def bound(D, b, h):
     return (D.shape[1] + 13) * 2.0 ** -24 * (np.abs(D).astype(np.float64) @ np.abs(h) + np.abs(b)[:, None])
 
 
-@pytest.mark.parametrize("V,H,n", [(33, 1, 33), (31, 31, 64), (129, 32, 65), (257, 33, 96), (1000, 63, 97), (1000, 65, 257), (4001, 100, 160), (2049, 129, 700),
-                                   (9001, 37, 1100), (30011, 500, 37), (33333, 64, 128), (50001, 96, 192), (8191, 300, 320), (12345, 1000, 40)])
+SIZES = [(33, 1, 33), (31, 31, 64), (129, 32, 65), (257, 33, 96), (1000, 63, 97), (1000, 65, 257), (4001, 100, 160), (2049, 129, 700),
+         (9001, 37, 1100), (30011, 500, 37), (33333, 64, 128), (50001, 96, 192), (8191, 300, 320), (12345, 1000, 40),
+         # the tiles that none of these takes, and matrices of 64 MiB and more, whose loads have the streaming hint, with rows left over
+         (2996, 64, 963), (4493, 64, 901), (11978, 64, 963), (18964, 64, 777), (16469, 64, 901), (16801, 1000, 33), (33601, 500, 97)]
+
+
+@pytest.mark.parametrize("V,H,n", SIZES)
 def test_logits_and_block_pairs(ctx, V, H, n):
     D, b, h = operands(V, H, n)
     x, pairs = logits_and_blocks(ctx, D, b, h)

@@ -250,6 +250,13 @@ inline int zr_small_gemm_shape(int M, int N, int K, int nseg, int z, int a_pack,
   return best;
 }
 
+// Groups a wave has in flight: all it has, up to 64 registers of operands.
+inline int zr_small_gemm_depth(int shape, int K, int nseg, int a_pack) {
+  const int kg = a_pack == 2 ? 32 : 16, mine = (nseg * ((K + kg - 1) / kg) + 7) / 8;
+  if (shape == 0) return mine <= 2 ? 2 : (mine <= 4 ? 4 : 8);
+  return shape == 1 ? (mine <= 3 ? 3 : 6) : 4;
+}
+
 // ---- sums over the columns of an attention node's backward pass (rows_with_sum): workgroups that share the columns of 32 rows
 
 // us of both sums' kernels, an element-wise one and a separate sum / one workgroup that walks all columns / in parts: H = 64, 64 columns 9.6 /

@@ -303,20 +303,14 @@ int zr_small_gemm(zr_ctx* ctx, const ZrGemmDesc& d, const unsigned short* const 
   const unsigned grid = (unsigned)(a.rows * a.n_tiles + 7) / 8 * 8;
   const int amode = d.a_pack == 2 ? (a.Blo[0] ? ZR_A_PACK8_BF16 : ZR_A_PACK8_BF16_1T)
                                   : (d.a_pack ? ZR_A_PACK4 : (d.trans_a ? ZR_A_TRANS : ZR_A_NN));
-  // groups in flight: all a wave has, up to 64 registers of operands
-  const int kg = d.a_pack == 2 ? 32 : 16, mine = (d.nseg * ((a.K + kg - 1) / kg) + kWaves - 1) / kWaves;
-  if (shape == 0 && mine <= 2)
-    launch<1, 1, 2>(a, amode, grid, ctx->stream);
-  else if (shape == 0 && mine <= 4)
-    launch<1, 1, 4>(a, amode, grid, ctx->stream);
-  else if (shape == 0)
-    launch<1, 1, 8>(a, amode, grid, ctx->stream);
-  else if (shape == 1 && mine <= 3)
-    launch<1, 2, 3>(a, amode, grid, ctx->stream);
-  else if (shape == 1)
-    launch<1, 2, 6>(a, amode, grid, ctx->stream);
-  else
-    launch<2, 2, 4>(a, amode, grid, ctx->stream);
+  switch (10 * shape + zr_small_gemm_depth(shape, a.K, a.nseg, d.a_pack)) {
+    case 2: launch<1, 1, 2>(a, amode, grid, ctx->stream); break;
+    case 4: launch<1, 1, 4>(a, amode, grid, ctx->stream); break;
+    case 8: launch<1, 1, 8>(a, amode, grid, ctx->stream); break;
+    case 13: launch<1, 2, 3>(a, amode, grid, ctx->stream); break;
+    case 16: launch<1, 2, 6>(a, amode, grid, ctx->stream); break;
+    default: launch<2, 2, 4>(a, amode, grid, ctx->stream); break;
+  }
   ZR_LAUNCH_CHECK("small_gemm_kernel");
   return ZR_OK;
 }
