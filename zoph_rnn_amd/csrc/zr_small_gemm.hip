@@ -52,7 +52,8 @@ __device__ __forceinline__ zr_f32x4 shifted(zr_f32x4 v, int d) {
 
 // ONE: one segment, ungrouped.  No load then needs an entry of a table of arguments by a computed index, which took a second trip for arguments
 // ahead of the first loads and others inside the loop: 885 x 126 x 98 5.0 -> 4.5 us, 1026 x 105 x 1030 11.7 -> 9.8, 2535 x 34 x 1463
-// 15.7 -> 13.2.
+// 15.7 -> 13.2.  Not for bf16 matrices: the compiler then keeps so many addresses in registers that some forms spill (a decode step at H = 1024, 64
+// columns 122 -> 129 us).
 template <int TM, int TN, int AMODE, int PF, bool ONE>
 __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a) {
   constexpr bool BF16 = zr_is_bf16_mode(AMODE), LO = AMODE == ZR_A_PACK8_BF16;
@@ -263,10 +264,13 @@ __global__ void __launch_bounds__(64 * kWaves, 2) small_gemm_kernel(SmallArgs a)
 
 template <int TM, int TN, int AMODE, int PF>
 void launch_mode(const SmallArgs& a, unsigned grid, hipStream_t stream) {
-  if (a.nseg == 1 && !a.groups)
-    small_gemm_kernel<TM, TN, AMODE, PF, true><<<grid, 64 * kWaves, 0, stream>>>(a);
-  else
-    small_gemm_kernel<TM, TN, AMODE, PF, false><<<grid, 64 * kWaves, 0, stream>>>(a);
+  if constexpr (!zr_is_bf16_mode(AMODE)) {
+    if (a.nseg == 1 && !a.groups) {
+      small_gemm_kernel<TM, TN, AMODE, PF, true><<<grid, 64 * kWaves, 0, stream>>>(a);
+      return;
+    }
+  }
+  small_gemm_kernel<TM, TN, AMODE, PF, false><<<grid, 64 * kWaves, 0, stream>>>(a);
 }
 
 template <int TM, int TN, int PF>
