@@ -1,4 +1,5 @@
-"""Products large enough for the bf16 matrix cores with every fp32 operand as three bf16 terms, and what feeds them."""
+"""Products large enough for the bf16 matrix cores with every fp32 operand as three bf16 terms, and what feeds them.  (The forward product of a prepared
+output layer here is zr_logits.hip's; the split product takes one from 4 GiB on, tests/test_gpu_logits_split.py.)"""
 import numpy as np
 import pytest
 
@@ -146,7 +147,7 @@ def test_lstm_weight_gradients(ctx, H, T, mb):
 
 @pytest.mark.parametrize("V,H,n", [(20000, 500, 257), (20001, 503, 512), (10001, 1000, 400), (12000, 1000, 1024)])
 def test_prepared_output_layer_is_rounded_in_short_chains(ctx, V, H, n):
-    """A probability is off by its logit's error, in proportion.  The logit of a large one is a sum that grows steadily, so the
+    """With sums of 32 k (zr_logits.hip; a bound for 16).  A probability is off by its logit's error, in proportion.  The logit of a large one is a sum that grows steadily, so the
     partial sums have a third of the final square on average: K / 16 additions, each a relative 2.5e-8 in the 2-norm (mantissas
     spread evenly in their logarithm), and the bias.  The exponential, its argument, the sum and the division add a part in
     10^7.  (Measured: two thirds of that.  With the six products of 16 k added one by one twice to three times as much.)"""

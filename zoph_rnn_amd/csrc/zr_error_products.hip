@@ -4,8 +4,8 @@
 // A workgroup has 64 x 64 outputs of one product, its four waves take the groups of 8 k in turn, straight from the k-interleaved copies of
 // both operands into registers, and split what they multiply; their sums are added through LDS in a fixed order.  A die takes a contiguous
 // range of the tiles, all column tiles of a row in turn, so that its level-two cache sees every element of the matrices once.
-// Bound by the conversions beside the matrix instructions and the trips to the caches: a full diagonal of 4 layers of H = 1000 at 128 columns
-// (8.2 GFLOP) takes 81 us on the fp32 instructions and 53 here (the sweep of 12 steps 1190 -> 922).  Error of a product against 64 bits, here and
+// Bound by the conversions beside the matrix instructions (61 % of a SIMD's cycles and 48.5 %, one wave a SIMD): a full diagonal of 4 layers of H = 1000 at 128
+// columns (8.2 GFLOP) takes 81 us on the fp32 instructions and 53 to 57 here (the sweep of 12 steps 1190 -> 922).  Error of a product against 64 bits, here and
 // there: H = 300 1.3e-7 to 1.6e-7 / 1.9e-7 to 2.4e-7, 1000 1.4e-7 to 2.6e-7 / 3.5e-7 to 4.7e-7 (with one chain of sums 3.7e-7).
 #include "zr_internal.h"
 #include "zr_mfma_core.h"

@@ -104,7 +104,7 @@ int zr_ctx_scratch_if_room(zr_ctx* ctx, int slot, size_t bytes, void** out);
 typedef float zr_f32x16 __attribute__((ext_vector_type(16)));
 typedef float zr_f32x4 __attribute__((ext_vector_type(4)));
 
-// Generic multi-segment GEMM: C = sum_s op(A_s) * B_s, then an epilogue.  Up to 3 segments.
+// Generic multi-segment GEMM: C = sum_s op(A_s) * B_s, then an epilogue.  Up to 3 segments, 4 on zr_small_gemm.
 enum ZrEpilogue {
   ZR_EPI_STORE = 0,           // C = acc (+ bias[m] if bias)
   ZR_EPI_TANH = 1,            // C = tanhf(acc)
@@ -114,7 +114,7 @@ enum ZrEpilogue {
 
 struct ZrGemmDesc {
   int M, N;
-  int nseg;  // up to 3 (4 where zr_small_gemm takes the product)
+  int nseg;  // up to 3 (4 where zr_small_gemm takes the product, on plain matrices)
   int K[4];
   const float* A[4];
   int lda[4];

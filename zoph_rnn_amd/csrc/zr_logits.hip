@@ -8,8 +8,9 @@
 // into LDS, one step ahead, and read by all waves.  The twelve products of 32 k are added up from zero and their sum is added to the
 // accumulator: short chains, one rounding at the accumulator's size.  An accumulator that comes out infinite or NaN is computed again with
 // fp32 instructions (the terms of an infinite operand are infinity and NaN).
-// Bound by the matrix cores: 50000 x 128 x 1000 takes 89 us (12.8 GFLOP, 77 of bf16 work), which is 1.13 PFLOP/s on the compute units that have eight
-// row blocks -- six do on average -- and large bf16 products reach 1.2 on this card.  The fp32 instructions took 110 to 124; 64 columns of 30011 x 500 31 -> 22.
+// Bound by matrix instructions and conversions together: at 50000 x 128 x 1000 the matrix pipes of the 200 compute units that have a tile are busy for 57 %,
+// the vector instructions take 44 % of their cycles.  It takes 89 to 92 us (12.8 GFLOP, 77 of bf16 work); the fp32 instructions took 110 to
+// 124; 64 columns of 30011 x 500 31 -> 22.
 // Error of the logits against 64 bits, relative 2-norm, here and with the fp32 instructions: H = 64 7.6e-8 / 8.7e-8, 200 9.1e-8 / 1.36e-7, 500
 // 1.09e-7 / 2.06e-7, 1000 1.35e-7 / 2.1e-7 to 2.9e-7.
 // Tried and dropped at 128 columns: one chain of dependent instructions a column block instead of two in turn (107 against 103 us the whole

@@ -32,5 +32,5 @@ struct LstmSweep {
 
 // Resident workgroups of the kernel on tiles of 32 * tn columns that the device can hold at once (0: unknown / query failed).
 int zr_sweep_capacity(zr_ctx* ctx, int tn);
-// H a multiple of 8 from 64 on, T of at least 1; the counters are cleared, P.hp has its size, and the workgroups fit the device.
+// H a multiple of 8, T of at least 1; the counters are cleared, P.hp has its size, and the workgroups fit the device.
 int zr_sweep_launch(zr_ctx* ctx, const LstmSweep& P, int tn);

@@ -9,16 +9,16 @@
 // refill of the operand pipeline from a cold start; the cell state never leaves registers.
 //
 // Eight waves: wave w has gate w % 4 and, of every 64 k, the first or second 32 (w / 4).  Its weights come from memory straight
-// into its registers, three steps of 64 k ahead and on into the next time step, and are split there: no other wave of the
+// into its registers, four steps of 64 k ahead and on into the next time step, and are split there: no other wave of the
 // workgroup needs them.  The activations' terms go through LDS: h is handed from node to node already split, 16-byte items of 8 k of one
 // term; embedding columns and h0 are split on their way in.  The two waves on a SIMD split and multiply in turn.  Twelve products of 32 k
 // are summed from zero before they reach the accumulator (short chains, one rounding at its size).
 // A loop over steps has no branch: waits for producers come before it or at the start of four steps, what lies past the end is
-// loaded as zero.  (With branches around loads the compiler waits for all of them at once: 3100 us for the 2600 below.)
+// loaded as zero.  (With branches around loads the compiler waits for all of them at once: the sweep named next took 3100 us.)
 //
-// Bound by the matrix cores' rate under load and the hand-overs: 4 layers of H = 1000, 128 columns, 50 steps 3258 -> 2487 us (fp32 matrix instructions
-// before), 409.6 GFLOP = 165 TFLOP/s, 0.99 PFLOP/s of bf16 work where large bf16 products reach 1.2 on this card; a steady step 48 us.  64
-// columns of it, 20 steps, 770 -> 705 (32-column tiles, whose weights are split for half the products).  Error of h against 64 bits, here and
+// Bound by the matrix cores' rate under load and the hand-overs: 4 layers of H = 1000, 128 columns, 50 steps 3250 us on the fp32 matrix instructions,
+// 2490 to 2710 here by the run, 2600 on average: 409.6 GFLOP = 158 TFLOP/s, 0.95 PFLOP/s of bf16 work where large bf16 products reach 1.2 on this card; a
+// steady step 49 to 52 us.  64 columns of it, 20 steps, 770 -> 705 (32-column tiles, whose weights are split for half the products).  Error of h against 64 bits, here and
 // with the fp32 instructions: H = 64 1.5e-7 / 1.6e-7, 512 1.9e-7 / 2.3e-7, 1000 2.1e-7 / 5.1e-7.
 //
 // Hand-over through memory: h is written twice, to the caller's array (plain stores, visible at kernel end) and as three terms
@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(512, 2) lstm_sweep_kernel(LstmSweep P) {
   zr_f32x4 ar[RING][4];
   // Segment 0: the input from below, 1: h of (l, t-1).  Layers above the first take the recurrent segment first: it only needs the layer's own
   // previous step, so a layer can trail the one below it by half a step instead of a whole one (the pipeline of layers fills and
-  // drains in half the time: 4 layers of H = 1000, 128 columns, 50 steps 2600 against 2655 us) and the wait for the layer below hides behind half a K loop.
+  // drains in half the time: 2 % of a sweep of 4 layers of H = 1000, 128 columns, 50 steps) and the wait for the layer below hides behind half a K loop.
   // The order is fixed per layer, so that no bit of the result depends on timing.
   auto seg_of = [&](int v) { return (v >= nit) != (l > 0) ? 1 : 0; };
   auto load_a = [&](zr_f32x4 (&a)[4], int v) {
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(512, 2) lstm_sweep_kernel(LstmSweep P) {
           split_a(a[2], a[3], x[1]);
         else
           split_a(next[0], next[1], x[0]);
-        // matrix instructions and the conversions in turn (left to the compiler: 2800 us for the 2600 below)
+        // matrix instructions and the conversions in turn (left to the compiler: 8 % slower)
 #pragma unroll
         for (int i = 0; i < 6 * TN; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);

@@ -270,7 +270,7 @@ inline int zr_attn_sum_parts(int mb) { return mb <= 512 ? 1 : (mb + 255) / 256; 
 // Estimated time, us: (steps of 32 k + what filling and the epilogue take) * a step of the workgroups that share a compute unit (one of four
 // waves alone; two of four or one of eight, whose matrix instructions fill it), times the rounds: within 11 % of 2700 measured
 // launches (V = 1000 .. 50000, H = 64 .. 1000, 33 to 1000 columns), and the choice is 4 % from the best tile on average.
-// Against the kernels before, the product alone, us: 50000 x 128 x 1000 123 -> 98, 192 columns 173 -> 125 (in turn with other kernels), 30011 x 33 x 500 30 ->
+// Against the kernels before, the product alone, us: 50000 x 128 x 1000 123 -> 89 to 92, 192 columns 173 -> 125 to 133, 30011 x 33 x 500 30 ->
 // 21, 33333 x 700 x 500 206 -> 171, 50000 x 128 x 333 79 -> 39, 16000 x 700 x 200 172 -> 53, 1000 x 64 x 64 8.9 -> 5.1.  Beyond 1024 columns the split product on the
 // plain matrix keeps what it takes, but for half-empty tiles: it has 256-column tiles and fewer conversions, and the estimate above does not know
 // the clock a launch of milliseconds runs at (50000 x 6400 x 1000 3.93 ms there, 4.09 here and 1.4 ms more inside a training
