@@ -1013,7 +1013,22 @@ int zr_lstm_node_backward(zr_ctx* ctx, const zr_lstm_train* layer, int mb, const
                                                             d_c_prev, d_mask01, d_err_above, d_err_h_next,
                                                             d_err_c_next, d_err_c_prev, H, mb, d_dgates);
   ZR_LAUNCH_CHECK("lstm_node_backward_kernel");
-  // the two error products share their right-hand side: one batched launch
+  // the two error products share their right-hand side: one batched launch, straight to where the caller wants the results -- but through
+  // scratch where these overlap each other (d_err_below then wins) or d_dgates, which the launch reads
+  const size_t n = (size_t)H * mb;
+  auto apart = [](const float* a, size_t na, const float* b, size_t nb) {
+    return (uintptr_t)(a + na) <= (uintptr_t)b || (uintptr_t)(b + nb) <= (uintptr_t)a;
+  };
+  const bool direct = apart(d_err_h_prev, n, d_dgates, 4 * n) &&
+                      (!d_err_below || (apart(d_err_below, n, d_err_h_prev, n) && apart(d_err_below, n, d_dgates, 4 * n)));
+  float *to_h = d_err_h_prev, *to_below = d_err_below;
+  if (!direct) {
+    void* scratch = nullptr;
+    rc = zr_ctx_scratch(ctx, 1, sizeof(float) * 2 * n, &scratch);
+    if (rc) return rc;
+    to_h = (float*)scratch;
+    if (d_err_below) to_below = to_h + n;
+  }
   ZrGemmDesc g = {};
   g.M = H;
   g.N = mb;
@@ -1026,12 +1041,16 @@ int zr_lstm_node_backward(zr_ctx* ctx, const zr_lstm_train* layer, int mb, const
   g.strideA = 4LL * H * H;
   g.B[0] = d_dgates;
   g.ldb[0] = 4 * H;
-  g.C = d_err_h_prev;
+  g.C = to_h;
   g.ldc = H;
   g.batch = d_err_below ? 2 : 1;
-  g.strideC = d_err_below ? float_offset(d_err_h_prev, d_err_below) : 0;
+  g.strideC = d_err_below ? float_offset(to_h, to_below) : 0;
   g.epilogue = ZR_EPI_STORE;
-  return zr_gemm_launch(ctx, g);
+  rc = zr_gemm_launch(ctx, g);
+  if (rc || direct) return rc;
+  ZR_HIP(hipMemcpyAsync(d_err_h_prev, to_h, sizeof(float) * n, hipMemcpyDeviceToDevice, ctx->stream));
+  if (d_err_below) ZR_HIP(hipMemcpyAsync(d_err_below, to_below, sizeof(float) * n, hipMemcpyDeviceToDevice, ctx->stream));
+  return ZR_OK;
 }
 
 int zr_attn_set_error_tables(zr_ctx* ctx, zr_attn* a, float* const* h_err_tables, int n) {
