@@ -91,36 +91,77 @@ softmax_error_kernel(float* __restrict__ x, int V, int n, int cols, const float*
   *(vec*)(sums + (size_t)blockIdx.y * V + v) = s;
 }
 
-// Double-precision column statistics straight from the logits (outputdist_perplexity_kernel accumulates in
-// double, reference: src/custom_kernels.h:583-660).  One workgroup per column, two passes over the column.
-__global__ void __launch_bounds__(256)
-softmax_colstats_f64_kernel(const float* __restrict__ logits, int V, double* __restrict__ colstats) {
-  __shared__ double s[256];
-  const int n = blockIdx.x;
-  const int tid = threadIdx.x;
+// Double-precision column statistics (outputdist_perplexity_kernel accumulates in double, reference:
+// src/custom_kernels.h:583-660).  The column's largest logit comes from the product's block pairs, whose maxima are of the
+// very values it stored, so the logits are read once, and are on their way while the pairs are folded.  gridDim.y workgroups
+// share a column: one (colstats = max, log sum) unless the columns alone would leave compute units idle; of several each
+// leaves its part of the sum in sums[column][part].
+// Bound by the logits' way from memory and the 64-bit exponentials together.  700 columns of 33333: 89 us with two passes of
+// single loads by 256 threads, 32 us so.
+constexpr int kF64Threads = 512;
+__global__ void __launch_bounds__(kF64Threads)
+softmax_colstats_f64_kernel(const float* __restrict__ logits, int V, const float* __restrict__ pairs, int nblocks, double* __restrict__ colstats,
+                            double* __restrict__ sums) {
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  constexpr int WAVES = kF64Threads / 64, U = 4, SPAN = 4 * kF64Threads;
+  __shared__ float s_m[WAVES];
+  __shared__ double s_s[WAVES];
+  const int n = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float* x = logits + (size_t)n * V;
-  double mx = -1.7976931348623157e308;
-  for (int i = tid; i < V; i += 256) mx = fmax(mx, (double)x[i]);
-  s[tid] = mx;
+  const int share = (V / 4 + (int)gridDim.y - 1) / (int)gridDim.y * 4;  // the last workgroup also takes the V % 4 left over
+  const int begin = min((int)blockIdx.y * share, V), end = blockIdx.y + 1 == gridDim.y ? V : min(begin + share, V);
+  f32x4u v[U];
+  auto load = [&](int at) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = at + 4 * tid + SPAN * u;
+      v[u] = f32x4u{-INFINITY, -INFINITY, -INFINITY, -INFINITY};  // adds exp(-inf) = 0
+      if (i + 4 <= end) {
+        v[u] = *(const f32x4u*)(x + i);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (i + e < end) v[u][e] = x[i + e];
+      }
+    }
+  };
+  load(begin);
+  float m = -INFINITY;
+  const f32x2* pp = (const f32x2*)(pairs + (size_t)n * nblocks * 2);
+  for (int b = tid; b < nblocks; b += kF64Threads) m = fmaxf(m, pp[b].x);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  if (lane == 0) s_m[wave] = m;
   __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st) s[tid] = fmax(s[tid], s[tid + st]);
-    __syncthreads();
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) m = fmaxf(m, s_m[w]);
+  const double mx = fmax(-1.7976931348623157e308, (double)m);
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int at = begin; at < end; at += SPAN * U) {
+    f32x4u now[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) now[u] = v[u];
+    if (at + SPAN * U < end) load(at + SPAN * U);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[e] += exp((double)now[u][e] - mx);
   }
-  mx = s[0];
+  double total = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off, 64);
+  if (lane == 0) s_s[wave] = total;
   __syncthreads();
-  double sum = 0.0;
-  for (int i = tid; i < V; i += 256) sum += exp((double)x[i] - mx);
-  s[tid] = sum;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st) s[tid] += s[tid + st];
-    __syncthreads();
-  }
-  if (tid == 0) {
-    colstats[2 * n] = mx;
-    colstats[2 * n + 1] = log(s[0]);
-  }
+  if (tid != 0) return;
+  total = 0.0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) total += s_s[w];
+  if (blockIdx.y == 0) colstats[2 * n] = mx;
+  if (gridDim.y == 1)
+    colstats[2 * n + 1] = log(total);
+  else
+    sums[(size_t)n * gridDim.y + blockIdx.y] = total;
 }
 
 __global__ void __launch_bounds__(256)
@@ -131,9 +172,10 @@ softmax_logprob_f64_kernel(const float* __restrict__ logits, double* __restrict_
   if (i < V) out[(size_t)n * V + i] = ((double)logits[(size_t)n * V + i] - colstats[2 * n]) - colstats[2 * n + 1];
 }
 
-// loss = sum over unmasked columns of log p[target[b], b]; single workgroup, fixed summation order.
+// loss = sum over unmasked columns of log p[target[b], b]; single workgroup, fixed summation order.  parts: workgroups of
+// softmax_colstats_f64_kernel that shared a column.
 __global__ void __launch_bounds__(256)
-softmax_loss_kernel(const float* __restrict__ logits, int V, int mb, const double* __restrict__ colstats,
+softmax_loss_kernel(const float* __restrict__ logits, int V, int mb, const double* __restrict__ colstats, const double* __restrict__ sums, int parts,
                     const int* __restrict__ target, const int* __restrict__ mask01, double* __restrict__ loss,
                     int* __restrict__ flags) {
   __shared__ double s[256];
@@ -146,7 +188,13 @@ softmax_loss_kernel(const float* __restrict__ logits, int V, int mb, const doubl
         atomicAdd(&flags[0], 1);
         t = t < 0 ? 0 : V - 1;
       }
-      acc += ((double)logits[(size_t)b * V + t] - colstats[2 * b]) - colstats[2 * b + 1];
+      double lsum = colstats[2 * b + 1];
+      if (parts > 1) {
+        lsum = 0.0;
+        for (int q = 0; q < parts; ++q) lsum += sums[(size_t)b * parts + q];
+        lsum = log(lsum);
+      }
+      acc += ((double)logits[(size_t)b * V + t] - colstats[2 * b]) - lsum;
     }
   }
   s[tid] = acc;
@@ -442,7 +490,7 @@ int zr_softmax_logprob_f64(zr_ctx* ctx, const float* d_D, const float* d_b_d, in
   rc = logits_with_partials(ctx, d_D, d_b_d, V, H, d_h, mb, d_logits_scratch, &partials, &nblocks);
   if (rc) return rc;
   double* colstats = (double*)stats_ptr(partials, nblocks, mb);
-  softmax_colstats_f64_kernel<<<mb, 256, 0, ctx->stream>>>(d_logits_scratch, V, colstats);
+  softmax_colstats_f64_kernel<<<mb, kF64Threads, 0, ctx->stream>>>(d_logits_scratch, V, partials, nblocks, colstats, nullptr);
   ZR_LAUNCH_CHECK("softmax_colstats_f64_kernel");
   dim3 grid((V + 255) / 256, mb);
   softmax_logprob_f64_kernel<<<grid, 256, 0, ctx->stream>>>(d_logits_scratch, d_logp, V, colstats);
@@ -462,11 +510,20 @@ int zr_softmax_loss(zr_ctx* ctx, const float* d_D, const float* d_b_d, int V, in
   rc = logits_with_partials(ctx, d_D, d_b_d, V, H, d_h, mb, d_logits_scratch, &partials, &nblocks);
   if (rc) return rc;
   double* colstats = (double*)stats_ptr(partials, nblocks, mb);
-  softmax_colstats_f64_kernel<<<mb, 256, 0, ctx->stream>>>(d_logits_scratch, V, colstats);
+  // enough workgroups for two a compute unit, each with at least one round of loads
+  int parts = (2 * ctx->cu_count + mb - 1) / mb;
+  const int rounds = V / (4 * kF64Threads * 4);
+  parts = parts < rounds ? parts : rounds;
+  parts = parts > 16 ? 16 : (parts < 1 ? 1 : parts);
+  void* sums = nullptr;
+  if (parts > 1) {  // (the product is done with this buffer)
+    if (zr_ctx_scratch(ctx, 0, sizeof(double) * (size_t)parts * mb, &sums) != ZR_OK) parts = 1;
+  }
+  softmax_colstats_f64_kernel<<<dim3(mb, parts), kF64Threads, 0, ctx->stream>>>(d_logits_scratch, V, partials, nblocks, colstats, (double*)sums);
   ZR_LAUNCH_CHECK("softmax_colstats_f64_kernel");
   // the loss cell lives in the partials area, which is dead once the column stats exist
   double* d_loss = (double*)partials;
-  softmax_loss_kernel<<<1, 256, 0, ctx->stream>>>(d_logits_scratch, V, mb, colstats, d_target, d_mask01, d_loss,
+  softmax_loss_kernel<<<1, 256, 0, ctx->stream>>>(d_logits_scratch, V, mb, colstats, (const double*)sums, parts, d_target, d_mask01, d_loss,
                                                   ctx->d_flags);
   ZR_LAUNCH_CHECK("softmax_loss_kernel");
   ZR_HIP(hipMemcpyAsync(h_loss, d_loss, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
