@@ -262,6 +262,12 @@ int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const flo
                       int V, const float* d_cprev, const int* d_mask01, float clip, int mb, float* d_h, float* d_c,
                       float* const d_gates[4], float* d_hp, int shape);
 
+// The same on bf16 weights (zr_lstm_rows_bf16.hip): every segment's input as bf16 terms, k-interleaved by 8 (lo[0] null: one term); out_hi / out_lo: h
+// in that form too (null: not wanted).
+int zr_lstm_rows_bf16_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const unsigned short* const hi[3], const unsigned short* const lo[3],
+                           const float* d_cprev, const int* d_mask01, float clip, int mb, float* d_h, float* d_c, float* const d_gates[4],
+                           unsigned short* out_hi, unsigned short* out_lo, int shape);
+
 // The attention step in one launch (zr_attn_step.hip).  a->d_hpack must hold h_t k-interleaved.  *took = 0: the
 // conditions do not hold and nothing was launched (the caller goes on with one launch per stage).
 struct zr_attn;

@@ -1334,6 +1334,12 @@ static int lstm_step_impl(zr_ctx* ctx, const zr_lstm_weights* w, const float* d_
       return zr_lstm_rows_step(ctx, w, nseg, U.in, d_gather_ids, V, d_cprev, d_mask01, clip_threshold, mb, d_h, d_c,
                                d_gates, U.hp, shape);
   }
+  if (w->bf16 && vec && !ctx->lstm_kernel && !ctx->lstm_tn && !ctx->lstm_ksplit && !ctx->lstm_kparts) {
+    const int shape = zr_lstm_rows_bf16_shape(H, mb, ctx->cu_count);
+    if (shape >= 0)
+      return zr_lstm_rows_bf16_step(ctx, w, nseg, (const unsigned short* const*)U.inp, U.inp_lo, d_cprev, d_mask01, clip_threshold, mb, d_h, d_c,
+                                    d_gates, U.hsplit_hi, U.hsplit_lo, shape);
+  }
   return launch_fused(ctx, L, vec);
 }
 

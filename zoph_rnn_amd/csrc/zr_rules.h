@@ -67,6 +67,21 @@ inline int zr_lstm_rows_shape(int H, int mb, int nseg, bool vec, int cus) {
   return rounds * (4.0 + 0.0115 * H * nseg) < zr_fused_us(1, H, mb, nseg, vec, cus) ? 3 : -1;
 }
 
+// The same for a node on bf16 weights (zr_lstm_rows_bf16.hip against lstm_fused_kernel's 32-row tiles); shapes 1 to 3 as above.  us of a
+// node, two terms (one term), in a decoder step of four layers: H = 512, 64 columns 12.1 -> 6.2 on 8 x 32 tiles (10.7 -> 5.2), 1024, 12
+// columns 15.4 -> 7.9 (14.2 -> 7.1), 1024, 64 17.3 -> 9.6, 1024, 128 17.2 -> 13.7 on 8 x 64, 2000, 64 35.0 -> 30.0.  Any of the tiles wins while its
+// workgroups are within one a compute unit, the narrowest the most; 8 x 16 against 8 x 32 only where it fills more of the chip (1024, 32 columns
+// 8.1 / 9.5; 512, 37 6.1 / 6.0).  In a second round the activations, which every row tile reads, are too much: 1024, 192 columns 17.5 against
+// 21.6 and 24.0, 768, 192 14.3 / 18.2; but for three 32-column tiles where 64-column ones are two rounds as well, 1104, 80 columns 16.4 / 14.2.
+inline int zr_lstm_rows_bf16_shape(int H, int mb, int cus) {
+  const long long rows = H / 8;
+  if (4LL * H * ((H + 31) / 32 * 32) >= 1LL << 31 || 8LL * H * mb >= 1LL << 31) return -1;  // 32-bit offsets
+  if (H > 512 && mb > 16 && rows * ((mb + 15) / 16) <= cus) return 1;
+  if (rows * ((mb + 31) / 32) <= cus) return 2;
+  if (rows * ((mb + 63) / 64) <= cus) return 3;
+  return mb > 64 && mb <= 96 && 4 * rows * 3 <= 7LL * cus ? 2 : -1;
+}
+
 // ---- the sweep of a stack (zr_lstm_stack_forward): one launch per diagonal, one launch with streamed weights
 // (lstm_sweep_kernel), or with its weights in registers (lstm_resident_kernel).  Estimates in us; the least one is taken.
 // Against 1812 sizes (H = 64 .. 2000, 1 to 4 layers, 1 to 256 columns, 12 and 50 steps; all that fit measured for each) the
