@@ -286,7 +286,6 @@ __global__ void __launch_bounds__(256)
 beam_select_blocks_kernel(const float* __restrict__ logits, const float* __restrict__ blocks, int V, int K, int nblocks,
                           float* __restrict__ cand_p, int* __restrict__ cand_w, float* __restrict__ colstats_out) {
   __shared__ float s_m[4], s_s[4];
-  __shared__ float s_stats[2];
   __shared__ unsigned s_tau_wave[4];
   __shared__ int s_blk[kSelBlockCap];
   __shared__ unsigned long long s_cand[kSelCandCap];
@@ -298,13 +297,11 @@ beam_select_blocks_kernel(const float* __restrict__ logits, const float* __restr
   const float* x = logits + (size_t)col * V;
   const float* pairs = blocks + (size_t)col * nblocks * 2;
   if (tid == 0) s_nblk = 0, s_count = 0;
-  float mx, sum, bm;
-  zr_softmax_fold_column(pairs, nblocks, s_m, s_s, mx, sum, &bm);
+  float c_max, c_sum;
+  const float bm = zr_softmax_fold_column(pairs, nblocks, s_m, s_s, c_max, c_sum, [] {});
   if (tid == 0) {
-    s_stats[0] = mx;
-    s_stats[1] = sum;
-    colstats_out[2 * col] = mx;
-    colstats_out[2 * col + 1] = sum;
+    colstats_out[2 * col] = c_max;
+    colstats_out[2 * col + 1] = c_sum;
   }
   // the bound: K-th largest thread value inside each wave (bitonic sort of the 64 lanes), largest of the four waves
   {
@@ -320,7 +317,6 @@ beam_select_blocks_kernel(const float* __restrict__ logits, const float* __restr
     if (lane == K - 1) s_tau_wave[wave] = v;
   }
   __syncthreads();
-  const float c_max = s_stats[0], c_sum = s_stats[1];
   unsigned tu = s_tau_wave[0];
 #pragma unroll
   for (int w = 1; w < 4; ++w) tu = s_tau_wave[w] > tu ? s_tau_wave[w] : tu;

@@ -151,6 +151,21 @@ inline ZrResidentPlan zr_sweep_resident_plan(int nl, int H, int mb, int T, const
   return plan;
 }
 
+// ---- normalising the output matrix (softmax_normalize_kernel): 16-byte accesses a thread, and whether its workgroups fold the block pairs
+
+// Every workgroup folds its column's V / 32 pairs: cheaper than a launch for it until there are some 2.5 million to fold, us folding /
+// in two launches: 30001 x 256 (1.9) 14.4 / 15.5, 50000 x 128 (2.6 with four accesses) 15.0 / 15.2, 80000 x 64 (3.2) 14.4 / 13.4, 10000 x 3000 (2.8) 44 / 41, 50000
+// x 256 (5.2) 20.9 / 20.5.  Two accesses a thread, 40000 x 64 10.2 against 10.8 with four; four where columns start at odd
+// addresses: 30011 x 37 5.6 against 6.4.
+struct ZrNormalizePlan {
+  int accesses;
+  bool fold;
+};
+inline ZrNormalizePlan zr_softmax_normalize_plan(int V, int n) {
+  if ((double)((V + 4095) / 4096) * n * ((V + 31) / 32) > 2.7e6) return {2, false};
+  return {V <= 1024 ? 1 : (V % 4 ? 4 : 2), true};
+}
+
 // ---- the output layer's error pass (softmax_error_kernel): columns a workgroup adds up, one after another
 
 // 32 keep the partial sums of the bias gradient small against the matrix.  Fewer where 1024-row blocks of 32 columns would

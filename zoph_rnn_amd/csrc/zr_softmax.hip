@@ -14,46 +14,64 @@ softmax_colstats_kernel(const float* __restrict__ partials, int nblocks, float* 
   __shared__ float s_m[4], s_s[4];
   const int n = blockIdx.x;
   float mx, sum;
-  zr_softmax_fold_column(partials + (size_t)n * nblocks * 2, nblocks, s_m, s_s, mx, sum, nullptr);
+  zr_softmax_fold_column(partials + (size_t)n * nblocks * 2, nblocks, s_m, s_s, mx, sum, [] {});
   if (threadIdx.x == 0) {
     colstats[2 * n] = mx;
     colstats[2 * n + 1] = sum;
   }
 }
 
-// out = exp(x - max) / sum   (MODE 0)   or   (x - max) - log(sum)   (MODE 1).  16-byte accesses when VEC.  One access
-// per thread: four per thread, loaded before the first is used, measured slower (11.1 against 9.4 us at 50000 x 128).
-template <int MODE, bool VEC>
+// out = exp(x - max) / sum   (MODE 0)   or   (x - max) - log(sum)   (MODE 1); in and out may be the same matrix.  A
+// workgroup takes 1024 * U rows of one column, U 16-byte accesses a thread at any alignment.  FOLD: it folds the column's block pairs itself,
+// while its logits are on their way, which saves the launch of softmax_colstats_kernel; else `pairs` holds that one's statistics.
+// Both launches before / this one, us: 10000 x 8 6.0 -> 3.9, 30011 x 37 (odd columns had 4-byte accesses) 8.9 -> 5.6, 40000 x 64 11.4 ->
+// 10.2, 50000 x 128 16.1 -> 15.0.  Bound by memory from there on, with the statistics in a launch of their own: 80000 x 256 30 us, the fold
+// by every workgroup 34; 80001 x 256 41.7 -> 29.8 by the accesses' width.
+template <int MODE, int U, bool FOLD>
 __global__ void __launch_bounds__(256)
-softmax_normalize_kernel(const float* in, float* out, int V, const float* __restrict__ colstats) {
+softmax_normalize_kernel(const float* in, float* out, int V, const float* __restrict__ pairs, int nblocks) {
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  __shared__ float s_m[4], s_s[4];
   const int n = blockIdx.y;
-  const float mx = colstats[2 * n];
-  const float sum = colstats[2 * n + 1];
-  const float lsum = logf(sum);
   const float* x = in + (size_t)n * V;
   float* y = out + (size_t)n * V;
-  if (VEC) {
-    const int i4 = blockIdx.x * 256 + threadIdx.x;
-    if (i4 * 4 < V) {
-      zr_f32x4 v = ((const zr_f32x4*)x)[i4];
-      zr_f32x4 r;
-      if (MODE == 0) {
-        // expf(x - max) / sum, as the reference divides (custom_kernels.h:574-576)
-        r.x = expf(v.x - mx) / sum;
-        r.y = expf(v.y - mx) / sum;
-        r.z = expf(v.z - mx) / sum;
-        r.w = expf(v.w - mx) / sum;
+  const int first = (blockIdx.x * U * 256 + threadIdx.x) * 4;
+  f32x4u v[U];
+  auto load = [&] {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = first + 1024 * u;
+      if (i + 4 <= V) {
+        v[u] = *(const f32x4u*)(x + i);
       } else {
-        r.x = (v.x - mx) - lsum;
-        r.y = (v.y - mx) - lsum;
-        r.z = (v.z - mx) - lsum;
-        r.w = (v.w - mx) - lsum;
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (i + e < V) v[u][e] = x[i + e];
       }
-      ((zr_f32x4*)y)[i4] = r;
     }
+  };
+  float mx, sum;
+  if constexpr (FOLD) {
+    zr_softmax_fold_column(pairs + (size_t)n * nblocks * 2, nblocks, s_m, s_s, mx, sum, load);
   } else {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < V) y[i] = (MODE == 0) ? expf(x[i] - mx) / sum : (x[i] - mx) - lsum;
+    mx = pairs[2 * n], sum = pairs[2 * n + 1];
+    load();
+  }
+  const float lsum = MODE == 1 ? logf(sum) : 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = first + 1024 * u;
+    f32x4u r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)  // expf(x - max) / sum, as the reference divides (custom_kernels.h:574-576)
+      r[e] = MODE == 0 ? expf(v[u][e] - mx) / sum : (v[u][e] - mx) - lsum;
+    if (i + 4 <= V) {
+      *(f32x4u*)(y + i) = r;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (i + e < V) y[i + e] = r[e];
+    }
   }
 }
 
@@ -204,6 +222,25 @@ softmax_loss_kernel(const float* __restrict__ logits, int V, int mb, const doubl
     __syncthreads();
   }
   if (tid == 0) loss[0] = s[0];
+}
+
+template <int MODE>
+int launch_normalize(zr_ctx* ctx, const float* in, float* out, int V, int mb, const float* pairs, int nblocks, float* colstats) {
+  const ZrNormalizePlan plan = zr_softmax_normalize_plan(V, mb);
+  const dim3 grid((V + 1024 * plan.accesses - 1) / (1024 * plan.accesses), mb);
+  if (!plan.fold) {
+    const int rc = zr_softmax_colstats_launch(ctx, pairs, nblocks, mb, colstats);
+    if (rc) return rc;
+    softmax_normalize_kernel<MODE, 2, false><<<grid, 256, 0, ctx->stream>>>(in, out, V, colstats, nblocks);
+  } else if (plan.accesses == 1) {
+    softmax_normalize_kernel<MODE, 1, true><<<grid, 256, 0, ctx->stream>>>(in, out, V, pairs, nblocks);
+  } else if (plan.accesses == 2) {
+    softmax_normalize_kernel<MODE, 2, true><<<grid, 256, 0, ctx->stream>>>(in, out, V, pairs, nblocks);
+  } else {
+    softmax_normalize_kernel<MODE, 4, true><<<grid, 256, 0, ctx->stream>>>(in, out, V, pairs, nblocks);
+  }
+  ZR_LAUNCH_CHECK("softmax_normalize_kernel");
+  return ZR_OK;
 }
 
 // d_h_packed: optional k-interleaved copy of d_h ([H/4][mb][4]); used when the product runs on the registered fp32 copy
@@ -409,28 +446,14 @@ int zr_softmax_forward_packed(zr_ctx* ctx, const float* d_D, const float* d_b_d,
                             with_blocks ? d_out + zr_softmax_blocks_offset_floats(V, mb) : nullptr);
   if (rc) return rc;
   if (with_blocks) return ZR_OK;
-  // ZR_SOFTMAX_LOGITS: the column statistics go behind the logits in the caller's buffer and no normalised matrix is
-  // written -- a consumer that needs only a few entries per column (the beam search) normalises those itself
-  float* colstats = logits_only ? d_out + (size_t)V * mb : (float*)stats_ptr(partials, nblocks, mb);
-  softmax_colstats_kernel<<<mb, 256, 0, ctx->stream>>>(partials, nblocks, colstats);
-  ZR_LAUNCH_CHECK("softmax_colstats_kernel");
-  if (logits_only) return ZR_OK;
-  const bool vec = (V % 4 == 0) && (((uintptr_t)logits & 15u) == 0) && (((uintptr_t)d_out & 15u) == 0);
-  if (vec) {
-    dim3 grid((V / 4 + 255) / 256, mb);
-    if (mode == ZR_SOFTMAX_PROB)
-      softmax_normalize_kernel<0, true><<<grid, 256, 0, ctx->stream>>>(logits, d_out, V, colstats);
-    else
-      softmax_normalize_kernel<1, true><<<grid, 256, 0, ctx->stream>>>(logits, d_out, V, colstats);
-  } else {
-    dim3 grid((V + 255) / 256, mb);
-    if (mode == ZR_SOFTMAX_PROB)
-      softmax_normalize_kernel<0, false><<<grid, 256, 0, ctx->stream>>>(logits, d_out, V, colstats);
-    else
-      softmax_normalize_kernel<1, false><<<grid, 256, 0, ctx->stream>>>(logits, d_out, V, colstats);
+  if (logits_only) {
+    // ZR_SOFTMAX_LOGITS: the column statistics go behind the logits in the caller's buffer and no normalised matrix is
+    // written -- a consumer that needs only a few entries per column (the beam search) normalises those itself
+    return zr_softmax_colstats_launch(ctx, partials, nblocks, mb, d_out + (size_t)V * mb);
   }
-  ZR_LAUNCH_CHECK("softmax_normalize_kernel");
-  return ZR_OK;
+  float* colstats = (float*)stats_ptr(partials, nblocks, mb);
+  return mode == ZR_SOFTMAX_PROB ? launch_normalize<0>(ctx, logits, d_out, V, mb, partials, nblocks, colstats)
+                                 : launch_normalize<1>(ctx, logits, d_out, V, mb, partials, nblocks, colstats);
 }
 
 int zr_softmax_error_chunks(int V, int n) { return (n + zr_softmax_error_cols(V, n) - 1) / zr_softmax_error_cols(V, n); }
