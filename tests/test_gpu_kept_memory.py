@@ -1,0 +1,112 @@
+"""Device memory that a context keeps from destroyed handles and zr_free (csrc/zr_runtime.hip): reuse in stream order, the errors there were, and
+nothing kept where another context or a caller's stream could still use a block."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import Layer
+from zoph_rnn_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def ctx():
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+def raw_free(ctx, ptr):
+    return capi.load().zr_free(ctx.h, ctypes.c_void_p(ptr))
+
+
+def test_a_freed_block_is_handed_out_again_and_freeing_it_twice_is_an_error(ctx):
+    a = ctx.zeros((1 << 20,))
+    ptr = a.ptr
+    a.free()
+    assert raw_free(ctx, ptr) != 0
+    b = ctx.empty((1 << 20,))
+    assert b.ptr == ptr
+    small = ctx.empty((1000,))
+    assert small.ptr != ptr
+    b.free()
+
+
+def test_weights_packed_again_while_the_old_ones_are_in_use(ctx):
+    """A training loop's pack: the new weights' block is the old one's, which a queued sweep still reads."""
+    H, mb, T, V, L = 200, 24, 40, 64, 2
+    cfgs = [synth.encoder_config(H=H, mb=mb, T=T, V=V, L=L) for _ in range(2)]
+    g = synth.rng(900, 1)
+    for ly in cfgs[1]["layers"]:
+        for k in ("M", "Wh"):
+            ly[k] = [np.asfortranarray(synth.uniform(g, (H, H))) for _ in range(4)]
+    embed, ids = ctx.array(cfgs[0]["embed"]), ctx.array(np.abs(cfgs[0]["ids"]).reshape(-1).astype(np.int32))
+    ones, z = ctx.array(np.ones(mb * T, np.int32)), ctx.zeros((H, mb))
+    mats = [[Layer(ctx, ly) for ly in c["layers"]] for c in cfgs]  # (matrices on the device; packed again below)
+
+    def pack(which):
+        return [ctx.lstm_pack(ly.M, ly.Wh, ly.b, H) for ly in mats[which]]
+
+    def sweep(w, h, c):
+        ctx.lstm_stack_forward(w, embed, V, ids, ones, T, mb, [z] * L, [z] * L, h, c)
+
+    def buffers():
+        return [ctx.empty((H * mb * T,)) for _ in range(L)], [ctx.empty((H * mb * T,)) for _ in range(L)]
+
+    want = []
+    for which in (0, 1):
+        w, (h, c) = pack(which), buffers()
+        sweep(w, h, c)
+        ctx.sync()
+        want.append([a.get() for a in h + c])
+        for x in w:
+            ctx.lstm_weights_destroy(x)
+    assert not np.array_equal(want[0][-1], want[1][-1])
+    outs = [buffers() for _ in range(8)]
+    w = pack(0)
+    for i, (h, c) in enumerate(outs):  # no wait in between
+        sweep(w, h, c)
+        for x in w:
+            ctx.lstm_weights_destroy(x)
+        w = pack((i + 1) % 2)
+    ctx.sync()
+    for i, (h, c) in enumerate(outs):
+        for a, b in zip(h + c, want[i % 2]):
+            assert np.array_equal(a.get(), b)
+    for x in w + [ly.w for m in mats for ly in m]:
+        ctx.lstm_weights_destroy(x)
+
+
+def test_beyond_the_bound_blocks_are_given_back(ctx):
+    """Freeing 80 blocks of 24 MiB keeps at most 512 MiB of them."""
+    blocks = [ctx.empty((6 << 20,)) for _ in range(80)]
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    for b in blocks:
+        b.free()
+    given_back = torch.cuda.mem_get_info()[0] - before
+    assert given_back >= 80 * (24 << 20) - (512 << 20) - (64 << 20)
+
+
+def test_nothing_is_kept_with_another_context_or_stream(ctx):
+    a = ctx.empty((12 << 20,))
+    other = capi.Context(0)
+    before = torch.cuda.mem_get_info()[0]
+    a.free()
+    assert torch.cuda.mem_get_info()[0] - before >= 40 << 20
+    other.close()
+    b = ctx.empty((12 << 20,))
+    b.free()  # kept now
+    before = torch.cuda.mem_get_info()[0]
+    s = torch.cuda.Stream()
+    capi._chk(capi.load().zr_ctx_set_stream(ctx.h, ctypes.c_void_p(s.cuda_stream)))
+    assert torch.cuda.mem_get_info()[0] - before >= 40 << 20
+    c = ctx.empty((12 << 20,))
+    before = torch.cuda.mem_get_info()[0]
+    c.free()
+    assert torch.cuda.mem_get_info()[0] - before >= 40 << 20
+    ctx.sync()
+    capi._chk(capi.load().zr_ctx_set_stream(ctx.h, None))

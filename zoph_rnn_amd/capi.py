@@ -63,6 +63,8 @@ SYMBOLS = [
     "zr_attn_backward", "zr_dropout_apply", "zr_uniform_fill", "zr_add_inplace",
 ]
 
+MAX_MULTI = 32  # arrays of one zr_gather_columns_multi call
+
 _lib = None
 
 

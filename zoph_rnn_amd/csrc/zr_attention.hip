@@ -605,9 +605,8 @@ int zr_attn_create(zr_ctx* ctx, int H, int mb, int D, const float* d_W_a, const 
   const size_t tbytes = (sizeof(float*) * longest_sent + 255) & ~(size_t)255;
   const size_t fbytes = sizeof(float) * (3 * n + W * mb + mb);
   const size_t fpad = (fbytes + 255) & ~(size_t)255;
-  char* base = nullptr;
-  if (hipMalloc((void**)&base, tbytes + fpad + sizeof(int) * W * mb) != hipSuccess) {
-    (void)hipGetLastError();
+  char* base = (char*)zr_dev_alloc(ctx, tbytes + fpad + sizeof(int) * W * mb);
+  if (!base) {
     delete a;
     return zr_set_error(ZR_ENOMEM, "zr_attn_create: allocation failed");
   }
@@ -619,9 +618,11 @@ int zr_attn_create(zr_ctx* ctx, int H, int mb, int D, const float* d_W_a, const 
   a->d_align = f + 3 * n;
   a->d_pt = f + 3 * n + W * mb;
   a->d_idx = (int*)(base + tbytes + fpad);
-  hipError_t e = hipMemcpy((void*)a->d_table, h_hs_table, sizeof(float*) * longest_sent, hipMemcpyHostToDevice);
+  // (on the stream: what a kept block was last used for may still be queued there)
+  hipError_t e = hipMemcpyAsync((void*)a->d_table, h_hs_table, sizeof(float*) * longest_sent, hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
-    (void)hipFree(base);
+    (void)zr_dev_free(ctx, base);
     delete a;
     return zr_set_error(ZR_EHIP, "zr_attn_create: table upload failed: %s", hipGetErrorString(e));
   }
@@ -639,11 +640,8 @@ int zr_attn_use_bf16_weights(zr_ctx* ctx, zr_attn* a) {
   const size_t per = (size_t)H * ldp;
   if (!a->d_bf16) {
     // the four matrices, then room for h_t as two bf16 terms (split once per step for its three products)
-    if (hipMalloc((void**)&a->d_bf16, sizeof(unsigned short) * (4 * per + 6 * (size_t)H * a->mb)) != hipSuccess) {
-      (void)hipGetLastError();
-      a->d_bf16 = nullptr;
-      return zr_set_error(ZR_ENOMEM, "zr_attn_use_bf16_weights: allocation failed");
-    }
+    a->d_bf16 = (unsigned short*)zr_dev_alloc(ctx, sizeof(unsigned short) * (4 * per + 6 * (size_t)H * a->mb));
+    if (!a->d_bf16) return zr_set_error(ZR_ENOMEM, "zr_attn_use_bf16_weights: allocation failed");
   }
   a->ldp = ldp;
   const float* src[4] = {a->W_p, a->W_a, a->W_c1, a->W_c2};
@@ -693,12 +691,8 @@ int zr_attn_prepare(zr_ctx* ctx, zr_attn* a) {
   const int ldp = (H + 31) / 32 * 32, kp = (H + 7) / 8 * 8;
   const size_t per = (size_t)kp * ldp;
   if (!a->d_pack32) {
-    if (hipMalloc((void**)&a->d_pack32, sizeof(float) * (4 * per + 3 * (size_t)H * a->mb + 3 * (size_t)ldp * a->mb + 32)) !=
-        hipSuccess) {
-      (void)hipGetLastError();
-      a->d_pack32 = nullptr;
-      return zr_set_error(ZR_ENOMEM, "zr_attn_prepare: allocation failed");
-    }
+    a->d_pack32 = (float*)zr_dev_alloc(ctx, sizeof(float) * (4 * per + 3 * (size_t)H * a->mb + 3 * (size_t)ldp * a->mb + 32));
+    if (!a->d_pack32) return zr_set_error(ZR_ENOMEM, "zr_attn_prepare: allocation failed");
   }
   a->ldp32 = ldp;
   a->kp32 = kp;
@@ -722,11 +716,10 @@ int zr_attn_destroy(zr_ctx* ctx, zr_attn* a) {
   if (!a) return ZR_OK;
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
-  ZR_HIP(hipStreamSynchronize(ctx->stream));
-  if (a->d_bf16) (void)hipFree(a->d_bf16);
-  if (a->d_pack32) (void)hipFree(a->d_pack32);
-  if (a->d_err_table) (void)hipFree((void*)a->d_err_table);
-  (void)hipFree((void*)a->d_table);
+  (void)zr_dev_free(ctx, a->d_bf16);
+  (void)zr_dev_free(ctx, a->d_pack32);
+  (void)zr_dev_free(ctx, (void*)a->d_err_table);
+  (void)zr_dev_free(ctx, (void*)a->d_table);
   delete a;
   return ZR_OK;
 }

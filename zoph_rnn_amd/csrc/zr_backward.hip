@@ -744,15 +744,14 @@ int zr_lstm_train_create(zr_ctx* ctx, const float* const d_M[4], const float* co
   for (int g = 0; g < 4; ++g) ZR_CHECK_ARG(d_M[g] && d_Wh[g], "zr_lstm_train_create: null matrix for gate %d", g);
   zr_lstm_train* w = new zr_lstm_train();
   w->H = H;
-  w->d_stack = nullptr;
-  w->d_stack_pack = nullptr;
   w->ldp = (H + 31) / 32 * 32;
   w->kp = (4 * H + 7) / 8 * 8;
   const size_t per = 4 * (size_t)H * H;
-  if (hipMalloc((void**)&w->d_stack, sizeof(float) * 2 * per) != hipSuccess ||
-      hipMalloc((void**)&w->d_stack_pack, sizeof(float) * 2 * (size_t)w->kp * w->ldp) != hipSuccess) {
-    (void)hipGetLastError();
-    if (w->d_stack) (void)hipFree(w->d_stack);
+  w->d_stack = (float*)zr_dev_alloc(ctx, sizeof(float) * 2 * per);
+  w->d_stack_pack = (float*)zr_dev_alloc(ctx, sizeof(float) * 2 * (size_t)w->kp * w->ldp);
+  if (!w->d_stack || !w->d_stack_pack) {
+    (void)zr_dev_free(ctx, w->d_stack);
+    (void)zr_dev_free(ctx, w->d_stack_pack);
     delete w;
     return zr_set_error(ZR_ENOMEM, "zr_lstm_train_create: allocation failed (H = %d)", H);
   }
@@ -778,9 +777,8 @@ int zr_lstm_train_destroy(zr_ctx* ctx, zr_lstm_train* w) {
   if (!w) return ZR_OK;
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
-  ZR_HIP(hipStreamSynchronize(ctx->stream));
-  if (w->d_stack) (void)hipFree(w->d_stack);
-  if (w->d_stack_pack) (void)hipFree(w->d_stack_pack);
+  (void)zr_dev_free(ctx, w->d_stack);
+  (void)zr_dev_free(ctx, w->d_stack_pack);
   delete w;
   return ZR_OK;
 }
@@ -1061,11 +1059,8 @@ int zr_attn_set_error_tables(zr_ctx* ctx, zr_attn* a, float* const* h_err_tables
                a->longest_sent);
   for (int t = 0; t < n; ++t) ZR_CHECK_ARG(h_err_tables[t] != nullptr, "zr_attn_set_error_tables: entry %d is null", t);
   if (!a->d_err_table) {
-    if (hipMalloc((void**)&a->d_err_table, sizeof(float*) * n) != hipSuccess) {
-      (void)hipGetLastError();
-      a->d_err_table = nullptr;
-      return zr_set_error(ZR_ENOMEM, "zr_attn_set_error_tables: allocation failed");
-    }
+    a->d_err_table = (float**)zr_dev_alloc(ctx, sizeof(float*) * n);
+    if (!a->d_err_table) return zr_set_error(ZR_ENOMEM, "zr_attn_set_error_tables: allocation failed");
   }
   ZR_HIP(hipStreamSynchronize(ctx->stream));
   ZR_HIP(hipMemcpy((void*)a->d_err_table, h_err_tables, sizeof(float*) * n, hipMemcpyHostToDevice));

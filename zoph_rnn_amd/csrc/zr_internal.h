@@ -11,6 +11,7 @@
 #define ZR_MAX_COUNTERS 4096
 #define ZR_MAX_STEP_FLAGS 16384
 #define ZR_MAX_PACKED_D 8
+#define ZR_MAX_KEPT 32
 
 struct zr_ctx {
   int device;
@@ -48,6 +49,17 @@ struct zr_ctx {
   size_t scratch_bytes;
   void* d_scratch2;
   size_t scratch2_bytes;
+  // device memory of destroyed handles and of zr_free, kept for the next allocation of its size (zr_runtime.hip)
+  struct KeptBlock {
+    void* p;
+    size_t bytes;
+    bool idle;  // no work that uses it can be queued anywhere; else only on own_stream
+  } kept[ZR_MAX_KEPT];  // oldest first
+  int n_kept;
+  size_t kept_bytes;
+  int foreign_stream;  // a caller's stream has been set once: nothing is kept any more
+  void* h_pinned;      // page-locked host memory that kernels write small results to (grown on demand)
+  size_t pinned_bytes;
   // the device's statically allocated scratch array (zr_runtime.hip), resolved when the context is created
   void* d_static_scratch;
   // while set, zr_ctx_scratch hands out these fixed buffers (slot 0 / slot 1) and never allocates
@@ -90,6 +102,13 @@ int zr_set_error(int code, const char* fmt, ...);
 int zr_bind_device(zr_ctx* ctx);
 // Number of contexts of this process that are alive on `device`.
 int zr_live_contexts(int device);
+// Device memory of a handle: hipMalloc, or a kept block of about the size.  May hold anything, and what is queued on ctx's own
+// stream may still use it (any_stream: nothing queued anywhere uses it).  nullptr: no memory.
+void* zr_dev_alloc(zr_ctx* ctx, size_t bytes, bool any_stream = false);
+// Gives it back, or keeps it; `idle` as for a kept block.  Null is fine.
+int zr_dev_free(zr_ctx* ctx, void* p, bool idle = false);
+// At least `bytes` of page-locked host memory, good until the next call; *dev is where a kernel finds it.
+int zr_ctx_pinned(zr_ctx* ctx, size_t bytes, void** host, void** dev);
 // Returns a context-owned scratch buffer of at least `bytes` (slot 0 or 1).
 int zr_ctx_scratch(zr_ctx* ctx, int slot, size_t bytes, void** out);
 // The same for a call that has a way without it: ZR_ENOMEM, with the buffer there is left as it is, where the device has no

@@ -1157,12 +1157,11 @@ static int pack_weights(zr_ctx* ctx, const char* who, bool bf16, const float* co
   w->ldw = ldw;
   w->kp = kp;
   w->nseg = nseg;
-  w->d_W = nullptr;
-  w->d_bias = nullptr;
-  if (hipMalloc((void**)&w->d_W, esize * HH * 4 * nseg) != hipSuccess ||
-      hipMalloc((void**)&w->d_bias, sizeof(float) * 4 * (size_t)H) != hipSuccess) {
-    (void)hipGetLastError();
-    if (w->d_W) (void)hipFree(w->d_W);
+  w->d_W = zr_dev_alloc(ctx, esize * HH * 4 * nseg);
+  w->d_bias = (float*)zr_dev_alloc(ctx, sizeof(float) * 4 * (size_t)H);
+  if (!w->d_W || !w->d_bias) {
+    (void)zr_dev_free(ctx, w->d_W);
+    (void)zr_dev_free(ctx, w->d_bias);
     delete w;
     return zr_set_error(ZR_ENOMEM, "%s: allocation failed (H = %d, nseg = %d)", who, H, nseg);
   }
@@ -1181,8 +1180,8 @@ static int pack_weights(zr_ctx* ctx, const char* who, bool bf16, const float* co
     rc = zr_pack4_multi_launch(ctx, 4 * nseg, mats, H, H, H, ldw, kp, (float*)w->d_W, 4, d_b, w->d_bias);
   }
   if (rc != ZR_OK) {
-    (void)hipFree(w->d_W);
-    (void)hipFree(w->d_bias);
+    (void)zr_dev_free(ctx, w->d_W);
+    (void)zr_dev_free(ctx, w->d_bias);
     delete w;
     return ZR_EHIP;
   }
@@ -1204,9 +1203,8 @@ int zr_lstm_weights_destroy(zr_ctx* ctx, zr_lstm_weights* w) {
   if (!w) return ZR_OK;
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
-  ZR_HIP(hipStreamSynchronize(ctx->stream));
-  if (w->d_W) (void)hipFree(w->d_W);
-  if (w->d_bias) (void)hipFree(w->d_bias);
+  (void)zr_dev_free(ctx, w->d_W);
+  (void)zr_dev_free(ctx, w->d_bias);
   delete w;
   return ZR_OK;
 }

@@ -52,6 +52,89 @@ int zr_bind_device(zr_ctx* ctx) {
   return ZR_OK;
 }
 
+// ---- kept device memory
+//
+// hipMalloc and hipFree take 10 to 300 us, and hipFree waits for the whole device: a training step that packs its layers' new weights
+// (destroy, create) drained the queue at every layer, a translation paid for its 100 MB and its handles each time (decode object of one sentence:
+// created 340 and closed in 70 us, of 16 sentences 530 and 380).  So a context keeps what is given back, up to 32 blocks and
+// 512 MiB, none larger than half of that, oldest out first.
+// A block of a handle is reused without waiting for the work that is queued on it, which is sound as long as all of that, and all
+// that comes, is on the context's own stream: nothing is kept where a caller's stream has ever been set or another context is alive.
+// What callers hold themselves (zr_malloc) may be in use on any stream of theirs, so zr_free waits for the device as hipFree
+// did, and zr_malloc for this stream where it hands out a handle's block.
+constexpr size_t kKeptTotal = (size_t)512 << 20, kKeptLargest = (size_t)256 << 20;
+
+static void drop_kept(zr_ctx* ctx, int i) {
+  (void)hipFree(ctx->kept[i].p);  // (waits for the device)
+  ctx->kept_bytes -= ctx->kept[i].bytes;
+  for (--ctx->n_kept; i < ctx->n_kept; ++i) ctx->kept[i] = ctx->kept[i + 1];
+}
+static void drop_all_kept(zr_ctx* ctx) {
+  while (ctx->n_kept) drop_kept(ctx, ctx->n_kept - 1);
+}
+
+void* zr_dev_alloc(zr_ctx* ctx, size_t bytes, bool any_stream) {
+  int best = -1;
+  for (int i = 0; i < ctx->n_kept; ++i)
+    if (ctx->kept[i].bytes >= bytes && ctx->kept[i].bytes - bytes <= bytes / 8 + 4096 && (best < 0 || ctx->kept[i].bytes < ctx->kept[best].bytes))
+      best = i;
+  if (best >= 0 && (!any_stream || ctx->kept[best].idle || hipStreamSynchronize(ctx->own_stream) == hipSuccess)) {
+    void* p = ctx->kept[best].p;
+    ctx->kept_bytes -= ctx->kept[best].bytes;
+    for (--ctx->n_kept; best < ctx->n_kept; ++best) ctx->kept[best] = ctx->kept[best + 1];
+    return p;
+  }
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  if (!ctx->n_kept) return nullptr;
+  drop_all_kept(ctx);
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+int zr_dev_free(zr_ctx* ctx, void* p, bool idle) {
+  if (!p) return ZR_OK;
+  for (int i = 0; i < ctx->n_kept; ++i)
+    if (ctx->kept[i].p == p) return zr_set_error(ZR_EHIP, "device memory %p is freed twice", p);
+  hipDeviceptr_t base = nullptr;
+  size_t bytes = 0;
+  hipPointerAttribute_t attr;
+  const bool keep = !ctx->foreign_stream && zr_live_contexts(ctx->device) == 1 && hipMemGetAddressRange(&base, &bytes, (hipDeviceptr_t)p) == hipSuccess &&
+                    base == (hipDeviceptr_t)p && bytes <= kKeptLargest && hipPointerGetAttributes(&attr, p) == hipSuccess &&
+                    attr.type == hipMemoryTypeDevice && attr.device == ctx->device;
+  if (!keep) {
+    (void)hipGetLastError();
+    if (!idle) ZR_HIP(hipStreamSynchronize(ctx->stream));
+    ZR_HIP(hipFree(p));
+    return ZR_OK;
+  }
+  while (ctx->n_kept == ZR_MAX_KEPT || (ctx->n_kept && ctx->kept_bytes + bytes > kKeptTotal)) drop_kept(ctx, 0);
+  ctx->kept[ctx->n_kept++] = {p, bytes, idle};
+  ctx->kept_bytes += bytes;
+  return ZR_OK;
+}
+
+int zr_ctx_pinned(zr_ctx* ctx, size_t bytes, void** host, void** dev) {
+  if (ctx->pinned_bytes < bytes) {
+    ZR_HIP(hipStreamSynchronize(ctx->stream));
+    if (ctx->h_pinned) ZR_HIP(hipHostFree(ctx->h_pinned));
+    ctx->h_pinned = nullptr;
+    ctx->pinned_bytes = 0;
+    const size_t want = bytes + bytes / 4 + 4096;
+    if (hipHostMalloc(&ctx->h_pinned, want, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->h_pinned = nullptr;
+      return zr_set_error(ZR_ENOMEM, "allocation of %zu bytes of page-locked host memory failed", want);
+    }
+    ctx->pinned_bytes = want;
+  }
+  *host = ctx->h_pinned;
+  ZR_HIP(hipHostGetDevicePointer(dev, ctx->h_pinned, 0));
+  return ZR_OK;
+}
+
 int zr_ctx_scratch(zr_ctx* ctx, int slot, size_t bytes, void** out) {
   if (ctx->fixed_scratch) {
     if (bytes > ctx->fixed_bytes[slot])
@@ -72,6 +155,12 @@ int zr_ctx_scratch(zr_ctx* ctx, int slot, size_t bytes, void** out) {
     size_t want = bytes + bytes / 4;
     if (hipMalloc(buf, want) != hipSuccess) {
       (void)hipGetLastError();
+      *buf = nullptr;
+      drop_all_kept(ctx);
+      if (hipMalloc(buf, want) != hipSuccess) *buf = nullptr;
+      (void)hipGetLastError();
+    }
+    if (!*buf) {
       return zr_set_error(ZR_ENOMEM, "scratch allocation of %zu bytes failed", want);
     }
     *cap = want;
@@ -85,7 +174,7 @@ int zr_ctx_scratch_if_room(zr_ctx* ctx, int slot, size_t bytes, void** out) {
     return zr_set_error(ZR_ENOMEM, "%zu bytes of scratch memory are more than ZR_OPT_LSTM_SWEEP_SCRATCH", bytes);
   const size_t cap = slot == 0 ? ctx->scratch_bytes : ctx->scratch2_bytes;
   size_t free_bytes = 0, total = 0;
-  if (cap < bytes && hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes + cap < bytes + bytes / 4)
+  if (cap < bytes && hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes + ctx->kept_bytes + cap < bytes + bytes / 4)
     return zr_set_error(ZR_ENOMEM, "no room for %zu bytes of scratch memory", bytes);
   (void)hipGetLastError();
   return zr_ctx_scratch(ctx, slot, bytes, out);
@@ -164,6 +253,8 @@ int zr_ctx_destroy(zr_ctx* ctx) {
   if (!ctx) return ZR_OK;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  drop_all_kept(ctx);
+  if (ctx->h_pinned) (void)hipHostFree(ctx->h_pinned);
   if (ctx->d_scratch) (void)hipFree(ctx->d_scratch);
   if (ctx->d_scratch2) (void)hipFree(ctx->d_scratch2);
   if (ctx->d_flags) (void)hipFree(ctx->d_flags);
@@ -234,6 +325,12 @@ int zr_ctx_query(zr_ctx* ctx, int what, int* h_value) {
 
 int zr_ctx_set_stream(zr_ctx* ctx, void* hip_stream) {
   ZR_CHECK_ARG(ctx != nullptr, "null context");
+  if (hip_stream && !ctx->foreign_stream) {
+    ctx->foreign_stream = 1;
+    const int rc = zr_bind_device(ctx);
+    if (rc) return rc;
+    drop_all_kept(ctx);
+  }
   ctx->stream = hip_stream ? (hipStream_t)hip_stream : ctx->own_stream;
   return ZR_OK;
 }
@@ -299,20 +396,16 @@ int zr_malloc(zr_ctx* ctx, size_t bytes, void** d_out) {
   ZR_CHECK_ARG(d_out != nullptr, "zr_malloc: out is null");
   *d_out = nullptr;
   if (bytes == 0) bytes = 4;
-  if (hipMalloc(d_out, bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    return zr_set_error(ZR_ENOMEM, "hipMalloc of %zu bytes failed", bytes);
-  }
-  return ZR_OK;
+  *d_out = zr_dev_alloc(ctx, bytes, true);
+  return *d_out ? ZR_OK : zr_set_error(ZR_ENOMEM, "hipMalloc of %zu bytes failed", bytes);
 }
 
 int zr_free(zr_ctx* ctx, void* d_ptr) {
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
   if (!d_ptr) return ZR_OK;
-  ZR_HIP(hipStreamSynchronize(ctx->stream));
-  ZR_HIP(hipFree(d_ptr));
-  return ZR_OK;
+  ZR_HIP(hipDeviceSynchronize());
+  return zr_dev_free(ctx, d_ptr, true);
 }
 
 int zr_h2d(zr_ctx* ctx, void* d_dst, const void* h_src, size_t bytes) {

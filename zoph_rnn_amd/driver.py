@@ -101,11 +101,12 @@ class BeamDecode:
         rep = self._rep
         rep.set(np.repeat(np.arange(n_sent, dtype=np.int32), beam))
         n = H * n_sent
-        for t in range(S):
-            ctx.gather_columns(h_all[L - 1].at(t * n), H, rep, self.cols, self.tables[t])
-        for l in range(L):
-            ctx.gather_columns(h_all[l].at((S - 1) * n), H, rep, self.cols, self.h[0][l])
-            ctx.gather_columns(c_all[l].at((S - 1) * n), H, rep, self.cols, self.c[0][l])
+        src = [h_all[L - 1].at(t * n) for t in range(S)]
+        dst = self.tables + self.h[0] + self.c[0]
+        for x in (h_all, c_all):
+            src += [x[l].at((S - 1) * n) for l in range(L)]
+        for i in range(0, len(src), capi.MAX_MULTI):
+            ctx.gather_columns_multi(src[i:i + capi.MAX_MULTI], H, rep, n_sent, self.cols, dst[i:i + capi.MAX_MULTI])
         lens = np.repeat(np.asarray(src_lens, np.int32), beam)
         self.d_batch_info.set(np.concatenate([lens, S - lens]).astype(np.int32))
         ctx.sync()
