@@ -730,6 +730,25 @@ int transpose_launch(zr_ctx* ctx, const float* src, int rows, int cols, float* d
   return ZR_OK;
 }
 
+// Whether a result of a backward sweep lies on an operand: lstm_backward_redo_kernel reads the operands again.
+bool backward_overlaps(int nl, int H, int T, int mb, const float* const c0[], const float* const c[], const float* const gates[], const float* top,
+                       const float* const hT[], const float* const cT[], float* const dg[], const float* below, float* const h0[], float* const ec0[]) {
+  const size_t n = sizeof(float) * (size_t)H * mb;
+  auto meets = [](const float* a, size_t na, const float* b, size_t nb) {
+    return a && b && (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+  };
+  auto on_operand = [&](const float* out, size_t bytes) {
+    bool hit = meets(out, bytes, top, n * T);
+    for (int l = 0; l < nl; ++l)
+      hit = hit || meets(out, bytes, c0[l], n) || meets(out, bytes, c[l], n * T) || meets(out, bytes, gates[l], 4 * n * T) ||
+            (hT && meets(out, bytes, hT[l], n)) || (cT && meets(out, bytes, cT[l], n));
+    return hit;
+  };
+  bool hit = on_operand(below, n * T);
+  for (int l = 0; l < nl; ++l) hit = hit || on_operand(dg[l], 4 * n * T) || on_operand(h0[l], n) || on_operand(ec0[l], n);
+  return hit;
+}
+
 }  // namespace
 
 extern "C" {
@@ -824,6 +843,20 @@ int zr_lstm_stack_backward_clamped(zr_ctx* ctx, int nl, const zr_lstm_train* con
                  "zr_lstm_stack_backward: null buffer for layer %d", l);
   }
   const size_t n = (size_t)H * mb;
+  // All time steps of the layers in one launch or a few, where that fits and is estimated faster; as in the forward sweep only
+  // for the only context on the device and on its own stream.
+  const bool alone = zr_live_contexts(ctx->device) == 1 && ctx->stream == ctx->own_stream;
+  if (ctx->lstm_sweep >= 2 || (ctx->lstm_sweep == 0 && ctx->gemm_cfg == 0 && alone)) {
+    const ZrBackPlan plan = zr_backward_resident_plan(ctx, nl, H, mb, T, d_err_below0 != nullptr);
+    if (plan.at_once && (ctx->lstm_sweep >= 2 || zr_back_takes(plan, nl)) &&
+        !backward_overlaps(nl, H, T, mb, d_c0, d_c_all, d_gates_all, d_err_top, d_err_hT, d_err_cT, d_dgates_all, d_err_below0, d_err_h0, d_err_c0)) {
+      const float* stacks[16];
+      for (int l = 0; l < nl; ++l) stacks[l] = layers[l]->d_stack;
+      rc = zr_backward_resident_sweep(ctx, plan, nl, stacks, H, T, mb, d_mask01, d_c0, d_c_all, d_gates_all, d_err_top, d_err_hT, d_err_cT,
+                                      d_dgates_all, d_err_below0, d_err_h0, d_err_c0, err_clip);
+      if (rc != ZR_ENOMEM) return rc;
+    }
+  }
   // The grid is walked by anti-diagonals d = l + t, highest first: node (l, t) needs the errors of (l+1, t) and
   // (l, t+1), both on diagonal d+1, so the nodes of a diagonal are independent and share two launches (the gate
   // derivatives of all of them, then all their error products as one grouped GEMM).

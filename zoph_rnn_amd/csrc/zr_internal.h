@@ -36,6 +36,8 @@ struct zr_ctx {
   int cu_count;      // compute units of the device
   int sweep_capacity[3];  // resident workgroups of lstm_sweep_kernel<TN> (0: not asked yet, -1: unknown)
   int resident_capacity[4][3];  // the same for lstm_resident_kernel, by size class and column class
+  int back_capacity[ZR_BACK_CLASSES];  // the same for lstm_backward_resident_kernel, by size class
+  int back_epoch;       // its launches so far: what d_flags[4] holds when the last one was abandoned
   int stack_step_capacity;  // the same for lstm_decoder_stack_kernel (the lesser of its two tile widths)
   int attn_step_capacity[3];  // the same for attn_step_kernel<8 / 16 / 32>
   int attn_single;      // ZR_OPT_ATTN_SINGLE_LAUNCH
@@ -275,6 +277,13 @@ int zr_lstm_resident_sweep(zr_ctx* ctx, const ZrResidentPlan& plan, int nl, cons
                            const float* d_embed, int V, const int* d_ids_nonneg, const int* d_mask01, int T, int mb,
                            const float* const d_h0[], const float* const d_c0[], float clip_threshold,
                            float* const d_h_all[], float* const d_c_all[], float* const d_gates_all[]);
+
+// The backward sweep with the weights held in registers (zr_backward_resident.hip).  stacks: [2][H x 4H] of a layer as zr_lstm_train has them.
+ZrBackPlan zr_backward_resident_plan(zr_ctx* ctx, int nl, int H, int mb, int T, bool below);
+int zr_backward_resident_sweep(zr_ctx* ctx, const ZrBackPlan& plan, int nl, const float* const stacks[], int H, int T, int mb, const int* d_mask01,
+                               const float* const d_c0[], const float* const d_c_all[], const float* const d_gates_all[], const float* d_err_top,
+                               const float* const d_err_hT[], const float* const d_err_cT[], float* const d_dgates_all[], float* d_err_below0,
+                               float* const d_err_h0[], float* const d_err_c0[], float err_clip);
 
 // One node on tiles of 4 or 8 hidden rows (zr_lstm_rows.hip).  shape: as zr_lstm_rows_shape has it (zr_rules.h); d_hp: h also k-interleaved [H/4][mb][4] (null: not wanted).
 int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const float* const in[3], const int* d_gather_ids,

@@ -151,6 +151,38 @@ inline ZrResidentPlan zr_sweep_resident_plan(int nl, int H, int mb, int T, const
   return plan;
 }
 
+// ---- the backward sweep of a stack: a launch or two per diagonal, or one launch with its weights in registers
+// (lstm_backward_resident_kernel)
+
+// Where a layer's workgroups of 16 rows x 16 columns fit the device they win with up to four launches, at 24 steps, us per diagonal / in
+// registers: 2 x 100, 100 columns 225 / 106, 3 x 200, 64 307 / 136, 4 x 200, 128 (two launches) 403 / 282, 2 x 500, 64 405 / 230, 3 x 500, 128 (three) 799 /
+// 564, 4 x 500, 128 (four) 850 / 752; but with eight, 8 x 300, 128 821 / 1099, 8 x 500, 128 1219 / 1536: the layers no longer overlap.
+constexpr int kBackLaunches = 4;
+constexpr int ZR_BACK_CLASSES = 5;
+inline int zr_back_size_class(int H) { return H <= 128 ? 0 : (H <= 256 ? 1 : (H <= 320 ? 2 : (H <= 384 ? 3 : 4))); }
+struct ZrBackPlan {
+  int size_class, at_once, flag_stride;  // layers a launch; 0: it does not fit
+  bool below;                            // the last launch also makes the error to the input from below
+  int capacity;                          // workgroups the device holds at once
+};
+// capacity: workgroups the device holds at once; below: whether the caller wants the error to the input from below.
+inline ZrBackPlan zr_back_plan(int nl, int H, int mb, int T, bool below, int capacity, int flags) {
+  ZrBackPlan plan = {zr_back_size_class(H), 0, 0, false, capacity};
+  const int tiles = (H + 15) / 16, n_tiles = (mb + 15) / 16;
+  plan.flag_stride = (tiles + 31) / 32 * 32;
+  const long long per = (long long)tiles * n_tiles;
+  long long fit = capacity / per;
+  if (fit > nl) fit = nl;
+  while (fit > 0 && fit * n_tiles * plan.flag_stride > flags) --fit;
+  if (fit < 1) return plan;
+  plan.at_once = (int)fit;
+  const int last = nl % plan.at_once ? nl % plan.at_once : plan.at_once;
+  plan.below = below && (last + 1) * per <= capacity;
+  return plan;
+}
+
+inline bool zr_back_takes(const ZrBackPlan& plan, int nl) { return plan.at_once > 0 && (nl + plan.at_once - 1) / plan.at_once <= kBackLaunches; }
+
 // ---- normalising the output matrix (softmax_normalize_kernel): 16-byte accesses a thread, and whether its workgroups fold the block pairs
 
 // Every workgroup folds its column's V / 32 pairs: cheaper than a launch for it until there are some 2.5 million to fold, us folding /
