@@ -375,3 +375,12 @@ inline ZrLogitsPlan zr_logits_plan(int V, int cols, int H, int cus) {
 // us of a call, one launch / two (the second is the time to launch them): 300 values 4.2 / 7.0, 40000 4.2 / 7.0, 90000 5.6 / 7.0, 131072 6.6 / 7.0,
 // 160000 7.6 / 7.0, 250000 10.0 / 6.9.  A quarter of that with four bytes a load.
 inline bool zr_sgd_small(long long n, bool vec) { return n <= (vec ? 112000 : 28000); }
+
+// One launch whose workgroups exchange their sums (sgd_fused_kernel): 16-byte accesses a thread, 0: not this one.  us, that above / two launches /
+// this one with two, four, eight accesses: 28000 4.1 / 7.0 / 4.1, 4.4, 4.8; 90000 6.5 / 6.9 / 4.3, 4.7, 6.0; 250000 - / 7.0 / 4.9, 5.0, 6.3; 500000 - / 7.2 / 5.7, 6.1,
+// 7.0; 1000000 - / 8.4 / 6.9, 6.8, 7.9; 2000000 - / 10.2 / -, 8.8, 9.0; 4000000 - / 14.0 / -, -, 11.4.  With one access more workgroups meet: 500000 6.1.
+constexpr int kSgdThreads = 1024, kSgdSlots = 128;
+inline int zr_sgd_fused_accesses(long long n) {
+  constexpr long long most = 4LL * kSgdThreads * kSgdSlots;  // with one access
+  return n <= 28000 || n > 8 * most ? 0 : (n <= 2 * most ? 2 : (n <= 4 * most ? 4 : 8));
+}

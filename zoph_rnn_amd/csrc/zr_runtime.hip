@@ -202,13 +202,15 @@ int zr_ctx_create(int device, zr_ctx** out) {
     return zr_set_error(ZR_EHIP, "hipStreamCreate failed: %s", hipGetErrorString(e));
   }
   c->stream = c->own_stream;
-  e = hipMalloc((void**)&c->d_flags, (32 + ZR_MAX_COUNTERS + ZR_MAX_STEP_FLAGS) * sizeof(int));
+  const size_t flag_bytes = (32 + ZR_MAX_COUNTERS + ZR_MAX_STEP_FLAGS) * sizeof(int), slot_bytes = kSgdSlots * sizeof(unsigned long long);
+  e = hipMalloc((void**)&c->d_flags, flag_bytes + slot_bytes);
   if (e != hipSuccess) {
     (void)hipStreamDestroy(c->own_stream);
     delete c;
     return zr_set_error(ZR_ENOMEM, "flag allocation failed: %s", hipGetErrorString(e));
   }
-  (void)hipMemset(c->d_flags, 0, (32 + ZR_MAX_COUNTERS + ZR_MAX_STEP_FLAGS) * sizeof(int));
+  (void)hipMemset(c->d_flags, 0, flag_bytes + slot_bytes);
+  c->d_sgd_slots = (unsigned long long*)((char*)c->d_flags + flag_bytes);
   c->d_counters = c->d_flags + 32;  // (a line apart from the flags)
   c->d_step_flags = c->d_counters + ZR_MAX_COUNTERS;
   {
