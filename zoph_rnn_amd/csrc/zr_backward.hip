@@ -1066,6 +1066,8 @@ static int weight_gradients(zr_ctx* ctx, int H, int T, int mb, const float* d_dg
   const long long K = (long long)T * mb;
   ZR_CHECK_ARG(K < (1LL << 31) / 4, "zr_lstm_weight_gradients: T * mb = %lld too large", K);
   void* scratch = nullptr;
+  if (zr_weight_gradients_takes(H, K, ctx->cu_count))
+    return zr_weight_gradients(ctx, H, (int)K, mb, d_dgates, d_in_all, d_h0, d_h_all, d_dM_stack, d_dWh_stack, d_db, accumulate);
   if (zr_split_gemm_takes(4 * H, H, (int)K)) {
     // the split product reads both operands as they lie; the previous states [h0, h_1 .. h_{T-1}] side by side
     const size_t first = sizeof(float) * (size_t)H * mb;

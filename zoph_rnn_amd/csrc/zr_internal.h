@@ -287,6 +287,10 @@ int zr_backward_resident_sweep(zr_ctx* ctx, const ZrBackPlan& plan, int nl, cons
                                const float* const d_err_hT[], const float* const d_err_cT[], float* const d_dgates_all[], float* d_err_below0,
                                float* const d_err_h0[], float* const d_err_c0[], float err_clip);
 
+// Weight and bias gradients of a layer over N columns, the first mb of the other right-hand side in d_h0 (zr_weight_gradients.hip).  No scratch.
+int zr_weight_gradients(zr_ctx* ctx, int H, int N, int mb, const float* d_dgates, const float* d_in_all, const float* d_h0, const float* d_h_all,
+                        float* d_dM, float* d_dWh, float* d_db, int accumulate);
+
 // One node on tiles of 4 or 8 hidden rows (zr_lstm_rows.hip).  shape: as zr_lstm_rows_shape has it (zr_rules.h); d_hp: h also k-interleaved [H/4][mb][4] (null: not wanted).
 int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const float* const in[3], const int* d_gather_ids,
                       int V, const float* d_cprev, const int* d_mask01, float clip, int mb, float* d_h, float* d_c,

@@ -261,6 +261,20 @@ inline bool zr_outer_takes(int count, int M, int N, int K) {
   return K <= (count > 1 || (long long)M * N >= 300000 ? 256 : 96) && !zr_split_gemm_takes(M, N, K);
 }
 
+// ---- weight gradients of a layer over N columns: one launch in fp32 (weight_gradients_kernel), or transposes and products (on the bf16 matrix cores
+// where the split product takes them) and row sums
+
+// us, those / this one (steps x minibatch): H = 64, 20 x 8 20 / 9, 100, 20 x 20 21 / 14, 300, 35 x 20 40 / 21, 500, 24 x 64 99 / 78, 700, 20 x 20 94 / 55; but few tiles that each
+// walk many columns, 64, 50 x 64 40 / 76, 200, 50 x 64 69 / 79, and what the bf16 matrix cores do faster, 500, 60 x 128 262 / 367, 1000, 12 x 64 136 / 162.
+// Estimates of both, within 10 % here and 30 % there.
+inline bool zr_weight_gradients_takes(int H, long long N, int cus) {
+  const long long tiles = (4LL * H + 63) / 64 * ((H + 63) / 64) * 2;
+  const double gflop = 16.0e-9 * H * H * N;
+  const double here = 4.0 + (double)((tiles + cus - 1) / cus) * (2.5 + 0.0235 * N);
+  const double there = 20.0 + gflop / 0.13 + (gflop < 2.5 ? 10.0 * gflop : 25.0);
+  return here <= 0.9 * there;
+}
+
 // ---- grouped products (the error products of a diagonal of the backward sweep, K = 4H): `tiles` of 32 x 32 with K over eight
 // waves, or 64 x 64 tiles (64 x 32 up to 32 columns)
 
