@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(256) row_sum_kernel(const float* __restrict__ 
   }
 }
 
-// C_g (M x N) += A_g (M x K) B_g^T for up to two independent problems (blockIdx.z), all column-major without padding: the
+// C_g (M x N) += A_g (M x K) B_g^T for up to four independent problems (blockIdx.z), all column-major without padding: the
 // weight gradients of a single attention or feed-input node, K = the minibatch.  Both operands have their rows contiguous
 // for every k, which is how the matrix instruction wants them: a half-wave reads 32 rows of one column, no transpose and no
 // LDS.  A wave has a 32 x 32 tile, A's rows on the lanes so that C is read and written 32 consecutive floats at a time.
@@ -265,9 +265,9 @@ __global__ void __launch_bounds__(256) row_sum_kernel(const float* __restrict__ 
 // Two of 500 x 500 at 64 columns 7.1 us, the launch included; the 20 target nodes of an encoder-decoder training step (2 x 500,
 // 64 columns) took 9.15 ms with a transpose and a tiled product each, 8.35 with this (W_c1^T e and W_c2^T e joined as well).
 struct OuterProducts {
-  const float* A[2];
-  const float* B[2];
-  float* C[2];
+  const float* A[4];
+  const float* B[4];
+  float* C[4];
 };
 __global__ void __launch_bounds__(256) outer_accumulate_kernel(OuterProducts P, int M, int N, int K) {
   constexpr int U = 16;  // instructions (of two k) a round; the next round's operands are in flight meanwhile
@@ -1285,15 +1285,12 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   ZR_LAUNCH_CHECK("attn_bwd_e_kernel");
   if ((rc = add_sums(grads->d_out_bias))) return rc;
   const bool outer = zr_outer_takes(2, H, H, mb);
-  if (outer) {
-    rc = outer_launch(ctx, OuterProducts{{e, e}, {d_c_t, d_h_t}, {grads->d_W_c1, grads->d_W_c2}}, 2, H, H, mb);
-    if (rc) return rc;
-  } else {
+  if (!outer) {
     if ((rc = outer_acc(e, d_c_t, grads->d_W_c1))) return rc;                   // :437
     if ((rc = outer_acc(e, d_h_t, grads->d_W_c2))) return rc;                   // :443
   }
   {
-    // W_c1^T e and W_c2^T e (:464, :476), one launch
+    // W_c1^T e and W_c2^T e (:464, :476), and W_a^T h of the forward pass again, one launch
     ZrGemmDesc g = {};
     g.M = H;
     g.N = mb;
@@ -1305,10 +1302,10 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
     g.ldc = H;
     g.batch = 1;
     g.epilogue = ZR_EPI_STORE;
-    g.groups = 2;
-    g.gA[0] = a->W_c1, g.gA[1] = a->W_c2;
-    g.gB[0] = g.gB[1] = e;
-    g.gC[0] = err_ct, g.gC[1] = d_err_h_t;
+    g.groups = 3;
+    g.gA[0] = a->W_c1, g.gA[1] = a->W_c2, g.gA[2] = a->W_a;
+    g.gB[0] = g.gB[1] = e, g.gB[2] = d_h_t;
+    g.gC[0] = err_ct, g.gC[1] = d_err_h_t, g.gC[2] = a->d_q;
     if ((rc = zr_gemm_launch(ctx, g))) return rc;
   }
   attn_bwd_align_kernel<<<dim3(W, mb), 256, 0, ctx->stream>>>(err_ct, a->d_table, a->d_err_table, d_batch_info, d_indices,
@@ -1323,12 +1320,11 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   if ((rc = add_sums(grads->d_v_p))) return rc;
   if (!outer && (rc = outer_acc(tw, d_h_t, grads->d_W_p))) return rc;           // :545
   if ((rc = product(a->W_p, 1, tw, d_err_h_t, 1, ZR_EPI_STORE))) return rc;     // :551
-  if ((rc = product(a->W_a, 1, d_h_t, a->d_q, 0, ZR_EPI_STORE))) return rc;     // W_a^T h of the forward pass again
   attn_bwd_hs_kernel<<<dim3(mb, (H + 255) / 256), 256, 0, ctx->stream>>>(a->d_q, a->d_table, a->d_err_table, d_batch_info, d_indices, scal, H, mb,
                                                   W, a->longest_sent, hs_sum);
   ZR_LAUNCH_CHECK("attn_bwd_hs_kernel");
-  if (outer)
-    rc = outer_launch(ctx, OuterProducts{{tw, d_h_t}, {d_h_t, hs_sum}, {grads->d_W_p, grads->d_W_a}}, 2, H, H, mb);
+  if (outer)  // all four weight gradients
+    rc = outer_launch(ctx, OuterProducts{{e, e, tw, d_h_t}, {d_c_t, d_h_t, d_h_t, hs_sum}, {grads->d_W_c1, grads->d_W_c2, grads->d_W_p, grads->d_W_a}}, 4, H, H, mb);
   else
     rc = outer_acc(d_h_t, hs_sum, grads->d_W_a);                                // :632
   if (rc) return rc;
