@@ -771,8 +771,8 @@ int zr_decoder_step(zr_ctx* ctx, int nl, const zr_lstm_weights* const layers[], 
   if (rc) return rc;
   if (!attn)
     return zr_softmax_forward_packed(ctx, d_D, d_b_d, V_out, layers[0]->H, top, nullptr, mb, mode, d_out, nullptr);
-  // h~ k-interleaved only for an output product that reads it so (zr_logits_plan's reads it as it lies)
-  const bool htpack = packed && (ctx->gemm_cfg != 0 || !zr_logits_plan(V_out, mb, attn->H, ctx->cu_count).tn);
+  // h~ k-interleaved only for an output product that reads it so (zr_logits_plan's and the narrow one read it as it lies)
+  const bool htpack = packed && (ctx->gemm_cfg != 0 || !(zr_logits_plan(V_out, mb, attn->H, ctx->cu_count).tn || zr_logits_narrow_takes(V_out, mb, attn->H)));
   rc = attn_step_impl(ctx, attn, d_batch_info, top, d_mask01, d_htild, d_alignments, d_indices, d_p_t, d_c_ctx,
                       (pack32 || split16) && wrote, htpack ? attn->d_htpack : nullptr);
   if (rc) return rc;

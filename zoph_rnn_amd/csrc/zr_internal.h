@@ -237,6 +237,10 @@ int zr_split_gemm(zr_ctx* ctx, int M, int N, int K, const float* A, long long ld
 int zr_logits_split(zr_ctx* ctx, int V, int cols, int H, const float* packed, int ldp, const float* h, long long ldh, float* C,
                     long long ldc, const float* bias, float* partials, bool stream, int tn, int waves);
 
+// The same for up to 16 columns (zr_logits_narrow.hip), H of at least 4.
+int zr_logits_narrow(zr_ctx* ctx, int V, int cols, int H, const float* packed, int ldp, const float* h, long long ldh, float* C, long long ldc,
+                     const float* bias, float* partials, bool stream);
+
 struct zr_lstm_weights {
   int H;
   int nseg;        // 2 (M, Wh) or 3 (+Q)

@@ -284,14 +284,16 @@ int logits_with_partials(zr_ctx* ctx, const float* d_D, const float* d_b_d, int 
     }
   }
   const bool stream = (size_t)V * H * (d.a_pack == 2 ? 2 : 4) >= ((size_t)64 << 20);
-  if (plan.tn) {
+  const bool narrow = d.a_pack == 1 && ctx->gemm_cfg == 0 && zr_logits_narrow_takes(V, mb, H);
+  if (plan.tn || narrow) {
     if (ctx->fixed_scratch && mb <= 1024 && V >= 2048 && H % 8 == 0 && ((uintptr_t)d_h & 15u) == 0) {
       // nothing of it is used here; the limit of the entry point does not follow the kernel
       void* p = nullptr;
       rc = zr_ctx_scratch(ctx, 0, sizeof(float) * (size_t)H * mb, &p);
       if (rc) return rc;
     }
-    rc = zr_logits_split(ctx, V, mb, H, d.A[0], d.lda[0], d_h, H, d_logits, V, d_b_d, (float*)scratch, stream, plan.tn, plan.waves);
+    rc = narrow ? zr_logits_narrow(ctx, V, mb, H, d.A[0], d.lda[0], d_h, H, d_logits, V, d_b_d, (float*)scratch, stream)
+                : zr_logits_split(ctx, V, mb, H, d.A[0], d.lda[0], d_h, H, d_logits, V, d_b_d, (float*)scratch, stream, plan.tn, plan.waves);
     if (rc) return rc;
     *partials_out = (float*)scratch;
     *nblocks_out = nblocks;
