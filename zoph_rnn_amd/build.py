@@ -7,7 +7,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libzoph_rnn_hip.so")
-SOURCES = ["zr_runtime.hip", "zr_elementwise.hip", "zr_gemm.hip", "zr_lstm.hip", "zr_lstm_sweep.hip", "zr_lstm_resident.hip", "zr_lstm_rows.hip", "zr_lstm_rows_bf16.hip", "zr_split_gemm.hip", "zr_small_gemm.hip", "zr_logits.hip", "zr_logits_narrow.hip",
+SOURCES = ["zr_runtime.hip", "zr_elementwise.hip", "zr_gemm.hip", "zr_lstm.hip", "zr_lstm_sweep.hip", "zr_lstm_resident.hip", "zr_lstm_rows.hip", "zr_lstm_rows_bf16.hip", "zr_split_gemm.hip", "zr_small_gemm.hip", "zr_logits.hip", "zr_logits_narrow.hip", "zr_logits_bf16.hip",
            "zr_softmax.hip", "zr_attention.hip", "zr_attn_step.hip", "zr_beam.hip", "zr_backward.hip", "zr_backward_resident.hip", "zr_weight_gradients.hip", "zr_error_products.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",

@@ -1252,6 +1252,9 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
         hi += 2 * e;
       }
     }
+    if (d.epilogue == ZR_EPI_SOFTMAX_PARTIAL && d.nseg == 1 && ctx->gemm_cfg == 0 && zr_logits_bf16_takes(d.M, d.N, d.K[0]))
+      return zr_logits_bf16(ctx, d.M, d.N, d.K[0], (const unsigned short*)d.A[0], d.lda[0], (const unsigned short*)ga.B[0], ga.Blo[0], d.C, d.ldc, d.bias,
+                            d.partials, d.stream_a != 0);
     if (small >= 0) return zr_small_gemm(ctx, d, (const unsigned short* const*)ga.B, ga.Blo, small);
     if (d.nseg == 1 && d.M >= 8192 && d.N > 32 && d.N <= 1024 &&
         (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL)) {

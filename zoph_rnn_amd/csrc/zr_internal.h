@@ -237,6 +237,9 @@ int zr_split_gemm(zr_ctx* ctx, int M, int N, int K, const float* A, long long ld
 int zr_logits_split(zr_ctx* ctx, int V, int cols, int H, const float* packed, int ldp, const float* h, long long ldh, float* C,
                     long long ldc, const float* bias, float* partials, bool stream, int tn, int waves);
 
+// The same on a prepared bf16 matrix for up to 64 columns, of which hi and lo (or null) are the bf16 terms (zr_split_pack_x_launch's layout).
+int zr_logits_bf16(zr_ctx* ctx, int V, int cols, int H, const unsigned short* packed, int ldp, const unsigned short* hi, const unsigned short* lo, float* C,
+                   long long ldc, const float* bias, float* partials, bool stream);
 // The same for up to 16 columns (zr_logits_narrow.hip), H of at least 4.
 int zr_logits_narrow(zr_ctx* ctx, int V, int cols, int H, const float* packed, int ldp, const float* h, long long ldh, float* C, long long ldc,
                      const float* bias, float* partials, bool stream);

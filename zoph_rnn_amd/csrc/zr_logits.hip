@@ -17,6 +17,7 @@
 // call), the matrix split a step ahead (spills), activations two steps ahead (106), two groups of waves in opposite phases, one
 // splitting while the other multiplies (108).
 #include "zr_internal.h"
+#include "zr_logits_epilogue.h"
 #include "zr_mfma_core.h"
 
 namespace {
@@ -189,48 +190,7 @@ __global__ void __launch_bounds__(64 * W, 2) logits_split_kernel(LogitsArgs a) {
     }
   }
 
-  // A lane has one column of each 32 x 32 block and sixteen of its rows: logits, and (max, sum exp) of the block's column.
-  const int nblocks = (a.M + 31) >> 5;
-  const bool whole = m0 + 32 <= a.M;
-  float b[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int m = m0 + 8 * (r >> 2) + 4 * half + (r & 3);
-    b[r] = a.bias[m < a.M ? m : a.M - 1];
-  }
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + 32 * j + jl;
-    float x[16], mx = -INFINITY, se = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      x[r] = acc[j][r] + b[r];
-      if (whole || m0 + 8 * (r >> 2) + 4 * half + (r & 3) < a.M) mx = fmaxf(mx, x[r]);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      if (whole || m0 + 8 * (r >> 2) + 4 * half + (r & 3) < a.M) se += __builtin_amdgcn_exp2f((x[r] - mx) * 1.4426950408889634f);
-    se += __shfl_xor(se, 32, 64);
-    if (n < a.N) {
-      float* c = a.C + (long long)n * a.ldc + m0 + 4 * half;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (whole) {
-          *(f32x4u*)(c + 8 * q) = f32x4u{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (m0 + 8 * q + 4 * half + e < a.M) c[8 * q + e] = x[4 * q + e];
-        }
-      }
-      if (half == 0) {
-        float* pp = a.partials + ((long long)n * nblocks + (m0 >> 5)) * 2;
-        pp[0] = mx;
-        pp[1] = se;
-      }
-    }
-  }
+  zr_logits_epilogue<TN>(acc, m0, n0, a.M, a.N, a.C, a.ldc, a.bias, a.partials, lane);
 }
 
 template <int TN, int W, int PD>

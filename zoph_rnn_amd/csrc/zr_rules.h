@@ -391,6 +391,15 @@ inline bool zr_logits_narrow_takes(int V, int cols, int H) {
   return (((long long)H + 7) / 8 * 8 + 160) * (((long long)V + 31) / 32) * 32 * 4 < 1LL << 32;  // 32-bit offsets
 }
 
+// The same on a prepared bf16 matrix for up to 64 columns (zr_logits_bf16.hip) instead of gemm_rows_kernel or, up to 32 columns, gemm_kernel, whose workgroups split K over
+// their waves: a wave here walks all of K, which few rows pay for.  us of a call, those / this one, 37 columns: 10000 x 512 11.7 / 10.9, 20000 x 1024 18.1 / 16.4,
+// 33333 x 512 19.4 / 15.6, 50000 x 64 19.5 / 10.4, 50000 x 1024 34.8 / 27.0, 80000 x 2000 87.4 / 67.5; 8 columns 50000 x 256 10.7 / 8.3, 80000 x 2000 60.4 / 55.1; and
+// 8192 x 256 8.5 / 9.2, 8192 x 1024 10.7 / 14.8, 16384 x 1024 13.3 / 15.4, 24000 x 2000 24.7 / 24.2 (8 columns 20.1 / 20.7 the other way).
+inline bool zr_logits_bf16_takes(int V, int cols, int H) {
+  if (cols > 64 || H % 16 != 0 || V < 10000 || V < 19LL * H) return false;
+  return ((long long)H / 8 + 56) * (((long long)V + 31) / 32) * 32 * 16 < 1LL << 32;  // 32-bit offsets, up to seven chunks behind the last one
+}
+
 // ---- the clipped update of one matrix (zr_sgd_update): one launch whose workgroups each read the whole gradient, or a launch for the
 // norm and one for the update
 
