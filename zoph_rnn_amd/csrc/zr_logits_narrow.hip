@@ -4,12 +4,12 @@
 // A wave owns 32 rows and all columns on the 16 x 16 x 4 instruction, whose operands are one 16-byte load a lane for 16 k in the k-interleaved
 // layout, five groups of 16 k ahead.  Waves are workgroups of their own, so that they spread evenly over the compute units; where four waves of 64 rows (1 KB of
 // neighbouring memory a k-block) are just about a workgroup a compute unit those are taken (50000 x 1000 31.8 us against 33.3, 60000 36.1 against 37.2;
-// but 40000 28.5 against 27.5, 80000 x 768 50.1 against 40.7).  gemm_stream_kernel's 32 x 32 x 2 instructions leave
-// more than half of their columns empty at this width: 30 us of them in a row at 50000 x 1000, on one wave a SIMD, beside 41 us for the whole
-// launch.  The activations are read as they lie.  No LDS, no barrier.
-// Bound: the matrix's way from memory, 6.3 TB/s.  gemm_stream_kernel with its re-layout of the activations where needed / this one, us: 50000 x 1000 x 12 40.4 -> 31.8,
+// but 40000 28.5 against 27.5, 80000 x 768 50.1 against 40.7).  32 x 32 x 2 instructions leave more than half of their columns empty at this
+// width: 30 us of them in a row at 50000 x 1000, on one wave a SIMD, beside 41 us for the launch that had them.  The activations are read as they lie.  No LDS, no barrier.
+// Bound: the matrix's way from memory, 6.3 TB/s.  That launch with its re-layout of the activations where needed / this one, us: 50000 x 1000 x 12 40.4 -> 31.8,
 // 50000 x 500 33.1 -> 17.3, 30000 x 1000 38.2 -> 18.8, 30011 x 333 x 10 (K % 8 != 0, another kernel) 15.1 -> 7.8, 10000 x 100 x 8 7.8 -> 4.8.  More groups in
-// flight (six, eight) 1 to 5 % slower.
+// flight (six, eight) 1 to 5 % slower.  Mean error against 64 bits with eight sums an output, with two, and before, 1e-9: H = 300 3.8, 6.2, 4.8; 500 5.9, 10.2, 7.7;
+// 1000 11, 20, 27: the same time.
 #include "zr_internal.h"
 #include "zr_mfma_core.h"
 
@@ -32,6 +32,7 @@ struct NarrowArgs {
 template <int TM, int PF, int W, int WAUX>
 __global__ void __launch_bounds__(64 * W, 2) logits_narrow_kernel(NarrowArgs a) {
   constexpr int T = 2 * TM;  // 16-row tiles
+  constexpr int NA = 8;      // sums an output, in turn over k: the shorter they are the less they round
   const int lane = threadIdx.x & 63, cl = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * W + (threadIdx.x >> 6)));
   const int m0 = 32 * TM * wave;
@@ -59,12 +60,12 @@ __global__ void __launch_bounds__(64 * W, 2) logits_narrow_kernel(NarrowArgs a) 
     const int k0 = 16 * g + 4 * kq, ks = k0 < a.K - 4 ? k0 : a.K - 4;
     q.x = *(const f32x4u*)(col + ks);
   };
-  zr_f32x4 acc[2][T];
+  zr_f32x4 acc[NA][T];
 #pragma unroll
-  for (int q = 0; q < 2; ++q)
+  for (int q = 0; q < NA; ++q)
 #pragma unroll
     for (int t = 0; t < T; ++t) acc[q][t] = zr_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto mma = [&](Frag& q, int g) {
+  auto mma = [&](Frag& q, int g, int first) {
     if (16 * (g + 1) > a.K) {  // the columns end inside this group: shift the moved load back, zero what lies behind
       const int d = 16 * g + 4 * kq - (a.K - 4);
       const zr_f32x4 v = q.x;
@@ -78,7 +79,7 @@ __global__ void __launch_bounds__(64 * W, 2) logits_narrow_kernel(NarrowArgs a) 
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int t = 0; t < T; ++t) acc[e & 1][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.w[t][e], q.x[e], acc[e & 1][t], 0, 0, 0);
+      for (int t = 0; t < T; ++t) acc[first + e][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.w[t][e], q.x[e], acc[first + e][t], 0, 0, 0);
   };
   const int last = groups - 1;
 #pragma unroll
@@ -88,13 +89,13 @@ __global__ void __launch_bounds__(64 * W, 2) logits_narrow_kernel(NarrowArgs a) 
 #pragma unroll
     for (int s = 0; s < PF + 1; ++s) {
       load(f[(s + PF) % (PF + 1)], g + s + PF < last ? g + s + PF : last);
-      mma(f[s], g + s);
+      mma(f[s], g + s, (s & 1) * 4);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 #pragma unroll
   for (int s = 0; s < PF; ++s)
-    if (g + s < groups) mma(f[s], g + s);
+    if (g + s < groups) mma(f[s], g + s, (s & 1) * 4);
 
   // A lane has one column and rows 4 kq .. 4 kq + 3 of every 16-row tile.
   const int nblocks = (a.M + 31) >> 5;
@@ -108,7 +109,10 @@ __global__ void __launch_bounds__(64 * W, 2) logits_narrow_kernel(NarrowArgs a) 
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = mb + 16 * h + 4 * kq + r;
-        x[h][r] = acc[0][2 * b + h][r] + acc[1][2 * b + h][r] + a.bias[m < a.M ? m : a.M - 1];
+        float v = 0.0f;
+#pragma unroll
+        for (int q = 0; q < NA; q += 2) v += acc[q][2 * b + h][r] + acc[q + 1][2 * b + h][r];
+        x[h][r] = v + a.bias[m < a.M ? m : a.M - 1];
         if (m < a.M) mx = fmaxf(mx, x[h][r]);
       }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
