@@ -1,5 +1,5 @@
 """The output layer's product on a prepared fp32 matrix for up to 16 columns (csrc/zr_logits_narrow.hip): edges of its 16-row tiles and 32-row blocks, of its
-groups of 16 k and their ring, both forms, and activations that are infinite.  Tolerance: H products and their sums, each rounded once, in two chains
+groups of 16 k and their ring, both forms, and activations that are infinite; and the split product's one 32-column block at 17 to 32 columns.  Tolerance: H products and their sums, each rounded once, in two chains
 (test_gpu_logits_split.py's bound)."""
 import numpy as np
 import pytest
@@ -32,6 +32,13 @@ def check(D, b, h, x, pairs):
                                    (4097, 333, 12), (8191, 640, 5), (9000, 1000, 16), (10001, 81, 7), (30011, 500, 12), (49152, 12, 16), (50001, 20, 3), (50000, 96, 12),
                                    (65536, 33, 2), (65537, 8, 1), (50001, 400, 11), (20011, 1003, 10)])
 def test_logits_and_block_pairs(ctx, V, H, n):
+    D, b, h = operands(V, H, n)
+    check(D, b, h, *logits_and_blocks(ctx, D, b, h))
+
+
+@pytest.mark.parametrize("V,H,n", [(1, 1, 17), (33, 31, 31), (257, 128, 32), (8192, 200, 18), (8449, 264, 32), (10001, 63, 25), (20480, 1000, 17), (30011, 500, 32), (33333, 333, 29),
+                                   (50001, 96, 24)])
+def test_one_block_of_columns(ctx, V, H, n):
     D, b, h = operands(V, H, n)
     check(D, b, h, *logits_and_blocks(ctx, D, b, h))
 

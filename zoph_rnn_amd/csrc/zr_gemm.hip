@@ -31,7 +31,6 @@ struct GemmArgs {
   // k-interleaved by 8 ([K/8][N][8]); see zr_split_pack_multi_kernel
   const unsigned short* Blo[3];
   int accum;  // ZR_EPI_STORE only: C += result instead of C = result
-  int stream_a;  // the weights are fetched with the streaming hint (ZrGemmDesc::stream_a)
   // groups > 0: blockIdx.z = group * batch + batch index; the group picks A, B and C from these tables
   int groups, batch;
   const float* gA[8];
@@ -127,7 +126,7 @@ __device__ __forceinline__ void softmax_partial_epilogue(const GemmArgs& a, floa
 // epilogue.  `active` false: same control flow (barriers), nothing stored.  PF = prefetch distance in k-groups.
 // BUF (k-interleaved fp32 operands on both sides, K % 8 == 0, every row and column of the tile in range, operands below
 // 4 GiB): the K loop fetches through buffer descriptors with the pinned schedule of zr_mma_segment_u.
-template <int TM, int TN, int KS, int AMODE, bool VEC, int EPI, int PF, bool BUF = false, int WAUX = 0>
+template <int TM, int TN, int KS, int AMODE, bool VEC, int EPI, int PF, bool BUF = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0, bool active, int z, float* redp,
                                           int kslice, int lane) {
   const int jl = lane & 31;
@@ -181,7 +180,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0, boo
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) xoffb[tn] = 16u * (unsigned)(cols[tn] + half * a.N);
       const unsigned woffb = 16u * (unsigned)(m0 + jl + half * (int)a.lda[s]);
-      zr_mma_segment_ring<TM, TN, KS, PF, WAUX>(acc, zr_make_rsrc(a.A[s]), wsoff, woffb, 32u * (unsigned)a.lda[s],
+      zr_mma_segment_ring<TM, TN, KS, PF>(acc, zr_make_rsrc(a.A[s]), wsoff, woffb, 32u * (unsigned)a.lda[s],
                                        zr_make_rsrc(a.B[s]), xoffb, 32u * (unsigned)a.N, a.K[s], kslice);
     } else if constexpr (zr_is_bf16_mode(AMODE)) {
       const unsigned short* wbase[TM];
@@ -404,17 +403,12 @@ __global__ void __launch_bounds__(256) gemm_rows_kernel(GemmArgs a, int row_chun
   }
 }
 
-// Tall weight matrix (k-interleaved) times at most 32 columns: the output layer at the width the reference decodes at
-// (one sentence, minibatch = beam).  The product is a stream of the matrix through the chip -- 200 MB for 1.2 GFLOP at
-// 50 000 x 1000 x 12 -- so what matters is bytes in flight and how memory sees the fetches.  K split over the waves of a
-// workgroup means a cross-wave sum through LDS and a ramp per pass (the row-range kernel: 50 us, 3.9 TB/s).  Here every
-// WAVE takes two neighbouring 32-row blocks over all of K on its own, a ring of 10 fetch stages deep, two workgroups per
-// compute unit: no LDS, no barrier, and the soft-max partials of a block are the wave's own rows.  Measured at
-// 50 000 x 12 x 1000 (kernel time): one block per wave, ring of 12: 49.6 us; two blocks, ring of 10: 40.2 us (5.0 TB/s;
-// a wave's two weight fetches of a stage are 1 KB of contiguous memory instead of 512 bytes); two blocks, ring of 14:
-// 51.9; three blocks, ring of 8: 57.4; four blocks, ring of 6: 73.3 (too few bytes in flight).
+// Tall weight matrix (k-interleaved, 8192 rows and more: the attention node's of a model that wide) times at most 32 columns: a stream of the matrix
+// through the chip, so what matters is bytes in flight and how memory sees the fetches.  K split over the waves of a workgroup means a cross-wave sum
+// through LDS and a ramp per pass (the row-range kernel: 50 us, 3.9 TB/s at 50000 x 12 x 1000).  Here every WAVE takes two neighbouring 32-row blocks over
+// all of K on its own (1 KB of neighbouring memory a stage), a ring of 10 fetch stages deep, two workgroups per compute unit: no LDS, no barrier.  40.2 us (5.0
+// TB/s); one block per wave, ring of 12: 49.6; two blocks, ring of 14: 51.9; three, ring of 8: 57.4; four, ring of 6: 73.3 (too few bytes in flight).
 // K % 8 == 0, k-interleaved activations.
-template <int EPI, int WAUX>
 __global__ void __launch_bounds__(256, 2) gemm_stream_kernel(GemmArgs a) {
   constexpr int PF = 10;
   const int lane = threadIdx.x & 63;
@@ -423,9 +417,9 @@ __global__ void __launch_bounds__(256, 2) gemm_stream_kernel(GemmArgs a) {
   const int blocks = (a.M + 31) >> 5;  // (the packed matrix holds exactly these rows: nothing beyond them is fetched)
   const int pairs = blocks >> 1;
   for (int b = wave; b < pairs; b += n_waves)
-    gemm_tile<2, 1, 1, ZR_A_PACK4, true, EPI, PF, true, WAUX>(a, b * 64, 0, true, 0, nullptr, 0, lane);
+    gemm_tile<2, 1, 1, ZR_A_PACK4, true, ZR_EPI_STORE, PF, true>(a, b * 64, 0, true, 0, nullptr, 0, lane);
   if ((blocks & 1) && wave == pairs % n_waves)  // an odd block at the end, on its own
-    gemm_tile<1, 1, 1, ZR_A_PACK4, true, EPI, PF, true, WAUX>(a, (blocks - 1) * 32, 0, true, 0, nullptr, 0, lane);
+    gemm_tile<1, 1, 1, ZR_A_PACK4, true, ZR_EPI_STORE, PF, true>(a, (blocks - 1) * 32, 0, true, 0, nullptr, 0, lane);
 }
 
 // Soft-max-partial epilogue for accumulators held the other way round: lane = column (n0 + 32*tn + lane % 32),
@@ -1219,7 +1213,6 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
   ZR_CHECK_ARG(!d.Cpack || (d.epilogue == ZR_EPI_TANH_BIAS_MASK && d.batch <= 1 && d.groups == 0),
                "gemm: a k-interleaved second result needs the tanh-bias-mask epilogue and a single problem");
   ga.accum = d.accumulate;
-  ga.stream_a = d.stream_a;
   if (d.epilogue == ZR_EPI_TANH_BIAS_MASK) ZR_CHECK_ARG(d.bias && d.mask, "gemm: bias/mask required");
   ZR_CHECK_ARG(!d.accumulate || d.epilogue == ZR_EPI_STORE, "gemm: accumulate needs the plain store epilogue");
   if (d.epilogue == ZR_EPI_SOFTMAX_PARTIAL) ZR_CHECK_ARG(d.bias && d.partials, "gemm: bias/partials required");
@@ -1344,22 +1337,15 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
     if (vec && d.nseg == 1 && zcount == 1 && d.M >= 8192 && d.N <= 1024 && ctx->gemm_cfg != 11 &&
         (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL)) {
       const int n32 = (d.N + 31) / 32;
-      if (d.N <= 32 && ga.b_pack4 && d.K[0] % 8 == 0 && ctx->gemm_cfg == 0 &&
+      if (d.epilogue == ZR_EPI_STORE && d.N <= 32 && ga.b_pack4 && d.K[0] % 8 == 0 && ctx->gemm_cfg == 0 &&
           (long long)d.K[0] * ga.lda[0] * 4 + 4096 < (1LL << 32)) {
-        // one 32-row block per wave while there are waves (three workgroups per compute unit), more beyond that
-        // two neighbouring 32-row blocks per wave (their fetches are 1 KB of contiguous memory), two workgroups per
-        // compute unit, one pair per wave while there are waves
+        // one pair of 32-row blocks per wave while there are waves
         const int pairs = ((d.M + 31) / 32 + 1) / 2;
         const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
         int wgs = (pairs + 3) / 4;
         if (wgs > 2 * cus) wgs = 2 * cus;
         ga.m_tiles = ga.n_tiles = 0;
-        if (d.epilogue == ZR_EPI_STORE)
-          gemm_stream_kernel<ZR_EPI_STORE, 0><<<wgs, 256, 0, ctx->stream>>>(ga);
-        else if (ga.stream_a)
-          gemm_stream_kernel<ZR_EPI_SOFTMAX_PARTIAL, ZR_AUX_STREAM><<<wgs, 256, 0, ctx->stream>>>(ga);
-        else
-          gemm_stream_kernel<ZR_EPI_SOFTMAX_PARTIAL, 0><<<wgs, 256, 0, ctx->stream>>>(ga);
+        gemm_stream_kernel<<<wgs, 256, 0, ctx->stream>>>(ga);
         ZR_LAUNCH_CHECK("gemm_stream_kernel");
         return ZR_OK;
       }

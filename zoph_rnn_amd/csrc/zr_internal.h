@@ -167,7 +167,7 @@ struct ZrGemmDesc {
   unsigned short* Clo;
   int accumulate;   // ZR_EPI_STORE only: C += product (+ bias) instead of C = ...
   // A is read once per step and is a large part of the memory-side cache: fetch it with the non-temporal hint so that
-  // it does not push out what the rest of the step reads again (honoured by the kernel of the output layer's product)
+  // it does not push out what the rest of the step reads again (honoured by zr_logits_bf16)
   int stream_a;
   // groups > 0: that many independent problems of the same shape in one launch (at most 8; one segment, plain store
   // epilogue, no bias): problem g multiplies gA[g] (instead of A[0]) with gB[g] (instead of B[0]) into gC[g]

@@ -1,4 +1,4 @@
-// The output layer's product on a prepared fp32 matrix, V x H times H x columns, beyond 32 columns: the bf16 matrix cores with every operand as
+// The output layer's product on a prepared fp32 matrix, V x H times H x columns, beyond 16 columns: the bf16 matrix cores with every operand as
 // three exact bf16 terms (zr_split_gemm.hip says why that loses nothing), the matrix straight from memory into the registers
 // of the one wave that multiplies it.
 //
@@ -10,7 +10,7 @@
 // fp32 instructions (the terms of an infinite operand are infinity and NaN).
 // Bound by matrix instructions and conversions together: at 50000 x 128 x 1000 the matrix pipes of the 200 compute units that have a tile are busy for 57 %,
 // the vector instructions take 44 % of their cycles.  It takes 89 to 92 us (12.8 GFLOP, 77 of bf16 work); the fp32 instructions took 110 to
-// 124; 64 columns of 30011 x 500 31 -> 22.
+// 124; 64 columns of 30011 x 500 31 -> 22, 32 columns 20.9 -> 17.2, of 50000 x 300 27.3 -> 15.9.
 // Error of the logits against 64 bits, relative 2-norm, here and with the fp32 instructions: H = 64 7.6e-8 / 8.7e-8, 200 9.1e-8 / 1.36e-7, 500
 // 1.09e-7 / 2.06e-7, 1000 1.35e-7 / 2.1e-7 to 2.9e-7.
 // Tried and dropped at 128 columns: one chain of dependent instructions a column block instead of two in turn (107 against 103 us the whole

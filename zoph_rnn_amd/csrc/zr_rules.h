@@ -359,8 +359,12 @@ struct ZrLogitsPlan {
 inline ZrLogitsPlan zr_logits_plan(int V, int cols, int H, int cus) {
   ZrLogitsPlan plan = {0, 0};
   const long long blocks = (V + 31) / 32, n32 = (cols + 31) / 32;
+  // Up to 16 columns: zr_logits_narrow.hip.  Up to 32, us, the other kernels / this one: K % 8 == 0 (a wave of theirs walks all of K on fp32 instructions), 8192 x 256 17.0
+  // / 9.0, 20000 x 512 24.4 / 15.1, 50000 x 1000 43.2 / 37.4, 80000 x 512 47.1 / 43.5; otherwise 30011 x 500 20.9 / 17.2, 50000 x 300 27.3 / 15.9, 9000 x 250 8.2 / 9.1; few
+  // rows 4000 x 128 8.4 / 6.4, 1000 x 128 6.5 / 6.2, 1000 x 200 7.5 / 8.4, 4000 x 1000 12.0 / 24.5.
+  if (cols <= 16 || (cols <= 32 && H > 128 && V < (H % 8 == 0 ? 8192 : 24576))) return plan;
   // 32-bit offsets into the matrix, and a few steps past it
-  if (cols <= 32 || (((long long)H + 7) / 8 * 8 + 160) * blocks * 32 * 4 >= 1LL << 32) return plan;
+  if ((((long long)H + 7) / 8 * 8 + 160) * blocks * 32 * 4 >= 1LL << 32) return plan;
   const int steps = (H + 31) / 32;
   double best = 0.0;
   for (int tn = 1; tn <= 6; ++tn)
@@ -383,11 +387,11 @@ inline ZrLogitsPlan zr_logits_plan(int V, int cols, int H, int cus) {
   return plan;
 }
 
-// The same for up to 16 columns (zr_logits_narrow.hip) instead of gemm_stream_kernel and, below 8192 rows or with K % 8 != 0, the others: faster by 20 to
+// The same for up to 16 columns (zr_logits_narrow.hip) instead of 32-column instructions and, below 8192 rows or with K % 8 != 0, the others: faster by 20 to
 // 65 % at every size (V = 1000 .. 80000, H = 64 .. 1000) but few rows of a long K, which one wave then walks alone: us, those / this one, 4000 x 1000 11.4 /
 // 12.1, 1000 x 1000 9.2 / 12.0, 2000 x 500 9.8 / 7.3, 4000 x 200 8.9 / 4.8, 8192 x 300 6.4 / 5.2, 10000 x 1000 37.8 / 12.7.
 inline bool zr_logits_narrow_takes(int V, int cols, int H) {
-  if (cols > 16 || H < 4 || (V < 8192 && H > 640)) return false;
+  if (cols > 16 || H < 4 || (V < 8192 && H > 600)) return false;
   return (((long long)H + 7) / 8 * 8 + 160) * (((long long)V + 31) / 32) * 32 * 4 < 1LL << 32;  // 32-bit offsets
 }
 
