@@ -203,9 +203,9 @@ def bench_decoder_step(ctx, steps, warmup, H=1000, mb=128, S=50, V=50000, L=4, D
                        parts["attention_us"], flops=f_attn, nbytes=4 * H * H * wb + slots * H * mb * 4, peak_tflops=peak,
                        note="a chain of dependent stages: %.0f MB of source states and matrices, %.2f GFLOP"
                             % ((4 * H * H * wb + slots * H * mb * 4) / 1e6, f_attn / 1e9)),
-        # (fp32 beyond 32 columns: three bf16 terms an operand; up to 32 a stream of the matrix)
-        roofline_entry("output-layer logits + column statistics (logits_split_kernel / gemm_stream_kernel / gemm_bf16_lds_kernel, "
-                       "softmax_colstats_kernel)", "hbm" if bf16 or mb <= 32 else "mfma", parts["logits_and_colstats_us"],
+        # (fp32 beyond 16 columns: three bf16 terms an operand; up to 16 a stream of the matrix)
+        roofline_entry("output-layer logits + column statistics (logits_split_kernel / logits_narrow_kernel / gemm_bf16_lds_kernel / "
+                       "logits_bf16_kernel, softmax_colstats_kernel)", "hbm" if bf16 or mb <= 16 else "mfma", parts["logits_and_colstats_us"],
                        flops=f_logits, nbytes=V * H * wb + V * mb * 4, peak_tflops=peak if bf16 else PEAK_SPLIT_FP32_TFLOPS),
         roofline_entry("softmax_normalize_kernel", "hbm", norm_us, nbytes=2.0 * V * mb * 4),
     ]
