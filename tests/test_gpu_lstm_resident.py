@@ -185,6 +185,12 @@ def test_node_on_narrow_row_tiles(ctx, H, mb):
         layer.close()
 
 
+# ... and 4-row tiles beyond H = 512, two of which share the lines of the weights: odd numbers of them, the last size that has them
+@pytest.mark.parametrize("H,mb", [(515, 1), (530, 16), (1021, 9), (1024, 16)])
+def test_node_on_pairs_of_row_tiles(ctx, H, mb):
+    test_node_on_narrow_row_tiles(ctx, H, mb)
+
+
 # Infinite values where a k-group is only partly filled: beside an infinity nothing may be multiplied by a zero that stands
 # for "not there".  H = 9, 100 and 101: the moved load of an embedding column's tail; 104: thirteen row tiles, whose last
 # 16-column k-group is half empty; 300 at 40 columns: 32-column tiles.

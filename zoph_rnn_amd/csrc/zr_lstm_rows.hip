@@ -5,7 +5,7 @@
 // workgroups whose K loops are many times longer than the weights' way from memory, and dividing K across workgroups as
 // well costs a round of partial tiles through memory.  Tiles of 4 or 8 rows put a node on 8 (4) times as many workgroups
 // with no exchange between them: one LDS sum of the 8 waves and the cell.
-// What bounds it: the weights' way from the memory-side cache at narrow batches, the matrix pipe at wide ones.
+// What bounds it: the weights' way from the memory-side cache at narrow batches (H = 1000, 12 columns: 36 MB in 10.9 us, 3.3 TB/s), the matrix pipe at wide ones.
 //
 // Inputs are read as they lie (columns of H floats, gathered from the embedding for a bottom layer), four consecutive k a
 // lane with one 16-byte load that only needs 4-byte alignment, so any H >= 8 runs here: the last load of a column is moved
@@ -13,6 +13,7 @@
 #include "zr_internal.h"
 #include "zr_math.h"
 #include "zr_mfma_core.h"
+#include "zr_rules.h"
 
 namespace {
 
@@ -46,10 +47,13 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
   constexpr int NOUT = (ROWS * COLS + 511) / 512;
   constexpr int NS = PF + 1;
   __shared__ float red[kWaves * COLS * kRedLd];
-  // Workgroup ids congruent mod 8 share a die: the column tiles of a row tile, which read the same weights, go together.
-  const int id = blockIdx.x;
-  const int jt = (id / (8 * P.n_tiles)) * 8 + (id & 7);
-  const int nt = (id >> 3) % P.n_tiles;
+  // Workgroup ids congruent mod 8 share a die: the column tiles of a row tile, which read the same weights, go together, and so do two row tiles of
+  // four, whose rows are the halves of the weights' 128-byte lines (apart, every line is fetched by two dies: a node of H = 1000 at 12 columns 14.3 us
+  // against 10.9, of H = 500 7.2 against 7.0).
+  constexpr int RT = ROWS == 4 ? 2 : 1;
+  const int id = blockIdx.x, slots = RT * P.n_tiles, at = (id >> 3) % slots;
+  const int jt = ((id / (8 * slots)) * 8 + (id & 7)) * RT + at % RT;
+  const int nt = at / RT;
   if (jt >= P.j_tiles) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -130,7 +134,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) lstm_rows_kernel(LstmRows P) {
   // kernels divide K further.  Error of h against 64 bits at H = 1024, one column 2.6e-7 with one accumulator, 1.7e-7 with four
   // (K split across workgroups 1.7e-7), with feed-input 3.3e-7, 1.9e-7 (1.9e-7); H = 500 at 128 columns 2.0e-7, 1.6e-7 with
   // two (1.6e-7).  Costs 0 to 1.5 %.
-  constexpr int NACC = NARROW && ROWS == 8 ? 4 : 2;
+  constexpr int NACC = NARROW ? 4 : 2;
   acc16 acc[2][TN];
   zr_f32x4 acc4[NACC][NB];
 #pragma unroll
@@ -255,10 +259,12 @@ int zr_lstm_rows_step(zr_ctx* ctx, const zr_lstm_weights* w, int nseg, const flo
   P.ldw = w->ldw;
   P.kp = w->kp;
   P.clip = clip;
+  if (shape == 1 && zr_lstm_rows_halves(P.H, mb, ctx->cu_count)) shape = 0;
   const int rows = shape == 0 ? 4 : 8, cols = shape <= 1 ? 16 : (shape == 2 ? 32 : 64);
   P.j_tiles = (P.H + rows - 1) / rows;
   P.n_tiles = (mb + cols - 1) / cols;
-  const unsigned grid = (unsigned)((P.j_tiles + 7) / 8 * 8 * P.n_tiles);
+  const int rt = rows == 4 ? 2 : 1;  // row tiles side by side on a die
+  const unsigned grid = (unsigned)(((P.j_tiles + rt - 1) / rt + 7) / 8 * 8 * rt * P.n_tiles);
   if (shape == 0)
     lstm_rows_kernel<4, 1, true, 8><<<grid, 64 * kWaves, 0, ctx->stream>>>(P);
   else if (shape == 1)

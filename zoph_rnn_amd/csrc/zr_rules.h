@@ -44,10 +44,9 @@ inline double zr_fused_us(int units, int H, int mb, int nseg, bool vec, int cus)
 
 // Tile by size, one node of H = 1000 / 500 / 300 at up to 128 columns, us (the register-streaming kernel of zr_lstm.hip
 // with K split across workgroups: 16-27 / 30-33 / 23-30):
-//   4 x 16:  13.0 at 12 columns /  6.4 at 12, 8.6 at 37 /  5.5 at 20      8 x 16:  11.5 at 12, 12.0 at 32 / 7.4 at 37 / 6.1
+//   4 x 16:  10.9 at 12 columns /  7.0 at 12, 9.6 at 37 /  5.4 at 20      8 x 16:  12.7 at 12, 12.0 at 32 / 8.2 at 37 / 6.4
 //   8 x 32:  17.0 at 64 / 11.7 at 128 / 7.7 at 100                        8 x 64:  26.5 at 128 / 16.8 at 128
-// The smallest tile that keeps the workgroups within one per compute unit wins, except that 4 x 16 tiles of H > 512 read the
-// activations once too often (13.0 against 11.5).  Wide tiles of a long K range lose to the streaming kernel where that has
+// The smallest tile that keeps the workgroups within one per compute unit wins (4 x 16 beyond H = 512: zr_lstm_rows_halves).  Wide tiles of a long K range lose to the streaming kernel where that has
 // its whole-group form (H = 2000, 64 columns: 71 against 48), and so does any second round of workgroups there (H = 1000, 192
 // columns: 42-65 against 37).  For 8 x 64 tiles it is a matter of how well the older kernels' own tiles fit the chip: H =
 // 1000, 128 columns 27.2 against 26.1 and 96 columns 25.9 against 36.3; H % 8 != 0, in rounds, H = 1001, 192 columns
@@ -66,6 +65,10 @@ inline int zr_lstm_rows_shape(int H, int mb, int nseg, bool vec, int cus) {
   if (H % 8 == 0 && (rounds > 1 || H > 1024)) return -1;
   return rounds * (4.0 + 0.0115 * H * nseg) < zr_fused_us(1, H, mb, nseg, vec, cus) ? 3 : -1;
 }
+
+// 8 x 16 tiles as twice as many of 4 x 16, whose two halves of a line go to the same die, while those are within one a compute unit: us of a node, 8 x 16 / 4 x 16, 16
+// columns, H = 513 8.9 / 7.7, 600 10.1 / 8.9, 800 11.4 / 10.0, 1000 12.9 / 11.2, 1024 12.6 / 11.0; one column, 1000 11.9 / 10.6.
+inline bool zr_lstm_rows_halves(int H, int mb, int cus) { return (long long)((H + 3) / 4) * ((mb + 15) / 16) <= cus; }
 
 // The same for a node on bf16 weights (zr_lstm_rows_bf16.hip against lstm_fused_kernel's 32-row tiles); shapes 1 to 3 as above.  us of a
 // node, two terms (one term), in a decoder step of four layers: H = 512, 64 columns 12.1 -> 6.2 on 8 x 32 tiles (10.7 -> 5.2), 1024, 12
