@@ -129,6 +129,20 @@ def test_beam_with_frequent_eof_and_penalty(ctx):
     _decode_both(ctx, 60, 5, 4, 7, max_len=12, penalty=0.3, seed=7, eof_boost=4.0)
 
 
+@pytest.mark.parametrize("beam,first", [(31, 6.0), (31, 0.0), (22, 6.0)])
+def test_beam_passes_over_words_that_take_no_slot(ctx, monkeypatch, beam, first):
+    """<START> and <EOF> at the head of every column: of a sentence's up to 992 candidates more than 64 are passed before the beam is full."""
+    def dist(g, V, cols, peaky=2.0, eof_boost=0.0):
+        logits = g.standard_normal(size=(V, cols)) * 0.3
+        logits[0] += first
+        logits[1] += eof_boost
+        e = np.exp(logits - logits.max(axis=0))
+        return np.asfortranarray((e / e.sum(axis=0)).astype(np.float32))
+
+    monkeypatch.setitem(globals(), "_random_dist", dist)
+    _decode_both(ctx, 2000, beam, 2, 4, max_len=9, penalty=0.1, seed=beam, eof_boost=6.0)
+
+
 def test_beam_batching_does_not_change_a_sentence(ctx):
     """16 sentences decoded together give, per sentence, what a single-sentence decode gives."""
     V, beam, n_sent, steps, max_len = 300, 12, 16, 5, 10

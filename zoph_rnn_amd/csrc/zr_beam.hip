@@ -299,6 +299,16 @@ beam_select_blocks_kernel(const float* __restrict__ logits, const float* __restr
   const float* x = logits + (size_t)col * V;
   const float* pairs = blocks + (size_t)col * nblocks * 2;
   if (tid == 0) s_nblk = 0, s_count = 0;
+  // the maxima of the first 2048 blocks, for the list below, on their way beside the fold's pairs
+  float pm[8];
+  auto load_maxima = [&](int b0) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int b = b0 + tid + 256 * u;
+      pm[u] = b < nblocks ? pairs[2 * b] : -INFINITY;
+    }
+  };
+  load_maxima(0);
   float c_max, c_sum;
   const float bm = zr_softmax_fold_column(pairs, nblocks, s_m, s_s, c_max, c_sum, [] {});
   if (tid == 0) {
@@ -328,14 +338,9 @@ beam_select_blocks_kernel(const float* __restrict__ logits, const float* __restr
     topk_unkey((unsigned long long)tu << 32, tp, tw);  // (no thread value at all: -inf, which lists every block)
     tp -= 1e-6f + 5e-7f * (fabsf(tp) + fabsf(c_max));
   }
-  // candidate blocks (the maxima again, eight loads in flight per thread)
+  // candidate blocks
   for (int b0 = 0; b0 < nblocks; b0 += 2048) {
-    float pm[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int b = b0 + tid + 256 * u;
-      pm[u] = b < nblocks ? pairs[2 * b] : -INFINITY;
-    }
+    if (b0) load_maxima(b0);
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       if (pm[u] >= tp && pm[u] > -INFINITY) {
@@ -348,14 +353,23 @@ beam_select_blocks_kernel(const float* __restrict__ logits, const float* __restr
   const int nblk = s_nblk;
   bool exact = nblk > kSelBlockCap;
   if (!exact) {
-    // candidate words: a half-wave per block
+    // candidate words: a half-wave per block, eight blocks of each in flight
     const int hw = tid >> 5, l32 = tid & 31;
-    for (int i = hw; i < nblk; i += 8) {
-      const int v = s_blk[i] * 32 + l32;
-      const float q = v < V ? x[v] : -INFINITY;
-      if (q >= tp && q > -INFINITY) {
-        const int pos = atomicAdd(&s_count, 1);
-        if (pos < kSelCandCap) s_cand[pos] = topk_key(expf(q - c_max) / c_sum, v);
+    for (int i0 = hw; i0 < nblk; i0 += 64) {
+      int v[8];
+      float q[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int i = i0 + 8 * u;
+        v[u] = i < nblk ? s_blk[i] * 32 + l32 : V;
+        q[u] = v[u] < V ? x[v[u]] : -INFINITY;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        if (q[u] >= tp && q[u] > -INFINITY) {
+          const int pos = atomicAdd(&s_count, 1);
+          if (pos < kSelCandCap) s_cand[pos] = topk_key(expf(q[u] - c_max) / c_sum, v[u]);
+        }
       }
     }
     __syncthreads();
@@ -404,7 +418,8 @@ beam_select_blocks_kernel(const float* __restrict__ logits, const float* __restr
 }
 
 // Cross-column merge and bookkeeping for one sentence per workgroup (expand_hypothesis_without_fsa,
-// src/decoder.h:1214-1315).
+// src/decoder.h:1214-1315).  Bound: two trips to memory and the launch, then the sentence rows' copy: one sentence of beam 12 6.6 us, sixteen 8.5; with the slots
+// filled by one thread, and its reads one after another, 9.4 and 10.2.
 __global__ void __launch_bounds__(256)
 beam_merge_kernel(int beam, int K, int max_len, int hyp_cap, float penalty, int index, int current_index,
                   const float* __restrict__ cand_p, const int* __restrict__ cand_w, float* scores,
@@ -435,6 +450,21 @@ beam_merge_kernel(int beam, int K, int max_len, int hyp_cap, float penalty, int 
   int* st = sent + (size_t)s * beam * max_len;
   int* stt = sent_tmp + (size_t)s * beam * max_len;
 
+  // Everything the ranking reads is asked for at once; the count by the thread that updates it at the end, and handed on through shared memory: a wave that
+  // came late to a load of its own could otherwise see the updated one.
+  if (tid == 0) s_base = hyp_count[s];
+  constexpr int MINE = (MAXC + 255) / 256;
+  const int all_cand = ((index == 0) ? 1 : beam) * K;
+  float p_mine[MINE], sc_mine[MINE];
+  int w_mine[MINE];
+#pragma unroll
+  for (int u = 0; u < MINE; ++u) {
+    const int a = tid + 256 * u, i = a / K;
+    if (a < all_cand) {
+      const size_t ci = ((size_t)s * beam + i) * K + (K - 1 - a % K);
+      p_mine[u] = cand_p[ci], w_mine[u] = cand_w[ci], sc_mine[u] = sc[i];
+    }
+  }
   // live columns: all of them, or column 0 only at the first step; stop at the first dead slot (:1188-1191)
   if (tid < 64) {  // beam < 64: one ballot over the slots finds the first dead one
     const int all = (index == 0) ? 1 : beam;
@@ -445,12 +475,13 @@ beam_merge_kernel(int beam, int K, int max_len, int hyp_cap, float penalty, int 
   const int live = s_ncand / K;
   // candidate a = i*K + q of live column i: the reference pops its per-column heap in ascending probability and
   // pushes into the global heap, so q counts ranks from the worst (rank K-1) to the best (rank 0)
-  for (int a = tid; a < live * K; a += 256) {
-    const int i = a / K, r = K - 1 - a % K;
-    const size_t ci = ((size_t)s * beam + i) * K + r;
-    c_val[a] = logf(cand_p[ci]) + sc[i];
+#pragma unroll
+  for (int q = 0; q < MINE; ++q) {
+    const int a = tid + 256 * q, i = a / K, r = K - 1 - a % K;
+    if (a >= live * K) break;
+    c_val[a] = logf(p_mine[q]) + sc_mine[q];
     c_col[a] = i;
-    c_word[a] = cand_w[ci];
+    c_word[a] = w_mine[q];
     unsigned u = __float_as_uint(c_val[a]);
     u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
     c_key[a] = ((unsigned long long)u << 32) | (unsigned)(0x7fffffff - (i * K + r));
@@ -466,34 +497,34 @@ beam_merge_kernel(int beam, int K, int max_len, int hyp_cap, float penalty, int 
     c_order[rank] = a;
   }
   __syncthreads();
-  if (tid == 0) {
-    int slot = 0, nfin = 0, pos = 0;
-    while (slot < beam) {
-      if (pos >= n) {  // global heap empty: filler slots (src/decoder.h:1231-1249)
-        s_parent[slot] = -1;
-        s_word[slot] = -1;
-        s_score[slot] = 0.0f;
-        ++slot;
-        continue;
+  // In that order, until the beam is full: <START> is never selected, <EOF> is a finished hypothesis and takes no slot, any other word does.  64
+  // candidates at a time by one wave, which counts the words ahead of each.
+  if (tid < 64) {
+    int slot = 0, nfin = 0;
+    for (int p0 = 0; p0 < n && slot < beam; p0 += 64) {
+      const int a = p0 + tid < n ? c_order[p0 + tid] : -1;
+      const int w = a >= 0 ? c_word[a] : 0;
+      const unsigned long long ahead = (1ull << tid) - 1, taken = __ballot(w != 0 && w != 1);
+      const int at = slot + __popcll(taken & ahead);
+      const unsigned long long eof = __ballot(w == 1 && at < beam);
+      if (at < beam && w == 1) {
+        const int f = nfin + __popcll(eof & ahead);
+        s_fin_parent[f] = c_col[a];
+        s_fin_score[f] = c_val[a] + penalty;
+      } else if (at < beam && w != 0) {
+        s_parent[at] = c_col[a];
+        s_word[at] = w;
+        s_score[at] = c_val[a] + penalty;
       }
-      const int a = c_order[pos++];
-      const int w = c_word[a];
-      if (w == 0) continue;  // <START> never selected
-      if (w == 1) {          // <EOF>: finished hypothesis, no beam slot consumed
-        s_fin_parent[nfin] = c_col[a];
-        s_fin_score[nfin] = c_val[a] + penalty;
-        ++nfin;
-      } else {
-        s_parent[slot] = c_col[a];
-        s_word[slot] = w;
-        s_score[slot] = c_val[a] + penalty;
-        ++slot;
-      }
+      slot += __popcll(taken);
+      nfin += __popcll(eof);
     }
-    s_nfin = nfin;
-    // read here, by the thread that updates it at the end, and handed on through shared memory: a wave that came late
-    // to a load of its own could otherwise see the updated count
-    s_base = hyp_count[s];
+    if (tid < beam && tid >= slot) {  // global heap empty: filler slots (src/decoder.h:1231-1249)
+      s_parent[tid] = -1;
+      s_word[tid] = -1;
+      s_score[tid] = 0.0f;
+    }
+    if (tid == 0) s_nfin = nfin;
   }
   __syncthreads();
   // finished hypotheses: parent's words [0, current_index+1) then <EOF>
