@@ -86,6 +86,7 @@ __global__ void __launch_bounds__(64 * W, 2) logits_bf16_kernel(Logits16Args a) 
   auto step = [&](int c, const zr_u32x4 (&v)[STEPS], const zr_u32x4* x, zr_u32x4 (&vn)[STEPS], zr_u32x4* xn) {
     __builtin_amdgcn_s_waitcnt(0x0F70 | (NI + STEPS));  // vmcnt
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");  // nothing behind the barrier is read before it (a fence would wait for every load)
     __builtin_amdgcn_sched_barrier(0);
     load_x(c + 2, xn);
     load_a(vn, c + 2);
