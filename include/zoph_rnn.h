@@ -530,7 +530,7 @@ int zr_lstm_feed_backward(zr_ctx* ctx, const float* const d_Q[4], int H, int mb,
  *   d_h_t: the h_t the forward step read (d_h_t_att: after the layer's dropout where that is on);
  *   d_h_tild, d_alignments, d_indices, d_p_t, d_c_t: outputs of that zr_attn_step call;
  *   d_err_htild: error of h~ (d_d_ERRt_ht_tild; the caller has added the feed-input error, :416);
- *   d_err_h_t (H x mb, overwritten): error of h_t (d_ERRnTOt_ht_p1, before the dropout of :647); may be d_err_htild;
+ *   d_err_h_t (H x mb, overwritten): error of h_t (d_ERRnTOt_ht_p1, before the dropout of :647); may be d_err_htild or d_c_t;
  *   grads: the layer's six gradient arrays, ACCUMULATED into (beta = 1 in the reference);
  *   the errors of the source states are ADDED into the arrays registered with zr_attn_set_error_tables, entry t for
  *   the source position stored in hs table t (d_total_hs_error, src/attention_layer.hpp:106-160). */

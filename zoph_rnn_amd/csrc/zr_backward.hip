@@ -833,13 +833,15 @@ int transpose_launch(zr_ctx* ctx, const float* src, int rows, int cols, float* d
   return ZR_OK;
 }
 
+// Whether na bytes at a and nb bytes at b share any (null: no).
+bool meets(const float* a, size_t na, const float* b, size_t nb) {
+  return a && b && (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+}
+
 // Whether a result of a backward sweep lies on an operand: lstm_backward_redo_kernel reads the operands again.
 bool backward_overlaps(int nl, int H, int T, int mb, const float* const c0[], const float* const c[], const float* const gates[], const float* top,
                        const float* const hT[], const float* const cT[], float* const dg[], const float* below, float* const h0[], float* const ec0[]) {
   const size_t n = sizeof(float) * (size_t)H * mb;
-  auto meets = [](const float* a, size_t na, const float* b, size_t nb) {
-    return a && b && (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
-  };
   auto on_operand = [&](const float* out, size_t bytes) {
     bool hit = meets(out, bytes, top, n * T);
     for (int l = 0; l < nl; ++l)
@@ -1242,7 +1244,9 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   };
 
   // C (H x H) += A (H x mb) * B^T for B H x mb (cuBLAS gemm N, T with beta = 1 in the reference)
+  const bool outer = zr_outer_takes(2, H, H, mb);
   auto outer_acc = [&](const float* A, const float* B, float* C) -> int {
+    if (outer) return outer_launch(ctx, OuterProducts{{A}, {B}, {C}}, 1, H, H, mb);
     int r = transpose_launch(ctx, B, H, mb, tr, mb, 0);
     if (r) return r;
     ZrGemmDesc g = {};
@@ -1284,8 +1288,12 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   attn_bwd_e_kernel<<<row_blocks, 1024, 0, ctx->stream>>>(d_err_htild, d_h_tild, d_mask01, H, mb, e, parts > 1 ? sums : grads->d_out_bias);  // :456
   ZR_LAUNCH_CHECK("attn_bwd_e_kernel");
   if ((rc = add_sums(grads->d_out_bias))) return rc;
-  const bool outer = zr_outer_takes(2, H, H, mb);
-  if (!outer) {
+  // All four weight gradients in one launch at the end, where d_c_t is still there by then and no two of them are added into the same memory
+  float* const dW[4] = {grads->d_W_c1, grads->d_W_c2, grads->d_W_p, grads->d_W_a};
+  bool joined = outer && !meets(d_err_h_t, sizeof(float) * n, d_c_t, sizeof(float) * n);
+  for (int i = 0; i < 4; ++i)
+    for (int k = 0; k < i; ++k) joined = joined && !meets(dW[i], sizeof(float) * (size_t)H * H, dW[k], sizeof(float) * (size_t)H * H);
+  if (!joined) {
     if ((rc = outer_acc(e, d_c_t, grads->d_W_c1))) return rc;                   // :437
     if ((rc = outer_acc(e, d_h_t, grads->d_W_c2))) return rc;                   // :443
   }
@@ -1318,13 +1326,13 @@ int zr_attn_backward(zr_ctx* ctx, zr_attn* a, const int* d_batch_info, const flo
   attn_bwd_vp_wp_kernel<<<row_blocks, 1024, 0, ctx->stream>>>(a->d_tanh1, a->v_p, col, H, mb, tw, parts > 1 ? sums : grads->d_v_p);  // :536
   ZR_LAUNCH_CHECK("attn_bwd_vp_wp_kernel");
   if ((rc = add_sums(grads->d_v_p))) return rc;
-  if (!outer && (rc = outer_acc(tw, d_h_t, grads->d_W_p))) return rc;           // :545
+  if (!joined && (rc = outer_acc(tw, d_h_t, grads->d_W_p))) return rc;           // :545
   if ((rc = product(a->W_p, 1, tw, d_err_h_t, 1, ZR_EPI_STORE))) return rc;     // :551
   attn_bwd_hs_kernel<<<dim3(mb, (H + 255) / 256), 256, 0, ctx->stream>>>(a->d_q, a->d_table, a->d_err_table, d_batch_info, d_indices, scal, H, mb,
                                                   W, a->longest_sent, hs_sum);
   ZR_LAUNCH_CHECK("attn_bwd_hs_kernel");
-  if (outer)  // all four weight gradients
-    rc = outer_launch(ctx, OuterProducts{{e, e, tw, d_h_t}, {d_c_t, d_h_t, d_h_t, hs_sum}, {grads->d_W_c1, grads->d_W_c2, grads->d_W_p, grads->d_W_a}}, 4, H, H, mb);
+  if (joined)
+    rc = outer_launch(ctx, OuterProducts{{e, e, tw, d_h_t}, {d_c_t, d_h_t, d_h_t, hs_sum}, {dW[0], dW[1], dW[2], dW[3]}}, 4, H, H, mb);
   else
     rc = outer_acc(d_h_t, hs_sum, grads->d_W_a);                                // :632
   if (rc) return rc;
