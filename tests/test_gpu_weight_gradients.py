@@ -56,3 +56,34 @@ def test_gradients_of_one_node_are_added(ctx, H, mb):
     check(out[0].get().reshape(H, 4 * H), dg, x, old[0].reshape(H, 4 * H).astype(np.float64))
     check(out[1].get().reshape(H, 4 * H), dg, h0, old[1].reshape(H, 4 * H).astype(np.float64))
     check(out[2].get()[None, :], dg, np.ones((mb, 1), np.float32), old[2][None, :].astype(np.float64))
+
+
+@pytest.mark.parametrize("H,T,mb", [(33, 5, 13), (100, 20, 20)])
+def test_results_that_share_memory_are_formed_one_after_another(ctx, H, T, mb):
+    dg, x, h0, h = operands(H, T, mb)
+    flat = lambda v: ctx.array(v.reshape(-1))
+    prev = np.concatenate([h0, h[:(T - 1) * mb]])
+    as_rows = lambda d: d.get().reshape(-1, order="F").reshape(H, 4 * H)
+    dM, dWh, db = ctx.empty((H, 4 * H)), ctx.empty((H, 4 * H)), ctx.empty((4 * H,))
+    ctx.lstm_weight_gradients(H, T, mb, flat(dg), flat(x), flat(h0), flat(h), dM, dM, db)  # the later one stays
+    ctx.sync()
+    check(as_rows(dM), dg, prev)
+    # over the columns that only it reads
+    n = max(T * mb * H, 4 * H * H)
+    x_and_dM = ctx.array(np.concatenate([x.reshape(-1), np.zeros(n - T * mb * H, np.float32)]))
+    ctx.lstm_weight_gradients(H, T, mb, flat(dg), x_and_dM, flat(h0), flat(h), x_and_dM, dWh, db)
+    ctx.sync()
+    check(x_and_dM.get()[:4 * H * H].reshape(H, 4 * H), dg, x)
+    check(as_rows(dWh), dg, prev)
+    check(db.get()[None, :], dg, np.ones((T * mb, 1), np.float32))
+
+
+@pytest.mark.parametrize("H,mb", [(5, 3), (64, 16), (100, 70)])
+def test_gradients_of_one_node_added_into_one_array(ctx, H, mb):
+    dg, x, h0, _ = operands(H, 1, mb)
+    flat = lambda v: ctx.array(v.reshape(-1))
+    dW, db = ctx.zeros((4 * H * H,)), ctx.zeros((4 * H,))
+    ctx.lstm_node_gradients(H, mb, flat(dg), flat(x), flat(h0), dW, dW, db)
+    ctx.sync()
+    check(dW.get().reshape(H, 4 * H), np.concatenate([dg, dg]), np.concatenate([x, h0]))
+    check(db.get()[None, :], dg, np.ones((mb, 1), np.float32))

@@ -1068,7 +1068,19 @@ static int weight_gradients(zr_ctx* ctx, int H, int T, int mb, const float* d_dg
   const long long K = (long long)T * mb;
   ZR_CHECK_ARG(K < (1LL << 31) / 4, "zr_lstm_weight_gradients: T * mb = %lld too large", K);
   void* scratch = nullptr;
-  if (zr_weight_gradients_takes(H, K, ctx->cu_count))
+  // (in one launch only results with memory of their own: the older routes write them one after another)
+  const size_t f = sizeof(float), hh = 4 * f * H * H, col = f * H;
+  const struct {
+    const float* p;
+    size_t bytes;
+  } out[3] = {{d_dM_stack, hh}, {d_dWh_stack, hh}, {d_db, 4 * col}},
+    in[4] = {{d_dgates, 4 * col * K}, {d_in_all, col * K}, {d_h0, col * mb}, {d_h_all, col * (K - mb)}};
+  bool apart = true;
+  for (int i = 0; i < 3; ++i) {
+    for (int k = 0; k < i; ++k) apart = apart && !meets(out[i].p, out[i].bytes, out[k].p, out[k].bytes);
+    for (int k = 0; k < 4; ++k) apart = apart && !meets(out[i].p, out[i].bytes, in[k].p, in[k].bytes);
+  }
+  if (apart && zr_weight_gradients_takes(H, K, ctx->cu_count))
     return zr_weight_gradients(ctx, H, (int)K, mb, d_dgates, d_in_all, d_h0, d_h_all, d_dM_stack, d_dWh_stack, d_db, accumulate);
   if (zr_split_gemm_takes(4 * H, H, (int)K)) {
     // the split product reads both operands as they lie; the previous states [h0, h_1 .. h_{T-1}] side by side
