@@ -127,3 +127,22 @@ def test_results_on_operands_take_the_launches_per_diagonal(ctx):
     compare(([by_column(x, T, mb, 4 * H) for x in dg], by_column(top, T, mb, H), [x.get() for x in eh], [by_column(x, mb, H) for x in cT]), want)
     for w in layers:
         ctx.lstm_train_destroy(w)
+
+
+def test_results_on_one_another_are_written_in_the_diagonals_order(ctx):
+    """One array for the error to every layer's initial h: the last layer's stays."""
+    L, H, mb, T = 3, 64, 8, 4
+    c = case(L, H, mb, T, True)
+    flat = lambda x: ctx.array(np.ascontiguousarray(np.swapaxes(x, -1, -2), np.float32).reshape(-1))
+    layers = [ctx.lstm_train_create([ctx.array(w) for w in c["M"][l]], [ctx.array(w) for w in c["Wh"][l]], H) for l in range(L)]
+    dg, ec, eh = [ctx.empty((T * mb * 4 * H,)) for _ in range(L)], [ctx.empty((H, mb)) for _ in range(L)], ctx.empty((H, mb))
+    ctx.lstm_stack_backward(layers, T, mb, ctx.array(c["mask"].reshape(-1)), [flat(x) for x in c["c0"]], [flat(x) for x in c["c"]],
+                            [flat(np.stack(g)) for g in c["gates"]], flat(c["top"]), dg, [eh] * L, ec, err_hT=[flat(x) for x in c["hT"]],
+                            err_cT=[flat(x) for x in c["cT"]])
+    ctx.sync()
+    want = reference(c, 0.0)
+    assert_close(eh.get(), want[2][L - 1], what="error to h_0 of the last layer")
+    for l in range(L):
+        assert_close(ec[l].get(), want[3][l], what="error to c_0, layer %d" % l)
+    for w in layers:
+        ctx.lstm_train_destroy(w)

@@ -838,19 +838,25 @@ bool meets(const float* a, size_t na, const float* b, size_t nb) {
   return a && b && (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
 }
 
-// Whether a result of a backward sweep lies on an operand: lstm_backward_redo_kernel reads the operands again.
+// Whether a result of a backward sweep lies on an operand (lstm_backward_redo_kernel reads those again) or on another result (the launches
+// per diagonal write them in one order).
 bool backward_overlaps(int nl, int H, int T, int mb, const float* const c0[], const float* const c[], const float* const gates[], const float* top,
                        const float* const hT[], const float* const cT[], float* const dg[], const float* below, float* const h0[], float* const ec0[]) {
   const size_t n = sizeof(float) * (size_t)H * mb;
-  auto on_operand = [&](const float* out, size_t bytes) {
-    bool hit = meets(out, bytes, top, n * T);
+  const float* out[1 + 3 * 16];
+  size_t bytes[1 + 3 * 16];
+  int results = 0;
+  auto result = [&](const float* p, size_t b) { out[results] = p, bytes[results++] = b; };
+  result(below, n * T);
+  for (int l = 0; l < nl; ++l) result(dg[l], 4 * n * T), result(h0[l], n), result(ec0[l], n);
+  bool hit = false;
+  for (int i = 0; i < results; ++i) {
+    for (int k = 0; k < i; ++k) hit = hit || meets(out[i], bytes[i], out[k], bytes[k]);
+    hit = hit || meets(out[i], bytes[i], top, n * T);
     for (int l = 0; l < nl; ++l)
-      hit = hit || meets(out, bytes, c0[l], n) || meets(out, bytes, c[l], n * T) || meets(out, bytes, gates[l], 4 * n * T) ||
-            (hT && meets(out, bytes, hT[l], n)) || (cT && meets(out, bytes, cT[l], n));
-    return hit;
-  };
-  bool hit = on_operand(below, n * T);
-  for (int l = 0; l < nl; ++l) hit = hit || on_operand(dg[l], 4 * n * T) || on_operand(h0[l], n) || on_operand(ec0[l], n);
+      hit = hit || meets(out[i], bytes[i], c0[l], n) || meets(out[i], bytes[i], c[l], n * T) || meets(out[i], bytes[i], gates[l], 4 * n * T) ||
+            (hT && meets(out[i], bytes[i], hT[l], n)) || (cT && meets(out[i], bytes[i], cT[l], n));
+  }
   return hit;
 }
 
