@@ -70,13 +70,18 @@ int zr_ctx_set_option(zr_ctx* ctx, int option, int value);
  *     that has only served calls that allocate nothing).  Does not wait.
  *   ZR_QUERY_ATTN_PATH: which schedule the last zr_attn_step (or the attention part of zr_decoder_step) on this
  *     context took -- 0 none yet, ZR_ATTN_PATH_SINGLE_LAUNCH, ZR_ATTN_PATH_THREE_LAUNCHES or ZR_ATTN_PATH_SEPARATE.
- *     Does not wait. */
+ *     Does not wait.
+ *   ZR_QUERY_WAITS_REPAIRED: waits for the stream; which of the last launches gave up a wait and formed what it had waited
+ *     for again (the results are right all the same): ZR_REPAIRED_SGD_UPDATE, the last clipped update of one matrix in one
+ *     launch. */
 int zr_ctx_query(zr_ctx* ctx, int what, int* h_value);
 #define ZR_QUERY_LSTM_STACK_PATH 1
 #define ZR_QUERY_LSTM_SWEEP_ABANDONED 2
 #define ZR_QUERY_ATTN_PATH 3
 #define ZR_QUERY_SCRATCH_KIB 4
 #define ZR_QUERY_LSTM_SWEEP_KERNEL 5
+#define ZR_QUERY_WAITS_REPAIRED 6
+#define ZR_REPAIRED_SGD_UPDATE 1
 #define ZR_LSTM_SWEEP_STREAMED 1 /* weights streamed from the caches in every time step */
 #define ZR_LSTM_SWEEP_RESIDENT 2 /* weights held in registers */
 #define ZR_ATTN_PATH_SINGLE_LAUNCH 1  /* projections, window / scores / context and output product in one launch */
@@ -112,7 +117,9 @@ const char* zr_version(void);
                                         one does.  The environment variable ZR_LSTM_SWEEP presets this option for every
                                         context created */
 #define ZR_OPT_LSTM_SWEEP_SPIN 8     /* polls a workgroup of that launch spends on one wait before it gives up
-                                        (0 = default, about a second); giving up is reported by zr_ctx_sync */
+                                        (0 = default, about a second); giving up is reported by zr_ctx_sync.  Also the
+                                        polls of the clipped update in one launch (0 = 4096), whose workgroups then form the
+                                        norm from the whole gradient: to the same bits, reported by ZR_QUERY_WAITS_REPAIRED only */
 
 #define ZR_OPT_BF16_ACTIVATION_TERMS 9 /* products against bf16 weights (zr_lstm_pack_weights_bf16, zr_softmax_prepare_bf16,
                                         zr_attn_use_bf16_weights): 2 (default) = every fp32 activation enters as two
@@ -122,7 +129,8 @@ const char* zr_version(void);
 #define ZR_OPT_LSTM_STEP_WAIT_EXTRA 10 /* for tests of the give-up path of zr_lstm_decoder_step's single launch: the
                                         waits of a layer for the layer below expect this many arrivals more than there
                                         will be, so each of them runs to ZR_OPT_LSTM_SWEEP_SPIN polls and gives up
-                                        whatever the timing (0 = off, the default) */
+                                        whatever the timing (0 = off, the default); the waits of the clipped update in one
+                                        launch likewise */
 #define ZR_OPT_ATTN_SINGLE_LAUNCH 11 /* the attention step as ONE launch whose workgroups hand over through device
                                         memory (prepared fp32 matrices, H a multiple of 8 up to 1024, at most 64 window
                                         slots, all workgroups resident at once, own stream, only context on the

@@ -1,6 +1,6 @@
 """The clipped update in one launch whose workgroups exchange their sums (sgd_fused_kernel in csrc/zr_backward.hip): edges of its workgroups and of the
 sizes that take two, four and eight accesses a thread, any alignment, waits that are given up, and launch numbers that start again.
-Tolerance as in test_gpu_sgd_small.py (the sum's last 16 bits, 2^-37 of it, are nothing beside the norm's rounding to fp32)."""
+Tolerance as in test_gpu_sgd_small.py; the same bits whether or not a wait was given up."""
 import numpy as np
 import pytest
 
@@ -72,3 +72,58 @@ def test_non_finite_gradients(ctx, special):
     # a norm that is no number is not above the threshold (the plain step); an infinite one makes every finite step zero, the infinite one NaN
     step = np.where(np.isnan(g), np.nan, np.float32(0.1)) if np.isnan(special) else np.where(np.isinf(g), np.nan, 0.0)
     assert np.array_equal(dw.get(), (np.float32(1) + step).astype(np.float32), equal_nan=True)
+
+
+def test_the_sum_keeps_its_64_bits(ctx):
+    """A gradient of two values whose norm lies just above the middle of two floats: the sum of squares with 37 bits would round the other way."""
+    r = np.random.default_rng(5)
+    x, y = (r.uniform(1, 2, 1 << 20).astype(np.float32) for _ in range(2))
+    total = x.astype(np.float64) ** 2 + y.astype(np.float64) ** 2
+    short = (total.view(np.uint64) & ~np.uint64(0xffff)).view(np.float64)
+    norm = lambda s: np.sqrt(s).astype(np.float32)
+    step = lambda s, v: (np.float32(1.0) / norm(s)) * v
+    at = np.flatnonzero((step(total, x) != step(short, x)) | (step(total, y) != step(short, y)))
+    assert len(at) >= 8
+    for i in at[:8]:
+        g = np.zeros(40000, np.float32)
+        g[7], g[11] = x[i], y[i]
+        w = ctx.zeros((40000,))
+        ctx.sgd_update(w, ctx.array(g), 40000, 1.0, 1.0, 1.0)
+        ctx.sync()
+        got = w.get()
+        assert (got[7], got[11]) == (step(total[i:i + 1], x[i])[0], step(total[i:i + 1], y[i])[0])
+
+
+@pytest.mark.parametrize("n", [28001, 40000, 250001, M + 3, 4 * M])
+def test_workgroups_that_gave_up_arrive_at_the_same_bits(ctx, n):
+    r = np.random.default_rng(n)
+    w, g = r.uniform(-1, 1, n).astype(np.float32), ctx.array(r.normal(0, 3, n).astype(np.float32))
+    got = []
+    for extra in (0, 3):  # (waits for a number that is never stored)
+        ctx.set_option(capi.ZR_OPT_LSTM_STEP_WAIT_EXTRA, extra)
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 50 if extra else 0)
+        try:
+            dw = ctx.array(w)
+            ctx.sgd_update(dw, g, n, 0.05, 0.5, 0.7)
+            repaired = ctx.query(capi.ZR_QUERY_WAITS_REPAIRED)
+            got.append(dw.get())
+        finally:
+            ctx.set_option(capi.ZR_OPT_LSTM_STEP_WAIT_EXTRA, 0)
+            ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)
+        assert repaired == (capi.ZR_REPAIRED_SGD_UPDATE if extra else 0)
+    assert np.array_equal(got[0], got[1])
+
+
+def test_beside_another_context_two_launches(ctx):
+    """No waits where another context's work may hold the compute units."""
+    check(ctx, 250000, 0, 0, 0.5)
+    ctx.set_option(capi.ZR_OPT_LSTM_STEP_WAIT_EXTRA, 3)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 50)
+    other = capi.Context(0)
+    try:
+        check(ctx, 250000, 0, 0, 0.5)
+        assert ctx.query(capi.ZR_QUERY_WAITS_REPAIRED) == 0
+    finally:
+        other.close()
+        ctx.set_option(capi.ZR_OPT_LSTM_STEP_WAIT_EXTRA, 0)
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)

@@ -465,102 +465,123 @@ __global__ void __launch_bounds__(1024) sgd_small_kernel(float* __restrict__ W, 
   for (i = 4 * n4 + first; i < n; i += stride) W[i] += f * g[i];
 }
 
-// The update of a matrix of up to two million values (ZR_CLIP_MATRIX_NORM) in one launch: a workgroup keeps its values of the gradient
+// The update of a matrix of up to four million values (ZR_CLIP_MATRIX_NORM) in one launch: a workgroup keeps its values of the gradient
 // and of W in registers, leaves its sum of squares in a slot and waits for those of the others, which every workgroup adds up in the same
-// order.  A slot is one 64-bit word: a sum, whose last 16 bits (2^-37 of it) are the launch's number, so that nothing has to be ordered
-// between two stores and nothing cleared.  A workgroup that waits too long (others hold the compute units) forms the norm from the whole
-// gradient itself, which nobody writes.  W and g do not overlap.
-// Bound by the trips: to memory for the values, to a slot and back: a 500 x 500 matrix 4.9 us against 7.0 in two launches, 1000 x 1000 6.8 against 8.4.
+// order.  A slot is two 64-bit words: the halves of a sum, each behind the launch's number, so that nothing has to be ordered
+// between two stores and nothing cleared.  A workgroup that waits too long (others hold the compute units) forms the others' sums itself, from the
+// gradient, which nobody writes, just as they do: every value of the matrix is scaled by the same factor either way.  W and g do not overlap.
+// Bound by the trips: to memory for the values, to a slot and back: a 500 x 500 matrix 4.8 us a call against 7.3 in two launches, 1000 x 1000 5.6 against 7.3.
+// (With 48-bit sums in one word each 5.0 and 6.2.)
 // (With a count of departures instead of the number 9.0 and 23.6: hundreds of additions to one word.)
+typedef float sgd_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// The values of workgroup `group`: 4 * U of every thread, zeros behind the end.
 template <int U>
-__global__ void __launch_bounds__(kSgdThreads) sgd_fused_kernel(float* __restrict__ W, const float* __restrict__ g, long long n, float scale, float threshold,
-                                                                float lr, unsigned long long* __restrict__ slots, unsigned epoch, int spin_limit) {
-  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-  constexpr int WAVES = kSgdThreads / 64;
-  __shared__ double s[WAVES];
-  __shared__ double s_total;
-  __shared__ int s_alone;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, groups = (int)gridDim.x;
-  const long long first = 4 * ((long long)blockIdx.x * U * kSgdThreads + tid);
-  f32x4u x[U], w[U];
+__device__ __forceinline__ void sgd_load(const float* __restrict__ from, long long n, int group, sgd_f32x4 (&x)[U]) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const long long i = first + 4LL * kSgdThreads * u;
-    x[u] = w[u] = f32x4u{0.0f, 0.0f, 0.0f, 0.0f};
+    const long long i = 4 * (((long long)group * U + u) * kSgdThreads + threadIdx.x);
+    x[u] = sgd_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     if (i + 4 <= n) {
-      x[u] = *(const f32x4u*)(g + i);
+      x[u] = *(const sgd_f32x4*)(from + i);
     } else {
 #pragma unroll
       for (int e = 0; e < 3; ++e)
-        if (i + e < n) x[u][e] = g[i + e];
+        if (i + e < n) x[u][e] = from[i + e];
     }
   }
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const long long i = first + 4LL * kSgdThreads * u;
-    if (i + 4 <= n) {
-      w[u] = *(const f32x4u*)(W + i);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 3; ++e)
-        if (i + e < n) w[u][e] = W[i + e];
-    }
-  }
-  auto workgroup_sum = [&](double v) {  // on thread 0; the others' values differ
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) s[wave] = v;
-    __syncthreads();
-    v = 0.0;
-#pragma unroll
-    for (int q = 0; q < WAVES; ++q) v += s[q];
-    return v;
-  };
+}
+
+// The sum of the workgroup's squares, on every thread.  s: a double for each wave.
+template <int U>
+__device__ __forceinline__ double sgd_squares(const sgd_f32x4 (&x)[U], double* s) {
   double acc[4] = {};
 #pragma unroll
   for (int u = 0; u < U; ++u)
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] += (double)x[u][e] * (double)x[u][e];
-  double total = workgroup_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
-  if (groups > 1) {
-    if (tid == 0) {
-      unsigned long long bits = (unsigned long long)__double_as_longlong(total);
-      if (total != total) bits = 0x7ff8000000000000ull;  // (its payload may be in the last bits)
-      __hip_atomic_store(slots + blockIdx.x, (bits & ~0xffffull) | epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  double v = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = 0.0;
+#pragma unroll
+  for (int q = 0; q < kSgdThreads / 64; ++q) v += s[q];
+  return v;
+}
+
+// expected: the number that is waited for, `epoch` but in tests.  gave_up: set to `epoch` where a wait was given up.
+template <int U>
+__global__ void __launch_bounds__(kSgdThreads) sgd_fused_kernel(float* __restrict__ W, const float* __restrict__ g, long long n, float scale, float threshold,
+                                                                float lr, unsigned long long* __restrict__ slots, unsigned epoch, unsigned expected,
+                                                                int* __restrict__ gave_up, int spin_limit) {
+  __shared__ double s[kSgdThreads / 64];
+  __shared__ double s_parts[kSgdSlots];
+  __shared__ double s_total;
+  __shared__ int s_alone;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, groups = (int)gridDim.x;
+  sgd_f32x4 x[U], w[U];
+  sgd_load<U>(g, n, (int)blockIdx.x, x);
+  sgd_load<U>(W, n, (int)blockIdx.x, w);
+  const double mine = sgd_squares<U>(x, s);
+  if (tid < 2) {  // the high half first
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(mine);
+    __hip_atomic_store(slots + 2 * blockIdx.x + tid, (unsigned long long)epoch << 32 | (tid ? bits & 0xffffffffu : bits >> 32), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  }
+  auto total_of = [&](auto&& part) {  // on every lane of a wave
+    double sum = 0.0;
+    for (int i = lane; i < groups; i += 64) sum += part(i);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    return sum;
+  };
+  if (wave == 0) {
+    bool all = true;
+    int spins = 0;
+    const double sum = total_of([&](int i) {
+      unsigned long long hi, lo;
+      for (;;) {
+        hi = __hip_atomic_load(slots + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lo = __hip_atomic_load(slots + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (hi >> 32 == expected && lo >> 32 == expected) break;
+        if (++spins >= spin_limit) {
+          all = false;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      return __longlong_as_double((long long)(hi << 32 | (lo & 0xffffffffu)));
+    });
+    const bool got = __all(all);
+    if (lane == 0) s_total = sum, s_alone = got ? 0 : 1;
+  }
+  __syncthreads();
+  if (s_alone) {
+    if (tid == 0) __hip_atomic_store(gave_up, (int)epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int q = 0; q < groups; ++q) {
+      sgd_f32x4 y[U];
+      sgd_load<U>(g, n, q, y);
+      const double part = sgd_squares<U>(y, s);
+      if (tid == 0) s_parts[q] = part;
+      __syncthreads();
     }
     if (wave == 0) {
-      double sum = 0.0;
-      bool all = true;
-      int spins = 0;
-      for (int i = lane; i < groups; i += 64) {
-        unsigned long long bits;
-        while (((bits = __hip_atomic_load(slots + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & 0xffffu) != epoch && ++spins < spin_limit)
-          __builtin_amdgcn_s_sleep(1);
-        all = all && (bits & 0xffffu) == epoch;
-        sum += __longlong_as_double((long long)(bits & ~0xffffull));
-      }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-      const bool got = __all(all);
-      if (lane == 0) s_total = sum, s_alone = got ? 0 : 1;
+      const double sum = total_of([&](int i) { return s_parts[i]; });
+      if (lane == 0) s_total = sum;
     }
     __syncthreads();
-    total = s_total;
-    if (s_alone) {
-      double a = 0.0;
-      for (long long i = tid; i < n; i += kSgdThreads) a += (double)g[i] * (double)g[i];
-      total = workgroup_sum(a);
-    }
   }
-  const float norm = (float)sqrt(total) * fabsf(scale);
+  const float norm = (float)sqrt(s_total) * fabsf(scale);
   const float f = lr * (norm > threshold ? threshold / norm : 1.0f) * scale;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const long long i = first + 4LL * kSgdThreads * u;
+    const long long i = 4 * (((long long)blockIdx.x * U + u) * kSgdThreads + tid);
 #pragma unroll
     for (int e = 0; e < 4; ++e) w[u][e] += f * x[u][e];
     if (i + 4 <= n) {
-      *(f32x4u*)(W + i) = w[u];
+      *(sgd_f32x4*)(W + i) = w[u];
     } else {
 #pragma unroll
       for (int e = 0; e < 3; ++e)
@@ -1610,17 +1631,19 @@ int zr_sgd_update_clipped(zr_ctx* ctx, float* d_W, const float* d_grad, long lon
   if (n == 0) return ZR_OK;
   const int vec = aligned16(d_W) && aligned16(d_grad) ? 1 : 0;
   const bool apart = (uintptr_t)(d_W + n) <= (uintptr_t)d_grad || (uintptr_t)(d_grad + n) <= (uintptr_t)d_W;
-  if (clip_mode == ZR_CLIP_MATRIX_NORM && apart && ctx->stream == ctx->own_stream) {  // (its slots are the context's)
+  // (the slots are the context's; beside another context's work the waits could run out)
+  if (clip_mode == ZR_CLIP_MATRIX_NORM && apart && ctx->stream == ctx->own_stream && zr_live_contexts(ctx->device) == 1) {
     if (const int u = zr_sgd_fused_accesses(n)) {
       const unsigned groups = (unsigned)((n + 4LL * kSgdThreads * u - 1) / (4 * kSgdThreads * u));
       if (++ctx->sgd_epoch > 0xffff) {  // (no slot may hold the number of a launch long past)
-        rc = zr_memset_zero(ctx, ctx->d_sgd_slots, kSgdSlots * sizeof(unsigned long long));
-        if (rc) return rc;
+        if ((rc = zr_memset_zero(ctx, ctx->d_sgd_slots, 2 * kSgdSlots * sizeof(unsigned long long)))) return rc;
+        if ((rc = zr_memset_zero(ctx, ctx->d_flags + 5, sizeof(int)))) return rc;
         ctx->sgd_epoch = 1;
       }
       const int spin = ctx->sweep_spin > 0 ? ctx->sweep_spin : 4096;
       auto kernel = u == 2 ? sgd_fused_kernel<2> : (u == 4 ? sgd_fused_kernel<4> : sgd_fused_kernel<8>);
-      kernel<<<groups, kSgdThreads, 0, ctx->stream>>>(d_W, d_grad, n, scale, threshold, learning_rate, ctx->d_sgd_slots, (unsigned)ctx->sgd_epoch, spin);
+      kernel<<<groups, kSgdThreads, 0, ctx->stream>>>(d_W, d_grad, n, scale, threshold, learning_rate, ctx->d_sgd_slots, (unsigned)ctx->sgd_epoch,
+                                                      (unsigned)(ctx->sgd_epoch + ctx->step_wait_extra), ctx->d_flags + 5, spin);
       ZR_LAUNCH_CHECK("sgd_fused_kernel");
       return ZR_OK;
     }

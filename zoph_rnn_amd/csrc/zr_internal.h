@@ -27,8 +27,8 @@ struct zr_ctx {
   int lstm_kernel;   // 0 auto, 1 register-streaming kernel, 2 LDS / split-K kernel
   int lstm_kparts;   // K parts per segment for the split-K kernel (0 auto)
   int* d_counters;   // ZR_MAX_COUNTERS arrival counters, zero between launches
-  unsigned long long* d_sgd_slots;  // kSgdSlots sums of sgd_fused_kernel's workgroups, their last 16 bits the launch's number
-  int sgd_epoch;                    // that number of the last launch, 1 to 65535
+  unsigned long long* d_sgd_slots;  // kSgdSlots sums of sgd_fused_kernel's workgroups, two words each: the launch's number and half of the sum
+  int sgd_epoch;                    // that number of the last launch, 1 to 65535; d_flags[5] holds it where workgroups of that launch gave up
   int* d_step_flags; // ZR_MAX_STEP_FLAGS flags of lstm_resident_kernel (the first 32 hold its departure count), zero between launches
   int lstm_sweep;    // whole-sweep LSTM kernels: 0 auto, 1 never, 2 / 3 streamed / resident weights whenever the launch fits
   int sweep_spin;    // polls before a waiting workgroup of that kernel gives up (0: default)

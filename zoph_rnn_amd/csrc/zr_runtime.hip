@@ -202,7 +202,7 @@ int zr_ctx_create(int device, zr_ctx** out) {
     return zr_set_error(ZR_EHIP, "hipStreamCreate failed: %s", hipGetErrorString(e));
   }
   c->stream = c->own_stream;
-  const size_t flag_bytes = (32 + ZR_MAX_COUNTERS + ZR_MAX_STEP_FLAGS) * sizeof(int), slot_bytes = kSgdSlots * sizeof(unsigned long long);
+  const size_t flag_bytes = (32 + ZR_MAX_COUNTERS + ZR_MAX_STEP_FLAGS) * sizeof(int), slot_bytes = 2 * kSgdSlots * sizeof(unsigned long long);
   e = hipMalloc((void**)&c->d_flags, flag_bytes + slot_bytes);
   if (e != hipSuccess) {
     (void)hipStreamDestroy(c->own_stream);
@@ -318,6 +318,15 @@ int zr_ctx_query(zr_ctx* ctx, int what, int* h_value) {
       // the caller's data; all four go down together, and the caller's re-run starts from a clean slate.
       if (flag != 0) ZR_HIP(hipMemset(ctx->d_flags, 0, 4 * sizeof(int)));
       *h_value = flag != 0 ? 1 : 0;
+      return ZR_OK;
+    }
+    case ZR_QUERY_WAITS_REPAIRED: {
+      int rc = zr_bind_device(ctx);
+      if (rc) return rc;
+      ZR_HIP(hipStreamSynchronize(ctx->stream));
+      int gave_up[2] = {0, 0};
+      ZR_HIP(hipMemcpy(gave_up, ctx->d_flags + 4, sizeof(gave_up), hipMemcpyDeviceToHost));
+      *h_value = ctx->sgd_epoch && gave_up[1] == ctx->sgd_epoch ? ZR_REPAIRED_SGD_UPDATE : 0;
       return ZR_OK;
     }
     default:
