@@ -52,3 +52,31 @@ def test_infinite_logits(ctx):
     ctx.softmax_forward(dD, ctx.array(b), V, H, dh, n, capi.ZR_SOFTMAX_PROB, p)
     ctx.sync()
     assert np.all(p.get()[off] == 0.0) and np.allclose(p.get()[~off], 1.0 / np.sum(~off), rtol=1e-6)
+
+
+def fold_of_one_large_logit(e, block):
+    """The sum of 256 blocks, one a thread, in the kernels' order: 32 e each, but 1 in `block`."""
+    p = np.full(256, np.float32(32) * np.float32(e), np.float32)
+    p[block] = 1
+    w, lanes = p.reshape(4, 64), np.arange(64)
+    for off in (32, 16, 8, 4, 2, 1):
+        w = w + w[:, lanes ^ off]
+    return (w[0, 0] + w[1, 0]) + (w[2, 0] + w[3, 0])
+
+
+@pytest.mark.parametrize("d", [9.732, 9.7779999, 10.41, 10.5, 10.782])
+def test_blocks_far_below_one_large_logit(ctx, d):
+    """The blocks' exponentials are those of expf, within one unit in the last place: exp2 of the rounded d * log2 e is off by 5 to 8 of them at
+    these distances, all in the same direction."""
+    V, H, block = 8192, 16, 77
+    d = np.float32(d)
+    b = np.zeros(V, np.float32)
+    b[32 * block:32 * block + 32] = -1e30  # (nothing beside the one)
+    b[32 * block + 3] = d
+    out = ctx.empty((V + 2,))
+    ctx.softmax_forward(ctx.zeros((V, H)), ctx.array(b), V, H, ctx.zeros((H, 1)), 1, capi.ZR_SOFTMAX_LOGITS, out)
+    ctx.sync()
+    mx, total = out.get()[V:]
+    e = np.float32(np.exp(-np.float64(d)))
+    assert mx == d
+    assert fold_of_one_large_logit(np.nextafter(e, np.float32(0)), block) <= total <= fold_of_one_large_logit(np.nextafter(e, np.float32(1)), block)

@@ -188,17 +188,19 @@ inline bool zr_back_takes(const ZrBackPlan& plan, int nl) { return plan.at_once 
 
 // ---- normalising the output matrix (softmax_normalize_kernel): 16-byte accesses a thread, and whether its workgroups fold the block pairs
 
-// Every workgroup folds its column's V / 32 pairs: cheaper than a launch for it until there are some 2.5 million to fold, us folding /
-// in two launches: 30001 x 256 (1.9) 14.4 / 15.5, 50000 x 128 (2.6 with four accesses) 15.0 / 15.2, 80000 x 64 (3.2) 14.4 / 13.4, 10000 x 3000 (2.8) 44 / 41, 50000
-// x 256 (5.2) 20.9 / 20.5.  Two accesses a thread, 40000 x 64 10.2 against 10.8 with four; four where columns start at odd
-// addresses: 30011 x 37 5.6 against 6.4.
+// Every workgroup folds its column's V / 32 pairs: cheaper than a launch for it until there are some 1.25 million to fold (counted for four accesses a
+// thread), 2.2 million up to 32768 rows, a few pairs a thread.  us behind the product, folding with two accesses a thread / with four / in a launch of its own: 50000 x 48 (0.98)
+// 10.5 / 10.8 / 11.0, 40000 x 96 (1.2) 13.8 / 14.1 / 13.3, 50000 x 64 (1.3) 12.7 / 13.4 / 12.5, 80000 x 64 (3.2) 15.1 / 14.9 / 13.6; 30000 x 128 (0.96) 14.2 / 10.2 / 13.6,
+// 20000 x 600 (1.9) 22.1 / 19.0 / 21.0, 30001 x 384 (2.9) 20.5 / 20.4 / 19.0.  Two accesses where there is little to fold, 50000 x 1 3.7 / 4.2; four where columns start
+// at odd addresses: 30011 x 37 6.7 / 5.7.
 struct ZrNormalizePlan {
   int accesses;
   bool fold;
 };
 inline ZrNormalizePlan zr_softmax_normalize_plan(int V, int n) {
-  if ((double)((V + 4095) / 4096) * n * ((V + 31) / 32) > 2.7e6) return {2, false};
-  return {V <= 1024 ? 1 : (V % 4 ? 4 : 2), true};
+  const double folds = (double)((V + 4095) / 4096) * n * ((V + 31) / 32);
+  if (folds > (V <= 32768 ? 2.2e6 : 1.25e6)) return {2, false};
+  return {V <= 1024 ? 1 : (V % 4 || folds > 0.9e6 ? 4 : 2), true};
 }
 
 // ---- the output layer's error pass (softmax_error_kernel): columns a workgroup adds up, one after another

@@ -24,9 +24,9 @@ softmax_colstats_kernel(const float* __restrict__ partials, int nblocks, float* 
 // out = exp(x - max) / sum   (MODE 0)   or   (x - max) - log(sum)   (MODE 1); in and out may be the same matrix.  A
 // workgroup takes 1024 * U rows of one column, U 16-byte accesses a thread at any alignment.  FOLD: it folds the column's block pairs itself,
 // while its logits are on their way, which saves the launch of softmax_colstats_kernel; else `pairs` holds that one's statistics.
-// Both launches before / this one, us: 10000 x 8 6.0 -> 3.9, 30011 x 37 (odd columns had 4-byte accesses) 8.9 -> 5.6, 40000 x 64 11.4 ->
-// 10.2, 50000 x 128 16.1 -> 15.0.  Bound by memory from there on, with the statistics in a launch of their own: 80000 x 256 30 us, the fold
-// by every workgroup 34; 80001 x 256 41.7 -> 29.8 by the accesses' width.
+// Both launches before / this one, us: 10000 x 8 6.0 -> 2.8, 30011 x 37 (odd columns had 4-byte accesses) 8.9 -> 5.7, 40000 x 64 11.6 -> 10.8,
+// 30000 x 128 14.3 -> 10.2.  Bound by memory from there on, with the statistics in a launch of their own: 50000 x 128 15.4 us, the fold by every workgroup 16.4; 80000 x 256
+// 29.6 and 34.5; 80001 x 256 41.4 -> 30.1 by the accesses' width.
 template <int MODE, int U, bool FOLD>
 __global__ void __launch_bounds__(256)
 softmax_normalize_kernel(const float* in, float* out, int V, const float* __restrict__ pairs, int nblocks) {

@@ -8,7 +8,8 @@
 
 // All 256 threads of a workgroup call this with the column's pairs ([nblocks][2] floats, contiguous) and have the column's (max,
 // sum) on return.  The maximum first, then every block's sum scaled to it once: one exponential a pair, where a running pair
-// takes two for every pair and for every step of the butterfly.  `behind_loads` is called once the first 2048 pairs are on
+// takes two for every pair and for every step of the butterfly.  (expf: in a column with all blocks a distance d below one large logit the
+// errors have one sign, and exp2 of a rounded d * log2 e is off by d * 2^-24.)  `behind_loads` is called once the first 2048 pairs are on
 // their way; returns the largest block maximum this thread saw (-inf if none).  s_m, s_s: four floats of shared memory each.
 template <class F>
 __device__ __forceinline__ float zr_softmax_fold_column(const float* __restrict__ pairs, int nblocks, float* s_m, float* s_s,
@@ -36,7 +37,7 @@ __device__ __forceinline__ float zr_softmax_fold_column(const float* __restrict_
   __syncthreads();
   mx = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
   // (a block at the maximum counts as it is: also where both are infinite)
-  auto scaled = [&](const zr_f32x2& p) { return p.x == mx ? p.y : p.y * __builtin_amdgcn_exp2f((p.x - mx) * 1.4426950408889634f); };
+  auto scaled = [&](const zr_f32x2& p) { return p.x == mx ? p.y : p.y * expf(p.x - mx); };
   float s = 0.0f;
 #pragma unroll
   for (int u = 0; u < 8; ++u)
