@@ -141,6 +141,10 @@ const char* zr_version(void);
                                         left).  The streamed sweep needs 6 * (L * (T + 1) + T) * H bytes a column (columns in
                                         eights), the resident one 4 * L * (T + 1) * H; a schedule there is no memory for
                                         is passed over, with ZR_OPT_LSTM_SWEEP = 2 and 3 too */
+#define ZR_OPT_KEEP_MEMORY 13 /* 1 (default): device memory of destroyed handles and of zr_free stays with the context for its
+                                 next requests, at most 32 blocks and 512 MiB, while it is the only context on its
+                                 device and has never been given a stream; 0: what is kept goes back to the device now,
+                                 and nothing is kept from then on */
 
 /* full_matrix_setup / cudaMalloc / cudaMemcpy / cudaMemset call sites (src/BZ_CUDA_UTIL.h:358-399 and the
  * layer constructors, e.g. src/LSTM.hpp:23-42). */

@@ -110,3 +110,67 @@ def test_nothing_is_kept_with_another_context_or_stream(ctx):
     assert torch.cuda.mem_get_info()[0] - before >= 40 << 20
     ctx.sync()
     capi._chk(capi.load().zr_ctx_set_stream(ctx.h, None))
+
+
+def free_bytes():
+    return torch.cuda.mem_get_info()[0]
+
+
+MIB = 1 << 20
+
+
+def keep(ctx, mib, blocks=1):
+    for b in [ctx.empty((mib << 18,)) for _ in range(blocks)]:
+        b.free()
+
+
+def test_another_context_has_what_was_kept_given_back(ctx):
+    keep(ctx, 200)
+    before = free_bytes()
+    other = capi.Context(0)
+    assert free_bytes() - before >= 150 * MIB
+    other.close()
+
+
+def test_an_output_layer_is_prepared_with_memory_that_was_kept(ctx):
+    """Memory for the copy of the matrix, which is no kept block's size, only with what the context keeps."""
+    V, H = 380000, 1000
+    need = (V + 31) // 32 * 32 * H * 4
+    D = torch.zeros((H, V), device="cuda")
+    torch.cuda.synchronize()
+    keep(ctx, 200, 2)
+    hog = []
+    try:
+        while free_bytes() > need - 150 * MIB and len(hog) < 8:
+            hog.append(torch.empty(free_bytes() - need + 200 * MIB, dtype=torch.uint8, device="cuda"))
+        assert free_bytes() < need
+        ctx.softmax_prepare(D.data_ptr(), V, H)
+        ctx.sync()
+        ctx.softmax_release(D.data_ptr())
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+
+
+def test_nothing_is_kept_without_the_option(ctx):
+    keep(ctx, 200)
+    before = free_bytes()
+    ctx.set_option(capi.ZR_OPT_KEEP_MEMORY, 0)
+    assert free_bytes() - before >= 150 * MIB
+    a = ctx.empty((50 << 20,))
+    before = free_bytes()
+    a.free()
+    assert free_bytes() - before >= 150 * MIB
+    ctx.set_option(capi.ZR_OPT_KEEP_MEMORY, 1)
+
+
+def test_freeing_waits_for_work_on_any_stream(ctx):
+    a = ctx.empty((1 << 20,))
+    s = torch.cuda.Stream()
+    done = torch.cuda.Event()
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(100_000_000)
+        done.record()
+    assert not done.query()
+    a.free()
+    assert done.query()

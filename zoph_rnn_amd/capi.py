@@ -24,6 +24,7 @@ ZR_OPT_BF16_ACTIVATION_TERMS = 9
 ZR_OPT_LSTM_STEP_WAIT_EXTRA = 10
 ZR_OPT_ATTN_SINGLE_LAUNCH = 11
 ZR_OPT_LSTM_SWEEP_SCRATCH = 12
+ZR_OPT_KEEP_MEMORY = 13
 ZR_QUERY_LSTM_STACK_PATH = 1
 ZR_QUERY_LSTM_SWEEP_ABANDONED = 2
 ZR_QUERY_ATTN_PATH = 3

@@ -62,6 +62,7 @@ struct zr_ctx {
   int n_kept;
   size_t kept_bytes;
   int foreign_stream;  // a caller's stream has been set once: nothing is kept any more
+  int keep_memory;     // ZR_OPT_KEEP_MEMORY
   void* h_pinned;      // page-locked host memory that kernels write small results to (grown on demand)
   size_t pinned_bytes;
   // the device's statically allocated scratch array (zr_runtime.hip), resolved when the context is created
@@ -109,8 +110,12 @@ int zr_live_contexts(int device);
 // Device memory of a handle: hipMalloc, or a kept block of about the size.  May hold anything, and what is queued on ctx's own
 // stream may still use it (any_stream: nothing queued anywhere uses it).  nullptr: no memory.
 void* zr_dev_alloc(zr_ctx* ctx, size_t bytes, bool any_stream = false);
-// Gives it back, or keeps it; `idle` as for a kept block.  Null is fine.
-int zr_dev_free(zr_ctx* ctx, void* p, bool idle = false);
+// Gives it back, or keeps it; callers: memory that a caller held, for whose streams this waits.  Null is fine.
+int zr_dev_free(zr_ctx* ctx, void* p, bool callers = false);
+// Gives memory of zr_dev_alloc back to the device (nothing is kept, nothing waited for but by hipFree).
+int zr_dev_release(void* p);
+// Gives back what the contexts on a device (or only one of them) keep; how many blocks.
+int zr_give_back_kept(int device, zr_ctx* only);
 // At least `bytes` of page-locked host memory, good until the next call; *dev is where a kernel finds it.
 int zr_ctx_pinned(zr_ctx* ctx, size_t bytes, void** host, void** dev);
 // Returns a context-owned scratch buffer of at least `bytes` (slot 0 or 1).

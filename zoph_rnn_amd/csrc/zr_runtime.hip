@@ -4,8 +4,11 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <unordered_map>
+#include <vector>
 
 #include "zr_internal.h"
 
@@ -62,57 +65,162 @@ int zr_bind_device(zr_ctx* ctx) {
 // that comes, is on the context's own stream: nothing is kept where a caller's stream has ever been set or another context is alive.
 // What callers hold themselves (zr_malloc) may be in use on any stream of theirs, so zr_free waits for the device as hipFree
 // did, and zr_malloc for this stream where it hands out a handle's block.
+// A second context on the device, and every allocation that fails, has the blocks of all contexts there given back first.
 constexpr size_t kKeptTotal = (size_t)512 << 20, kKeptLargest = (size_t)256 << 20;
 
-static void drop_kept(zr_ctx* ctx, int i) {
-  (void)hipFree(ctx->kept[i].p);  // (waits for the device)
-  ctx->kept_bytes -= ctx->kept[i].bytes;
-  for (--ctx->n_kept; i < ctx->n_kept; ++i) ctx->kept[i] = ctx->kept[i + 1];
-}
-static void drop_all_kept(zr_ctx* ctx) {
-  while (ctx->n_kept) drop_kept(ctx, ctx->n_kept - 1);
+struct Block {
+  size_t bytes;
+  int device;
+};
+struct Blocks {
+  std::mutex mu;                             // of everything here and of every context's kept blocks
+  std::unordered_map<void*, Block> handed;   // made by zr_dev_alloc and not given back
+  std::vector<zr_ctx*> contexts;             // of the process
+};
+static Blocks& blocks() {
+  static Blocks* b = new Blocks();  // (handles may be destroyed behind static objects)
+  return *b;
 }
 
-void* zr_dev_alloc(zr_ctx* ctx, size_t bytes, bool any_stream) {
-  int best = -1;
-  for (int i = 0; i < ctx->n_kept; ++i)
-    if (ctx->kept[i].bytes >= bytes && ctx->kept[i].bytes - bytes <= bytes / 8 + 4096 && (best < 0 || ctx->kept[i].bytes < ctx->kept[best].bytes))
-      best = i;
-  if (best >= 0 && (!any_stream || ctx->kept[best].idle || hipStreamSynchronize(ctx->own_stream) == hipSuccess)) {
-    void* p = ctx->kept[best].p;
-    ctx->kept_bytes -= ctx->kept[best].bytes;
-    for (--ctx->n_kept; best < ctx->n_kept; ++best) ctx->kept[best] = ctx->kept[best + 1];
-    return p;
+static void* take_kept(zr_ctx* ctx, int i) {
+  void* p = ctx->kept[i].p;
+  ctx->kept_bytes -= ctx->kept[i].bytes;
+  for (--ctx->n_kept; i < ctx->n_kept; ++i) ctx->kept[i] = ctx->kept[i + 1];
+  return p;
+}
+static void free_blocks(const std::vector<void*>& list) {
+  for (void* p : list) (void)hipFree(p);  // (waits for the device)
+}
+
+int zr_give_back_kept(int device, zr_ctx* only) {
+  std::vector<void*> list;
+  {
+    std::lock_guard<std::mutex> lock(blocks().mu);
+    for (zr_ctx* c : blocks().contexts)
+      while (c->device == device && (!only || c == only) && c->n_kept) list.push_back(take_kept(c, c->n_kept - 1));
   }
+  free_blocks(list);
+  return (int)list.size();
+}
+
+// On the list, and counted, before anything of the context is allocated: from here on nobody keeps blocks on its device.
+static void register_context(zr_ctx* ctx) {
+  {
+    std::lock_guard<std::mutex> lock(blocks().mu);
+    blocks().contexts.push_back(ctx);
+    if (ctx->device < 64) g_live[ctx->device].fetch_add(1);
+  }
+  if (zr_live_contexts(ctx->device) > 1) (void)zr_give_back_kept(ctx->device, nullptr);
+}
+static void unregister_context(zr_ctx* ctx) {
+  std::lock_guard<std::mutex> lock(blocks().mu);
+  auto& all = blocks().contexts;
+  all.erase(std::remove(all.begin(), all.end(), ctx), all.end());
+  if (ctx->device < 64) g_live[ctx->device].fetch_sub(1);
+}
+
+// hipMalloc, if need be once more behind the kept blocks.
+static void* hip_malloc(zr_ctx* ctx, size_t bytes) {
   void* p = nullptr;
   if (hipMalloc(&p, bytes) == hipSuccess) return p;
   (void)hipGetLastError();
-  if (!ctx->n_kept) return nullptr;
-  drop_all_kept(ctx);
+  if (!zr_give_back_kept(ctx->device, nullptr)) return nullptr;
   if (hipMalloc(&p, bytes) == hipSuccess) return p;
   (void)hipGetLastError();
   return nullptr;
 }
 
-int zr_dev_free(zr_ctx* ctx, void* p, bool idle) {
-  if (!p) return ZR_OK;
-  for (int i = 0; i < ctx->n_kept; ++i)
-    if (ctx->kept[i].p == p) return zr_set_error(ZR_EHIP, "device memory %p is freed twice", p);
-  hipDeviceptr_t base = nullptr;
-  size_t bytes = 0;
-  hipPointerAttribute_t attr;
-  const bool keep = !ctx->foreign_stream && zr_live_contexts(ctx->device) == 1 && hipMemGetAddressRange(&base, &bytes, (hipDeviceptr_t)p) == hipSuccess &&
-                    base == (hipDeviceptr_t)p && bytes <= kKeptLargest && hipPointerGetAttributes(&attr, p) == hipSuccess &&
-                    attr.type == hipMemoryTypeDevice && attr.device == ctx->device;
-  if (!keep) {
-    (void)hipGetLastError();
-    if (!idle) ZR_HIP(hipStreamSynchronize(ctx->stream));
-    ZR_HIP(hipFree(p));
-    return ZR_OK;
+void* zr_dev_alloc(zr_ctx* ctx, size_t bytes, bool any_stream) {
+  void* p = nullptr;
+  Block block = {bytes, ctx->device};
+  bool idle = false;
+  {
+    std::lock_guard<std::mutex> lock(blocks().mu);
+    int best = -1;
+    for (int i = 0; i < ctx->n_kept; ++i)
+      if (ctx->kept[i].bytes >= bytes && ctx->kept[i].bytes - bytes <= bytes / 8 + 4096 && (best < 0 || ctx->kept[i].bytes < ctx->kept[best].bytes))
+        best = i;
+    if (best >= 0) {
+      block.bytes = ctx->kept[best].bytes;
+      idle = ctx->kept[best].idle;
+      p = take_kept(ctx, best);
+    }
   }
-  while (ctx->n_kept == ZR_MAX_KEPT || (ctx->n_kept && ctx->kept_bytes + bytes > kKeptTotal)) drop_kept(ctx, 0);
-  ctx->kept[ctx->n_kept++] = {p, bytes, idle};
-  ctx->kept_bytes += bytes;
+  if (p && any_stream && !idle && hipStreamSynchronize(ctx->own_stream) != hipSuccess) {
+    (void)hipFree(p);
+    (void)hipGetLastError();
+    p = nullptr;
+  }
+  if (!p) {
+    p = hip_malloc(ctx, bytes);
+    block.bytes = bytes;
+  }
+  if (p) {
+    std::lock_guard<std::mutex> lock(blocks().mu);
+    blocks().handed[p] = block;
+  }
+  return p;
+}
+
+int zr_dev_free(zr_ctx* ctx, void* p, bool callers) {
+  if (!p) return ZR_OK;
+  auto may_keep = [&](const Block& b) {
+    return ctx->keep_memory && !ctx->foreign_stream && zr_live_contexts(ctx->device) == 1 && b.device == ctx->device && b.bytes <= kKeptLargest;
+  };
+  bool keep = false;
+  {
+    std::lock_guard<std::mutex> lock(blocks().mu);
+    auto it = blocks().handed.find(p);
+    hipDeviceptr_t base = nullptr;
+    size_t bytes = 0;
+    hipPointerAttribute_t attr;
+    if (it == blocks().handed.end() && hipMemGetAddressRange(&base, &bytes, (hipDeviceptr_t)p) == hipSuccess && base == (hipDeviceptr_t)p &&
+        hipPointerGetAttributes(&attr, p) == hipSuccess && attr.type == hipMemoryTypeDevice) {
+      bool kept = false;
+      for (zr_ctx* c : blocks().contexts)
+        for (int i = 0; i < c->n_kept; ++i) kept = kept || c->kept[i].p == p;
+      if (!kept) it = blocks().handed.emplace(p, Block{bytes, attr.device}).first;
+    }
+    (void)hipGetLastError();
+    if (it != blocks().handed.end()) {
+      keep = may_keep(it->second);
+    } else {
+      for (zr_ctx* c : blocks().contexts)
+        for (int i = 0; i < c->n_kept; ++i)
+          if (c->kept[i].p == p) return zr_set_error(ZR_EHIP, "device memory %p is freed twice", p);
+    }
+  }
+  if (callers)
+    ZR_HIP(hipDeviceSynchronize());
+  else if (!keep)
+    ZR_HIP(hipStreamSynchronize(ctx->stream));
+  std::vector<void*> list;
+  {
+    std::lock_guard<std::mutex> lock(blocks().mu);
+    const auto it = blocks().handed.find(p);
+    if (it != blocks().handed.end()) {
+      const Block b = it->second;
+      blocks().handed.erase(it);
+      if (keep && may_keep(b)) {
+        while (ctx->n_kept == ZR_MAX_KEPT || (ctx->n_kept && ctx->kept_bytes + b.bytes > kKeptTotal)) list.push_back(take_kept(ctx, 0));
+        ctx->kept[ctx->n_kept++] = {p, b.bytes, callers};
+        ctx->kept_bytes += b.bytes;
+        p = nullptr;
+      }
+    }
+  }
+  free_blocks(list);
+  if (p) ZR_HIP(hipFree(p));
+  return ZR_OK;
+}
+
+int zr_dev_release(void* p) {
+  if (!p) return ZR_OK;
+  {
+    std::lock_guard<std::mutex> lock(blocks().mu);
+    blocks().handed.erase(p);
+  }
+  ZR_HIP(hipFree(p));
   return ZR_OK;
 }
 
@@ -153,13 +261,7 @@ int zr_ctx_scratch(zr_ctx* ctx, int slot, size_t bytes, void** out) {
     *buf = nullptr;
     *cap = 0;
     size_t want = bytes + bytes / 4;
-    if (hipMalloc(buf, want) != hipSuccess) {
-      (void)hipGetLastError();
-      *buf = nullptr;
-      drop_all_kept(ctx);
-      if (hipMalloc(buf, want) != hipSuccess) *buf = nullptr;
-      (void)hipGetLastError();
-    }
+    *buf = hip_malloc(ctx, want);
     if (!*buf) {
       return zr_set_error(ZR_ENOMEM, "scratch allocation of %zu bytes failed", want);
     }
@@ -173,8 +275,12 @@ int zr_ctx_scratch_if_room(zr_ctx* ctx, int slot, size_t bytes, void** out) {
   if (ctx->sweep_scratch_kib && bytes > (size_t)ctx->sweep_scratch_kib << 10)
     return zr_set_error(ZR_ENOMEM, "%zu bytes of scratch memory are more than ZR_OPT_LSTM_SWEEP_SCRATCH", bytes);
   const size_t cap = slot == 0 ? ctx->scratch_bytes : ctx->scratch2_bytes;
-  size_t free_bytes = 0, total = 0;
-  if (cap < bytes && hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes + ctx->kept_bytes + cap < bytes + bytes / 4)
+  size_t free_bytes = 0, total = 0, kept = 0;
+  if (cap < bytes) {
+    std::lock_guard<std::mutex> lock(blocks().mu);
+    kept = ctx->kept_bytes;
+  }
+  if (cap < bytes && hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes + kept + cap < bytes + bytes / 4)
     return zr_set_error(ZR_ENOMEM, "no room for %zu bytes of scratch memory", bytes);
   (void)hipGetLastError();
   return zr_ctx_scratch(ctx, slot, bytes, out);
@@ -196,8 +302,11 @@ int zr_ctx_create(int device, zr_ctx** out) {
   zr_ctx* c = new zr_ctx();
   memset(c, 0, sizeof(*c));
   c->device = device;
+  c->keep_memory = 1;
+  register_context(c);
   hipError_t e = hipStreamCreate(&c->own_stream);  // default priority
   if (e != hipSuccess) {
+    unregister_context(c);
     delete c;
     return zr_set_error(ZR_EHIP, "hipStreamCreate failed: %s", hipGetErrorString(e));
   }
@@ -206,6 +315,7 @@ int zr_ctx_create(int device, zr_ctx** out) {
   e = hipMalloc((void**)&c->d_flags, flag_bytes + slot_bytes);
   if (e != hipSuccess) {
     (void)hipStreamDestroy(c->own_stream);
+    unregister_context(c);
     delete c;
     return zr_set_error(ZR_ENOMEM, "flag allocation failed: %s", hipGetErrorString(e));
   }
@@ -218,6 +328,7 @@ int zr_ctx_create(int device, zr_ctx** out) {
     if (rc) {
       (void)hipFree(c->d_flags);
       (void)hipStreamDestroy(c->own_stream);
+      unregister_context(c);
       delete c;
       return rc;
     }
@@ -246,7 +357,6 @@ int zr_ctx_create(int device, zr_ctx** out) {
   // ZR_LSTM_STACK_HELPERS=0 keeps the decoder step on its two-workgroups-per-tile schedules (timing comparisons)
   c->stack_helpers = 1;
   if (const char* e = getenv("ZR_LSTM_STACK_HELPERS")) c->stack_helpers = atoi(e) != 0 ? 1 : 0;
-  if (device < 64) g_live[device].fetch_add(1);
   *out = c;
   return ZR_OK;
 }
@@ -255,17 +365,17 @@ int zr_ctx_destroy(zr_ctx* ctx) {
   if (!ctx) return ZR_OK;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
-  drop_all_kept(ctx);
+  (void)zr_give_back_kept(ctx->device, ctx);
   if (ctx->h_pinned) (void)hipHostFree(ctx->h_pinned);
   if (ctx->d_scratch) (void)hipFree(ctx->d_scratch);
   if (ctx->d_scratch2) (void)hipFree(ctx->d_scratch2);
   if (ctx->d_flags) (void)hipFree(ctx->d_flags);
   for (int i = 0; i < ZR_MAX_PACKED_D; ++i)
-    if (ctx->packed_d[i].d_pack) (void)hipFree(ctx->packed_d[i].d_pack);
+    (void)zr_dev_release(ctx->packed_d[i].d_pack);
   if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
   if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
   (void)hipStreamDestroy(ctx->own_stream);
-  if (ctx->device >= 0 && ctx->device < 64) g_live[ctx->device].fetch_sub(1);
+  unregister_context(ctx);
   delete ctx;
   return ZR_OK;
 }
@@ -340,7 +450,7 @@ int zr_ctx_set_stream(zr_ctx* ctx, void* hip_stream) {
     ctx->foreign_stream = 1;
     const int rc = zr_bind_device(ctx);
     if (rc) return rc;
-    drop_all_kept(ctx);
+    (void)zr_give_back_kept(ctx->device, ctx);
   }
   ctx->stream = hip_stream ? (hipStream_t)hip_stream : ctx->own_stream;
   return ZR_OK;
@@ -388,6 +498,15 @@ int zr_ctx_set_option(zr_ctx* ctx, int option, int value) {
       ZR_CHECK_ARG(value == 0 || value == 1, "ZR_OPT_ATTN_SINGLE_LAUNCH must be 0 or 1");
       ctx->attn_single = value;
       return ZR_OK;
+    case ZR_OPT_KEEP_MEMORY:
+      ZR_CHECK_ARG(value == 0 || value == 1, "ZR_OPT_KEEP_MEMORY must be 0 or 1");
+      ctx->keep_memory = value;
+      if (!value) {
+        const int rc = zr_bind_device(ctx);
+        if (rc) return rc;
+        (void)zr_give_back_kept(ctx->device, ctx);
+      }
+      return ZR_OK;
     case ZR_OPT_BF16_ACTIVATION_TERMS:
       ZR_CHECK_ARG(value == 1 || value == 2, "ZR_OPT_BF16_ACTIVATION_TERMS must be 1 or 2");
       ctx->bf16_terms = value;
@@ -414,8 +533,6 @@ int zr_malloc(zr_ctx* ctx, size_t bytes, void** d_out) {
 int zr_free(zr_ctx* ctx, void* d_ptr) {
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
-  if (!d_ptr) return ZR_OK;
-  ZR_HIP(hipDeviceSynchronize());
   return zr_dev_free(ctx, d_ptr, true);
 }
 

@@ -362,11 +362,8 @@ static int softmax_prepare(zr_ctx* ctx, const char* who, const float* d_D, int V
     for (int i = 0; i < ZR_MAX_PACKED_D && slot < 0; ++i)
       if (!ctx->packed_d[i].key) slot = i;
     ZR_CHECK_ARG(slot >= 0, "%s: all %d slots are in use (zr_softmax_release one)", who, ZR_MAX_PACKED_D);
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-      (void)hipGetLastError();
-      return zr_set_error(ZR_ENOMEM, "%s: allocation of %zu bytes failed", who, bytes);
-    }
+    void* p = zr_dev_alloc(ctx, bytes);
+    if (!p) return zr_set_error(ZR_ENOMEM, "%s: allocation of %zu bytes failed", who, bytes);
     ctx->packed_d[slot].d_pack = p;
     ctx->packed_d[slot].V = V;
     ctx->packed_d[slot].H = H;
@@ -376,7 +373,7 @@ static int softmax_prepare(zr_ctx* ctx, const char* who, const float* d_D, int V
   rc = bf16 ? zr_pack8_bf16_launch(ctx, d_D, V, H, V, ldp, kp, (unsigned short*)ctx->packed_d[slot].d_pack)
             : zr_pack4_launch(ctx, d_D, V, H, V, ldp, kp, (float*)ctx->packed_d[slot].d_pack);
   if (rc) {
-    (void)hipFree(ctx->packed_d[slot].d_pack);
+    (void)zr_dev_release(ctx->packed_d[slot].d_pack);
     ctx->packed_d[slot] = zr_ctx::PackedD{};
     return rc;
   }
@@ -398,7 +395,7 @@ int zr_softmax_release(zr_ctx* ctx, const float* d_D) {
   for (int i = 0; i < ZR_MAX_PACKED_D; ++i) {
     if (ctx->packed_d[i].key == d_D && d_D) {
       ZR_HIP(hipStreamSynchronize(ctx->stream));
-      (void)hipFree(ctx->packed_d[i].d_pack);
+      (void)zr_dev_release(ctx->packed_d[i].d_pack);
       ctx->packed_d[i] = zr_ctx::PackedD{};
     }
   }
