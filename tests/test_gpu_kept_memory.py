@@ -174,3 +174,24 @@ def test_freeing_waits_for_work_on_any_stream(ctx):
     assert not done.query()
     a.free()
     assert done.query()
+
+
+def test_freeing_during_a_relaxed_capture_of_another_stream(ctx):
+    """As with hipFree, which such a capture allows."""
+    a = ctx.zeros((1 << 20,))
+    ctx.sync()
+    x = torch.zeros(1000, device="cuda")
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, capture_error_mode="relaxed"):
+        x.add_(1)
+        freed = raw_free(ctx, a.ptr)
+        a.ptr = 0
+        b = ctx.empty((1 << 20,))
+        x.add_(1)
+    assert freed == 0
+    for i in range(3):
+        g.replay()
+        b.set(np.full(1 << 20, i, np.float32))
+        torch.cuda.synchronize()
+        assert x[0].item() == 2.0 * (i + 1) and b.get()[5] == i

@@ -162,6 +162,15 @@ void* zr_dev_alloc(zr_ctx* ctx, size_t bytes, bool any_stream) {
   return p;
 }
 
+// Waits for all work on the device, as hipFree does; hipDeviceSynchronize would end a capture that goes on meanwhile on another stream, which
+// hipFree does not (relaxed mode).
+static bool wait_for_device() {
+  void* p = nullptr;
+  if (hipMalloc(&p, 4) == hipSuccess && hipFree(p) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 int zr_dev_free(zr_ctx* ctx, void* p, bool callers) {
   if (!p) return ZR_OK;
   auto may_keep = [&](const Block& b) {
@@ -190,10 +199,8 @@ int zr_dev_free(zr_ctx* ctx, void* p, bool callers) {
           if (c->kept[i].p == p) return zr_set_error(ZR_EHIP, "device memory %p is freed twice", p);
     }
   }
-  if (callers)
-    ZR_HIP(hipDeviceSynchronize());
-  else if (!keep)
-    ZR_HIP(hipStreamSynchronize(ctx->stream));
+  if (callers || !keep) ZR_HIP(hipStreamSynchronize(ctx->stream));
+  if (callers && keep) keep = wait_for_device();
   std::vector<void*> list;
   {
     std::lock_guard<std::mutex> lock(blocks().mu);
