@@ -164,6 +164,20 @@ def test_nothing_is_kept_without_the_option(ctx):
     ctx.set_option(capi.ZR_OPT_KEEP_MEMORY, 1)
 
 
+def hip():
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    return ctypes.CDLL(path)
+
+
+def test_memory_of_another_allocator_is_not_kept(ctx):
+    torch.cuda.synchronize()
+    p = ctypes.c_void_p()
+    assert hip().hipMalloc(ctypes.byref(p), ctypes.c_size_t(200 * MIB)) == 0
+    before = free_bytes()
+    assert raw_free(ctx, p.value) == 0
+    assert free_bytes() - before >= 150 * MIB
+
+
 def test_freeing_waits_for_work_on_any_stream(ctx):
     a = ctx.empty((1 << 20,))
     s = torch.cuda.Stream()

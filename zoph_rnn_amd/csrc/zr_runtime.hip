@@ -60,7 +60,7 @@ int zr_bind_device(zr_ctx* ctx) {
 // hipMalloc and hipFree take 10 to 300 us, and hipFree waits for the whole device: a training step that packs its layers' new weights
 // (destroy, create) drained the queue at every layer, a translation paid for its 100 MB and its handles each time (decode object of one sentence:
 // created 340 and closed in 70 us, of 16 sentences 530 and 380).  So a context keeps what is given back, up to 32 blocks and
-// 512 MiB, none larger than half of that, oldest out first.
+// 512 MiB, none larger than half of that, oldest out first, and only what zr_dev_alloc made.
 // A block of a handle is reused without waiting for the work that is queued on it, which is sound as long as all of that, and all
 // that comes, is on the context's own stream: nothing is kept where a caller's stream has ever been set or another context is alive.
 // What callers hold themselves (zr_malloc) may be in use on any stream of theirs, so zr_free waits for the device as hipFree
@@ -179,18 +179,7 @@ int zr_dev_free(zr_ctx* ctx, void* p, bool callers) {
   bool keep = false;
   {
     std::lock_guard<std::mutex> lock(blocks().mu);
-    auto it = blocks().handed.find(p);
-    hipDeviceptr_t base = nullptr;
-    size_t bytes = 0;
-    hipPointerAttribute_t attr;
-    if (it == blocks().handed.end() && hipMemGetAddressRange(&base, &bytes, (hipDeviceptr_t)p) == hipSuccess && base == (hipDeviceptr_t)p &&
-        hipPointerGetAttributes(&attr, p) == hipSuccess && attr.type == hipMemoryTypeDevice) {
-      bool kept = false;
-      for (zr_ctx* c : blocks().contexts)
-        for (int i = 0; i < c->n_kept; ++i) kept = kept || c->kept[i].p == p;
-      if (!kept) it = blocks().handed.emplace(p, Block{bytes, attr.device}).first;
-    }
-    (void)hipGetLastError();
+    const auto it = blocks().handed.find(p);
     if (it != blocks().handed.end()) {
       keep = may_keep(it->second);
     } else {
