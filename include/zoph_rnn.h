@@ -195,6 +195,9 @@ int zr_lstm_pack_weights(zr_ctx* ctx, const float* const d_M[4], const float* co
  * the results agree within 1e-4 relative.  Requires H % 16 == 0 and 16-byte aligned activations. */
 int zr_lstm_pack_weights_bf16(zr_ctx* ctx, const float* const d_M[4], const float* const d_Wh[4],
                               const float* const d_Q[4], const float* const d_b[4], int H, zr_lstm_weights** out);
+/* The destroy functions of handles (zr_lstm_weights, zr_lstm_train, zr_attn, zr_beam): on the context's own stream, and while it is the
+ * only context on the device, they do not wait for what is queued (ZR_OPT_KEEP_MEMORY); else they wait for the stream
+ * and return its error, with the handle left as it is. */
 int zr_lstm_weights_destroy(zr_ctx* ctx, zr_lstm_weights* w);
 
 /* One node forward step: LSTM_IH_Node::forward_prop_GPU after the gather (src/LSTM.hpp:133-399) and

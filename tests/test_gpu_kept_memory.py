@@ -209,3 +209,28 @@ def test_freeing_during_a_relaxed_capture_of_another_stream(ctx):
         b.set(np.full(1 << 20, i, np.float32))
         torch.cuda.synchronize()
         assert x[0].item() == 2.0 * (i + 1) and b.get()[5] == i
+
+
+def test_destroying_a_handle_returns_the_error_of_its_wait(ctx):
+    """On a stream that is being captured there is no waiting: an error, after which the handle is still there."""
+    H, beam = 64, 3
+    mats = [[ctx.zeros((H, H)) for _ in range(4)] for _ in range(2)]
+    vec = [ctx.zeros((H,)) for _ in range(4)]
+    L = capi.load()
+    handles = [(L.zr_lstm_weights_destroy, ctx.lstm_pack(mats[0], mats[1], vec, H)), (L.zr_lstm_train_destroy, ctx.lstm_train_create(mats[0], mats[1], H)),
+               (L.zr_attn_destroy, ctx.attn_create(H, beam, 2, mats[0][0], mats[0][1], vec[0], vec[1], mats[0][2], mats[0][3], [ctx.zeros((H, beam))])),
+               (L.zr_beam_destroy, ctx.beam_create(beam, 100, 1, 10, 0.0))]
+    ctx.sync()
+    lib, stream, graph = hip(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert lib.hipStreamCreate(ctypes.byref(stream)) == 0
+    capi._chk(L.zr_ctx_set_stream(ctx.h, stream))
+    for destroy, handle in handles:
+        assert lib.hipStreamBeginCapture(stream, 2) == 0  # relaxed
+        assert destroy(ctx.h, handle) == -2
+        lib.hipStreamEndCapture(stream, ctypes.byref(graph))
+        lib.hipGetLastError()
+    capi._chk(L.zr_ctx_set_stream(ctx.h, None))
+    for destroy, handle in handles:
+        assert destroy(ctx.h, handle) == 0
+    ctx.sync()
+    assert lib.hipStreamDestroy(stream) == 0

@@ -716,10 +716,13 @@ int zr_attn_destroy(zr_ctx* ctx, zr_attn* a) {
   if (!a) return ZR_OK;
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
-  (void)zr_dev_free(ctx, a->d_bf16);
-  (void)zr_dev_free(ctx, a->d_pack32);
-  (void)zr_dev_free(ctx, (void*)a->d_err_table);
-  (void)zr_dev_free(ctx, (void*)a->d_table);
+  if ((rc = zr_dev_free(ctx, a->d_bf16))) return rc;
+  a->d_bf16 = nullptr;
+  if ((rc = zr_dev_free(ctx, a->d_pack32))) return rc;
+  a->d_pack32 = nullptr;
+  if ((rc = zr_dev_free(ctx, (void*)a->d_err_table))) return rc;
+  a->d_err_table = nullptr;
+  if ((rc = zr_dev_free(ctx, (void*)a->d_table))) return rc;
   delete a;
   return ZR_OK;
 }

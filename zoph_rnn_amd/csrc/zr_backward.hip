@@ -928,8 +928,9 @@ int zr_lstm_train_destroy(zr_ctx* ctx, zr_lstm_train* w) {
   if (!w) return ZR_OK;
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
-  (void)zr_dev_free(ctx, w->d_stack);
-  (void)zr_dev_free(ctx, w->d_stack_pack);
+  if ((rc = zr_dev_free(ctx, w->d_stack))) return rc;
+  w->d_stack = nullptr;
+  if ((rc = zr_dev_free(ctx, w->d_stack_pack))) return rc;
   delete w;
   return ZR_OK;
 }

@@ -803,7 +803,7 @@ int zr_beam_destroy(zr_ctx* ctx, zr_beam* b) {
   if (!b) return ZR_OK;
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
-  (void)zr_dev_free(ctx, b->d_block);
+  if ((rc = zr_dev_free(ctx, b->d_block))) return rc;
   delete b;
   return ZR_OK;
 }

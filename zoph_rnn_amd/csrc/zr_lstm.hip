@@ -1203,8 +1203,9 @@ int zr_lstm_weights_destroy(zr_ctx* ctx, zr_lstm_weights* w) {
   if (!w) return ZR_OK;
   int rc = zr_bind_device(ctx);
   if (rc) return rc;
-  (void)zr_dev_free(ctx, w->d_W);
-  (void)zr_dev_free(ctx, w->d_bias);
+  if ((rc = zr_dev_free(ctx, w->d_W))) return rc;
+  w->d_W = nullptr;
+  if ((rc = zr_dev_free(ctx, w->d_bias))) return rc;
   delete w;
   return ZR_OK;
 }
