@@ -73,7 +73,12 @@ int zr_ctx_set_option(zr_ctx* ctx, int option, int value);
  *     Does not wait.
  *   ZR_QUERY_WAITS_REPAIRED: waits for the stream; which of the last launches gave up a wait and formed what it had waited
  *     for again (the results are right all the same): ZR_REPAIRED_SGD_UPDATE, the last clipped update of one matrix in one
- *     launch. */
+ *     launch; ZR_REPAIRED_LSTM_BACKWARD, the last backward sweep with its weights in registers (one workgroup a column
+ *     formed it again, after up to a second of waiting: a program that sees this often sets ZR_OPT_LSTM_SWEEP = 1).  Both
+ *     bits may be set.
+ *   ZR_QUERY_LSTM_BACKWARD_PATH: which schedule the last zr_lstm_stack_backward(_clamped) call on this context took -- 0 none yet,
+ *     ZR_LSTM_BACKWARD_PATH_DIAGONALS (one or two launches per diagonal) or ZR_LSTM_BACKWARD_PATH_RESIDENT (one launch
+ *     or a few, with the weights in registers).  Does not wait. */
 int zr_ctx_query(zr_ctx* ctx, int what, int* h_value);
 #define ZR_QUERY_LSTM_STACK_PATH 1
 #define ZR_QUERY_LSTM_SWEEP_ABANDONED 2
@@ -81,7 +86,11 @@ int zr_ctx_query(zr_ctx* ctx, int what, int* h_value);
 #define ZR_QUERY_SCRATCH_KIB 4
 #define ZR_QUERY_LSTM_SWEEP_KERNEL 5
 #define ZR_QUERY_WAITS_REPAIRED 6
+#define ZR_QUERY_LSTM_BACKWARD_PATH 7
 #define ZR_REPAIRED_SGD_UPDATE 1
+#define ZR_REPAIRED_LSTM_BACKWARD 2
+#define ZR_LSTM_BACKWARD_PATH_DIAGONALS 1
+#define ZR_LSTM_BACKWARD_PATH_RESIDENT 2
 #define ZR_LSTM_SWEEP_STREAMED 1 /* weights streamed from the caches in every time step */
 #define ZR_LSTM_SWEEP_RESIDENT 2 /* weights held in registers */
 #define ZR_ATTN_PATH_SINGLE_LAUNCH 1  /* projections, window / scores / context and output product in one launch */
@@ -115,11 +124,15 @@ const char* zr_version(void);
                                         1 never (one launch per diagonal), 2 a sweep whenever one fits, with streamed
                                         weights if that one does, 3 the same with its weights in registers if that
                                         one does.  The environment variable ZR_LSTM_SWEEP presets this option for every
-                                        context created */
+                                        context created.  zr_lstm_stack_backward(_clamped) likewise: 0 auto (all time
+                                        steps in one launch or a few with the weights in registers, H up to 512, under the
+                                        same conditions, else a launch or two per diagonal), 1 never, 2 and 3 whenever it
+                                        fits and no result shares memory with an operand or another result */
 #define ZR_OPT_LSTM_SWEEP_SPIN 8     /* polls a workgroup of that launch spends on one wait before it gives up
                                         (0 = default, about a second); giving up is reported by zr_ctx_sync.  Also the
-                                        polls of the clipped update in one launch (0 = 4096), whose workgroups then form the
-                                        norm from the whole gradient: to the same bits, reported by ZR_QUERY_WAITS_REPAIRED only */
+                                        polls of the backward sweep, which is then formed again, and of the clipped update
+                                        in one launch (0 = 4096), whose workgroups then form the norm from the whole
+                                        gradient, to the same bits: both reported by ZR_QUERY_WAITS_REPAIRED only */
 
 #define ZR_OPT_BF16_ACTIVATION_TERMS 9 /* products against bf16 weights (zr_lstm_pack_weights_bf16, zr_softmax_prepare_bf16,
                                         zr_attn_use_bf16_weights): 2 (default) = every fp32 activation enters as two
@@ -129,8 +142,8 @@ const char* zr_version(void);
 #define ZR_OPT_LSTM_STEP_WAIT_EXTRA 10 /* for tests of the give-up path of zr_lstm_decoder_step's single launch: the
                                         waits of a layer for the layer below expect this many arrivals more than there
                                         will be, so each of them runs to ZR_OPT_LSTM_SWEEP_SPIN polls and gives up
-                                        whatever the timing (0 = off, the default); the waits of the clipped update in one
-                                        launch likewise */
+                                        whatever the timing (0 = off, the default); the waits of the backward sweep
+                                        and of the clipped update in one launch likewise */
 #define ZR_OPT_ATTN_SINGLE_LAUNCH 11 /* the attention step as ONE launch whose workgroups hand over through device
                                         memory (prepared fp32 matrices, H a multiple of 8 up to 1024, at most 64 window
                                         slots, all workgroups resident at once, own stream, only context on the
@@ -139,8 +152,9 @@ const char* zr_version(void);
                                         single-launch LSTM schedules' and reported the same way */
 #define ZR_OPT_LSTM_SWEEP_SCRATCH 12 /* KiB of scratch memory that a sweep as one launch may use (0 = what the device has
                                         left).  The streamed sweep needs 6 * (L * (T + 1) + T) * H bytes a column (columns in
-                                        eights), the resident one 4 * L * (T + 1) * H; a schedule there is no memory for
-                                        is passed over, with ZR_OPT_LSTM_SWEEP = 2 and 3 too */
+                                        eights), the resident one 4 * L * (T + 1) * H, the backward sweep 256 * L * T *
+                                        ceil(H / 16) (all of it a quarter more, and it stays with the context); a schedule
+                                        there is no memory for is passed over, with ZR_OPT_LSTM_SWEEP = 2 and 3 too */
 #define ZR_OPT_KEEP_MEMORY 13 /* 1 (default): device memory of destroyed handles and of zr_free stays with the context for its
                                  next requests, at most 32 blocks and 512 MiB, while it is the only context on its
                                  device and has never been given a stream; 0: what is kept goes back to the device now,

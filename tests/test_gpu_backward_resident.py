@@ -65,6 +65,8 @@ def run(ctx, c, clip, want_below, option):
                                     flat(c["top"]), dg, eh, ec, err_hT=each(c["hT"]), err_cT=each(c["cT"]), d_err_below0=ein if want_below else None,
                                     err_clip=clip)
         ctx.sync()
+        if option >= 2:
+            assert ctx.query(capi.ZR_QUERY_LSTM_BACKWARD_PATH) == capi.ZR_LSTM_BACKWARD_PATH_RESIDENT
     finally:
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP, 0)
         for w in layers:
@@ -107,6 +109,25 @@ def test_an_abandoned_sweep_is_formed_again(ctx, L, H, mb, T):
     compare(run(ctx, c, 0.1, True, 3), reference(c, 0.1))
 
 
+@pytest.mark.parametrize("L,H,mb,T", [(1, 8, 1, 1), (1, 8, 3, 5), (3, 100, 20, 7), (2, 385, 24, 3), (5, 500, 50, 3), (9, 64, 16, 3)])
+@pytest.mark.parametrize("clip,below", [(0.1, True), (0.0, False)])
+def test_waits_that_cannot_end_are_given_up_and_the_sweep_formed_again(ctx, L, H, mb, T, clip, below):
+    """Every wait expects more slots than there are: each launch is abandoned, whatever the timing."""
+    c = case(L, H, mb, T, True)
+    ctx.set_option(capi.ZR_OPT_LSTM_STEP_WAIT_EXTRA, 1)
+    ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 30)
+    try:
+        got = run(ctx, c, clip, below, 3)
+        repaired = ctx.query(capi.ZR_QUERY_WAITS_REPAIRED)
+    finally:
+        ctx.set_option(capi.ZR_OPT_LSTM_STEP_WAIT_EXTRA, 0)
+        ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)
+    assert repaired & capi.ZR_REPAIRED_LSTM_BACKWARD
+    compare(got, reference(c, clip))
+    compare(run(ctx, c, clip, below, 3), reference(c, clip))
+    assert ctx.query(capi.ZR_QUERY_WAITS_REPAIRED) & capi.ZR_REPAIRED_LSTM_BACKWARD == 0
+
+
 def test_results_on_operands_take_the_launches_per_diagonal(ctx):
     """err_below0 written over err_top, err_c0 over err_cT: as before the single launch."""
     L, H, mb, T = 2, 64, 8, 4
@@ -122,6 +143,7 @@ def test_results_on_operands_take_the_launches_per_diagonal(ctx):
         ctx.sync()
     finally:
         ctx.set_option(capi.ZR_OPT_LSTM_SWEEP_SPIN, 0)
+    assert ctx.query(capi.ZR_QUERY_LSTM_BACKWARD_PATH) == capi.ZR_LSTM_BACKWARD_PATH_DIAGONALS
     want = reference(c, 0.0)
     by_column = lambda a, *s: a.get().reshape(*s).swapaxes(-1, -2)
     compare(([by_column(x, T, mb, 4 * H) for x in dg], by_column(top, T, mb, H), [x.get() for x in eh], [by_column(x, mb, H) for x in cT]), want)
@@ -140,9 +162,18 @@ def test_results_on_one_another_are_written_in_the_diagonals_order(ctx):
                             [flat(np.stack(g)) for g in c["gates"]], flat(c["top"]), dg, [eh] * L, ec, err_hT=[flat(x) for x in c["hT"]],
                             err_cT=[flat(x) for x in c["cT"]])
     ctx.sync()
+    assert ctx.query(capi.ZR_QUERY_LSTM_BACKWARD_PATH) == capi.ZR_LSTM_BACKWARD_PATH_DIAGONALS
     want = reference(c, 0.0)
     assert_close(eh.get(), want[2][L - 1], what="error to h_0 of the last layer")
     for l in range(L):
         assert_close(ec[l].get(), want[3][l], what="error to c_0, layer %d" % l)
     for w in layers:
         ctx.lstm_train_destroy(w)
+
+
+def test_without_an_option_the_same_sizes_take_one_launch(ctx):
+    """(what the two tests before this one would take if no memory were shared)"""
+    for L, H, mb, T in ((2, 64, 8, 4), (3, 64, 8, 4)):
+        c = case(L, H, mb, T, True)
+        compare(run(ctx, c, 0.0, True, 0), reference(c, 0.0))
+        assert ctx.query(capi.ZR_QUERY_LSTM_BACKWARD_PATH) == capi.ZR_LSTM_BACKWARD_PATH_RESIDENT

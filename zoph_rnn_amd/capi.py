@@ -31,7 +31,11 @@ ZR_QUERY_ATTN_PATH = 3
 ZR_QUERY_SCRATCH_KIB = 4
 ZR_QUERY_LSTM_SWEEP_KERNEL = 5
 ZR_QUERY_WAITS_REPAIRED = 6
+ZR_QUERY_LSTM_BACKWARD_PATH = 7
 ZR_REPAIRED_SGD_UPDATE = 1
+ZR_REPAIRED_LSTM_BACKWARD = 2
+ZR_LSTM_BACKWARD_PATH_DIAGONALS = 1
+ZR_LSTM_BACKWARD_PATH_RESIDENT = 2
 ZR_LSTM_SWEEP_STREAMED = 1
 ZR_LSTM_SWEEP_RESIDENT = 2
 ZR_ATTN_PATH_SINGLE_LAUNCH = 1

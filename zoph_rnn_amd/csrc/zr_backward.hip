@@ -987,9 +987,11 @@ int zr_lstm_stack_backward_clamped(zr_ctx* ctx, int nl, const zr_lstm_train* con
       for (int l = 0; l < nl; ++l) stacks[l] = layers[l]->d_stack;
       rc = zr_backward_resident_sweep(ctx, plan, nl, stacks, H, T, mb, d_mask01, d_c0, d_c_all, d_gates_all, d_err_top, d_err_hT, d_err_cT,
                                       d_dgates_all, d_err_below0, d_err_h0, d_err_c0, err_clip);
+      if (rc == ZR_OK) ctx->last_backward_path = ZR_LSTM_BACKWARD_PATH_RESIDENT;
       if (rc != ZR_ENOMEM) return rc;
     }
   }
+  ctx->last_backward_path = ZR_LSTM_BACKWARD_PATH_DIAGONALS;
   // The grid is walked by anti-diagonals d = l + t, highest first: node (l, t) needs the errors of (l+1, t) and
   // (l, t+1), both on diagonal d+1, so the nodes of a diagonal are independent and share two launches (the gate
   // derivatives of all of them, then all their error products as one grouped GEMM).

@@ -54,6 +54,7 @@ struct BackResident {
   int nl, T, H, mb, mbp, j_tiles, n_tiles;
   float clip;
   int spin_limit;
+  int wait_extra;                 // 0; in tests of giving up waits want so many slots more than there are
 };
 
 __device__ __forceinline__ float clamp_error(float v, float clip) { return v > clip ? clip : (v < -clip ? -clip : v); }
@@ -127,6 +128,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG <= 4 ? 4 : 2) lstm_backward_re
     bool dead = false;
     auto wait_for = [&](const int* flags, int target) {
       if (dead) return;
+      target += P.wait_extra;
       int spins = 0;
       bool gave_up = false;
       for (;;) {
@@ -296,7 +298,7 @@ __global__ void __launch_bounds__(64 * kWaves, NG <= 4 ? 4 : 2) lstm_backward_re
 }
 
 // The whole sweep of one column by one workgroup, where a launch above was abandoned.  The state between the steps lies in the launch's own
-// hand-over memory, which nobody reads any more: per column [nl][4][H] (error to h_{t-1}, to the layer below, gate errors are in LDS).
+// hand-over memory, which nobody reads any more: per column [2][nl][H], the errors to h_{t-1} and to c_{t-1} (gate errors are in LDS).
 __global__ void __launch_bounds__(512) lstm_backward_redo_kernel(BackResident P) {
   if (__hip_atomic_load(P.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != P.epoch) return;
   __shared__ float dg[4 * 512];
@@ -424,6 +426,7 @@ int zr_backward_resident_sweep(zr_ctx* ctx, const ZrBackPlan& plan, int nl, cons
   P.mb = mb;
   P.clip = err_clip;
   P.spin_limit = ctx->sweep_spin > 0 ? ctx->sweep_spin : (1 << 20);
+  P.wait_extra = ctx->step_wait_extra;
   const int per = P.j_tiles * P.n_tiles;
   for (int left = nl; left > 0; left -= P.layers) {
     P.l_top = left - 1;

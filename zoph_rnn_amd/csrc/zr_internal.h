@@ -33,12 +33,13 @@ struct zr_ctx {
   int lstm_sweep;    // whole-sweep LSTM kernels: 0 auto, 1 never, 2 / 3 streamed / resident weights whenever the launch fits
   int sweep_spin;    // polls before a waiting workgroup of that kernel gives up (0: default)
   int sweep_scratch_kib;  // ZR_OPT_LSTM_SWEEP_SCRATCH
-  int step_wait_extra;  // arrivals the decoder step's layer waits expect beyond the real ones (tests of giving up)
+  int step_wait_extra;  // ZR_OPT_LSTM_STEP_WAIT_EXTRA: arrivals that waits expect beyond the real ones (tests of giving up)
   int stack_helpers;    // 1 (default): the decoder step may run 32-column tiles with helper workgroups (zr_lstm.hip)
   int cu_count;      // compute units of the device
   int sweep_capacity[3];  // resident workgroups of lstm_sweep_kernel<TN> (0: not asked yet, -1: unknown)
   int resident_capacity[4][3];  // the same for lstm_resident_kernel, by size class and column class
   int back_capacity[ZR_BACK_CLASSES];  // the same for lstm_backward_resident_kernel, by size class
+  int last_backward_path;  // ZR_QUERY_LSTM_BACKWARD_PATH
   int back_epoch;       // its launches so far: what d_flags[4] holds when the last one was abandoned
   int stack_step_capacity;  // the same for lstm_decoder_stack_kernel (the lesser of its two tile widths)
   int attn_step_capacity[3];  // the same for attn_step_kernel<8 / 16 / 32>

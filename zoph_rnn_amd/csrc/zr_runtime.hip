@@ -407,6 +407,9 @@ int zr_ctx_query(zr_ctx* ctx, int what, int* h_value) {
     case ZR_QUERY_LSTM_SWEEP_KERNEL:
       *h_value = ctx->last_sweep_kernel;
       return ZR_OK;
+    case ZR_QUERY_LSTM_BACKWARD_PATH:
+      *h_value = ctx->last_backward_path;
+      return ZR_OK;
     case ZR_QUERY_SCRATCH_KIB:
       *h_value = (int)((ctx->scratch_bytes + ctx->scratch2_bytes + 1023) / 1024);
       return ZR_OK;
@@ -432,7 +435,8 @@ int zr_ctx_query(zr_ctx* ctx, int what, int* h_value) {
       ZR_HIP(hipStreamSynchronize(ctx->stream));
       int gave_up[2] = {0, 0};
       ZR_HIP(hipMemcpy(gave_up, ctx->d_flags + 4, sizeof(gave_up), hipMemcpyDeviceToHost));
-      *h_value = ctx->sgd_epoch && gave_up[1] == ctx->sgd_epoch ? ZR_REPAIRED_SGD_UPDATE : 0;
+      *h_value = (ctx->sgd_epoch && gave_up[1] == ctx->sgd_epoch ? ZR_REPAIRED_SGD_UPDATE : 0) |
+                 (ctx->back_epoch && gave_up[0] == ctx->back_epoch ? ZR_REPAIRED_LSTM_BACKWARD : 0);
       return ZR_OK;
     }
     default:
