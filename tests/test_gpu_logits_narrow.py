@@ -1,6 +1,6 @@
 """The output layer's product on a prepared fp32 matrix for up to 16 columns (csrc/zr_logits_narrow.hip): edges of its 16-row tiles and 32-row blocks, of its
-groups of 16 k and their ring, both forms, and activations that are infinite; and the split product's one 32-column block at 17 to 32 columns.  Tolerance: H products and their sums, each rounded once, in two chains
-(test_gpu_logits_split.py's bound)."""
+groups of 16 k and their ring, both forms, and activations that are infinite; and the split product's one 32-column block at 17 to 32 columns.  Tolerance: H products and their sums, each rounded
+once (test_gpu_logits_split.py's bound; the eight chains round less)."""
 import numpy as np
 import pytest
 
@@ -32,6 +32,12 @@ def check(D, b, h, x, pairs):
                                    (4097, 333, 12), (8191, 640, 5), (9000, 1000, 16), (10001, 81, 7), (30011, 500, 12), (49152, 12, 16), (50001, 20, 3), (50000, 96, 12),
                                    (65536, 33, 2), (65537, 8, 1), (50001, 400, 11), (20011, 1003, 10)])
 def test_logits_and_block_pairs(ctx, V, H, n):
+    D, b, h = operands(V, H, n)
+    check(D, b, h, *logits_and_blocks(ctx, D, b, h))
+
+
+@pytest.mark.parametrize("V,H,n", [(45568, 401, 2), (45569, 400, 12), (50001, 417, 3), (48900, 1003, 16), (65505, 402, 1), (65536, 399, 5), (65536, 401, 16), (65537, 404, 7)])
+def test_four_waves_of_64_rows_around_their_line(ctx, V, H, n):
     D, b, h = operands(V, H, n)
     check(D, b, h, *logits_and_blocks(ctx, D, b, h))
 

@@ -1,8 +1,11 @@
 """The clipped update of a matrix in one launch (sgd_small_kernel) around its block sizes, its limit and off 16-byte alignment.
 Tolerance: the factor's product, square root, quotient and two multiplications, 2^-24 each, times the step; one rounding of the step and one
 of the sum."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
 from zoph_rnn_amd import capi
 
@@ -45,3 +48,15 @@ def test_non_finite_gradient_reaches_every_value(ctx):
     # a norm that is no number is not above the threshold: the other values take the plain step
     want = np.where(np.isnan(g), np.nan, np.float32(1) + np.float32(0.1))
     assert np.array_equal(dw.get(), want.astype(np.float32), equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [27999, 28001, 65537, 112000, 112001, 250001])
+@pytest.mark.parametrize("off_w,off_g", [(0, 0), (1, 0)])
+def test_update_on_a_callers_stream(n, off_w, off_g):
+    """Where the workgroups' sums cannot be exchanged: this kernel to its limit, then two launches."""
+    c = capi.Context(0)
+    s = torch.cuda.Stream()
+    capi._chk(capi.load().zr_ctx_set_stream(c.h, ctypes.c_void_p(s.cuda_stream)))
+    test_update(c, n, off_w, off_g, 0.5)
+    capi._chk(capi.load().zr_ctx_set_stream(c.h, None))
+    c.close()

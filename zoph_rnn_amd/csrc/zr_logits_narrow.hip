@@ -2,9 +2,8 @@
 // at -- with the soft-max partials: a stream of the matrix through the chip, 200 MB for 1.2 GFLOP at 50000 x 1000 x 12.
 //
 // A wave owns 32 rows and all columns on the 16 x 16 x 4 instruction, whose operands are one 16-byte load a lane for 16 k in the k-interleaved
-// layout, five groups of 16 k ahead.  Waves are workgroups of their own, so that they spread evenly over the compute units; where four waves of 64 rows (1 KB of
-// neighbouring memory a k-block) are just about a workgroup a compute unit those are taken (50000 x 1000 31.8 us against 33.3, 60000 36.1 against 37.2;
-// but 40000 28.5 against 27.5, 80000 x 768 50.1 against 40.7).  32 x 32 x 2 instructions leave more than half of their columns empty at this
+// layout, five groups of 16 k ahead.  Waves are workgroups of their own, so that they spread evenly over the compute units, or four of them
+// with 64 rows each (1 KB of neighbouring memory a k-block; zr_logits_narrow_pairs).  32 x 32 x 2 instructions leave more than half of their columns empty at this
 // width: 30 us of them in a row at 50000 x 1000, on one wave a SIMD, beside 41 us for the launch that had them.  The activations are read as they lie.  No LDS, no barrier.
 // Bound: the matrix's way from memory, 6.3 TB/s.  That launch with its re-layout of the activations where needed / this one, us: 50000 x 1000 x 12 40.4 -> 31.8,
 // 50000 x 500 33.1 -> 17.3, 30000 x 1000 38.2 -> 18.8, 30011 x 333 x 10 (K % 8 != 0, another kernel) 15.1 -> 7.8, 10000 x 100 x 8 7.8 -> 4.8.  More groups in
@@ -158,8 +157,7 @@ void launch(const NarrowArgs& a, bool stream, hipStream_t st) {
 int zr_logits_narrow(zr_ctx* ctx, int V, int cols, int H, const float* packed, int ldp, const float* h, long long ldh, float* C, long long ldc,
                      const float* bias, float* partials, bool stream) {
   const NarrowArgs a = {V, cols, H, ldp, (H + 7) / 8 * 8, packed, h, ldh, C, ldc, bias, partials};
-  const int pairs = (V + 255) / 256;  // workgroups of four waves of 64 rows
-  if (pairs <= ctx->cu_count && 4 * pairs >= 3 * ctx->cu_count)
+  if (zr_logits_narrow_pairs(V, H, ctx->cu_count))
     launch<2, 4, 4>(a, stream, ctx->stream);
   else
     launch<1, 4, 1>(a, stream, ctx->stream);

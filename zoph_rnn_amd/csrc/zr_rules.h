@@ -160,6 +160,8 @@ inline ZrResidentPlan zr_sweep_resident_plan(int nl, int H, int mb, int T, const
 // Where a layer's workgroups of 16 rows x 16 columns fit the device they win with up to four launches, at 24 steps, us per diagonal / in
 // registers: 2 x 100, 100 columns 225 / 106, 3 x 200, 64 307 / 136, 4 x 200, 128 (two launches) 403 / 282, 2 x 500, 64 405 / 230, 3 x 500, 128 (three) 799 /
 // 564, 4 x 500, 128 (four) 850 / 752; but with eight, 8 x 300, 128 821 / 1099, 8 x 500, 128 1219 / 1536: the layers no longer overlap.
+// Sizes share a kernel by their k-groups a wave; the one for 257 to 320 against the next larger one: 2 x 300, 20 columns, 35 steps 207 / 221, 3 x 320, 64 182 / 194, 1 x 257, 20 112 /
+// 117.
 constexpr int kBackLaunches = 4;
 constexpr int ZR_BACK_CLASSES = 5;
 inline int zr_back_size_class(int H) { return H <= 128 ? 0 : (H <= 256 ? 1 : (H <= 320 ? 2 : (H <= 384 ? 3 : 4))); }
@@ -259,7 +261,8 @@ inline bool zr_split_gemm_takes_product(int M, int N, int K, bool k_fast_a, bool
 // ---- weight gradients of a single node (outer_accumulate_kernel), `count` products a launch, K = the minibatch
 
 // Against a transpose and the LDS-tiled product each, us of the whole call.  Two H x H at a time (zr_attn_backward): faster at
-// every size up to 256 columns, a third over all.  One 4H x H (zr_lstm_feed_backward): H = 1000, 128 columns 63 / 82, 200
+// every size up to 256 columns, a third over all; all four of a node in one launch, us of its whole backward pass against those: H = 64, 8 columns 33 / 52, 256 46 / 59; 500, 64
+// columns 48 / 75; 1000, 256 columns 127 / 172.  One 4H x H (zr_lstm_feed_backward): H = 1000, 128 columns 63 / 82, 200
 // 75 / 89; but small ones do not fill the chip with waves that each walk all columns: H = 64, 192 columns 20.8 / 19.1, 256
 // 23.2 / 19.5, H = 256, 192 columns 27.3 / 25.2, where 64 columns are 16.1 / 17.0 and 22.9 / 23.9.
 inline bool zr_outer_takes(int count, int M, int N, int K) {
@@ -398,6 +401,14 @@ inline ZrLogitsPlan zr_logits_plan(int V, int cols, int H, int cus) {
 inline bool zr_logits_narrow_takes(int V, int cols, int H) {
   if (cols > 16 || H < 4 || (V < 8192 && H > 600)) return false;
   return (((long long)H + 7) / 8 * 8 + 160) * (((long long)V + 31) / 32) * 32 * 4 < 1LL << 32;  // 32-bit offsets
+}
+
+// Its two forms: workgroups of four waves of 64 rows where they are just about one a compute unit and K is long, else waves of 32 rows.  us of a call
+// at 12 columns, the first / the second: 1000 at 44000 rows 29.7 / 29.7, 48000 30.8 / 32.3, 50000 31.6 / 33.4, 56000 34.0 / 36.6, 65536 38.2 / 40.9, 66000 61.2 / 46.2; 512 at 40000 16.2 / 14.8,
+// 56000 18.8 / 19.6; 333 at 50000 14.2 / 13.6, 56000 13.4 / 13.5; 200 at 56000 10.5 / 10.0, 65536 11.8 / 10.8; 64 at 50000 4.8 / 4.5.
+inline bool zr_logits_narrow_pairs(int V, int H, int cus) {
+  const int groups = (V + 255) / 256;
+  return H >= 400 && groups <= cus && 10 * groups >= 7 * cus;
 }
 
 // The same on a prepared bf16 matrix for up to 64 columns (zr_logits_bf16.hip) instead of gemm_rows_kernel or, up to 32 columns, gemm_kernel, whose workgroups split K over
