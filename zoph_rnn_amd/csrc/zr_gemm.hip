@@ -124,9 +124,7 @@ __device__ __forceinline__ void softmax_partial_epilogue(const GemmArgs& a, floa
 // One output tile of 32*TM rows x 32*TN columns at (m0, n0), computed by the KS waves that call this together
 // (kslice = this wave's K slice, redp = their KS*TN*16*64 floats of LDS): all segments, the split-K sum and the
 // epilogue.  `active` false: same control flow (barriers), nothing stored.  PF = prefetch distance in k-groups.
-// BUF (k-interleaved fp32 operands on both sides, K % 8 == 0, every row and column of the tile in range, operands below
-// 4 GiB): the K loop fetches through buffer descriptors with the pinned schedule of zr_mma_segment_u.
-template <int TM, int TN, int KS, int AMODE, bool VEC, int EPI, int PF, bool BUF = false>
+template <int TM, int TN, int KS, int AMODE, bool VEC, int EPI, int PF>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0, bool active, int z, float* redp,
                                           int kslice, int lane) {
   const int jl = lane & 31;
@@ -173,16 +171,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0, boo
   }
 
   for (int s = 0; s < a.nseg; ++s) {
-    if constexpr (BUF) {
-      unsigned wsoff[TM], xoffb[TN];
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm) wsoff[tm] = 512u * (unsigned)tm;  // 32 rows of 16 bytes
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) xoffb[tn] = 16u * (unsigned)(cols[tn] + half * a.N);
-      const unsigned woffb = 16u * (unsigned)(m0 + jl + half * (int)a.lda[s]);
-      zr_mma_segment_ring<TM, TN, KS, PF>(acc, zr_make_rsrc(a.A[s]), wsoff, woffb, 32u * (unsigned)a.lda[s],
-                                       zr_make_rsrc(a.B[s]), xoffb, 32u * (unsigned)a.N, a.K[s], kslice);
-    } else if constexpr (zr_is_bf16_mode(AMODE)) {
+    if constexpr (zr_is_bf16_mode(AMODE)) {
       const unsigned short* wbase[TM];
       unsigned woff[TM];
       const float* xcol[TN];
@@ -401,25 +390,6 @@ __global__ void __launch_bounds__(256) gemm_rows_kernel(GemmArgs a, int row_chun
       gemm_tile<1, 1, 4, AMODE, true, EPI, PF4 + 2>(a, blk * 32, n0 + sub * 32, true, 0, red, kslice, lane);
     __syncthreads();
   }
-}
-
-// Tall weight matrix (k-interleaved, 8192 rows and more: the attention node's of a model that wide) times at most 32 columns: a stream of the matrix
-// through the chip, so what matters is bytes in flight and how memory sees the fetches.  K split over the waves of a workgroup means a cross-wave sum
-// through LDS and a ramp per pass (the row-range kernel: 50 us, 3.9 TB/s at 50000 x 12 x 1000).  Here every WAVE takes two neighbouring 32-row blocks over
-// all of K on its own (1 KB of neighbouring memory a stage), a ring of 10 fetch stages deep, two workgroups per compute unit: no LDS, no barrier.  40.2 us (5.0
-// TB/s); one block per wave, ring of 12: 49.6; two blocks, ring of 14: 51.9; three, ring of 8: 57.4; four, ring of 6: 73.3 (too few bytes in flight).
-// K % 8 == 0, k-interleaved activations.
-__global__ void __launch_bounds__(256, 2) gemm_stream_kernel(GemmArgs a) {
-  constexpr int PF = 10;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-  const int n_waves = (int)gridDim.x * 4;
-  const int blocks = (a.M + 31) >> 5;  // (the packed matrix holds exactly these rows: nothing beyond them is fetched)
-  const int pairs = blocks >> 1;
-  for (int b = wave; b < pairs; b += n_waves)
-    gemm_tile<2, 1, 1, ZR_A_PACK4, true, ZR_EPI_STORE, PF, true>(a, b * 64, 0, true, 0, nullptr, 0, lane);
-  if ((blocks & 1) && wave == pairs % n_waves)  // an odd block at the end, on its own
-    gemm_tile<1, 1, 1, ZR_A_PACK4, true, ZR_EPI_STORE, PF, true>(a, (blocks - 1) * 32, 0, true, 0, nullptr, 0, lane);
 }
 
 // Soft-max-partial epilogue for accumulators held the other way round: lane = column (n0 + 32*tn + lane % 32),
@@ -1337,18 +1307,6 @@ int zr_gemm_launch(zr_ctx* ctx, const ZrGemmDesc& d) {
     if (vec && d.nseg == 1 && zcount == 1 && d.M >= 8192 && d.N <= 1024 && ctx->gemm_cfg != 11 &&
         (d.epilogue == ZR_EPI_STORE || d.epilogue == ZR_EPI_SOFTMAX_PARTIAL)) {
       const int n32 = (d.N + 31) / 32;
-      if (d.epilogue == ZR_EPI_STORE && d.N <= 32 && ga.b_pack4 && d.K[0] % 8 == 0 && ctx->gemm_cfg == 0 &&
-          (long long)d.K[0] * ga.lda[0] * 4 + 4096 < (1LL << 32)) {
-        // one pair of 32-row blocks per wave while there are waves
-        const int pairs = ((d.M + 31) / 32 + 1) / 2;
-        const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-        int wgs = (pairs + 3) / 4;
-        if (wgs > 2 * cus) wgs = 2 * cus;
-        ga.m_tiles = ga.n_tiles = 0;
-        gemm_stream_kernel<<<wgs, 256, 0, ctx->stream>>>(ga);
-        ZR_LAUNCH_CHECK("gemm_stream_kernel");
-        return ZR_OK;
-      }
       const int n_tiles = (n32 + 3) / 4;
       const int tn = (n32 + n_tiles - 1) / n_tiles;
       if (tn == 1) return launch_rows<1>(ctx, ga, d.epilogue, n_tiles);

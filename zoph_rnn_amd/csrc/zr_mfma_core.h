@@ -233,7 +233,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t zr_make_rsrc(const void* base)
 // The weight halves of the first PF ring stages of a segment, issued ahead of time (zr_mma_segment_u with WPRE then
 // fetches only the activation halves in its prologue): weights depend on nothing, so a caller that must wait for its
 // activations can have them in flight during the wait.
-template <int TM, int TN, int KS, int PF, int WAUX = 0>
+template <int TM, int TN, int KS, int PF>
 __device__ __forceinline__ void zr_preload_w(ZrFrag<TM, TN> (&f)[PF + 1], __amdgpu_buffer_rsrc_t wrsrc,
                                              const unsigned (&wsoff)[TM], unsigned woffb, unsigned wstep, int K,
                                              int kslice) {
@@ -245,7 +245,7 @@ __device__ __forceinline__ void zr_preload_w(ZrFrag<TM, TN> (&f)[PF + 1], __amdg
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
       const zr_u32x4 v =
-          __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + (unsigned)gl * wstep), WAUX);
+          __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + (unsigned)gl * wstep), 0);
       f[s].w[tm][0] = __uint_as_float(v.x);
       f[s].w[tm][1] = __uint_as_float(v.y);
       f[s].w[tm][2] = __uint_as_float(v.z);
@@ -254,7 +254,7 @@ __device__ __forceinline__ void zr_preload_w(ZrFrag<TM, TN> (&f)[PF + 1], __amdg
   }
 }
 
-template <int TM, int TN, int KS, int PF, bool WPRE = false, int WAUX = 0>
+template <int TM, int TN, int KS, int PF, bool WPRE = false>
 __device__ __forceinline__ void zr_mma_segment_u(zr_f32x16 (&acc)[TM][TN], __amdgpu_buffer_rsrc_t wrsrc,
                                                  const unsigned (&wsoff)[TM], unsigned woffb, unsigned wstep,
                                                  __amdgpu_buffer_rsrc_t xrsrc, const unsigned (&xoffb)[TN],
@@ -277,7 +277,7 @@ __device__ __forceinline__ void zr_mma_segment_u(zr_f32x16 (&acc)[TM][TN], __amd
     load_x(f, g);
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
-      const zr_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + ug * wstep), WAUX);
+      const zr_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)woffb, (int)(wsoff[tm] + ug * wstep), 0);
       f.w[tm][0] = __uint_as_float(v.x);
       f.w[tm][1] = __uint_as_float(v.y);
       f.w[tm][2] = __uint_as_float(v.z);
@@ -463,13 +463,13 @@ __device__ __forceinline__ void zr_mma_segment_split(zr_f32x16 (&acc)[TM][TN], _
 }
 
 // The same with a ring of its own (no weights fetched ahead).
-template <int TM, int TN, int KS, int PF, int WAUX = 0>
+template <int TM, int TN, int KS, int PF>
 __device__ __forceinline__ void zr_mma_segment_ring(zr_f32x16 (&acc)[TM][TN], __amdgpu_buffer_rsrc_t wrsrc,
                                                  const unsigned (&wsoff)[TM], unsigned woffb, unsigned wstep,
                                                  __amdgpu_buffer_rsrc_t xrsrc, const unsigned (&xoffb)[TN],
                                                  unsigned xstep, int K, int kslice) {
   ZrFrag<TM, TN> f[PF + 1];
-  zr_mma_segment_u<TM, TN, KS, PF, false, WAUX>(acc, wrsrc, wsoff, woffb, wstep, xrsrc, xoffb, xstep, K, kslice, f);
+  zr_mma_segment_u<TM, TN, KS, PF, false>(acc, wrsrc, wsoff, woffb, wstep, xrsrc, xoffb, xstep, K, kslice, f);
 }
 
 // Workgroup barrier that also publishes: when it returns, every store any thread of the workgroup issued before it
