@@ -5,8 +5,9 @@
 // several share a compute unit and one's loads fly beside another's products.
 // gemm_rows_kernel's workgroups split K over their waves instead: a sum through LDS for every few rows, no loads in flight meanwhile.
 // Four accumulators an output (terms, and steps of 16 k in turn), so that no chain is longer than there.
-// Bound: the matrix's way from memory.  50000 x 1024, us of a call: 64 columns 36.1 -> 30.7 (20 for the matrix alone at the rate of a large copy), 37 34.8 -> 27.0, 8 22.1
-// -> 20.8.  Three chunks ahead instead of two measured the same.
+// Bound: the matrix's way from memory at a few columns (8: 105 MB past L2 at 5.2 TB/s); at 37 and 64 neither memory (4.5 and 4.2 TB/s) nor the matrix pipes (busy
+// for a quarter) are full, the waits at the steps' barriers are left.  50000 x 1024, us of a call: 64 columns 36.1 -> 30.7, 37 34.8 -> 27.0, 8 22.1 -> 20.8.  Three chunks
+// ahead instead of two measured the same.
 #include "zr_internal.h"
 #include "zr_logits_epilogue.h"
 #include "zr_mfma_core.h"
