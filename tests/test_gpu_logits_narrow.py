@@ -42,6 +42,12 @@ def test_four_waves_of_64_rows_around_their_line(ctx, V, H, n):
     check(D, b, h, *logits_and_blocks(ctx, D, b, h))
 
 
+@pytest.mark.parametrize("V,H,n", [(125, 536, 9), (2047, 512, 3), (2048, 512, 5), (2048, 513, 16), (4001, 600, 2), (4001, 608, 12), (8191, 555, 7), (8192, 601, 12), (8193, 601, 2)])
+def test_few_rows_of_a_long_k(ctx, V, H, n):
+    D, b, h = operands(V, H, n)
+    check(D, b, h, *logits_and_blocks(ctx, D, b, h))
+
+
 @pytest.mark.parametrize("V,H,n", [(1, 1, 17), (33, 31, 31), (257, 128, 32), (8192, 200, 18), (8449, 264, 32), (10001, 63, 25), (20480, 1000, 17), (30011, 500, 32), (33333, 333, 29),
                                    (50001, 96, 24)])
 def test_one_block_of_columns(ctx, V, H, n):

@@ -396,10 +396,12 @@ inline ZrLogitsPlan zr_logits_plan(int V, int cols, int H, int cus) {
 }
 
 // The same for up to 16 columns (zr_logits_narrow.hip) instead of 32-column instructions and, below 8192 rows or with K % 8 != 0, the others: faster by 20 to
-// 65 % at every size (V = 1000 .. 80000, H = 64 .. 1000) but few rows of a long K, which one wave then walks alone: us, those / this one, 4000 x 1000 11.4 /
-// 12.1, 1000 x 1000 9.2 / 12.0, 2000 x 500 9.8 / 7.3, 4000 x 200 8.9 / 4.8, 8192 x 300 6.4 / 5.2, 10000 x 1000 37.8 / 12.7.
+// 65 % at every size (V = 1000 .. 80000, H = 64 .. 1000) but few rows of a long K, which one wave then walks alone while the others split it over eight from
+// K = 512 on: us, those / this one, 4000 x 1000 11.4 / 12.1, 500 x 504 9.2 / 7.6, 500 x 512 6.5 / 7.5, 2040 x 600 7.0 / 8.5, 2050 x 600 8.6 / 8.5, 2050 x 550 6.6 / 8.3, 8000 x 550
+// 6.6 / 8.3, 8192 x 777 7.7 / 10.2, 9000 x 550 11.1 / 8.4, 4000 x 200 8.9 / 4.8, 8192 x 300 6.4 / 5.2, 10000 x 1000 37.8 / 12.7.
 inline bool zr_logits_narrow_takes(int V, int cols, int H) {
-  if (cols > 16 || H < 4 || (V < 8192 && H > 600)) return false;
+  if (cols > 16 || H < 4) return false;
+  if (H >= 512 && (V < 2048 || (H % 8 ? V <= 8192 : V < 8192 && H > 600))) return false;
   return (((long long)H + 7) / 8 * 8 + 160) * (((long long)V + 31) / 32) * 32 * 4 < 1LL << 32;  // 32-bit offsets
 }
 
