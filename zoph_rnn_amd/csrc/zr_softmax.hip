@@ -162,9 +162,11 @@ softmax_colstats_f64_kernel(const float* __restrict__ logits, int V, const float
     for (int u = 0; u < U; ++u) now[u] = v[u];
     if (at + SPAN * U < end) load(at + SPAN * U);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      if (at + 4 * tid + SPAN * u >= end) break;  // (nothing but zeros: small vocabularies)
 #pragma unroll
       for (int e = 0; e < 4; ++e) sum[e] += exp((double)now[u][e] - mx);
+    }
   }
   double total = (sum[0] + sum[1]) + (sum[2] + sum[3]);
 #pragma unroll
