@@ -153,7 +153,8 @@ const char* zr_version(void);
 #define ZR_OPT_LSTM_SWEEP_SCRATCH 12 /* KiB of scratch memory that a sweep as one launch may use (0 = what the device has
                                         left).  The streamed sweep needs 6 * (L * (T + 1) + T) * H bytes a column (columns in
                                         eights), the resident one 4 * L * (T + 1) * H, the backward sweep 256 * L * T *
-                                        ceil(H / 16) (all of it a quarter more, and it stays with the context); a schedule
+                                        ceil(H / 16) (all of it a quarter more, and it stays with the context until one
+                                        of its allocations would fail); a schedule
                                         there is no memory for is passed over, with ZR_OPT_LSTM_SWEEP = 2 and 3 too */
 #define ZR_OPT_KEEP_MEMORY 13 /* 1 (default): device memory of destroyed handles and of zr_free stays with the context for its
                                  next requests, at most 32 blocks and 512 MiB, while it is the only context on its

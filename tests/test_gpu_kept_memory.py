@@ -152,6 +152,43 @@ def test_an_output_layer_is_prepared_with_memory_that_was_kept(ctx):
         torch.cuda.empty_cache()
 
 
+def test_a_sweeps_memory_serves_an_allocation_that_fails_without_it(ctx):
+    L, H, mb, T = 4, 512, 128, 40
+    r = np.random.default_rng(11)
+    draw = lambda *shape: ctx.array(r.random(shape, np.float32))
+    mats = [[ctx.array(synth.uniform(synth.rng(901, i), (H, H))) for _ in range(4)] for i in range(2)]
+    layers = [ctx.lstm_train_create(mats[0], mats[1], H) for _ in range(L)]
+    ones, top, c0 = ctx.array(np.ones(mb * T, np.int32)), draw(H * mb * T), [draw(H * mb) for _ in range(L)]
+    c, gates = [draw(H * mb * T) for _ in range(L)], [draw(4 * H * mb * T) for _ in range(L)]
+    dg, eh, ec = [[ctx.empty((k * H * mb,)) for _ in range(L)] for k in (4 * T, 1, 1)]
+
+    def sweep():
+        ctx.lstm_stack_backward(layers, T, mb, ones, c0, c, gates, top, dg, eh, ec)
+        ctx.sync()
+        return [x.get() for x in dg + eh + ec]
+
+    want = sweep()
+    path = ctx.query(capi.ZR_QUERY_LSTM_BACKWARD_PATH)
+    scratch = ctx.query(capi.ZR_QUERY_SCRATCH_KIB) << 10
+    assert path == capi.ZR_LSTM_BACKWARD_PATH_RESIDENT and scratch >= 150 * MIB
+    hog = []
+    try:
+        while free_bytes() > 600 * MIB and len(hog) < 8:
+            hog.append(torch.empty(free_bytes() - 512 * MIB, dtype=torch.uint8, device="cuda"))
+        need = free_bytes() + scratch // 2
+        p = ctypes.c_void_p()
+        assert capi.load().zr_malloc(ctx.h, ctypes.c_size_t(need), ctypes.byref(p)) == 0
+        assert ctx.query(capi.ZR_QUERY_SCRATCH_KIB) == 0
+        assert raw_free(ctx, p.value) == 0
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+    for a, b in zip(sweep(), want):
+        assert np.array_equal(a, b)
+    for w in layers:
+        ctx.lstm_train_destroy(w)
+
+
 def test_nothing_is_kept_without_the_option(ctx):
     keep(ctx, 200)
     before = free_bytes()

@@ -65,7 +65,8 @@ int zr_bind_device(zr_ctx* ctx) {
 // that comes, is on the context's own stream: nothing is kept where a caller's stream has ever been set or another context is alive.
 // What callers hold themselves (zr_malloc) may be in use on any stream of theirs, so zr_free waits for the device as hipFree
 // did, and zr_malloc for this stream where it hands out a handle's block.
-// A second context on the device, and every allocation that fails, has the blocks of all contexts there given back first.
+// A second context on the device, and every allocation that fails, has the blocks of all contexts there given back first, and an
+// allocation that fails all the same its own context's scratch buffers.
 constexpr size_t kKeptTotal = (size_t)512 << 20, kKeptLargest = (size_t)256 << 20;
 
 struct Block {
@@ -130,6 +131,18 @@ static void* hip_malloc(zr_ctx* ctx, size_t bytes) {
   return nullptr;
 }
 
+// Gives the context's scratch buffers back, which stay as large as the largest call so far made them (a backward sweep's hand-over memory: 315 MB for four
+// layers of 512, 128 columns, 60 steps).  Only where no graph can hold their addresses; nothing lies in them from call to call.
+static bool give_back_scratch(zr_ctx* ctx) {
+  if (ctx->foreign_stream || (!ctx->d_scratch && !ctx->d_scratch2) || hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+  if (ctx->d_scratch) (void)hipFree(ctx->d_scratch);
+  if (ctx->d_scratch2) (void)hipFree(ctx->d_scratch2);
+  ctx->d_scratch = ctx->d_scratch2 = nullptr;
+  ctx->scratch_bytes = ctx->scratch2_bytes = 0;
+  return true;
+}
+
+// Called at the entry points, before any scratch of theirs.
 void* zr_dev_alloc(zr_ctx* ctx, size_t bytes, bool any_stream) {
   void* p = nullptr;
   Block block = {bytes, ctx->device};
@@ -153,6 +166,7 @@ void* zr_dev_alloc(zr_ctx* ctx, size_t bytes, bool any_stream) {
   }
   if (!p) {
     p = hip_malloc(ctx, bytes);
+    if (!p && give_back_scratch(ctx)) p = hip_malloc(ctx, bytes);
     block.bytes = bytes;
   }
   if (p) {
