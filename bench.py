@@ -456,7 +456,7 @@ def main():
                     help="only run a plain copy kernel of known size (for scaling HBM traffic counters) and exit")
     args = ap.parse_args()
     if args.gpus != 1:
-        print("bench.py: this build runs on one GPU; --gpus %d is not supported (no cross-GPU path exists)" % args.gpus,
+        print("bench.py: the framework runs on one GPU; --gpus %d is not supported (no cross-GPU path exists)" % args.gpus,
               file=sys.stderr)
         sys.exit(2)
 

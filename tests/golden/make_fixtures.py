@@ -4,7 +4,7 @@ CPU oracle (oracle/libzoph_oracle.so, double accumulation) makes of them.
 The reference ships no expected outputs for this path (sample_data/ holds raw text only) and none of it can be
 compiled or imported here, so these vectors come from the oracle and serve two purposes: they freeze the oracle (a
 change to it that moves a result fails tests/test_golden_fixtures.py on the CPU), and they give the GPU tests inputs and
-expected outputs that do not depend on the oracle being built on the GPU box.
+expected outputs that do not depend on the oracle being built there.
 
 Run from the repository root:  python tests/golden/make_fixtures.py
 Each fixture is one .npz (numpy arrays only, loaded with allow_pickle=False).
